@@ -71,6 +71,7 @@ SIGNATURES = {
     "accel_memcpy_d2h": (C.c_int, [vp, vp, C.c_size_t]),
     "accel_dev_fill_u32": (C.c_int, [vp, C.c_uint32, C.c_size_t, vp]),
     "accel_dev_copy_u32": (C.c_int, [vp, vp, C.c_size_t, vp]),
+    "accel_release_memory": (C.c_int, []),
     "accel_stream_sync": (C.c_int, [vp]),
     "accel_create": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.POINTER(vp)]),
     "accel_preprocess": (C.c_int, [vp]),

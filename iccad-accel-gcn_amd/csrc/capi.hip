@@ -29,28 +29,30 @@ bool stream_is_capturing(hipStream_t s);
 int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int K, int N, int64_t ldx, int64_t ldz,
                     hipStream_t stream);      // dense.hip
 
+// Work that is queued on the null stream alone orders itself before whoever takes the memory
+// next (memory.hip); for a handle that other streams, or graphs, have used, the device is
+// waited for first.  Returns whether nothing uses the handle's memory any more.
+static bool settle(const accel_handle *h)
+{
+    if (!h->multi_stream && !h->captured && !(h->has_home && h->home)) return !h->has_home;
+    if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
+    return true;
+}
+
 void release_products(accel_handle *h)
 {
-    if (h->slab) {
-        (void)hipFree(h->slab);
-        h->slab = nullptr;
-    } else {
-        if (h->perm) (void)hipFree(h->perm);
-        if (h->s_indptr) (void)hipFree(h->s_indptr);
-        if (h->owns_sorted) {
-            if (h->s_idx) (void)hipFree(const_cast<int32_t *>(h->s_idx));
-            if (h->s_val) (void)hipFree(const_cast<float *>(h->s_val));
-        }
-    }
-    if (h->work) (void)hipFree(h->work);
-    if (h->long_slot) (void)hipFree(h->long_slot);
-    if (h->block4) (void)hipFree(h->block4);
-    if (h->partial) (void)hipFree(h->partial);
-    if (h->src_pos) (void)hipFree(h->src_pos);
+    const bool settled = settle(h);
+    give_memory(h->slab, settled);                     // perm, s_indptr and the sorted copy live in here
+    h->slab = nullptr;
+    give_memory(h->work, settled);
+    give_memory(h->long_slot, settled);
+    give_memory(h->block4, settled);
+    give_memory(h->partial, settled);
+    give_memory(h->src_pos, settled);
     h->src_pos = nullptr;
     h->val_stale = false;
-    // what other streams still hold was queued against the memory freed above (hipFree waits
-    // for the device), so the bookkeeping starts afresh
+    // what other streams still held was queued against the memory given back above and has
+    // finished, so the bookkeeping starts afresh
     if (h->writer_done) (void)hipEventDestroy(h->writer_done);
     for (auto &sl : h->slot) {
         if (sl.done) (void)hipEventDestroy(sl.done);
@@ -58,7 +60,7 @@ void release_products(accel_handle *h)
     }
     h->writer_done = nullptr; h->writer = nullptr; h->writer_pending = false;
     h->partial_slot = -1; h->next_victim = 0;
-    h->has_home = false; h->home = nullptr; h->multi_stream = false;
+    h->has_home = false; h->home = nullptr; h->multi_stream = false; h->captured = false;
     h->perm = nullptr; h->s_indptr = nullptr; h->s_idx = nullptr; h->s_val = nullptr;
     h->work = nullptr; h->long_slot = nullptr; h->row_done = nullptr; h->block4 = nullptr; h->partial = nullptr;
     h->n_units = h->n_long_units = 0;
@@ -208,7 +210,7 @@ static int single_stream(accel_handle *h, hipStream_t s, bool *single)
 int order_run(accel_handle *h, hipStream_t s, bool uses_partial, bool capturing, hipEvent_t *run_done)
 {
     *run_done = nullptr;
-    if (capturing) return ACCEL_OK;
+    if (capturing) { h->captured = true; return ACCEL_OK; }
     bool single = false;
     if (int rc = single_stream(h, s, &single)) return rc;
     if (single) return ACCEL_OK;
@@ -251,7 +253,7 @@ int order_run(accel_handle *h, hipStream_t s, bool uses_partial, bool capturing,
 // values it rewrites, and after an earlier update on another stream.
 int order_update(accel_handle *h, hipStream_t s, bool capturing)
 {
-    if (capturing) return ACCEL_OK;
+    if (capturing) { h->captured = true; return ACCEL_OK; }
     bool single = false;
     if (int rc = single_stream(h, s, &single)) return rc;
     if (single) return ACCEL_OK;
@@ -486,6 +488,13 @@ int accel_dev_copy_u32(void *dst_dev, const void *src_dev, size_t n_words, void 
     return copy_u32(dst_dev, src_dev, n_words, static_cast<hipStream_t>(stream));
 }
 
+int accel_release_memory(void)
+{
+    clear_error();
+    release_idle_memory();
+    return ACCEL_OK;
+}
+
 int accel_stream_sync(void *stream)
 {
     clear_error();
@@ -530,15 +539,13 @@ int accel_create(const int32_t *indptr, const int32_t *idx, const float *val, in
         // the kernels of accel_preprocess read these arrays: a host address would be a memory fault
         if (int rc = check_borrowed_csr(h, "accel_create")) { delete h; return rc; }
     } else {
-        void *a = nullptr, *b = nullptr, *c = nullptr;
         const size_t sa = sizeof(int32_t) * (size_t)(rows + 1);
         const size_t sb = sizeof(int32_t) * (size_t)nnz, sc = sizeof(float) * (size_t)nnz;
-        if (hipMalloc(&a, sa) != hipSuccess || hipMalloc(&b, sb ? sb : 4) != hipSuccess ||
-            hipMalloc(&c, sc ? sc : 4) != hipSuccess) {
-            (void)hipGetLastError();
-            if (a) (void)hipFree(a);
-            if (b) (void)hipFree(b);
-            if (c) (void)hipFree(c);
+        void *a = take_memory(sa, false), *b = take_memory(sb, false), *c = take_memory(sc, false);
+        if (!a || !b || !c) {
+            give_memory(a, true);
+            give_memory(b, true);
+            give_memory(c, true);
             delete h;
             set_error("device allocation for the CSR (%zu bytes) failed", sa + sb + sc);
             return ACCEL_ERR_ALLOC;
@@ -563,11 +570,12 @@ int accel_create(const int32_t *indptr, const int32_t *idx, const float *val, in
 int accel_destroy(accel_handle *h)
 {
     if (!h) return ACCEL_OK;
+    const bool settled = settle(h);                    // the kernels may read the CSR in place
     release_products(h);
     if (h->owns_input) {
-        (void)hipFree(const_cast<int32_t *>(h->indptr));
-        (void)hipFree(const_cast<int32_t *>(h->idx));
-        (void)hipFree(const_cast<float *>(h->val));
+        give_memory(const_cast<int32_t *>(h->indptr), settled);
+        give_memory(const_cast<int32_t *>(h->idx), settled);
+        give_memory(const_cast<float *>(h->val), settled);
     }
     delete h;
     return ACCEL_OK;
@@ -882,9 +890,8 @@ int accel_partition_gpu(const int32_t *indptr, int64_t rows, int32_t *block4_out
     if (int rc = need_gpu()) return rc;
     *n_blocks = 0;
     if (rows == 0) return ACCEL_OK;
-    void *dptr = nullptr;
-    if (hipMalloc(&dptr, sizeof(int32_t) * (size_t)(rows + 1)) != hipSuccess) {
-        (void)hipGetLastError();
+    void *dptr = take_memory(sizeof(int32_t) * (size_t)(rows + 1), false);
+    if (!dptr) {
         set_error("device allocation failed");
         return ACCEL_ERR_ALLOC;
     }
@@ -905,8 +912,8 @@ int accel_partition_gpu(const int32_t *indptr, int64_t rows, int32_t *block4_out
             rc = ACCEL_ERR_HIP;
         }
     }
-    if (b4) (void)hipFree(b4);
-    (void)hipFree(dptr);
+    give_memory(b4, false);
+    give_memory(dptr, false);
     return rc;
 }
 
@@ -943,7 +950,7 @@ int accel_reserve(accel_handle *h, int32_t max_N)
     if (!h) { set_error("accel_reserve: null handle"); return ACCEL_ERR_ARG; }
     if (!h->ready) { set_error("accel_reserve: call accel_preprocess first"); return ACCEL_ERR_STATE; }
     if (max_N <= 0) { set_error("accel_reserve: N must be positive, got %d", max_N); return ACCEL_ERR_ARG; }
-    return reserve_partial(h, (size_t)h->n_long_units * (size_t)max_N);
+    return reserve_partial(h, (size_t)h->n_long_units * (size_t)max_N, true);
 }
 
 int accel_run_static(accel_handle *h, const float *X, float *Y, int32_t N, void *stream)

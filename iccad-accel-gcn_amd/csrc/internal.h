@@ -139,6 +139,7 @@ struct accel_handle {
     hipStream_t home = nullptr;              // the one stream the handle has been used on so far
     bool has_home = false;
     bool multi_stream = false;               // a second stream has turned up: runs are tracked
+    bool captured = false;                   // a graph that uses the handle may be launched on any stream
     static constexpr int kMaxStreams = 4;
     struct StreamSlot {
         hipStream_t stream = nullptr;
@@ -153,6 +154,13 @@ struct accel_handle {
 };
 
 namespace accel {
+// memory.hip: device memory that outlives a handle.  take_memory returns null when there is
+// none; any_stream: the memory will first be used on another stream than the null stream.
+// give_memory returns it; settled: no kernel uses it any more (else: only kernels queued on the
+// null stream may).
+void *take_memory(size_t bytes, bool any_stream);
+void give_memory(void *p, bool settled);
+void release_idle_memory();
 // preprocess.hip
 struct SavedOrder {               // a degree-sort order read from a saved state
     bool identity;                // the rows were already in order: no permutation stored
@@ -173,7 +181,7 @@ int note_update(accel_handle *h, hipStream_t s, bool capturing);
 int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t stream,
                 hipEvent_t main_start = nullptr, hipEvent_t main_stop = nullptr, const float *bias = nullptr,
                 int relu = 0, bool static_partial = false, int ld = 0);
-int reserve_partial(accel_handle *h, size_t floats);
+int reserve_partial(accel_handle *h, size_t floats, bool any_stream);
 int fill_u32(void *dst, uint32_t v, size_t n, hipStream_t s);
 int copy_u32(void *dst, const void *src, size_t n, hipStream_t s);
 }  // namespace accel

@@ -367,9 +367,9 @@ __global__ __launch_bounds__(kThreads) void iota_kernel(uint32_t *out, int64_t n
     if (i < n) out[i] = (uint32_t)i;
 }
 
-// Temporaries of one preprocessing call come out of a few large device allocations
-// instead of one hipMalloc / hipFree each (a pair costs about 0.2 ms, and there are
-// some twenty temporaries).  Chunks are freed when the arena goes out of scope.
+// Temporaries of one preprocessing call come out of a few large pieces of device memory (there
+// are some twenty of them).  The pieces are given back when the arena goes out of scope; what
+// is still queued then is queued on the null stream.
 struct Arena {
     static constexpr int kMaxChunks = 32;
     char *chunk[kMaxChunks] = {};
@@ -378,7 +378,7 @@ struct Arena {
     size_t next_chunk = 0;         // size hint for the next chunk
     ~Arena()
     {
-        for (int i = 0; i < n_chunks; i++) (void)hipFree(chunk[i]);
+        for (int i = 0; i < n_chunks; i++) give_memory(chunk[i], false);
     }
     void *take(size_t bytes)
     {
@@ -386,11 +386,8 @@ struct Arena {
         if (n_chunks == 0 || used + bytes > cap) {
             if (n_chunks == kMaxChunks) return nullptr;
             const size_t want = std::max(bytes, next_chunk);
-            void *p = nullptr;
-            if (hipMalloc(&p, want) != hipSuccess) {
-                (void)hipGetLastError();
-                return nullptr;
-            }
+            void *p = take_memory(want, false);
+            if (!p) return nullptr;
             chunk[n_chunks++] = static_cast<char *>(p);
             cap = want;
             used = 0;
@@ -405,19 +402,15 @@ struct Arena {
 struct DevBuf {  // frees on scope exit; with an arena, the arena owns the memory
     void *p = nullptr;
     Arena *arena = nullptr;
+    bool any_stream = false;         // will be used on another stream than the null stream
     DevBuf() = default;
     explicit DevBuf(Arena *a) : arena(a) {}
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { if (p && !arena) (void)hipFree(p); }
+    ~DevBuf() { if (!arena) give_memory(p, false); }
     int alloc(size_t bytes)
     {
-        if (arena) {
-            p = arena->take(bytes);
-        } else if (hipMalloc(&p, bytes ? bytes : 4) != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
-        }
+        p = arena ? arena->take(bytes) : take_memory(bytes, any_stream);
         if (!p) {
             set_error("device allocation of %zu bytes failed", bytes);
             return ACCEL_ERR_ALLOC;
@@ -1399,6 +1392,7 @@ int build_source_positions(accel_handle *h, hipStream_t s)
     const int64_t rows = h->rows, n_long = h->n_split_rows, first_long = rows - n_long;
     const int64_t nnz_short = h->nnz_short;
     DevBuf map, tiles;
+    map.any_stream = tiles.any_stream = s != nullptr;
     if (int rc = map.alloc(sizeof(int32_t) * (size_t)h->nnz)) return rc;
     if (nnz_short > 0) {
         if (int rc = tiles.alloc(sizeof(int) * (size_t)(nnz_short / kPermuteTile + 2))) return rc;
@@ -1416,7 +1410,7 @@ int build_source_positions(accel_handle *h, hipStream_t s)
 }
 
 // s_val[p] = val[src_pos[p]]: four non-zeros per thread, the map read and the values written
-// as 16-byte vectors (both arrays come from hipMalloc and start 256-byte aligned).
+// as 16-byte vectors (both arrays start 256-byte aligned).
 __global__ __launch_bounds__(kThreads) void gather_values_kernel(const float *__restrict__ val,
                                                                  const int32_t *__restrict__ src_pos,
                                                                  float *__restrict__ s_val, int64_t nnz)

@@ -757,17 +757,17 @@ static int static_scratch_address(float **out)
 }
 
 // Grows the handle's partial-sum buffer to `floats` (never shrinks).  The old buffer is
-// freed: graphs captured with it must be captured again.
-int reserve_partial(accel_handle *h, size_t floats)
+// given back: graphs captured with it must be captured again.
+int reserve_partial(accel_handle *h, size_t floats, bool any_stream)
 {
     if (h->partial_floats >= floats) return ACCEL_OK;
-    if (h->partial_slot >= 0 && hipEventSynchronize(h->slot[h->partial_slot].done) != hipSuccess)
-        (void)hipGetLastError();                       // nobody reads the old one (hipFree waits for the device as well)
-    if (h->partial) (void)hipFree(h->partial);
-    h->partial = nullptr;
+    if (h->partial) {
+        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();     // nobody reads the old one
+        give_memory(h->partial, true);
+    }
     h->partial_floats = 0;
-    if (hipMalloc(reinterpret_cast<void **>(&h->partial), floats * sizeof(float)) != hipSuccess) {
-        (void)hipGetLastError();
+    h->partial = static_cast<float *>(take_memory(floats * sizeof(float), any_stream));
+    if (!h->partial) {
         set_error("device allocation of %zu bytes for long-row partial sums failed", floats * sizeof(float));
         return ACCEL_ERR_ALLOC;
     }
@@ -820,7 +820,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
                           "call accel_reserve(h, N) before the capture", N);
                 return ACCEL_ERR_STATE;
             }
-            if (int rc = reserve_partial(h, need)) return rc;
+            if (int rc = reserve_partial(h, need, stream != nullptr)) return rc;
         }
         partial = h->partial;
     }

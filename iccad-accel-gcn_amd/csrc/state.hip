@@ -72,7 +72,7 @@ struct PinnedBuf {   // host memory the GPU copies from and to directly
 
 struct DevMem {
     void *p = nullptr;
-    ~DevMem() { if (p) (void)hipFree(p); }
+    ~DevMem() { give_memory(p, false); }
 };
 
 }  // namespace
@@ -190,9 +190,8 @@ int accel_load_state(accel_handle *h, const char *path)
         const size_t bytes = sizeof(int32_t) * (size_t)hd.perm_words;
         if (int rc = host.alloc(bytes)) return rc;
         if (fread(host.p, 1, bytes, in.f) != bytes) { set_error("%s: truncated", path); return ACCEL_ERR_IO; }
-        if (hipMalloc(&dev.p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            dev.p = nullptr;
+        dev.p = take_memory(bytes, false);
+        if (!dev.p) {
             set_error("device allocation of %zu bytes failed", bytes);
             return ACCEL_ERR_ALLOC;
         }
