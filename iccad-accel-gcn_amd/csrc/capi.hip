@@ -63,6 +63,7 @@ void release_products(accel_handle *h)
     h->has_home = false; h->home = nullptr; h->multi_stream = false; h->captured = false;
     h->perm = nullptr; h->s_indptr = nullptr; h->s_idx = nullptr; h->s_val = nullptr;
     h->work = nullptr; h->long_slot = nullptr; h->row_done = nullptr; h->block4 = nullptr; h->partial = nullptr;
+    h->runs = h->first_chunk = h->chunk_row = nullptr;
     h->n_units = h->n_long_units = 0;
     h->partial_floats = 0; h->owns_sorted = false; h->ready = false;
 }

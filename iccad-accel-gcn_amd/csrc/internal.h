@@ -83,12 +83,13 @@ struct accel_handle {
     // preprocess products
     bool ready = false;
     bool identity_perm = false;       // input already degree-sorted: perm == iota
+    // perm, s_indptr, runs, the chunk tables and the owned s_idx / s_val live in one allocation, `slab`
     int32_t *perm = nullptr;          // [rows] new row -> caller's row (nullptr when identity)
     int32_t *s_indptr = nullptr;      // [rows+1] degree-sorted CSR
     const int32_t *s_idx = nullptr;   // [nnz]  (aliases idx when identity)
     const float *s_val = nullptr;     // [nnz]  (aliases val when identity)
     bool owns_sorted = false;
-    void *slab = nullptr;             // when set: perm, s_indptr and the owned s_idx / s_val live in this one allocation
+    void *slab = nullptr;
     int32_t *block4 = nullptr;        // [4*n_blocks]  the .block4 metadata (upstream ABI)
     // launch plan derived from block4 (see preprocess.hip, "work list")
     int32_t *work = nullptr;          // [4*n_units] one int4 per wavefront
@@ -117,7 +118,10 @@ struct accel_handle {
     int64_t n_split_rows = 0;         // rows with more than plan_split non-zeros
     int64_t n_big_rows = 0;           // of those, rows with more than 32 * plan_split
     int64_t nnz_short = 0;            // non-zeros of the rows that are not split
-    int64_t n_wide_rows = 0;          // rows with more than 1,024 non-zeros (regrouped by a workgroup each)
+    int64_t n_wide_rows = 0;          // rows with more than 1,024 non-zeros, regrouped in chunks
+    int64_t n_chunks = 0;             // ... of 4,096 non-zeros
+    int *runs = nullptr;              // first sorted row and first non-zero of each degree's run (SortedRows)
+    int *first_chunk = nullptr, *chunk_row = nullptr;     // chunks of each wide row, wide row of each chunk
     int64_t n_blocks = 0, n_long_blocks = 0, n_long_rows = 0, n_zero_rows = 0;
     int32_t max_degree = 0;
     double preprocess_ms = 0.0;

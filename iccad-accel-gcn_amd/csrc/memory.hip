@@ -29,7 +29,7 @@
 #include <unordered_map>
 #include <vector>
 
-#include "internal.h"
+#include "preprocess.h"
 
 namespace accel {
 namespace {
@@ -178,6 +178,37 @@ void give_memory(void *p, bool settled)
         expire(pl, gone);
     }
     free_idle(gone);
+}
+
+// Pinned blocks for the preprocessing's results, one per call that is under way; kept (a few KB
+// each, as many as calls have run at once).
+static std::mutex g_mail_mu;
+static std::vector<Mail *> g_mail;
+
+Mail *take_mail()
+{
+    Mail *m = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_mail_mu);
+        if (!g_mail.empty()) {
+            m = g_mail.back();
+            g_mail.pop_back();
+        }
+    }
+    if (!m && hipHostMalloc(reinterpret_cast<void **>(&m), sizeof(Mail), hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("allocation of pinned host memory failed");
+        return nullptr;
+    }
+    m->bad_index = m->bad_order = 0;
+    return m;
+}
+
+void give_mail(Mail *m)
+{
+    if (!m) return;
+    std::lock_guard<std::mutex> lock(g_mail_mu);
+    g_mail.push_back(m);
 }
 
 }  // namespace accel

@@ -1,0 +1,555 @@
+// The launch plan (work list) of a preprocessed matrix, built on the GPU.  One work unit per
+// wavefront, kWavesPerGroup units per workgroup, as int4 (x, y, z, w):
+//   x <= 384 : whole rows of one block4 entry (degree, first row, first non-zero,
+//              (w_nz << 16) + n_rows): the entry itself, or a run of its rows when
+//              the plan's unit is smaller than the entry;
+//   x  > 384 : a piece of a split row: partial-sum slot x - 385, row y, first
+//              non-zero z, length w <= plan_unit, all of one column group;
+//   w == 0   : padding, nothing to do.
+// Workgroups are dispatched to the eight dies round-robin (workgroup i runs on
+// die i % 8), so the list is laid out as eight interleaved queues.  Column group
+// g belongs to die g % 8.  A queue holds, in this order: the pieces of the rows
+// stored in 64 groups (the longest rows), one group after the other, largest
+// rows first; then the same for the rows with 32, 16 and 8 groups (the rows of
+// an 8-group bin in the order of the caller's row ids); then the
+// queue's share of the whole-row units.  While a die works through one group its
+// L2 only has to hold that group's share of X.
+// The whole-row units are put in the order of the caller's row ids (of each unit's
+// first row) and that sequence is cut into eight consecutive shares, one per queue,
+// sized so that all queues carry about the same load.  Graphs whose neighbouring
+// row ids have neighbouring columns (most graphs with a meaningful vertex order)
+// lose that locality to the degree sort; this gives it back: at any time a die
+// works on a narrow band of the caller's rows.
+//
+// Nothing here is sorted: the pass that placed the rows (place_rows in preprocess.hip) knows of
+// every row, in the caller's order, whether it starts a unit, so a scan of the counts per share
+// of rows puts the units in that order (list_units_kernel).  The pieces of a column group are
+// ordered by a scan over (class of rows, group, row of the class).  What bounds all of it is
+// the number of dependent launches (2 to 5 us each), not bytes: nine launches and no
+// synchronisation before the last, where there were 45 launches and two (110 of 440 us of
+// kernels at 2.45 M non-zeros, 400 us of 1.79 ms at 125 M).
+#include "preprocess.h"
+
+namespace accel {
+namespace {
+
+constexpr int kClasses = 4;                 // rows stored in 8, 16, 32, 64 column groups
+// The split rows' unit counts per group are laid out [class][group][rank in the class].
+struct ClassLayout {
+    int rows[kClasses];                     // split rows of each class
+    int base[kClasses];                     // where the class's counts start
+    int above[kClasses];                    // rows of the classes with more groups
+    int total;                              // counts in all
+};
+
+ClassLayout class_layout(int64_t n_split, const Mail *stats, int groups)
+{
+    ClassLayout c{};
+    if (groups) {
+        for (int i = 0; i < kClasses; i++) c.rows[i] = (kXcds << i) == groups ? (int)n_split : 0;
+    } else {
+        c.rows[1] = stats->stat[kStatRows16];
+        c.rows[2] = stats->stat[kStatRows32];
+        c.rows[3] = stats->stat[kStatRows64];
+        c.rows[0] = (int)n_split - c.rows[1] - c.rows[2] - c.rows[3];
+    }
+    for (int i = 0, at = 0; i < kClasses; i++) {
+        c.base[i] = at;
+        at += (kXcds << i) * c.rows[i];
+        c.total = at;
+    }
+    for (int i = kClasses - 1, n = 0; i >= 0; i--) {
+        c.above[i] = n;
+        n += c.rows[i];
+    }
+    return c;
+}
+
+constexpr int kScanItems = 8;
+constexpr int kScanTile = kThreads * kScanItems;
+inline int64_t scan_tiles(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
+
+// The part of the zeroed memory each user has: queue loads, the two scans' tickets, their
+// per-tile words (8 bytes each).
+constexpr int kZeroQueueLoad = 0, kZeroTickets = 8, kZeroWords = 16;
+
+__device__ __forceinline__ int64_t plan_index(int queue, int pos, int n_queues)
+{
+    // queue q, position p  ->  slot of wavefront (p % 4) in workgroup (p / 4) * n_queues + q
+    return ((int64_t)(pos / kWavesPerGroup) * n_queues + queue) * kWavesPerGroup + pos % kWavesPerGroup;
+}
+
+// Exclusive scan of the counts per share, in place, a workgroup per kind of count (kSum*);
+// the total goes behind the last share.
+__global__ __launch_bounds__(1024) void share_scan_kernel(int *__restrict__ sums, int n, int pitch)
+{
+    __shared__ int lds[16];
+    int *s = sums + (int64_t)blockIdx.x * pitch;
+    static_assert(kMaxShares <= 4 * 1024, "four shares per thread");
+    int v[4], acc = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = (int)threadIdx.x * 4 + j;
+        v[j] = i < n ? s[i] : 0;
+        acc += v[j];
+    }
+    int total, run = block_exclusive_sum<1024>(acc, lds, total);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = (int)threadIdx.x * 4 + j;
+        if (i < n) s[i] = run;
+        run += v[j];
+    }
+    if (threadIdx.x == 0) s[n] = total;
+}
+
+// One wavefront per share of the caller's rows: writes the units of whole rows that start in
+// it, the running cost and the number of heavy units before each, and the rank of each split row
+// of 8 column groups among those rows, all in the caller's order.
+__global__ __launch_bounds__(kThreads) void list_units_kernel(
+    SortedRows sr, int share, int n_shares, const int *__restrict__ sums, int pitch, UnitRule rule, int first_split,
+    int4 *__restrict__ units, int *__restrict__ running, int *__restrict__ heavy_before, int *__restrict__ rank8)
+{
+    __shared__ int run_row[kBins + 1], run_nz[kBins];
+    for (int i = threadIdx.x; i <= kBins; i += kThreads) run_row[i] = sr.run_row[i];
+    for (int i = threadIdx.x; i < kBins; i += kThreads) run_nz[i] = sr.run_nz[i];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, c = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
+    if (c == 0 && lane == 0) {
+        const int n = sums[kSumUnits * pitch + n_shares];
+        running[n] = sums[kSumCost * pitch + n_shares];
+        heavy_before[n] = sums[kSumHeavy * pitch + n_shares];
+    }
+    if (c >= n_shares) return;
+    int n_units = sums[kSumUnits * pitch + c], cost0 = sums[kSumCost * pitch + c];
+    int heavy0 = sums[kSumHeavy * pitch + c], rows8 = sums[kSumRows8 * pitch + c];
+    const int64_t r_end = min(sr.rows, (int64_t)(c + 1) * share);
+    for (int64_t r0 = (int64_t)c * share; r0 < r_end; r0 += 64) {
+        const int64_t r = r0 + lane;
+        const bool ok = r < r_end;
+        const int d = ok ? sr.indptr[r + 1] - sr.indptr[r] : 0;
+        const int p = ok ? (int)sr.place[r] : 0;
+        int n = 0, in_run = 0;
+        if (d > 0 && d <= rule.split) {
+            in_run = p - run_row[d];
+            n = unit_rows(d, in_run, run_row[d + 1] - run_row[d], rule);
+        }
+        const int nz = d * n;
+        const int cost = n > 0 ? unit_cost(nz, n, rule.cost_shift) : 0;
+        const unsigned long long heads = __ballot(n > 0), heavies = __ballot(n > 0 && nz > rule.light_nz);
+        int inc = cost;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(inc, off);
+            if (lane >= off) inc += t;
+        }
+        if (n > 0) {
+            int w, rpb;
+            slice_rule(d, w, rpb);
+            const int at = n_units + lanes_below(heads, lane);
+            units[at] = make_int4(d, p, run_nz[d] + in_run * d, (w << 16) + n);
+            running[at] = cost0 + inc - cost;
+            heavy_before[at] = heavy0 + lanes_below(heavies, lane);
+        }
+        const bool is8 = d > rule.split && row_groups(d, rule.groups) == kXcds;
+        const unsigned long long eights = __ballot(is8);
+        if (is8) rank8[p - first_split] = rows8 + lanes_below(eights, lane);
+        n_units += __popcll(heads);
+        cost0 += __shfl(inc, 63);
+        heavy0 += __popcll(heavies);
+        rows8 += __popcll(eights);
+    }
+}
+
+// A split row's place in its class: rows of 8 groups follow the caller's row ids, the longer
+// ones come largest first (they touch all of X whatever their id; the hub workload measured
+// 2 % faster that way: 2.31 against 2.36 ms at N = 256).
+struct SplitRow {
+    int d, groups, cls, rank;
+};
+__device__ __forceinline__ SplitRow split_row(const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
+                                              int lr, const int *__restrict__ rank8, const ClassLayout &cl, int forced)
+{
+    SplitRow s;
+    s.d = s_indptr[first_split + lr + 1] - s_indptr[first_split + lr];
+    s.groups = row_groups(s.d, forced);
+    s.cls = 31 - __clz(s.groups / kXcds);
+    s.rank = s.cls == 0 ? rank8[lr] : n_split - cl.above[s.cls] - 1 - lr;
+    return s;
+}
+
+// One wavefront per split row, lane = column group: pieces per group (into `bins`) and per row,
+// and what they cost per queue (column group g belongs to queue g % n_queues).
+__global__ __launch_bounds__(kThreads) void split_rows_kernel(
+    const int *__restrict__ gcount, const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
+    const int *__restrict__ rank8, ClassLayout cl, int forced, int piece, int cost_shift, int n_queues,
+    int *__restrict__ bins, int *__restrict__ row_units, int *__restrict__ row_done, int *__restrict__ queue_cost)
+{
+    __shared__ int part[kWaves4][kXcds];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int cost = 0;
+    for (int lr = (int)blockIdx.x * kWaves4 + w; lr < n_split; lr += (int)gridDim.x * kWaves4) {
+        const SplitRow s = split_row(s_indptr, first_split, n_split, lr, rank8, cl, forced);
+        const int c = lane < s.groups ? gcount[(int64_t)lr * kMaxGroups + lane] : 0;
+        const int u = (c + piece - 1) / piece;
+        if (lane < s.groups) bins[cl.base[s.cls] + lane * cl.rows[s.cls] + s.rank] = u;
+        if (c > 0) cost += ((c + 9 * u) >> cost_shift) + u;
+        const int total = wave_sum(u);
+        if (lane == 0) {
+            row_units[lr] = total;
+            row_done[lr] = 0;
+        }
+    }
+    cost += __shfl_xor(cost, 8);
+    cost += __shfl_xor(cost, 16);
+    cost += __shfl_xor(cost, 32);
+    if (lane < kXcds) part[w][lane] = cost;
+    __syncthreads();
+    if ((int)threadIdx.x < kXcds) {
+        for (int q = 1; q < kWaves4; q++) cost += part[q][threadIdx.x];
+        if (cost) atomicAdd(&queue_cost[threadIdx.x % n_queues], cost);
+    }
+}
+
+// out = exclusive scan of in over n ints, out[n] = the sum, in one launch (in place allowed).  A
+// workgroup takes the next tile by ticket, publishes its sum, and adds up what the tiles before it
+// have published: their sums, back to the first that already knows its prefix.  Tiles are taken in
+// order, so every tile a workgroup waits for belongs to a workgroup that is running and publishes
+// its sum before it waits for anything itself.  Words: value below, 1 = sum, 2 = prefix above
+// (one 64-bit access: no fence).
+__global__ __launch_bounds__(kThreads) void scan_kernel(const int *__restrict__ in, int64_t n, int *__restrict__ out,
+                                                        int *__restrict__ ticket, unsigned long long *__restrict__ word)
+{
+    __shared__ int lds[kWaves4], my_tile, my_prefix;
+    if (threadIdx.x == 0)
+        my_tile = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tile = my_tile;
+    const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
+    int v[kScanItems], acc = 0;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+        v[j] = base + j < n ? in[base + j] : 0;
+        acc += v[j];
+    }
+    int total;
+    const int exc = block_exclusive_sum<kThreads>(acc, lds, total);
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        if (lane == 0)
+            __hip_atomic_store(&word[tile], ((tile ? 1ull : 2ull) << 32) | (unsigned)total, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        int prefix = 0;
+        for (int look = tile - 1; look >= 0; look -= 64) {
+            const int t = look - lane;
+            unsigned long long s = 2ull << 32;                      // before the first tile: a prefix of 0
+            if (t >= 0)
+                while (((s = __hip_atomic_load(&word[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) == 0)
+                    __builtin_amdgcn_s_sleep(1);
+            const unsigned long long known = __ballot((s >> 32) == 2);
+            const int stop = known ? __ffsll((unsigned long long)known) - 1 : 63;   // the nearest known prefix
+            prefix += wave_sum(lane <= stop ? (int)(unsigned)s : 0);
+            if (known) break;
+        }
+        if (lane == 0) {
+            if (tile)
+                __hip_atomic_store(&word[tile], (2ull << 32) | (unsigned)(prefix + total), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            my_prefix = prefix;
+            if ((int64_t)(tile + 1) * kScanTile >= n) out[n] = prefix + total;
+        }
+    }
+    __syncthreads();
+    int run = my_prefix + exc;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+        if (base + j < n) out[base + j] = run;
+        run += v[j];
+    }
+}
+
+// Where everything goes in the list: computed by one workgroup, read by the kernels that write it.
+struct PlanHead {
+    int queue_long[kXcds];       // pieces in each queue
+    int cut[kXcds + 1];          // queue q takes the units whose running cost lies in [cut[q], cut[q + 1])
+    int first[kXcds + 1];        // first unit of each queue
+    int bin_off[kPlanBins];      // where the pieces of a (class, column group) bin start in their queue
+    int per_queue;               // units per queue, a multiple of kWavesPerGroup
+};
+
+__device__ __forceinline__ int queue_of(int running_cost, const int *cut)
+{
+    int q = 0;
+#pragma unroll
+    for (int i = 1; i < kXcds; i++) q += running_cost >= cut[i];
+    return q;
+}
+
+// Queue q takes max(0, level - its pieces' cost) of the whole-row units' cost, level being the
+// smallest common level that takes all of it.
+__global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ bins, ClassLayout cl, int n_split,
+                                                        const int *__restrict__ queue_cost,
+                                                        const int *__restrict__ running, const int *__restrict__ sums,
+                                                        int pitch, int n_shares, int n_queues,
+                                                        PlanHead *__restrict__ head, Mail *__restrict__ mail)
+{
+    static_assert(kXcds * 64 == 512, "one wavefront per queue");
+    __shared__ int at[kPlanBins + 1], off[kPlanBins], queue_long[kXcds], cut[kXcds + 1], first[kXcds + 1];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int n = sums[kSumUnits * pitch + n_shares];
+    if (t <= kPlanBins) {
+        int v = 0;
+        if (n_split > 0) {
+            if (t == kPlanBins) {
+                v = bins[cl.total];
+            } else {
+                int cls = 0;                                       // bins of a class: 8, 16, 32, 64 in turn
+                while (t >= plan_bin(kXcds << (cls + 1), 0)) cls++;
+                v = bins[cl.base[cls] + (t - plan_bin(kXcds << cls, 0)) * cl.rows[cls]];
+            }
+        }
+        at[t] = v;
+    }
+    __syncthreads();
+    if (t < n_queues) {
+        // a die first takes the pieces of the rows with the most groups (the longest rows), one
+        // group after the other, then those of the next class, ...
+        int pos = 0;
+        for (int ng = kMaxGroups; ng >= kXcds; ng /= 2)
+            for (int g = t; g < ng; g += n_queues) {
+                const int b = plan_bin(ng, g);
+                off[b] = pos;
+                pos += at[b + 1] - at[b];
+            }
+        queue_long[t] = pos;
+    }
+    if (t == 64) {
+        const long long short_cost = sums[kSumCost * pitch + n_shares];
+        long long lc[kXcds], lo = 0, hi = short_cost;
+        for (int q = 0; q < n_queues; q++) {
+            lc[q] = n_split > 0 ? queue_cost[q] : 0;
+            if (lc[q] + short_cost > hi) hi = lc[q] + short_cost;
+        }
+        while (lo < hi) {                                  // smallest level that takes all of it
+            const long long mid = (lo + hi) / 2;
+            long long taken = 0;
+            for (int q = 0; q < n_queues; q++) taken += mid > lc[q] ? mid - lc[q] : 0;
+            if (taken >= short_cost) hi = mid; else lo = mid + 1;
+        }
+        long long run = 0;
+        for (int q = 0; q < n_queues; q++) {
+            cut[q] = (int)(run < short_cost ? run : short_cost);
+            run += lo > lc[q] ? lo - lc[q] : 0;
+        }
+        for (int q = n_queues; q <= kXcds; q++) cut[q] = 0x7fffffff;   // queues that do not exist take nothing
+    }
+    __syncthreads();
+    // first[q]: the first unit whose running cost reaches cut[q]; wavefront q searches, 64 units per step
+    if (w < n_queues) {
+        int lo = 0, hi = n;                                // the answer lies in [lo, hi]
+        while (lo < hi) {
+            const int step = (hi - lo + 63) / 64;
+            const int i = lo + lane * step;
+            const bool below = i < hi && running[i] < cut[w];
+            const int k = __popcll(__ballot(below));       // the first k probes are below
+            if (k == 0) { hi = lo; break; }
+            const int nlo = lo + (k - 1) * step + 1, nhi = min(hi, lo + k * step);
+            lo = nlo; hi = nhi;
+        }
+        if (lane == 0) first[w] = w == 0 ? 0 : lo;
+    } else if (lane == 0) {
+        first[w] = n;
+    }
+    if (t == 0) first[kXcds] = n;
+    __syncthreads();
+    if (t < kPlanBins) head->bin_off[t] = n_split > 0 ? off[t] : 0;
+    if (t < kXcds) head->queue_long[t] = t < n_queues ? queue_long[t] : 0;
+    if (t <= kXcds) {
+        head->cut[t] = cut[t];
+        head->first[t] = first[t];
+    }
+    if (t == 0) {
+        int most = 0;
+        for (int q = 0; q < n_queues; q++) most = max(most, queue_long[q] + first[q + 1] - first[q]);
+        most = (most + kWavesPerGroup - 1) / kWavesPerGroup * kWavesPerGroup;
+        head->per_queue = most;
+        mail->per_queue = most;
+        mail->n_pieces = at[kPlanBins];
+        mail->n_units = n;
+    }
+}
+
+// One wavefront per split row, lane = column group: writes the row's pieces into the queues.
+__global__ __launch_bounds__(kThreads) void emit_pieces_kernel(
+    const int *__restrict__ gcount, const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
+    const int *__restrict__ slot, const int *__restrict__ bins, const int *__restrict__ rank8, ClassLayout cl,
+    int forced, int piece, const PlanHead *__restrict__ head, int n_queues, int room, int4 *__restrict__ work)
+{
+    if (head->per_queue > room) return;                // the host makes room and launches again
+    const int lane = threadIdx.x & 63;
+    const int lr = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
+    if (lr >= n_split) return;
+    const SplitRow s = split_row(s_indptr, first_split, n_split, lr, rank8, cl, forced);
+    const int c = lane < s.groups ? gcount[(int64_t)lr * kMaxGroups + lane] : 0;
+    const int u = (c + piece - 1) / piece;
+    int c_inc = c, u_inc = u;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int tc = __shfl_up(c_inc, o), tu = __shfl_up(u_inc, o);
+        if (lane >= o) { c_inc += tc; u_inc += tu; }
+    }
+    if (c == 0) return;
+    const int row = (int)(first_split + lr);
+    const int loc = s_indptr[row] + c_inc - c, sl = slot[lr] + u_inc - u;
+    const int bin0 = cl.base[s.cls] + lane * cl.rows[s.cls];
+    const int pos0 = head->bin_off[plan_bin(s.groups, lane)] + bins[bin0 + s.rank] - bins[bin0];
+    for (int k = 0, off = 0; off < c; k++, off += piece)
+        work[plan_index(lane % n_queues, pos0 + k, n_queues)] =
+            make_int4(kDegBound + 1 + sl + k, row, loc + off, min(piece, c - off));
+}
+
+// Inside its queue a unit goes behind the pieces, in the order of the caller's row ids,
+// except that the queue's last kTailLight light units (few non-zeros: short chains of
+// gathers) are held back and placed at the very end, so that a queue does not end on a
+// long chain.  They are the light units with the highest ids of the queue's share, i.e.
+// they lie in the band of rows the die is working on at that time anyway.
+// heavy_before[s] = heavy units among the first s, [n] = all.
+constexpr int kTailLight = 2048;             // two rounds of the 1,024 wavefronts a die holds
+__global__ __launch_bounds__(kThreads) void place_units_kernel(
+    const int4 *__restrict__ units, const int *__restrict__ running, const int *__restrict__ heavy_before, int n,
+    const PlanHead *__restrict__ head, int n_queues, int room, int4 *__restrict__ work)
+{
+    const int per_queue = head->per_queue;
+    if (per_queue > room) return;                      // the host makes room and launches again
+    const int tid = blockIdx.x * kThreads + threadIdx.x;
+    if (tid < n) {
+        const int q = queue_of(running[tid], head->cut);
+        const int f = head->first[q], n_q = head->first[q + 1] - f;
+        const int h0 = heavy_before[f];
+        const int light_all = n_q - (heavy_before[f + n_q] - h0);              // light units of this queue
+        const int light_me = (tid - f) - (heavy_before[tid] - h0);             // ... before this unit
+        const bool is_light = heavy_before[tid + 1] == heavy_before[tid];
+        const int kept = max(0, light_all - kTailLight);                 // light units that stay in line
+        int pos;
+        if (is_light && light_me >= kept)
+            pos = n_q - (light_all - light_me);                                // held back: the last ones
+        else
+            pos = (tid - f) - max(0, light_me - kept);                         // in line, minus those held back before it
+        work[plan_index(q, head->queue_long[q] + pos, n_queues)] = units[tid];
+    }
+    for (int q = 0; q < n_queues; q++) {               // the rest of the shorter queues: padding
+        const int len = head->queue_long[q] + head->first[q + 1] - head->first[q];
+        for (int pos = len + tid; pos < per_queue; pos += (int)gridDim.x * kThreads)
+            work[plan_index(q, pos, n_queues)] = make_int4(0, 0, 0, 0);
+    }
+}
+
+}  // namespace
+
+// Split rows are added up by the gather kernel itself (the wavefront that stores a row's last
+// piece does it: one launch) when the plan holds at most this many pieces, by a second kernel
+// otherwise.  In the kernel every piece ends on a wait for its stores and one atomic, some
+// microseconds of latency that nothing hides on a launch-bound matrix but that is still less
+// than a second launch costs; with many pieces it adds up to more.  Measured, runs queued
+// back to back, in-kernel against second kernel at N = 16 / 64 / 128: 96 pieces (1.9 M
+// non-zeros) 0.88 / 0.94 / 0.96; 5,160 (1.2 M) 0.88 / 0.90 / 0.96; 8,848 (1.6 M) 0.82 / 0.94 /
+// 0.98; 7,760 (2.4 M) 0.99 / 0.96 / 0.98; 68,608 (14 M) 1.01 / 1.02 / 1.02; 144,561 (27 M)
+// 1.24 / 1.08 / 1.09; 0.5 M pieces (115 M non-zeros, nearly every row split) 1.30 at N = 64.
+constexpr int64_t kFusedReduceMaxPieces = 16384;
+
+int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups)
+{
+    if (n_split == 0) return kZeroWords;
+    return kZeroWords + 2 * (scan_tiles(n_split) + scan_tiles(class_layout(n_split, stats, groups).total));
+}
+
+int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
+                    const int *share_sums, const int *gcount, const Mail *stats, int64_t n_short_units, int *zeroed,
+                    Mail *mail, hipStream_t s)
+{
+    // pieces of split rows hold up to piece_nz non-zeros, units of several whole rows up to unit_nz
+    const int piece_nz = std::max(h->plan_unit, h->plan_split), forced = rule.groups;
+    const int nq = h->plan_queues;                     // 8 interleaved queues, or 1 (plain order)
+    const int n_split = (int)h->n_split_rows;
+    const int64_t first_split = h->rows - n_split;
+    const ClassLayout cl = class_layout(n_split, stats, forced);
+    const int pitch = sh.pitch + kWaves4;
+    int rc;
+    int4 *units;
+    int *running, *heavy, *rank8 = nullptr, *row_units = nullptr, *bins = nullptr;
+    PlanHead *head;
+    if ((rc = tmp->alloc(&units, (size_t)n_short_units))) return rc;
+    if ((rc = tmp->alloc(&running, (size_t)n_short_units + 1))) return rc;
+    if ((rc = tmp->alloc(&heavy, (size_t)n_short_units + 1))) return rc;
+    if ((rc = tmp->alloc(&head, 1))) return rc;
+    // the slots of each split row, and behind them one counter per split row (zero between launches)
+    DevBuf dslot;
+    if ((rc = dslot.alloc(sizeof(int) * (size_t)(2 * (int64_t)n_split + 1)))) return rc;
+    int *slot = dslot.as<int>(), *row_done = slot + n_split + 1;
+    if (n_split > 0) {
+        if ((rc = tmp->alloc(&rank8, (size_t)n_split))) return rc;
+        if ((rc = tmp->alloc(&row_units, (size_t)n_split))) return rc;
+        if ((rc = tmp->alloc(&bins, (size_t)cl.total + 1))) return rc;
+    }
+    share_scan_kernel<<<dim3(kSums), dim3(1024), 0, s>>>(const_cast<int *>(share_sums), sh.n, pitch);
+    list_units_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(sr, sh.share, sh.n, share_sums, pitch, rule,
+                                                                  (int)first_split, units, running, heavy, rank8);
+    if (n_split > 0) {
+        const unsigned groups = std::min(grid_for((int64_t)n_split * 64), 512u);
+        split_rows_kernel<<<dim3(groups), dim3(kThreads), 0, s>>>(
+            gcount, sr.s_indptr, first_split, n_split, rank8, cl, forced, piece_nz, rule.cost_shift, nq, bins,
+            row_units, row_done, zeroed + kZeroQueueLoad);
+        unsigned long long *words = reinterpret_cast<unsigned long long *>(zeroed + kZeroWords);
+        scan_kernel<<<dim3((unsigned)scan_tiles(n_split)), dim3(kThreads), 0, s>>>(row_units, n_split, slot,
+                                                                                  zeroed + kZeroTickets, words);
+        scan_kernel<<<dim3((unsigned)scan_tiles(cl.total)), dim3(kThreads), 0, s>>>(
+            bins, cl.total, bins, zeroed + kZeroTickets + 1, words + scan_tiles(n_split));
+    }
+    plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, zeroed + kZeroQueueLoad, running, share_sums,
+                                                  pitch, sh.n, nq, head, mail);
+    // Room for the list, before its length is known: the queues are level in cost, not in units,
+    // so each gets half as much again as its share of the units.  Where that is not enough
+    // (queues of single light rows next to queues of full units) the kernels below write nothing,
+    // and a second round has the length.
+    const int64_t most = n_short_units + cl.total + (h->nnz - h->nnz_short) / piece_nz;
+    int64_t room = std::min(most, most / nq + most / (2 * nq) + 4096);
+    DevBuf dwork;
+    for (int round = 0;; round++) {
+        room = (room + kWavesPerGroup - 1) / kWavesPerGroup * kWavesPerGroup;
+        if (room * nq > (int64_t)0x7fffffff) {
+            set_error("the launch plan would exceed 2^31 work units");
+            return ACCEL_ERR_ARG;
+        }
+        if ((rc = dwork.alloc(sizeof(int4) * (size_t)(room * nq)))) return rc;
+        if (n_split > 0)
+            emit_pieces_kernel<<<dim3(grid_for((int64_t)n_split * 64)), dim3(kThreads), 0, s>>>(
+                gcount, sr.s_indptr, first_split, n_split, slot, bins, rank8, cl, forced, piece_nz, head, nq,
+                (int)room, dwork.as<int4>());
+        place_units_kernel<<<dim3(grid_for(std::max<int64_t>(n_short_units, kThreads))), dim3(kThreads), 0, s>>>(
+            units, running, heavy, (int)n_short_units, head, nq, (int)room, dwork.as<int4>());
+        ACCEL_HIP(hipGetLastError());
+        ACCEL_HIP(hipStreamSynchronize(s));
+        if (mail->per_queue <= room) break;
+        if (round > 0) {
+            set_error("internal: the launch plan does not fit its own length");
+            return ACCEL_ERR_STATE;
+        }
+        room = mail->per_queue;
+        give_memory(dwork.release(), true);
+    }
+    if (mail->n_units != (int)n_short_units) {
+        set_error("internal: %d units of whole rows, %lld were expected from the degree histogram", mail->n_units,
+                  (long long)n_short_units);
+        return ACCEL_ERR_STATE;
+    }
+    h->n_units = (int64_t)mail->per_queue * nq;
+    h->n_long_units = n_split > 0 ? mail->n_pieces : 0;
+    h->work = static_cast<int32_t *>(dwork.release());
+    h->long_slot = static_cast<int32_t *>(dslot.release());
+    h->row_done = h->long_slot + n_split + 1;
+    h->fused_reduce = h->plan_reduce_option == 1 ||
+                      (h->plan_reduce_option == 0 && h->n_long_units <= kFusedReduceMaxPieces);
+    return ACCEL_OK;
+}
+
+}  // namespace accel

@@ -1,0 +1,239 @@
+// Shared by the two halves of the preprocessing: preprocess.hip (sort, sorted CSR, partition)
+// and plan.hip (the launch plan).
+#pragma once
+#include <algorithm>
+
+#include "internal.h"
+
+namespace accel {
+
+constexpr int kThreads = 256;
+constexpr int kWaves4 = kThreads / 64;
+
+// Rows are sorted by degree through bins: bin d holds the rows of degree d = 0..384, the last
+// bin all longer rows.
+constexpr int kBins = kDegBound + 2;
+constexpr int kLongBin = kDegBound + 1;
+
+// Split rows of more than this many non-zeros are regrouped in pieces of kWideChunk by a
+// workgroup per piece, shorter ones by a wavefront each.
+constexpr int kWideRow = 1024;
+constexpr int kWideChunk = 4096;
+
+// A small block of pinned host memory that kernels write their results for the host into: the
+// host reads it after a synchronisation, with no copy queued in between.
+struct Mail {
+    int hist[kBins];          // rows per bin
+    // statistics of the rows (kStat* below)
+    int stat[16];
+    // from the later kernels
+    int bad_index;            // a column outside [0, cols)
+    int bad_order;            // a saved row order is not the degree order
+    int per_queue;            // units per queue of the launch plan, padding included
+    int n_pieces;             // pieces of split rows
+    int n_units;              // units of whole rows
+    int n_blocks;             // entries of the partition (only for rows in any order)
+};
+enum {
+    kStatBadIndptr, kStatUnsorted, kStatMaxDegree,        // these three: the largest value over all rows
+    kStatLongBlocks, kStatWideRows, kStatWideChunks,      // the others: sums
+    kStatRows16, kStatRows32, kStatRows64,                // rows stored in 16, 32, 64 column groups by row_groups' own rule
+    kStatBig, kStatBigAlt,                                // rows with more than 32 times a split threshold
+    kStatSampled, kStatLocal,                             // of the locality sample
+    kStatCount
+};
+Mail *take_mail();            // memory.hip; null when there is none
+void give_mail(Mail *m);
+struct MailHolder {
+    Mail *m;
+    MailHolder() : m(take_mail()) {}
+    ~MailHolder() { give_mail(m); }
+    MailHolder(const MailHolder &) = delete;
+    MailHolder &operator=(const MailHolder &) = delete;
+};
+
+// Temporaries of one preprocessing call come out of a few large pieces of device memory (there
+// are some twenty of them).  The pieces are given back when the arena goes out of scope; what
+// is still queued then is queued on the null stream.
+struct Arena {
+    static constexpr int kMaxChunks = 32;
+    char *chunk[kMaxChunks] = {};
+    size_t cap = 0, used = 0;      // of the newest chunk
+    int n_chunks = 0;
+    size_t next_chunk = 0;         // size hint for the next chunk
+    bool any_stream = false;       // will be used on another stream than the null stream
+    Arena() = default;
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    ~Arena()
+    {
+        for (int i = 0; i < n_chunks; i++) give_memory(chunk[i], any_stream);
+    }
+    void *take(size_t bytes)
+    {
+        bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
+        if (n_chunks == 0 || used + bytes > cap) {
+            if (n_chunks == kMaxChunks) return nullptr;
+            const size_t want = std::max(bytes, next_chunk);
+            void *p = take_memory(want, any_stream);
+            if (!p) return nullptr;
+            chunk[n_chunks++] = static_cast<char *>(p);
+            cap = want;
+            used = 0;
+            next_chunk = std::max<size_t>(next_chunk / 4, (size_t)1 << 20);   // later chunks: leftovers only
+        }
+        void *p = chunk[n_chunks - 1] + used;
+        used += bytes;
+        return p;
+    }
+    template <class T> int alloc(T **out, size_t count)
+    {
+        *out = static_cast<T *>(take(sizeof(T) * count));
+        if (*out) return ACCEL_OK;
+        set_error("device allocation of %zu bytes failed", sizeof(T) * count);
+        return ACCEL_ERR_ALLOC;
+    }
+};
+
+struct DevBuf {  // device memory that is given back on scope exit unless it is released
+    void *p = nullptr;
+    DevBuf() = default;
+    DevBuf(const DevBuf &) = delete;
+    DevBuf &operator=(const DevBuf &) = delete;
+    ~DevBuf() { give_memory(p, false); }
+    int alloc(size_t bytes, bool any_stream = false)
+    {
+        p = take_memory(bytes, any_stream);
+        if (p) return ACCEL_OK;
+        set_error("device allocation of %zu bytes failed", bytes);
+        return ACCEL_ERR_ALLOC;
+    }
+    template <class T> T *as() { return static_cast<T *>(p); }
+    void *release() { void *q = p; p = nullptr; return q; }
+};
+
+inline unsigned grid_for(int64_t n) { return (unsigned)((n + kThreads - 1) / kThreads); }
+
+// Exclusive scan of one value per thread over a workgroup of T threads; `lds` holds T / 64 ints.
+template <int T>
+__device__ __forceinline__ int block_exclusive_sum(int v, int *lds, int &total)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int inc = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(inc, off);
+        if (lane >= off) inc += t;
+    }
+    if (lane == 63) lds[w] = inc;
+    __syncthreads();
+    int prefix = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < T / 64; i++) {
+        const int t = lds[i];
+        if (i < w) prefix += t;
+        tot += t;
+    }
+    __syncthreads();
+    total = tot;
+    return prefix + inc - v;
+}
+
+__device__ __forceinline__ int wave_sum(int v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+
+// Lanes of this wavefront that are `valid` and hold the same value in the low `bits` bits of v.
+__device__ __forceinline__ unsigned long long wave_match(int v, int bits, bool valid)
+{
+    unsigned long long peers = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+        const bool bit = (v >> b) & 1;
+        const unsigned long long bal = __ballot(bit);
+        peers &= bit ? bal : ~bal;
+    }
+    return peers;
+}
+__device__ __forceinline__ int lanes_below(unsigned long long m, int lane)
+{
+    return __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// ---------------------------------------------------------------------------
+// What one pass over the caller's rows computes about the units of whole rows (plan.hip's
+// subject, formed here because the pass that sorts the rows has everything at hand).
+// ---------------------------------------------------------------------------
+// Rows a unit of whole rows may hold: as many as fit unit_nz non-zeros, at least one.
+__device__ __forceinline__ int rows_per_unit(int d, int unit_nz) { return max(1, unit_nz / d); }
+
+// What a unit costs, for levelling the queues: a gathered row of X per non-zero, a
+// written row of Y per row, a fixed part; scaled down (shift >= 2) so that the sum over
+// the matrix stays below 2^31.  (Counting units, or fixed parts of 64 or 200, measured the
+// same within noise.)
+__device__ __forceinline__ int unit_cost(int nz, int n_rows, int shift)
+{
+    return ((nz + n_rows + 8) >> shift) + 1;
+}
+
+struct UnitRule {
+    int split;          // rows of more non-zeros are split, shorter ones form units of whole rows
+    int unit_nz;        // most non-zeros of a unit of several whole rows
+    int groups;         // column groups of split rows: 0 by row_groups' rule, else forced
+    int cost_shift;
+    int light_nz;       // a unit of up to this many non-zeros is a light one
+};
+
+// The unit that the row of degree d (1..split), `in_run` rows into the sorted run of its degree
+// (`run_rows` rows long), starts: n rows, or 0 when it starts none.
+__device__ __forceinline__ int unit_rows(int d, int in_run, int run_rows, const UnitRule &u)
+{
+    int w, rpb;
+    slice_rule(d, w, rpb);
+    const int rpu = rows_per_unit(d, u.unit_nz);
+    const int off = in_run % rpb;
+    if (off % rpu != 0) return 0;
+    return min(min(rpu, rpb - off), run_rows - in_run);
+}
+
+// Per run of rows in the caller's order (one wavefront's share): units of whole rows that start
+// there, their cost, how many of them are not light, and split rows stored in 8 column groups.
+enum { kSumUnits, kSumCost, kSumHeavy, kSumRows8, kSums };
+
+// Rows in a share and shares of a matrix: at most kMaxShares shares (enough wavefronts to fill
+// the GPU; the bins of every share are scanned), of a multiple of 64 rows.
+constexpr int kMaxShares = 4096;
+struct Shares {
+    int64_t rows = 0;
+    int share = 64, n = 0, pitch = 0;         // rows per share, shares, shares rounded up to a multiple of 4
+    explicit Shares(int64_t r) : rows(r)
+    {
+        const int64_t want = (r + kMaxShares - 1) / kMaxShares;
+        share = (int)std::max<int64_t>(64, (want + 63) / 64 * 64);
+        n = (int)((r + share - 1) / share);
+        pitch = (n + kWaves4 - 1) / kWaves4 * kWaves4;
+    }
+    unsigned groups() const { return (unsigned)(pitch / kWaves4); }
+};
+
+// The sorted rows as the kernels see them.
+struct SortedRows {
+    int64_t rows = 0;
+    const int32_t *indptr = nullptr;          // the caller's
+    int32_t *s_indptr = nullptr;              // sorted
+    int32_t *perm = nullptr;                  // sorted row -> caller's row; null: in order already
+    uint32_t *place = nullptr;                // caller's row -> sorted row
+    const int *run_row = nullptr;             // [kBins + 1] first sorted row of each bin
+    const int *run_nz = nullptr;              // [kBins] first non-zero of each bin
+};
+
+// plan.hip
+int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
+                    const int *share_sums, const int *gcount, const Mail *stats, int64_t n_short_units, int *zeroed,
+                    Mail *mail, hipStream_t s);
+// ints that must be zero when build_work_list is called (place_rows clears them)
+int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups);
+
+}  // namespace accel
