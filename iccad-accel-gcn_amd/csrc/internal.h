@@ -121,7 +121,7 @@ struct accel_handle {
     int64_t n_wide_rows = 0;          // rows with more than 1,024 non-zeros, regrouped in chunks
     int64_t n_chunks = 0;             // ... of 4,096 non-zeros
     int *runs = nullptr;              // first sorted row and first non-zero of each degree's run (SortedRows)
-    int *first_chunk = nullptr, *chunk_row = nullptr;     // chunks of each wide row, wide row of each chunk
+    int *first_chunk = nullptr, *chunk_row = nullptr;     // first chunk of each long row, long row of each chunk
     int64_t n_blocks = 0, n_long_blocks = 0, n_long_rows = 0, n_zero_rows = 0;
     int32_t max_degree = 0;
     double preprocess_ms = 0.0;

@@ -25,7 +25,7 @@
 // every row, in the caller's order, whether it starts a unit, so a scan of the counts per share
 // of rows puts the units in that order (list_units_kernel).  The pieces of a column group are
 // ordered by a scan over (class of rows, group, row of the class).  What bounds all of it is
-// the number of dependent launches (2 to 5 us each), not bytes: nine launches and no
+// the number of dependent launches (2 to 5 us each), not bytes: five launches and no
 // synchronisation before the last, where there were 45 launches and two (110 of 440 us of
 // kernels at 2.45 M non-zeros, 400 us of 1.79 ms at 125 M).
 #include "preprocess.h"
@@ -65,42 +65,13 @@ ClassLayout class_layout(int64_t n_split, const Mail *stats, int groups)
     return c;
 }
 
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kThreads * kScanItems;
-inline int64_t scan_tiles(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
-
-// The part of the zeroed memory each user has: queue loads, the two scans' tickets, their
-// per-tile words (8 bytes each).
-constexpr int kZeroQueueLoad = 0, kZeroTickets = 8, kZeroWords = 16;
+// Zeroed memory: the queue loads, then the two scans' part.
+constexpr int kZeroQueueLoad = 8;
 
 __device__ __forceinline__ int64_t plan_index(int queue, int pos, int n_queues)
 {
     // queue q, position p  ->  slot of wavefront (p % 4) in workgroup (p / 4) * n_queues + q
     return ((int64_t)(pos / kWavesPerGroup) * n_queues + queue) * kWavesPerGroup + pos % kWavesPerGroup;
-}
-
-// Exclusive scan of the counts per share, in place, a workgroup per kind of count (kSum*);
-// the total goes behind the last share.
-__global__ __launch_bounds__(1024) void share_scan_kernel(int *__restrict__ sums, int n, int pitch)
-{
-    __shared__ int lds[16];
-    int *s = sums + (int64_t)blockIdx.x * pitch;
-    static_assert(kMaxShares <= 4 * 1024, "four shares per thread");
-    int v[4], acc = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = (int)threadIdx.x * 4 + j;
-        v[j] = i < n ? s[i] : 0;
-        acc += v[j];
-    }
-    int total, run = block_exclusive_sum<1024>(acc, lds, total);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = (int)threadIdx.x * 4 + j;
-        if (i < n) s[i] = run;
-        run += v[j];
-    }
-    if (threadIdx.x == 0) s[n] = total;
 }
 
 // One wavefront per share of the caller's rows: writes the units of whole rows that start in
@@ -211,63 +182,6 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(
     }
 }
 
-// out = exclusive scan of in over n ints, out[n] = the sum, in one launch (in place allowed).  A
-// workgroup takes the next tile by ticket, publishes its sum, and adds up what the tiles before it
-// have published: their sums, back to the first that already knows its prefix.  Tiles are taken in
-// order, so every tile a workgroup waits for belongs to a workgroup that is running and publishes
-// its sum before it waits for anything itself.  Words: value below, 1 = sum, 2 = prefix above
-// (one 64-bit access: no fence).
-__global__ __launch_bounds__(kThreads) void scan_kernel(const int *__restrict__ in, int64_t n, int *__restrict__ out,
-                                                        int *__restrict__ ticket, unsigned long long *__restrict__ word)
-{
-    __shared__ int lds[kWaves4], my_tile, my_prefix;
-    if (threadIdx.x == 0)
-        my_tile = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int tile = my_tile;
-    const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    int v[kScanItems], acc = 0;
-#pragma unroll
-    for (int j = 0; j < kScanItems; j++) {
-        v[j] = base + j < n ? in[base + j] : 0;
-        acc += v[j];
-    }
-    int total;
-    const int exc = block_exclusive_sum<kThreads>(acc, lds, total);
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        if (lane == 0)
-            __hip_atomic_store(&word[tile], ((tile ? 1ull : 2ull) << 32) | (unsigned)total, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        int prefix = 0;
-        for (int look = tile - 1; look >= 0; look -= 64) {
-            const int t = look - lane;
-            unsigned long long s = 2ull << 32;                      // before the first tile: a prefix of 0
-            if (t >= 0)
-                while (((s = __hip_atomic_load(&word[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) == 0)
-                    __builtin_amdgcn_s_sleep(1);
-            const unsigned long long known = __ballot((s >> 32) == 2);
-            const int stop = known ? __ffsll((unsigned long long)known) - 1 : 63;   // the nearest known prefix
-            prefix += wave_sum(lane <= stop ? (int)(unsigned)s : 0);
-            if (known) break;
-        }
-        if (lane == 0) {
-            if (tile)
-                __hip_atomic_store(&word[tile], (2ull << 32) | (unsigned)(prefix + total), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            my_prefix = prefix;
-            if ((int64_t)(tile + 1) * kScanTile >= n) out[n] = prefix + total;
-        }
-    }
-    __syncthreads();
-    int run = my_prefix + exc;
-#pragma unroll
-    for (int j = 0; j < kScanItems; j++) {
-        if (base + j < n) out[base + j] = run;
-        run += v[j];
-    }
-}
-
 // Where everything goes in the list: computed by one workgroup, read by the kernels that write it.
 struct PlanHead {
     int queue_long[kXcds];       // pieces in each queue
@@ -323,25 +237,34 @@ __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ 
             }
         queue_long[t] = pos;
     }
-    if (t == 64) {
+    if (w == 1) {
+        // the smallest level that takes all of it, 64 candidates at a time
         const long long short_cost = sums[kSumCost * pitch + n_shares];
-        long long lc[kXcds], lo = 0, hi = short_cost;
-        for (int q = 0; q < n_queues; q++) {
-            lc[q] = n_split > 0 ? queue_cost[q] : 0;
-            if (lc[q] + short_cost > hi) hi = lc[q] + short_cost;
+        long long lc[kXcds], lo = 0, hi = short_cost;      // the level lies in [lo, hi]
+#pragma unroll
+        for (int q = 0; q < kXcds; q++) {
+            lc[q] = q < n_queues ? (n_split > 0 ? queue_cost[q] : 0) : 0x7fffffffffffffffLL;
+            if (q < n_queues && lc[q] + short_cost > hi) hi = lc[q] + short_cost;
         }
-        while (lo < hi) {                                  // smallest level that takes all of it
-            const long long mid = (lo + hi) / 2;
+        while (lo < hi) {
+            const long long step = (hi - lo + 63) / 64, mid = lo + lane * step;
             long long taken = 0;
-            for (int q = 0; q < n_queues; q++) taken += mid > lc[q] ? mid - lc[q] : 0;
-            if (taken >= short_cost) hi = mid; else lo = mid + 1;
+#pragma unroll
+            for (int q = 0; q < kXcds; q++) taken += mid > lc[q] ? mid - lc[q] : 0;
+            const int k = __popcll(__ballot(mid < hi && taken < short_cost));     // the first k are too low
+            if (k == 0) break;
+            const long long first_low = lo;
+            lo = first_low + (k - 1) * step + 1;
+            if (first_low + k * step < hi) hi = first_low + k * step;
         }
-        long long run = 0;
-        for (int q = 0; q < n_queues; q++) {
-            cut[q] = (int)(run < short_cost ? run : short_cost);
-            run += lo > lc[q] ? lo - lc[q] : 0;
+        if (lane == 0) {
+            long long run = 0;
+            for (int q = 0; q < n_queues; q++) {
+                cut[q] = (int)(run < short_cost ? run : short_cost);
+                run += lo > lc[q] ? lo - lc[q] : 0;
+            }
+            for (int q = n_queues; q <= kXcds; q++) cut[q] = 0x7fffffff;   // queues that do not exist take nothing
         }
-        for (int q = n_queues; q <= kXcds; q++) cut[q] = 0x7fffffff;   // queues that do not exist take nothing
     }
     __syncthreads();
     // first[q]: the first unit whose running cost reaches cut[q]; wavefront q searches, 64 units per step
@@ -379,35 +302,8 @@ __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ 
     }
 }
 
-// One wavefront per split row, lane = column group: writes the row's pieces into the queues.
-__global__ __launch_bounds__(kThreads) void emit_pieces_kernel(
-    const int *__restrict__ gcount, const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
-    const int *__restrict__ slot, const int *__restrict__ bins, const int *__restrict__ rank8, ClassLayout cl,
-    int forced, int piece, const PlanHead *__restrict__ head, int n_queues, int room, int4 *__restrict__ work)
-{
-    if (head->per_queue > room) return;                // the host makes room and launches again
-    const int lane = threadIdx.x & 63;
-    const int lr = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
-    if (lr >= n_split) return;
-    const SplitRow s = split_row(s_indptr, first_split, n_split, lr, rank8, cl, forced);
-    const int c = lane < s.groups ? gcount[(int64_t)lr * kMaxGroups + lane] : 0;
-    const int u = (c + piece - 1) / piece;
-    int c_inc = c, u_inc = u;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int tc = __shfl_up(c_inc, o), tu = __shfl_up(u_inc, o);
-        if (lane >= o) { c_inc += tc; u_inc += tu; }
-    }
-    if (c == 0) return;
-    const int row = (int)(first_split + lr);
-    const int loc = s_indptr[row] + c_inc - c, sl = slot[lr] + u_inc - u;
-    const int bin0 = cl.base[s.cls] + lane * cl.rows[s.cls];
-    const int pos0 = head->bin_off[plan_bin(s.groups, lane)] + bins[bin0 + s.rank] - bins[bin0];
-    for (int k = 0, off = 0; off < c; k++, off += piece)
-        work[plan_index(lane % n_queues, pos0 + k, n_queues)] =
-            make_int4(kDegBound + 1 + sl + k, row, loc + off, min(piece, c - off));
-}
-
+// Writes the list.  The first workgroups take split rows, a wavefront each (lane = column group),
+// and write their pieces; the others the units of whole rows, one per thread.
 // Inside its queue a unit goes behind the pieces, in the order of the caller's row ids,
 // except that the queue's last kTailLight light units (few non-zeros: short chains of
 // gathers) are held back and placed at the very end, so that a queue does not end on a
@@ -415,32 +311,74 @@ __global__ __launch_bounds__(kThreads) void emit_pieces_kernel(
 // they lie in the band of rows the die is working on at that time anyway.
 // heavy_before[s] = heavy units among the first s, [n] = all.
 constexpr int kTailLight = 2048;             // two rounds of the 1,024 wavefronts a die holds
-__global__ __launch_bounds__(kThreads) void place_units_kernel(
-    const int4 *__restrict__ units, const int *__restrict__ running, const int *__restrict__ heavy_before, int n,
-    const PlanHead *__restrict__ head, int n_queues, int room, int4 *__restrict__ work)
+struct EmitArgs {
+    const int *gcount;
+    const int32_t *s_indptr;
+    int64_t first_split;
+    int n_split, piece_groups;               // split rows; workgroups that take them
+    const int *slot, *bins, *rank8;
+    ClassLayout cl;
+    int forced, piece;
+    const int4 *units;
+    const int *running, *heavy_before;
+    int n_units;
+    const PlanHead *head;
+    int n_queues, room;
+    int4 *work;
+};
+
+__device__ __forceinline__ void emit_pieces(const EmitArgs &a, int lr)
 {
-    const int per_queue = head->per_queue;
-    if (per_queue > room) return;                      // the host makes room and launches again
-    const int tid = blockIdx.x * kThreads + threadIdx.x;
-    if (tid < n) {
-        const int q = queue_of(running[tid], head->cut);
-        const int f = head->first[q], n_q = head->first[q + 1] - f;
-        const int h0 = heavy_before[f];
-        const int light_all = n_q - (heavy_before[f + n_q] - h0);              // light units of this queue
-        const int light_me = (tid - f) - (heavy_before[tid] - h0);             // ... before this unit
-        const bool is_light = heavy_before[tid + 1] == heavy_before[tid];
+    const int lane = threadIdx.x & 63;
+    const SplitRow s = split_row(a.s_indptr, a.first_split, a.n_split, lr, a.rank8, a.cl, a.forced);
+    const int c = lane < s.groups ? a.gcount[(int64_t)lr * kMaxGroups + lane] : 0;
+    const int u = (c + a.piece - 1) / a.piece;
+    int c_inc = c, u_inc = u;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int tc = __shfl_up(c_inc, o), tu = __shfl_up(u_inc, o);
+        if (lane >= o) { c_inc += tc; u_inc += tu; }
+    }
+    if (c == 0) return;
+    const int row = (int)(a.first_split + lr);
+    const int loc = a.s_indptr[row] + c_inc - c, sl = a.slot[lr] + u_inc - u;
+    const int bin0 = a.cl.base[s.cls] + lane * a.cl.rows[s.cls];
+    const int pos0 = a.head->bin_off[plan_bin(s.groups, lane)] + a.bins[bin0 + s.rank] - a.bins[bin0];
+    for (int k = 0, off = 0; off < c; k++, off += a.piece)
+        a.work[plan_index(lane % a.n_queues, pos0 + k, a.n_queues)] =
+            make_int4(kDegBound + 1 + sl + k, row, loc + off, min(a.piece, c - off));
+}
+
+__global__ __launch_bounds__(kThreads) void emit_plan_kernel(EmitArgs a)
+{
+    const int per_queue = a.head->per_queue;
+    if (per_queue > a.room) return;                    // the host makes room and launches again
+    if ((int)blockIdx.x < a.piece_groups) {
+        const int lr = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
+        if (lr < a.n_split) emit_pieces(a, lr);
+        return;
+    }
+    const int tid = ((int)blockIdx.x - a.piece_groups) * kThreads + threadIdx.x;
+    if (tid < a.n_units) {
+        const int q = queue_of(a.running[tid], a.head->cut);
+        const int f = a.head->first[q], n_q = a.head->first[q + 1] - f;
+        const int h0 = a.heavy_before[f], h_me = a.heavy_before[tid];
+        const int light_all = n_q - (a.heavy_before[f + n_q] - h0);            // light units of this queue
+        const int light_me = (tid - f) - (h_me - h0);                          // ... before this unit
+        const bool is_light = a.heavy_before[tid + 1] == h_me;
         const int kept = max(0, light_all - kTailLight);                 // light units that stay in line
         int pos;
         if (is_light && light_me >= kept)
             pos = n_q - (light_all - light_me);                                // held back: the last ones
         else
             pos = (tid - f) - max(0, light_me - kept);                         // in line, minus those held back before it
-        work[plan_index(q, head->queue_long[q] + pos, n_queues)] = units[tid];
+        a.work[plan_index(q, a.head->queue_long[q] + pos, a.n_queues)] = a.units[tid];
     }
-    for (int q = 0; q < n_queues; q++) {               // the rest of the shorter queues: padding
-        const int len = head->queue_long[q] + head->first[q + 1] - head->first[q];
-        for (int pos = len + tid; pos < per_queue; pos += (int)gridDim.x * kThreads)
-            work[plan_index(q, pos, n_queues)] = make_int4(0, 0, 0, 0);
+    const int all = ((int)gridDim.x - a.piece_groups) * kThreads;
+    for (int q = 0; q < a.n_queues; q++) {             // the rest of the shorter queues: padding
+        const int len = a.head->queue_long[q] + a.head->first[q + 1] - a.head->first[q];
+        for (int pos = len + tid; pos < per_queue; pos += all)
+            a.work[plan_index(q, pos, a.n_queues)] = make_int4(0, 0, 0, 0);
     }
 }
 
@@ -459,8 +397,8 @@ constexpr int64_t kFusedReduceMaxPieces = 16384;
 
 int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups)
 {
-    if (n_split == 0) return kZeroWords;
-    return kZeroWords + 2 * (scan_tiles(n_split) + scan_tiles(class_layout(n_split, stats, groups).total));
+    if (n_split == 0) return kZeroQueueLoad;
+    return kZeroQueueLoad + scan_zeroed(n_split) + scan_zeroed(class_layout(n_split, stats, groups).total);
 }
 
 int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
@@ -491,22 +429,19 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
         if ((rc = tmp->alloc(&row_units, (size_t)n_split))) return rc;
         if ((rc = tmp->alloc(&bins, (size_t)cl.total + 1))) return rc;
     }
-    share_scan_kernel<<<dim3(kSums), dim3(1024), 0, s>>>(const_cast<int *>(share_sums), sh.n, pitch);
     list_units_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(sr, sh.share, sh.n, share_sums, pitch, rule,
                                                                   (int)first_split, units, running, heavy, rank8);
     if (n_split > 0) {
-        const unsigned groups = std::min(grid_for((int64_t)n_split * 64), 512u);
+        // (each workgroup ends on eight atomics to the same eight words)
+        const unsigned groups = std::min(grid_for((int64_t)n_split * 64), 1024u);
         split_rows_kernel<<<dim3(groups), dim3(kThreads), 0, s>>>(
             gcount, sr.s_indptr, first_split, n_split, rank8, cl, forced, piece_nz, rule.cost_shift, nq, bins,
-            row_units, row_done, zeroed + kZeroQueueLoad);
-        unsigned long long *words = reinterpret_cast<unsigned long long *>(zeroed + kZeroWords);
-        scan_kernel<<<dim3((unsigned)scan_tiles(n_split)), dim3(kThreads), 0, s>>>(row_units, n_split, slot,
-                                                                                  zeroed + kZeroTickets, words);
-        scan_kernel<<<dim3((unsigned)scan_tiles(cl.total)), dim3(kThreads), 0, s>>>(
-            bins, cl.total, bins, zeroed + kZeroTickets + 1, words + scan_tiles(n_split));
+            row_units, row_done, zeroed);
+        int *z = zeroed + kZeroQueueLoad;
+        launch_scans({{{row_units, slot, n_split, 0, z}, {bins, bins, cl.total, 0, z + scan_zeroed(n_split)}}, {}}, 2, s);
     }
-    plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, zeroed + kZeroQueueLoad, running, share_sums,
-                                                  pitch, sh.n, nq, head, mail);
+    plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, zeroed, running, share_sums, pitch, sh.n, nq, head,
+                                                  mail);
     // Room for the list, before its length is known: the queues are level in cost, not in units,
     // so each gets half as much again as its share of the units.  Where that is not enough
     // (queues of single light rows next to queues of full units) the kernels below write nothing,
@@ -521,12 +456,11 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
             return ACCEL_ERR_ARG;
         }
         if ((rc = dwork.alloc(sizeof(int4) * (size_t)(room * nq)))) return rc;
-        if (n_split > 0)
-            emit_pieces_kernel<<<dim3(grid_for((int64_t)n_split * 64)), dim3(kThreads), 0, s>>>(
-                gcount, sr.s_indptr, first_split, n_split, slot, bins, rank8, cl, forced, piece_nz, head, nq,
-                (int)room, dwork.as<int4>());
-        place_units_kernel<<<dim3(grid_for(std::max<int64_t>(n_short_units, kThreads))), dim3(kThreads), 0, s>>>(
-            units, running, heavy, (int)n_short_units, head, nq, (int)room, dwork.as<int4>());
+        const int piece_groups = (int)grid_for((int64_t)n_split * 64);
+        const EmitArgs ea{gcount, sr.s_indptr, first_split, n_split, piece_groups, slot, bins, rank8, cl, forced, piece_nz,
+                          units, running, heavy, (int)n_short_units, head, nq, (int)room, dwork.as<int4>()};
+        emit_plan_kernel<<<dim3(piece_groups + grid_for(std::max<int64_t>(n_short_units, kThreads))), dim3(kThreads), 0,
+                           s>>>(ea);
         ACCEL_HIP(hipGetLastError());
         ACCEL_HIP(hipStreamSynchronize(s));
         if (mail->per_queue <= room) break;

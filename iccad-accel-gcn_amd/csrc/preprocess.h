@@ -203,20 +203,130 @@ __device__ __forceinline__ int unit_rows(int d, int in_run, int run_rows, const 
 enum { kSumUnits, kSumCost, kSumHeavy, kSumRows8, kSums };
 
 // Rows in a share and shares of a matrix: at most kMaxShares shares (enough wavefronts to fill
-// the GPU; the bins of every share are scanned), of a multiple of 64 rows.
-constexpr int kMaxShares = 4096;
+// the GPU; the bins of every share are scanned), of a multiple of 64 rows, 256 at least (a
+// wavefront reads and writes a counter per bin whatever the length of its share).
+constexpr int kMaxShares = 4096, kMinShare = 256;
 struct Shares {
     int64_t rows = 0;
-    int share = 64, n = 0, pitch = 0;         // rows per share, shares, shares rounded up to a multiple of 4
+    int share = kMinShare, n = 0, pitch = 0;  // rows per share, shares, shares rounded up to a multiple of 4
     explicit Shares(int64_t r) : rows(r)
     {
         const int64_t want = (r + kMaxShares - 1) / kMaxShares;
-        share = (int)std::max<int64_t>(64, (want + 63) / 64 * 64);
+        share = (int)std::max<int64_t>(kMinShare, (want + 63) / 64 * 64);
         n = (int)((r + share - 1) / share);
         pitch = (n + kWaves4 - 1) / kWaves4 * kWaves4;
     }
     unsigned groups() const { return (unsigned)(pitch / kWaves4); }
 };
+
+// Exclusive scan of the counts per share, in place, by a workgroup of 1,024 threads; the total goes
+// behind the last share.
+__device__ __forceinline__ void scan_shares(int *__restrict__ s, int n, int *lds /* 16 ints */)
+{
+    static_assert(kMaxShares <= 4 * 1024, "four shares per thread");
+    int v[4], acc = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = (int)threadIdx.x * 4 + j;
+        v[j] = i < n ? s[i] : 0;
+        acc += v[j];
+    }
+    int total, run = block_exclusive_sum<1024>(acc, lds, total);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = (int)threadIdx.x * 4 + j;
+        if (i < n) s[i] = run;
+        run += v[j];
+    }
+    if (threadIdx.x == 0) s[n] = total;
+}
+
+// ---------------------------------------------------------------------------
+// Exclusive scans of up to three arrays in one launch: out[i] = add + in[0] + ... + in[i - 1],
+// out[n] = the sum of all plus add (in place allowed).  A workgroup takes the next tile of its array
+// by ticket, publishes the tile's sum, and adds up what the tiles before it have published: their
+// sums, back to the first that already knows its prefix.  Tiles are taken in order, so every tile a
+// workgroup waits for belongs to a workgroup that is running and publishes its sum before it waits
+// for anything itself.  Words: value below, 1 = sum, 2 = prefix above (one 64-bit access: no
+// fence).  Tickets and words are zero on entry.
+// ---------------------------------------------------------------------------
+constexpr int kScanItems = 8;
+constexpr int kScanTile = kThreads * kScanItems;
+inline int64_t scan_tiles(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
+struct ScanJob {
+    const int *in;
+    int *out;
+    int64_t n;
+    int add;
+    int *zeroed;                              // scan_zeroed(n) ints, 8-byte aligned
+};
+inline int64_t scan_zeroed(int64_t n) { return 2 + 2 * scan_tiles(n); }
+struct ScanJobs {
+    ScanJob job[3];
+    int first[3];                             // first workgroup of each job
+};
+static __global__ __launch_bounds__(kThreads) void scan_kernel(ScanJobs jobs)
+{
+    __shared__ int lds[kWaves4], my_tile, my_prefix;
+    const int which = (int)blockIdx.x >= jobs.first[2] ? 2 : (int)blockIdx.x >= jobs.first[1] ? 1 : 0;
+    const ScanJob jb = jobs.job[which];
+    unsigned long long *word = reinterpret_cast<unsigned long long *>(jb.zeroed) + 1;
+    if (threadIdx.x == 0)
+        my_tile = __hip_atomic_fetch_add(jb.zeroed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tile = my_tile;
+    const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
+    int v[kScanItems], acc = 0;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+        v[j] = base + j < jb.n ? jb.in[base + j] : 0;
+        acc += v[j];
+    }
+    int total;
+    const int exc = block_exclusive_sum<kThreads>(acc, lds, total);
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        if (lane == 0)
+            __hip_atomic_store(&word[tile], ((tile ? 1ull : 2ull) << 32) | (unsigned)total, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        int prefix = 0;
+        for (int look = tile - 1; look >= 0; look -= 64) {
+            const int t = look - lane;
+            unsigned long long s = 2ull << 32;                      // before the first tile: a prefix of 0
+            if (t >= 0)
+                while (((s = __hip_atomic_load(&word[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) == 0)
+                    __builtin_amdgcn_s_sleep(1);
+            const unsigned long long known = __ballot((s >> 32) == 2);
+            const int stop = known ? __ffsll((unsigned long long)known) - 1 : 63;   // the nearest known prefix
+            prefix += wave_sum(lane <= stop ? (int)(unsigned)s : 0);
+            if (known) break;
+        }
+        if (lane == 0) {
+            if (tile)
+                __hip_atomic_store(&word[tile], (2ull << 32) | (unsigned)(prefix + total), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            my_prefix = prefix + jb.add;
+            if ((int64_t)(tile + 1) * kScanTile >= jb.n) jb.out[jb.n] = prefix + total + jb.add;
+        }
+    }
+    __syncthreads();
+    int run = my_prefix + exc;
+#pragma unroll
+    for (int j = 0; j < kScanItems; j++) {
+        if (base + j < jb.n) jb.out[base + j] = run;
+        run += v[j];
+    }
+}
+// The n_jobs jobs (1 to 3), each of at least one element.
+inline void launch_scans(ScanJobs jobs, int n_jobs, hipStream_t s)
+{
+    int at = 0;
+    for (int i = 0; i < 3; i++) {
+        jobs.first[i] = i < n_jobs ? at : 0x7fffffff;
+        if (i < n_jobs) at += (int)scan_tiles(jobs.job[i].n);
+    }
+    scan_kernel<<<dim3((unsigned)at), dim3(kThreads), 0, s>>>(jobs);
+}
 
 // The sorted rows as the kernels see them.
 struct SortedRows {

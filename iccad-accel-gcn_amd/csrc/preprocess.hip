@@ -61,10 +61,18 @@ __global__ __launch_bounds__(kThreads) void degree_kernel(DegreeArgs a, int *__r
 #pragma unroll
     for (int k = 0; k < kStatCount; k++) st[k] = 0;
     const int64_t r_end = min(a.rows, (int64_t)(c + 1) * a.share);
+    const int64_t r_first = (int64_t)c * a.share + lane;
+    int lo_next = r_first < r_end ? a.indptr[r_first] : 0, hi_next = r_first < r_end ? a.indptr[r_first + 1] : 0;
     for (int64_t r0 = (int64_t)c * a.share; r0 < r_end; r0 += 64) {
         const int64_t r = r0 + lane;
         const bool ok = r < r_end;
-        const int lo = ok ? a.indptr[r] : 0, hi = ok ? a.indptr[r + 1] : 0;
+        const int lo = lo_next, hi = hi_next;                // the next round's are on their way
+        if (r + 64 < r_end) {
+            lo_next = a.indptr[r + 64];
+            hi_next = a.indptr[r + 65];
+        } else {
+            lo_next = hi_next = 0;
+        }
         int before = __shfl_up(lo, 1);
         if (lane == 0) before = r > 0 ? a.indptr[r - 1] : lo;
         int d = hi - lo;
@@ -156,14 +164,23 @@ __global__ __launch_bounds__(kThreads) void bin_scan_kernel(int *__restrict__ bi
         return;
     }
     int *row = bins + (int64_t)b * pitch;
+    constexpr int kVecs = kMaxShares / (4 * kThreads);           // 16-byte vectors per thread, all loaded at once
+    int4 v[kVecs];
     int carry = 0;
-    for (int c0 = 0; c0 < pitch; c0 += 4 * kThreads) {           // pitch is a multiple of 4
-        const int c = c0 + 4 * (int)threadIdx.x;
-        int4 v = c < pitch ? *reinterpret_cast<const int4 *>(row + c) : make_int4(0, 0, 0, 0);
-        int total, run = block_exclusive_sum<kThreads>(v.x + v.y + v.z + v.w, lds, total);
+#pragma unroll
+    for (int j = 0; j < kVecs; j++) {
+        const int c = 4 * (j * kThreads + (int)threadIdx.x);
+        v[j] = c < pitch ? *reinterpret_cast<const int4 *>(row + c) : make_int4(0, 0, 0, 0);   // pitch is a multiple of 4
+    }
+#pragma unroll
+    for (int j = 0; j < kVecs; j++) {
+        const int c = 4 * (j * kThreads + (int)threadIdx.x);
+        if (4 * j * kThreads >= pitch) break;
+        int total, run = block_exclusive_sum<kThreads>(v[j].x + v[j].y + v[j].z + v[j].w, lds, total);
         run += carry;
         if (c < pitch)
-            *reinterpret_cast<int4 *>(row + c) = make_int4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
+            *reinterpret_cast<int4 *>(row + c) =
+                make_int4(run, run + v[j].x, run + v[j].x + v[j].y, run + v[j].x + v[j].y + v[j].z);
         carry += total;
     }
     if (threadIdx.x == 0) {
@@ -269,10 +286,13 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
     __builtin_amdgcn_wave_barrier();
     int n_units = 0, cost = 0, n_heavy = 0, n_rows8 = 0;
     const int64_t r_end = min(a.rows, (int64_t)(c + 1) * a.share);
+    const int64_t r_first = (int64_t)c * a.share + lane;
+    int d_next = r_first < r_end ? a.indptr[r_first + 1] - a.indptr[r_first] : 0;
     for (int64_t r0 = (int64_t)c * a.share; r0 < r_end; r0 += 64) {
         const int64_t r = r0 + lane;
         const bool ok = r < r_end;
-        const int d = ok ? a.indptr[r + 1] - a.indptr[r] : 0;
+        const int d = d_next;                                // the next round's is on its way
+        d_next = r + 64 < r_end ? a.indptr[r + 65] - a.indptr[r + 64] : 0;
         const int bin = min(d, kLongBin);
         const unsigned long long peers = wave_match(bin, 9, ok);
         const int rank = lanes_below(peers, lane);
@@ -314,16 +334,34 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Rows of more than 384 non-zeros: ranked by (degree, row).  Up to kRankMax of them are ranked by
-// comparing each with all (one launch; 8,192 rows: 10 us), more by a stable radix sort, 8 bits a pass.
+// Rows of more than 384 non-zeros: ranked by (degree, row).  Up to kFewLong of them one workgroup
+// does everything (ranks by comparing each with all, scans, blocks) in one launch, 8 us at 800
+// rows; up to kRankMax they are ranked the same way by many workgroups (8,192 rows: 10 us), more
+// by a stable radix sort, 8 bits a pass, and the rest is scans.
 // ---------------------------------------------------------------------------
+constexpr int kFewLong = 2048;
 constexpr int kRankMax = 8192;
 constexpr int kRankRows = 64;                 // rows ranked by a workgroup, by four threads each
+
+// How many of the n4 * 4 degrees at `tile` (LDS), the first of which is long row `at0`, rank before
+// long row j of degree d.  Equal degrees rank by row, which is the order they are listed in.
+__device__ __forceinline__ int count_before(const int4 *tile, int n4, int at0, int d, int j)
+{
+    int below = 0;
+#pragma unroll 4
+    for (int i = 0; i < n4; i++) {
+        const int4 e = tile[i];
+        const int at = at0 + 4 * i;
+        below += (e.x < d + (at < j)) + (e.y < d + (at + 1 < j)) + (e.z < d + (at + 2 < j)) + (e.w < d + (at + 3 < j));
+    }
+    return below;
+}
+
 __global__ __launch_bounds__(kThreads) void rank_long_rows_kernel(
     const int *__restrict__ deg, const uint32_t *__restrict__ row, int n, int64_t first_long,
     int32_t *__restrict__ perm, uint32_t *__restrict__ place, int *__restrict__ sorted_deg)
 {
-    __shared__ int tile[kThreads * 4];
+    __shared__ __attribute__((aligned(16))) int tile[kThreads * 4];
     __shared__ int part[4][kRankRows];
     const int j = (int)blockIdx.x * kRankRows + (threadIdx.x & 63), seg = threadIdx.x >> 6;
     const int d = j < n ? deg[j] : 0;
@@ -332,12 +370,7 @@ __global__ __launch_bounds__(kThreads) void rank_long_rows_kernel(
         __syncthreads();
         for (int i = threadIdx.x; i < kThreads * 4; i += kThreads) tile[i] = t0 + i < n ? deg[t0 + i] : INT_MAX;
         __syncthreads();
-        const int i0 = seg * kThreads;
-#pragma unroll 8
-        for (int i = 0; i < kThreads; i++) {
-            const int e = tile[i0 + i], at = t0 + i0 + i;
-            below += e < d || (e == d && at < j);
-        }
+        below += count_before(reinterpret_cast<const int4 *>(tile + seg * kThreads), kThreads / 4, t0 + seg * kThreads, d, j);
     }
     part[seg][threadIdx.x & 63] = below;
     __syncthreads();
@@ -348,6 +381,80 @@ __global__ __launch_bounds__(kThreads) void rank_long_rows_kernel(
         if (perm) perm[p] = (int32_t)r;
         if (place) place[r] = (uint32_t)p;
         sorted_deg[below] = d;
+    }
+}
+
+__host__ __device__ inline int blocks_of(int d) { return (d + kDegBound - 1) / kDegBound; }
+__host__ __device__ inline int chunks_of(int d) { return d > kWideRow ? (d + kWideChunk - 1) / kWideChunk : 0; }
+
+struct LongArgs {
+    const int *deg;                           // in the caller's order
+    const uint32_t *row;
+    int n;
+    int64_t first_long;                       // sorted row of the first
+    int nz0, block0;                          // non-zeros and blocks before them
+    int32_t *perm;                            // null: in order already
+    uint32_t *place;
+    int32_t *s_indptr;                        // null: not wanted
+    int4 *block4;
+    int *first_chunk, *chunk_row;             // of long row i (null: none is wide)
+};
+
+// Workgroup 0: the long rows, when there are few.  The others: one kind each of the counts per share
+// (kSum*), whose scan the launch plan needs and which have nothing to do with it but the launch.
+__global__ __launch_bounds__(1024) void few_long_rows_kernel(LongArgs a, int *__restrict__ sums, int sum_pitch,
+                                                             int n_shares)
+{
+    __shared__ int lds[16];
+    if (blockIdx.x > 0) {
+        scan_shares(sums + (int64_t)(blockIdx.x - 1) * sum_pitch, n_shares, lds);
+        return;
+    }
+    if (a.n == 0) return;
+    __shared__ __attribute__((aligned(16))) int deg[kFewLong];
+    __shared__ int sorted[kFewLong], first_block[kFewLong], loc[kFewLong];
+    const int t = threadIdx.x, n4 = (a.n + 3) / 4;
+    for (int i = t; i < n4 * 4; i += 1024) deg[i] = i < a.n ? a.deg[i] : INT_MAX;
+    __syncthreads();
+    for (int j = t; j < a.n; j += 1024) {
+        const int d = deg[j], below = count_before(reinterpret_cast<const int4 *>(deg), n4, 0, d, j);
+        sorted[below] = d;
+        const uint32_t r = a.row[j];
+        if (a.perm) a.perm[a.first_long + below] = (int32_t)r;
+        if (a.place) a.place[r] = (uint32_t)(a.first_long + below);
+    }
+    __syncthreads();
+    {
+        const int i = 2 * t, d0 = i < a.n ? sorted[i] : 0, d1 = i + 1 < a.n ? sorted[i + 1] : 0;
+        int tot;
+        const int nz = a.nz0 + block_exclusive_sum<1024>(d0 + d1, lds, tot);
+        const int blk = a.block0 + block_exclusive_sum<1024>(blocks_of(d0) + blocks_of(d1), lds, tot);
+        const int chk = block_exclusive_sum<1024>(chunks_of(d0) + chunks_of(d1), lds, tot);
+        if (i < a.n) {
+            loc[i] = nz;
+            first_block[i] = blk;
+            if (a.s_indptr) a.s_indptr[a.first_long + i] = nz;
+            if (a.first_chunk) a.first_chunk[i] = chk;
+        }
+        if (i + 1 < a.n) {
+            loc[i + 1] = nz + d0;
+            first_block[i + 1] = blk + blocks_of(d0);
+            if (a.s_indptr) a.s_indptr[a.first_long + i + 1] = nz + d0;
+            if (a.first_chunk) a.first_chunk[i + 1] = chk + chunks_of(d0);
+        }
+        if (a.first_chunk && t == 0) a.first_chunk[a.n] = tot;
+    }
+    __syncthreads();                                     // (global stores of this workgroup are read back below)
+    const int lane = t & 63;
+    for (int i = t >> 6; i < a.n; i += 16) {
+        const int d = sorted[i];
+        for (int k = lane; k < blocks_of(d); k += 64)
+            a.block4[first_block[i] + k] =
+                make_int4(d, (int)a.first_long + i, loc[i] + k * kDegBound, min(kDegBound, d - k * kDegBound));
+        if (a.first_chunk && chunks_of(d) > 0) {
+            const int c0 = a.first_chunk[i];
+            for (int k = lane; k < chunks_of(d); k += 64) a.chunk_row[c0 + k] = i;
+        }
     }
 }
 
@@ -428,6 +535,15 @@ __global__ __launch_bounds__(kThreads) void apply_long_order_kernel(
     sorted_deg[i] = (int)sorted_key[i];
 }
 
+__global__ __launch_bounds__(kThreads) void long_sizes_kernel(const int *__restrict__ sorted_deg, int n,
+                                                              int *__restrict__ blocks, int *__restrict__ chunks)
+{
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= n) return;
+    blocks[i] = blocks_of(sorted_deg[i]);
+    if (chunks) chunks[i] = chunks_of(sorted_deg[i]);
+}
+
 // Exclusive scan of n ints in place by one workgroup (the radix sort's counts).
 __global__ __launch_bounds__(1024) void small_scan_kernel(int *__restrict__ v, int64_t n)
 {
@@ -483,70 +599,64 @@ int sort_long_rows(Arena *tmp, const int *deg, const uint32_t *row, int n, int m
     return ACCEL_OK;
 }
 
-// One workgroup scans the sorted long rows: their first non-zeros (s_indptr, may be null), their
-// first blocks and, for the wide ones (the last n_wide), their first chunks.
-__global__ __launch_bounds__(1024) void long_scan_kernel(const int *__restrict__ sorted_deg, int n, int nz0,
-                                                         int32_t *__restrict__ s_indptr, int *__restrict__ first_block,
-                                                         int n_wide, int *__restrict__ first_chunk)
-{
-    __shared__ int lds[16];
-    int nz = nz0, blk = 0, chk = 0;
-    for (int b = 0; b < n; b += 1024 * kItems) {
-        const int at = b + (int)threadIdx.x * kItems;
-        int d[kItems], sz = 0, sb = 0, sc = 0;
-#pragma unroll
-        for (int j = 0; j < kItems; j++) {
-            d[j] = at + j < n ? sorted_deg[at + j] : 0;
-            sz += d[j];
-            sb += (d[j] + kDegBound - 1) / kDegBound;
-            sc += d[j] > kWideRow ? (d[j] + kWideChunk - 1) / kWideChunk : 0;
-        }
-        int tz, tb, tc;
-        int rz = nz + block_exclusive_sum<1024>(sz, lds, tz);
-        int rb = blk + block_exclusive_sum<1024>(sb, lds, tb);
-        int rc = chk + block_exclusive_sum<1024>(sc, lds, tc);
-#pragma unroll
-        for (int j = 0; j < kItems; j++) {
-            if (at + j < n) {
-                if (s_indptr) s_indptr[at + j] = rz;
-                first_block[at + j] = rb;
-                const int wide = at + j - (n - n_wide);
-                if (first_chunk && wide >= 0) first_chunk[wide] = rc;
-            }
-            rz += d[j];
-            rb += (d[j] + kDegBound - 1) / kDegBound;
-            rc += d[j] > kWideRow ? (d[j] + kWideChunk - 1) / kWideChunk : 0;
-        }
-        nz += tz;
-        blk += tb;
-        chk += tc;
-    }
-    if (first_chunk && threadIdx.x == 0) first_chunk[n_wide] = chk;
-}
-
 // One wavefront per long row: its block4 entries, and the row of each of its chunks.
-__global__ __launch_bounds__(kThreads) void long_blocks_kernel(
-    const int *__restrict__ sorted_deg, int n, int64_t first_long, const int32_t *__restrict__ loc_of,
-    const int *__restrict__ first_block, int block0, int n_wide, const int *__restrict__ first_chunk,
-    int4 *__restrict__ block4, int *__restrict__ chunk_row)
+__global__ __launch_bounds__(kThreads) void long_blocks_kernel(LongArgs a, const int *__restrict__ sorted_deg,
+                                                               const int32_t *__restrict__ loc_of,
+                                                               const int *__restrict__ first_block)
 {
     const int lane = threadIdx.x & 63, i = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
-    if (i >= n) return;
-    const int d = sorted_deg[i], row = (int)(first_long + i), loc = loc_of[row];
-    const int n_blk = (d + kDegBound - 1) / kDegBound, at = block0 + first_block[i];
-    for (int k = lane; k < n_blk; k += 64)
-        block4[at + k] = make_int4(d, row, loc + k * kDegBound, min(kDegBound, d - k * kDegBound));
-    const int wide = i - (n - n_wide);
-    if (chunk_row && wide >= 0) {
-        const int n_chk = (d + kWideChunk - 1) / kWideChunk, c0 = first_chunk[wide];
-        for (int k = lane; k < n_chk; k += 64) chunk_row[c0 + k] = wide;
+    if (i >= a.n) return;
+    const int d = sorted_deg[i], row = (int)(a.first_long + i), loc = loc_of[row], at = first_block[i];
+    for (int k = lane; k < blocks_of(d); k += 64)
+        a.block4[at + k] = make_int4(d, row, loc + k * kDegBound, min(kDegBound, d - k * kDegBound));
+    if (a.first_chunk && chunks_of(d) > 0) {
+        const int c0 = a.first_chunk[i];
+        for (int k = lane; k < chunks_of(d); k += 64) a.chunk_row[c0 + k] = i;
     }
+}
+
+// Ints that must be zero for place_long_rows (place_rows clears them).
+int64_t long_zeroed_ints(int64_t n) { return n > kFewLong ? 3 * scan_zeroed(n) : 0; }
+
+// The long rows' places, row pointers, blocks and chunks, and the scan of the counts per share (sums,
+// may be null).  in_order: the rows are sorted already, so they are listed in sorted order.
+int place_long_rows(Arena *tmp, const LongArgs &a, bool in_order, int max_degree, const int32_t *loc_of, int *zeroed,
+                    int *sums, const Shares &sh, hipStream_t s)
+{
+    const bool few = a.n <= kFewLong;
+    if (few || sums) {
+        LongArgs la = a;
+        if (!few) la.n = 0;
+        few_long_rows_kernel<<<dim3(1 + (sums ? kSums : 0)), dim3(1024), 0, s>>>(la, sums, sh.pitch + kWaves4, sh.n);
+    }
+    if (few) return ACCEL_OK;
+    int rc, *sorted_deg = const_cast<int *>(a.deg), *blocks, *chunks = nullptr;
+    if (!in_order) {
+        if ((rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
+        if ((rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
+            return rc;
+    }
+    if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
+    if (a.first_chunk && (rc = tmp->alloc(&chunks, (size_t)a.n))) return rc;
+    long_sizes_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(sorted_deg, a.n, blocks, chunks);
+    ScanJobs jobs{};
+    int n_jobs = 0;
+    auto add = [&](const int *in, int *out, int first) {
+        jobs.job[n_jobs] = {in, out, a.n, first, zeroed + n_jobs * scan_zeroed(a.n)};
+        n_jobs++;
+    };
+    add(blocks, blocks, a.block0);
+    if (a.s_indptr) add(sorted_deg, a.s_indptr + a.first_long, a.nz0);
+    if (chunks) add(chunks, a.first_chunk, 0);
+    launch_scans(jobs, n_jobs, s);
+    long_blocks_kernel<<<dim3(grid_for((int64_t)a.n * 64)), dim3(kThreads), 0, s>>>(a, sorted_deg, loc_of, blocks);
+    return ACCEL_OK;
 }
 
 // ---------------------------------------------------------------------------
-// Sorted copy of the non-zeros.  Each of the two outputs may be left out: the columns (idx_out
-// null), and the payload, which is the value of the non-zero or, when src_pos is set, its
-// position in the caller's arrays (what a later value update gathers through).  Columns outside
+// Sorted copy of the non-zeros: the columns (idx_out, may be null) and a payload, which is the
+// value of the non-zero or, when src_pos is set, its position in the caller's arrays (what a later
+// value update gathers through).  Columns outside
 // [0, cols) are reported to the host: every non-zero passes through here exactly once.
 // ---------------------------------------------------------------------------
 struct CopyArgs {
@@ -568,18 +678,22 @@ __device__ __forceinline__ void report_bad(const CopyArgs &a, bool bad)
     if (a.mail && __ballot(bad) && (threadIdx.x & 63) == 0) a.mail->bad_index = 1;
 }
 
-// Rows of up to 384 non-zeros: a workgroup copies kPermuteTile consecutive non-zeros of the sorted
-// matrix.  Which rows those are is a closed form of the position (runs of equal degree); their
-// source offsets are put in LDS, and where the tile lies inside one run, as nearly all do, each
-// thread finds the row of its non-zeros by a multiplication.  Bound by reading row segments of
-// some hundred bytes at arbitrary addresses (about twice their bytes in 128-byte lines).
+// Rows that stay whole (up to 384 non-zeros): a workgroup copies kPermuteTile consecutive non-zeros
+// of the sorted matrix.  Which rows those are is a closed form of the position (runs of equal
+// degree); their source offsets are put in LDS, and where the tile lies inside one run, as nearly
+// all do on a large matrix, each thread finds the row of its non-zeros by a multiplication.  Bound
+// by reading row segments of some hundred bytes at arbitrary addresses (about twice their bytes in
+// 128-byte lines).
 constexpr int kPermuteNz = 8;                        // non-zeros per thread
 constexpr int kPermuteTile = kThreads * kPermuteNz;  // non-zeros per workgroup
-__global__ __launch_bounds__(kThreads) void permute_rows_kernel(CopyArgs a, int n_take)
+struct PermuteLds {
+    int run_row[kBins + 1], run_nz[kBins];
+    int row_end[kPermuteTile + 1];                   // first non-zero of the row behind, per row of the tile
+    int shift[kPermuteTile + 1];                     // source position minus sorted position, per row
+};
+__device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, int tile, int n_take)
 {
-    __shared__ int row_end[kPermuteTile + 1];        // first non-zero of the row behind, per row of the tile
-    __shared__ int shift[kPermuteTile + 1];          // source position minus sorted position, per row
-    const int p0 = (int)blockIdx.x * kPermuteTile, p1 = min(p0 + kPermuteTile, n_take);
+    const int p0 = tile * kPermuteTile, p1 = min(p0 + kPermuteTile, n_take);
     // degrees of the rows that hold the tile's first and last non-zero: as many bins (from 1 up) as
     // start at or before it
     int d_first = 0, d_last = 0;
@@ -588,33 +702,32 @@ __global__ __launch_bounds__(kThreads) void permute_rows_kernel(CopyArgs a, int 
         int nz[kLoads];
 #pragma unroll
         for (int j = 0; j < kLoads; j++) nz[j] = a.sr.run_nz[1 + 64 * j + (threadIdx.x & 63)];
+        for (int i = threadIdx.x; i <= kBins; i += kThreads) l.run_row[i] = a.sr.run_row[i];
+        for (int i = threadIdx.x; i < kBins; i += kThreads) l.run_nz[i] = a.sr.run_nz[i];
 #pragma unroll
         for (int j = 0; j < kLoads; j++) {
             d_first += __popcll(__ballot(nz[j] <= p0));
             d_last += __popcll(__ballot(nz[j] <= p1 - 1));
         }
     }
-    const int row0 = a.sr.run_row[d_first] + (p0 - a.sr.run_nz[d_first]) / d_first;
-    const int row1 = a.sr.run_row[d_last] + (p1 - 1 - a.sr.run_nz[d_last]) / d_last;
+    __syncthreads();
+    const int row0 = l.run_row[d_first] + (p0 - l.run_nz[d_first]) / d_first;
+    const int row1 = l.run_row[d_last] + (p1 - 1 - l.run_nz[d_last]) / d_last;
     const int n_here = row1 - row0 + 1;              // at most kPermuteTile: every row holds a non-zero of the tile
     const bool one_run = d_first == d_last;
     for (int j = threadIdx.x; j < n_here; j += kThreads) {
         const int row = row0 + j;
-        int d = d_first;
-        if (!one_run) {
-            int lo = d_first, hi = d_last;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (a.sr.run_row[mid] <= row) lo = mid; else hi = mid - 1;
-            }
-            d = lo;
+        int lo = d_first, hi = d_last;               // the last bin that starts at or before the row
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (l.run_row[mid] <= row) lo = mid; else hi = mid - 1;
         }
-        const int start = a.sr.run_nz[d] + (row - a.sr.run_row[d]) * d;
-        row_end[j] = start + d;
-        shift[j] = a.sr.indptr[a.sr.perm ? a.sr.perm[row] : row] - start;
+        const int start = l.run_nz[lo] + (row - l.run_row[lo]) * lo;
+        l.row_end[j] = start + lo;
+        l.shift[j] = a.sr.indptr[a.sr.perm ? a.sr.perm[row] : row] - start;
     }
     __syncthreads();
-    const int start0 = one_run ? a.sr.run_nz[d_first] + (row0 - a.sr.run_row[d_first]) * d_first : 0;
+    const int start0 = l.row_end[0] - d_first;       // first non-zero of the tile's first row
     const float inv = 1.0f / (float)d_first;
     int src[kPermuteNz], col[kPermuteNz], pay[kPermuteNz];
     bool bad = false;
@@ -628,16 +741,16 @@ __global__ __launch_bounds__(kThreads) void permute_rows_kernel(CopyArgs a, int 
             int lo = 0, hi = n_here - 1;             // first j with row_end[j] > p
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
-                if (row_end[mid] > p) hi = mid; else lo = mid + 1;
+                if (l.row_end[mid] > p) hi = mid; else lo = mid + 1;
             }
             j = lo;
         }
-        src[q] = p + shift[j];
+        src[q] = p + l.shift[j];
     }
 #pragma unroll
     for (int q = 0; q < kPermuteNz; q++) {
         col[q] = a.idx[src[q]];
-        if (a.pay_out) pay[q] = payload(a, src[q]);
+        pay[q] = payload(a, src[q]);
     }
 #pragma unroll
     for (int q = 0; q < kPermuteNz; q++) {
@@ -645,7 +758,7 @@ __global__ __launch_bounds__(kThreads) void permute_rows_kernel(CopyArgs a, int 
         bad |= (uint32_t)col[q] >= a.cols;
         if (p >= p1) continue;
         if (a.idx_out) a.idx_out[p] = col[q];
-        if (a.pay_out) a.pay_out[p] = pay[q];
+        a.pay_out[p] = pay[q];
     }
     report_bad(a, bad);
 }
@@ -655,25 +768,24 @@ __global__ __launch_bounds__(kThreads) void permute_rows_kernel(CopyArgs a, int 
 // column group.  counts[lr * 64 + g] receives the size of each group (counts may be null).
 // Rows of up to R * 64 non-zeros: a wavefront per row.  The whole row is loaded at once, put in
 // order in LDS and written out in one piece per array: with stores straight from the ranks (up to
-// 64 groups under the same store instruction) and a second read of the columns the two
-// regrouping kernels took 0.49 ms for 62 M non-zeros.
+// 64 groups under the same store instruction) and a second read of the columns regrouping 62 M
+// non-zeros took 0.49 ms (0.33 ms so).
+template <int R> struct GroupLds {
+    int2 buf[kWaves4][R * 64];
+    int cnt[kWaves4][kMaxGroups];
+};
 template <int R>
-__global__ __launch_bounds__(kThreads) void group_rows_kernel(CopyArgs a, int64_t first_row, int lr0, int n_rows,
-                                                              int forced_groups, int *__restrict__ counts)
+__device__ __forceinline__ void group_row(const CopyArgs &a, GroupLds<R> &l, int64_t r, int lr, int forced_groups,
+                                          int *__restrict__ counts)
 {
     static_assert(kMaxGroups == 64, "one lane per column group");
-    __shared__ int2 buf[kWaves4][R * 64];
-    __shared__ int cnt[kWaves4][kMaxGroups];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = (int)blockIdx.x * kWaves4 + w;
-    if (i >= n_rows) return;                             // the whole wavefront leaves; no barriers below
-    const int64_t r = first_row + i;
     const int64_t src0 = a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r];
     const int64_t dst0 = a.sr.s_indptr[r];
     const int d = a.sr.s_indptr[r + 1] - (int)dst0;
     const int ng = row_groups(d, forced_groups), bits = 31 - __clz(ng);
-    int *my = cnt[w];
-    int2 *st = buf[w];
+    int *my = l.cnt[w];
+    int2 *st = l.buf[w];
     my[lane] = 0;
     __builtin_amdgcn_wave_barrier();
     int col[R], pay[R];
@@ -697,7 +809,7 @@ __global__ __launch_bounds__(kThreads) void group_rows_kernel(CopyArgs a, int64_
     report_bad(a, bad);
     __builtin_amdgcn_wave_barrier();
     const int c = my[lane];                              // lane g holds the size of group g
-    if (counts) counts[(int64_t)(lr0 + i) * kMaxGroups + lane] = c;
+    if (counts) counts[(int64_t)lr * kMaxGroups + lane] = c;
     int inc = c;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -728,18 +840,19 @@ __global__ __launch_bounds__(kThreads) void group_rows_kernel(CopyArgs a, int64_
         if (e < d) {
             const int2 v = st[e];
             if (a.idx_out) a.idx_out[dst0 + e] = v.x;
-            if (a.pay_out) a.pay_out[dst0 + e] = v.y;
+            a.pay_out[dst0 + e] = v.y;
         }
     }
 }
 
 // Longer rows ("wide") in chunks of kWideChunk non-zeros, a workgroup per chunk, so that a row of
 // 200,000 is 49 workgroups and not a chain of 200 rounds in one: count the chunk's groups, scan the
-// counts of each row's chunks, place.  chunk_row[c] = the wide row of chunk c, first_chunk[w] = the
-// first chunk of wide row w.
+// counts of each row's chunks, place.  chunk_row[c] = the long row of chunk c, first_chunk[i] = the
+// first chunk of long row i.
 struct WideArgs {
     const int *chunk_row, *first_chunk;
-    int64_t first_row;                        // sorted row of the first wide row
+    int64_t first_long;                       // sorted row of the first long row
+    int n_narrow;                             // long rows before the first wide one
     int forced_groups;
     int *chunk_count;                         // [chunks][64]: counts, then destinations
 };
@@ -749,17 +862,16 @@ struct WideChunk {
 };
 __device__ __forceinline__ WideChunk wide_chunk(const CopyArgs &a, const WideArgs &wa, int c)
 {
-    const int w = wa.chunk_row[c];
-    const int64_t r = wa.first_row + w;
-    const int d = a.sr.s_indptr[r + 1] - a.sr.s_indptr[r], off = (c - wa.first_chunk[w]) * kWideChunk;
+    const int i = wa.chunk_row[c];
+    const int64_t r = wa.first_long + i;
+    const int d = a.sr.s_indptr[r + 1] - a.sr.s_indptr[r], off = (c - wa.first_chunk[i]) * kWideChunk;
     return {(int64_t)a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r] + off, min(kWideChunk, d - off),
             row_groups(d, wa.forced_groups)};
 }
 
-__global__ __launch_bounds__(kThreads) void wide_count_kernel(CopyArgs a, WideArgs wa)
+__device__ __forceinline__ void wide_count(const CopyArgs &a, const WideArgs &wa, int *cnt, int c)
 {
-    __shared__ int cnt[kMaxGroups];
-    const WideChunk ch = wide_chunk(a, wa, (int)blockIdx.x);
+    const WideChunk ch = wide_chunk(a, wa, c);
     if ((int)threadIdx.x < kMaxGroups) cnt[threadIdx.x] = 0;
     __syncthreads();
     int col[kWideChunk / kThreads];
@@ -778,7 +890,45 @@ __global__ __launch_bounds__(kThreads) void wide_count_kernel(CopyArgs a, WideAr
     }
     report_bad(a, bad);
     __syncthreads();
-    if ((int)threadIdx.x < kMaxGroups) wa.chunk_count[(int64_t)blockIdx.x * kMaxGroups + threadIdx.x] = cnt[threadIdx.x];
+    if ((int)threadIdx.x < kMaxGroups) wa.chunk_count[(int64_t)c * kMaxGroups + threadIdx.x] = cnt[threadIdx.x];
+}
+
+// All of the above in one launch (on a small matrix each would take its few microseconds after the
+// other): workgroups take, in this order, chunks of wide rows to count, split rows of up to 1,024 and
+// of up to 384 non-zeros (four each), tiles of whole rows.
+constexpr int kSmallRounds = kDegBound / 64, kMidRounds = kWideRow / 64;
+struct CopyPlan {
+    int n_chunks, n_mid, n_small;             // chunks; split rows
+    int mid_groups, small_groups;             // workgroups for the split rows
+    int64_t first_mid, first_small;           // sorted rows
+    int n_take;                               // non-zeros of whole rows
+    int *counts;                              // [split row][64], or null
+};
+__global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArgs wa, CopyPlan cp)
+{
+    union Lds {
+        PermuteLds permute;
+        GroupLds<kMidRounds> mid;
+        GroupLds<kSmallRounds> small;
+        int cnt[kMaxGroups];
+    };
+    __shared__ __attribute__((aligned(16))) char raw[sizeof(Lds)];
+    Lds &l = *reinterpret_cast<Lds *>(raw);
+    int b = blockIdx.x;
+    if (b < cp.n_chunks) { wide_count(a, wa, l.cnt, b); return; }
+    b -= cp.n_chunks;
+    if (b < cp.mid_groups) {                  // a wavefront without a row leaves; no barriers inside
+        const int i = b * kWaves4 + (threadIdx.x >> 6);
+        if (i < cp.n_mid) group_row<kMidRounds>(a, l.mid, cp.first_mid + i, cp.n_small + i, wa.forced_groups, cp.counts);
+        return;
+    }
+    b -= cp.mid_groups;
+    if (b < cp.small_groups) {
+        const int i = b * kWaves4 + (threadIdx.x >> 6);
+        if (i < cp.n_small) group_row<kSmallRounds>(a, l.small, cp.first_small + i, i, wa.forced_groups, cp.counts);
+        return;
+    }
+    permute_rows(a, l.permute, b - cp.small_groups, cp.n_take);
 }
 
 // A workgroup per wide row turns the counts of its chunks into destinations in the sorted arrays
@@ -786,17 +936,17 @@ __global__ __launch_bounds__(kThreads) void wide_count_kernel(CopyArgs a, WideAr
 __global__ __launch_bounds__(kThreads) void wide_scan_kernel(CopyArgs a, WideArgs wa, int lr0, int *__restrict__ counts)
 {
     __shared__ int part[kWaves4][kMaxGroups];
-    const int w = blockIdx.x, g = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int c0 = wa.first_chunk[w], n = wa.first_chunk[w + 1] - c0;
+    const int w = blockIdx.x, g = threadIdx.x & 63, q = threadIdx.x >> 6, i = wa.n_narrow + w;
+    const int c0 = wa.first_chunk[i], n = wa.first_chunk[i + 1] - c0;
     const int per = (n + kWaves4 - 1) / kWaves4, from = c0 + min(n, q * per), to = c0 + min(n, (q + 1) * per);
     int sum = 0;
     for (int c = from; c < to; c++) sum += wa.chunk_count[(int64_t)c * kMaxGroups + g];
     part[q][g] = sum;
     __syncthreads();
     int total = 0, before = 0;
-    for (int i = 0; i < kWaves4; i++) {
-        if (i < q) before += part[i][g];
-        total += part[i][g];
+    for (int k = 0; k < kWaves4; k++) {
+        if (k < q) before += part[k][g];
+        total += part[k][g];
     }
     if (q == 0 && counts) counts[(int64_t)(lr0 + w) * kMaxGroups + g] = total;
     int inc = total;                                     // every wavefront scans the 64 totals
@@ -805,7 +955,7 @@ __global__ __launch_bounds__(kThreads) void wide_scan_kernel(CopyArgs a, WideArg
         const int t = __shfl_up(inc, off);
         if (g >= off) inc += t;
     }
-    int run = a.sr.s_indptr[wa.first_row + w] + inc - total + before;
+    int run = a.sr.s_indptr[wa.first_long + i] + inc - total + before;
     for (int c = from; c < to; c++) {
         int *p = wa.chunk_count + (int64_t)c * kMaxGroups + g;
         const int v = *p;
@@ -872,7 +1022,7 @@ __global__ __launch_bounds__(kThreads) void wide_place_kernel(CopyArgs a, WideAr
         const int2 v = buf[e];
         const int64_t to = (int64_t)off[col_group(v.x, ch.ng)] + e;
         if (a.idx_out) a.idx_out[to] = v.x;
-        if (a.pay_out) a.pay_out[to] = v.y;
+        a.pay_out[to] = v.y;
     }
 }
 
@@ -1154,24 +1304,6 @@ static RunTotals run_totals(const int *hist, int most, int unit_nz)
     return t;
 }
 
-// The sorted long rows' products: degrees in order, first non-zeros, blocks, chunks.
-struct LongRows {
-    int n = 0, n_wide = 0, n_chunks = 0;
-    int *deg = nullptr;                       // in the caller's order
-    uint32_t *row = nullptr;
-    int *sorted_deg = nullptr, *first_block = nullptr;
-    int *first_chunk = nullptr, *chunk_row = nullptr;      // [n_wide + 1], [n_chunks]
-    int alloc(Arena *tmp)
-    {
-        int rc;
-        if ((rc = tmp->alloc(&deg, (size_t)n))) return rc;
-        if ((rc = tmp->alloc(&row, (size_t)n))) return rc;
-        if ((rc = tmp->alloc(&sorted_deg, (size_t)n))) return rc;
-        return tmp->alloc(&first_block, (size_t)n);
-    }
-    static size_t bytes(int64_t n) { return (size_t)n * 16 + 1024; }
-};
-
 // Partition a row order as given (no sort): the GPU counterpart of running
 // block_level_partition.py on one *.new_indptr file.
 int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
@@ -1192,10 +1324,14 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
         return partition_any_order(&tmp, indptr_dev, rows, block4_dev, n_blocks, mail, s);
     }
     const RunTotals rt = run_totals(mail->hist, kDegBound, kDegBound);
-    LongRows lo;
-    lo.n = mail->hist[kLongBin];
-    tmp.next_chunk = LongRows::bytes(lo.n) + (1 << 12);
-    if ((rc = lo.alloc(&tmp))) return rc;
+    const int n_long = mail->hist[kLongBin];
+    const int64_t n_zeroed = long_zeroed_ints(n_long);
+    tmp.next_chunk = (size_t)n_long * 12 + (size_t)n_zeroed * 4 + (1 << 12);
+    int *long_deg, *zeroed;
+    uint32_t *long_row;
+    if ((rc = tmp.alloc(&long_deg, (size_t)n_long))) return rc;
+    if ((rc = tmp.alloc(&long_row, (size_t)n_long))) return rc;
+    if ((rc = tmp.alloc(&zeroed, (size_t)n_zeroed))) return rc;
     *n_blocks = rt.blocks + mail->stat[kStatLongBlocks];
     DevBuf b4;
     if ((rc = b4.alloc(sizeof(int4) * (size_t)*n_blocks))) return rc;
@@ -1204,12 +1340,15 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
     pa.bins = bins; pa.bin_total = bin_total;
     pa.rule = UnitRule{kDegBound, kDegBound, 0, 2, 0};
     pa.block4 = b4.as<int4>();
-    pa.long_deg = lo.deg; pa.long_row = lo.row;
+    pa.long_deg = long_deg; pa.long_row = long_row;
+    pa.zero = zeroed; pa.n_zero = n_zeroed;
     place_rows_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(pa);
-    if (lo.n > 0) {                           // in order already: their place is the order they were listed in
-        long_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(lo.deg, lo.n, 0, nullptr, lo.first_block, 0, nullptr);
-        long_blocks_kernel<<<dim3(grid_for((int64_t)lo.n * 64)), dim3(kThreads), 0, s>>>(
-            lo.deg, lo.n, rows - lo.n, indptr_dev, lo.first_block, (int)rt.blocks, 0, nullptr, b4.as<int4>(), nullptr);
+    if (n_long > 0) {
+        LongArgs la{};
+        la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
+        la.nz0 = (int)rt.nnz; la.block0 = (int)rt.blocks;
+        la.block4 = b4.as<int4>();
+        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, nullptr, sh, s))) return rc;
     }
     ACCEL_HIP(hipGetLastError());
     *block4_dev = static_cast<int32_t *>(b4.release());
@@ -1269,21 +1408,23 @@ static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, i
 {
     const int64_t rows = h->rows;
     const int n_split = (int)h->n_split_rows, n_long = (int)h->n_long_rows, n_wide = (int)h->n_wide_rows;
-    if (nnz_short > 0)
-        permute_rows_kernel<<<dim3((unsigned)((nnz_short + kPermuteTile - 1) / kPermuteTile)), dim3(kThreads), 0, s>>>(
-            a, (int)nnz_short);
-    const int n_small = n_split - n_long, n_mid = n_long - n_wide;
-    constexpr int kSmallRounds = kDegBound / 64, kMidRounds = kWideRow / 64;
-    if (n_small > 0)
-        group_rows_kernel<kSmallRounds><<<dim3(grid_for((int64_t)n_small * 64)), dim3(kThreads), 0, s>>>(
-            a, rows - n_split, 0, n_small, h->plan_groups, counts);
-    if (n_mid > 0)
-        group_rows_kernel<kMidRounds><<<dim3(grid_for((int64_t)n_mid * 64)), dim3(kThreads), 0, s>>>(
-            a, rows - n_long, n_small, n_mid, h->plan_groups, counts);
-    if (n_wide > 0) {
-        WideArgs wa{h->chunk_row, h->first_chunk, rows - n_wide, h->plan_groups, nullptr};
+    WideArgs wa{h->chunk_row, h->first_chunk, rows - n_long, n_long - n_wide, h->plan_groups, nullptr};
+    if (n_wide > 0)
         if (int rc = tmp->alloc(&wa.chunk_count, (size_t)h->n_chunks * kMaxGroups)) return rc;
-        wide_count_kernel<<<dim3((unsigned)h->n_chunks), dim3(kThreads), 0, s>>>(a, wa);
+    CopyPlan cp{};
+    cp.n_chunks = (int)h->n_chunks;
+    cp.n_mid = n_long - n_wide;
+    cp.n_small = n_split - n_long;
+    cp.mid_groups = (int)grid_for((int64_t)cp.n_mid * 64);
+    cp.small_groups = (int)grid_for((int64_t)cp.n_small * 64);
+    cp.first_mid = rows - n_long;
+    cp.first_small = rows - n_split;
+    cp.n_take = (int)nnz_short;
+    cp.counts = counts;
+    const int64_t groups = (int64_t)cp.n_chunks + cp.mid_groups + cp.small_groups +
+                           (nnz_short + kPermuteTile - 1) / kPermuteTile;
+    if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp);
+    if (n_wide > 0) {
         wide_scan_kernel<<<dim3((unsigned)n_wide), dim3(kThreads), 0, s>>>(a, wa, n_split - n_wide, counts);
         wide_place_kernel<<<dim3((unsigned)h->n_chunks), dim3(kThreads), 0, s>>>(a, wa);
     }
@@ -1470,20 +1611,20 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     UnitRule rule{h->plan_split, h->plan_unit, h->plan_groups, 2, std::max(24, h->plan_unit / 4)};
     // total cost = about (nnz + 10 rows) >> shift + units < 2^31
     while (((nnz + 10 * rows) >> rule.cost_shift) + rows >= ((int64_t)1 << 30)) rule.cost_shift++;
-    const int64_t n_zeroed = plan_zeroed_ints(n_split, mail, h->plan_groups);
-    LongRows lo;
-    lo.n = (int)h->n_long_rows;
-    lo.n_wide = (int)h->n_wide_rows;
-    lo.n_chunks = (int)h->n_chunks;
-    tmp.next_chunk = (size_t)rows * 4 + LongRows::bytes(lo.n) + (size_t)n_zeroed * 4 +
-                     (size_t)kSums * (sh.pitch + kWaves4) * 4 + (size_t)n_split * (256 + 24) +
-                     (size_t)lo.n_chunks * 260 + (size_t)whole.units * 24 + 16 * (size_t)(binned.nnz / 384) + (1 << 16);
-    uint32_t *place;
-    int *sums, *zeroed, *gcount = nullptr;
+    const int n_long = (int)h->n_long_rows, n_wide = (int)h->n_wide_rows;
+    const int64_t plan_zeroed = plan_zeroed_ints(n_split, mail, h->plan_groups);
+    const int64_t n_zeroed = plan_zeroed + long_zeroed_ints(n_long);
+    tmp.next_chunk = (size_t)rows * 4 + (size_t)n_long * (n_long > kFewLong ? 48 : 8) + (size_t)n_zeroed * 4 +
+                     (size_t)kSums * (sh.pitch + kWaves4) * 4 + (size_t)n_split * (256 + 8) +
+                     (size_t)plan_zeroed * kScanTile / 2 * 4 + (size_t)h->n_chunks * 260 + (size_t)whole.units * 24 +
+                     (1 << 16);
+    uint32_t *place, *long_row;
+    int *sums, *zeroed, *long_deg, *gcount = nullptr;
     if ((rc = tmp.alloc(&place, (size_t)rows))) return rc;
     if ((rc = tmp.alloc(&sums, (size_t)kSums * (sh.pitch + kWaves4)))) return rc;
     if ((rc = tmp.alloc(&zeroed, (size_t)n_zeroed))) return rc;
-    if ((rc = lo.alloc(&tmp))) return rc;
+    if ((rc = tmp.alloc(&long_deg, (size_t)n_long))) return rc;
+    if ((rc = tmp.alloc(&long_row, (size_t)n_long))) return rc;
     if (n_split > 0 && (rc = tmp.alloc(&gcount, (size_t)n_split * kMaxGroups))) return rc;
     // Split rows (more than plan_split non-zeros: the last n_split rows of the sorted order) are
     // stored grouped by column group; all other rows keep their non-zero order.  The caller's
@@ -1493,7 +1634,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     const size_t b_sip = pad(sizeof(int32_t) * (size_t)(rows + 1));
     const size_t b_perm = h->identity_perm ? 0 : pad(sizeof(int32_t) * (size_t)rows);
     const size_t b_runs = pad(sizeof(int) * (2 * kBins + 1));
-    const size_t b_chk = lo.n_wide ? pad(sizeof(int) * (size_t)(lo.n_wide + 1 + lo.n_chunks)) : 0;
+    const size_t b_chk = n_wide ? pad(sizeof(int) * (size_t)(n_long + 1 + h->n_chunks)) : 0;
     const size_t b_nz = own_copy ? pad(sizeof(int32_t) * (size_t)nnz) : 0;
     DevBuf slab, b4;
     if ((rc = slab.alloc(b_sip + b_perm + b_runs + b_chk + 2 * b_nz))) return rc;
@@ -1506,12 +1647,10 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     h->runs = reinterpret_cast<int *>(at);
     at += b_runs;
     h->first_chunk = b_chk ? reinterpret_cast<int *>(at) : nullptr;
-    h->chunk_row = b_chk ? h->first_chunk + lo.n_wide + 1 : nullptr;
+    h->chunk_row = b_chk ? h->first_chunk + n_long + 1 : nullptr;
     at += b_chk;
     int32_t *s_idx = reinterpret_cast<int32_t *>(at);
     float *s_val = reinterpret_cast<float *>(at + b_nz);
-    lo.first_chunk = h->first_chunk;
-    lo.chunk_row = h->chunk_row;
 
     // ---- sort: perm, place, s_indptr, block4 ------------------------------------------
     PlaceArgs pa{};
@@ -1520,19 +1659,16 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     pa.perm = h->perm; pa.place = place; pa.s_indptr = h->s_indptr;
     pa.block4 = b4.as<int4>();
     pa.run_row = h->runs; pa.run_nz = h->runs + kBins + 1;
-    pa.long_deg = lo.deg; pa.long_row = lo.row;
+    pa.long_deg = long_deg; pa.long_row = long_row;
     pa.sums = sums; pa.zero = zeroed; pa.n_zero = n_zeroed;
     place_rows_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(pa);
-    if (lo.n > 0) {
-        const int64_t first_long = rows - lo.n;
-        if ((rc = sort_long_rows(&tmp, lo.deg, lo.row, lo.n, h->max_degree, first_long, h->perm, place, lo.sorted_deg, s)))
-            return rc;
-        long_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(lo.sorted_deg, lo.n, (int)binned.nnz, h->s_indptr + first_long,
-                                                       lo.first_block, lo.n_wide, lo.first_chunk);
-        long_blocks_kernel<<<dim3(grid_for((int64_t)lo.n * 64)), dim3(kThreads), 0, s>>>(
-            lo.sorted_deg, lo.n, first_long, h->s_indptr, lo.first_block, (int)binned.blocks, lo.n_wide, lo.first_chunk,
-            b4.as<int4>(), lo.chunk_row);
-    }
+    LongArgs la{};
+    la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
+    la.nz0 = (int)binned.nnz; la.block0 = (int)binned.blocks;
+    la.perm = h->perm; la.place = place; la.s_indptr = h->s_indptr;
+    la.block4 = b4.as<int4>();
+    la.first_chunk = h->first_chunk; la.chunk_row = h->chunk_row;
+    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, sums, sh, s))) return rc;
     if (given && !h->identity_perm)
         compare_order_kernel<<<dim3(grid_for(rows)), dim3(kThreads), 0, s>>>(
             reinterpret_cast<const uint32_t *>(h->perm), given->perm_dev, rows, mail);
