@@ -17,7 +17,7 @@ CSRC = PKG / "csrc"
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libaccelgcn.so"
 BIN_DIR = PKG / "bin"
-SOURCES = ["capi.hip", "preprocess.hip", "plan.hip", "spmm.hip", "state.hip", "dense.hip", "memory.hip", "spmm_accel.cpp"]
+SOURCES = ["capi.hip", "preprocess.hip", "plan.hip", "spmm.hip", "state.hip", "dense.hip", "memory.hip", "transfer.hip", "spmm_accel.cpp"]
 ARCH = "gfx950"
 
 
@@ -59,7 +59,7 @@ def build(verbose: bool = False) -> Path:
     if failed:
         raise RuntimeError("hipcc failed:\n" + "\n".join(f"--- {s}\n{o}" for s, o in failed))
     tmp = out.with_suffix(".so.tmp")
-    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", str(tmp)]
+    cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", *objs, "-o", str(tmp)]
     subprocess.run(cmd, check=True)
     os.replace(tmp, out)
     for o in objs:

@@ -891,27 +891,20 @@ int accel_partition_gpu(const int32_t *indptr, int64_t rows, int32_t *block4_out
     if (int rc = need_gpu()) return rc;
     *n_blocks = 0;
     if (rows == 0) return ACCEL_OK;
-    void *dptr = take_memory(sizeof(int32_t) * (size_t)(rows + 1), false);
+    const size_t bytes = sizeof(int32_t) * (size_t)(rows + 1);
+    void *dptr = take_memory(bytes, false);
     if (!dptr) {
         set_error("device allocation failed");
         return ACCEL_ERR_ALLOC;
     }
-    int rc = ACCEL_OK;
     int32_t *b4 = nullptr;
     int64_t nb = 0;
-    if (hipMemcpy(dptr, indptr, sizeof(int32_t) * (size_t)(rows + 1), hipMemcpyHostToDevice) != hipSuccess) {
-        set_error("upload of indptr failed");
-        rc = ACCEL_ERR_HIP;
-    }
+    int rc = upload(dptr, indptr, bytes, nullptr);
     if (!rc) rc = partition_only_device(static_cast<int32_t *>(dptr), rows, indptr[rows], &b4, &nb);
     if (!rc) {
         *n_blocks = nb;
         const int64_t take = std::min(nb, cap);
-        if (take > 0 &&
-            hipMemcpy(block4_out, b4, sizeof(int32_t) * 4 * (size_t)take, hipMemcpyDeviceToHost) != hipSuccess) {
-            set_error("download of the metadata failed");
-            rc = ACCEL_ERR_HIP;
-        }
+        if (take > 0) rc = download(block4_out, b4, sizeof(int32_t) * 4 * (size_t)take, nullptr);
     }
     give_memory(b4, false);
     give_memory(dptr, false);

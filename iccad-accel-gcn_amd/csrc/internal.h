@@ -165,6 +165,10 @@ namespace accel {
 void *take_memory(size_t bytes, bool any_stream);
 void give_memory(void *p, bool settled);
 void release_idle_memory();
+// transfer.hip: ordinary host memory to and from the device, queued on s; upload returns when src has
+// been read, download when dst has been written
+int upload(void *dst, const void *src, size_t bytes, hipStream_t s);
+int download(void *dst, const void *src, size_t bytes, hipStream_t s);
 // preprocess.hip
 struct SavedOrder {               // a degree-sort order read from a saved state
     bool identity;                // the rows were already in order: no permutation stored

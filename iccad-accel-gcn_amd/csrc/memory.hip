@@ -103,9 +103,7 @@ void expire(Pool &pl, std::vector<Idle> &gone)
     pl.idle.resize(keep);
 }
 
-}  // namespace
-
-void release_idle_memory()
+void release_idle_device_memory()
 {
     Pool &pl = pool();
     std::vector<Idle> gone;
@@ -115,6 +113,8 @@ void release_idle_memory()
     }
     free_idle(gone);
 }
+
+}  // namespace
 
 void *take_memory(size_t bytes, bool any_stream)
 {
@@ -148,7 +148,7 @@ void *take_memory(size_t bytes, bool any_stream)
     }
     if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
-        release_idle_memory();
+        release_idle_device_memory();
         if (hipMalloc(&p, want) != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;
@@ -182,14 +182,17 @@ void give_memory(void *p, bool settled)
 
 // Pinned blocks for the preprocessing's results, one per call that is under way; kept (a few KB
 // each, as many as calls have run at once).
-static std::mutex g_mail_mu;
+static std::mutex g_host_mu;
 static std::vector<Mail *> g_mail;
+// Pinned buffers for transfers: at most kIdleStages are kept (16 MiB each at most).
+constexpr size_t kIdleStages = 2;
+static std::vector<Stage *> g_stage;
 
 Mail *take_mail()
 {
     Mail *m = nullptr;
     {
-        std::lock_guard<std::mutex> lock(g_mail_mu);
+        std::lock_guard<std::mutex> lock(g_host_mu);
         if (!g_mail.empty()) {
             m = g_mail.back();
             g_mail.pop_back();
@@ -207,8 +210,78 @@ Mail *take_mail()
 void give_mail(Mail *m)
 {
     if (!m) return;
-    std::lock_guard<std::mutex> lock(g_mail_mu);
+    std::lock_guard<std::mutex> lock(g_host_mu);
     g_mail.push_back(m);
+}
+
+static void free_stage(Stage *s)
+{
+    if (s->busy) (void)hipEventSynchronize(s->last);
+    for (hipEvent_t e : s->event)
+        if (e) (void)hipEventDestroy(e);
+    if (s->last) (void)hipEventDestroy(s->last);
+    if (s->p) (void)hipHostFree(s->p);
+    (void)hipGetLastError();
+    delete s;
+}
+
+Stage *take_stage(size_t bytes)
+{
+    const size_t want = std::min(std::max(bytes, (size_t)1 << 20), kStageBytes);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    Stage *s = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_host_mu);
+        for (size_t i = g_stage.size(); i-- > 0 && !s;)
+            if (g_stage[i]->bytes >= want && g_stage[i]->device == dev) {
+                s = g_stage[i];
+                g_stage.erase(g_stage.begin() + (long)i);
+            }
+    }
+    if (s) {
+        if (s->busy && hipEventSynchronize(s->last) != hipSuccess) (void)hipGetLastError();
+        s->busy = false;
+        return s;
+    }
+    s = new Stage;
+    s->bytes = want;
+    s->device = dev;
+    bool ok = hipHostMalloc(&s->p, want, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t &e : s->event)
+        if (ok) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (ok) ok = hipEventCreateWithFlags(&s->last, hipEventDisableTiming) == hipSuccess;
+    if (ok) return s;
+    (void)hipGetLastError();
+    free_stage(s);
+    set_error("allocation of %zu bytes of pinned host memory failed", want);
+    return nullptr;
+}
+
+void give_stage(Stage *s)
+{
+    if (!s) return;
+    Stage *gone = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_host_mu);
+        g_stage.push_back(s);
+        if (g_stage.size() > kIdleStages) {
+            gone = g_stage.front();
+            g_stage.erase(g_stage.begin());
+        }
+    }
+    if (gone) free_stage(gone);
+}
+
+void release_idle_memory()
+{
+    release_idle_device_memory();
+    std::vector<Stage *> stages;
+    {
+        std::lock_guard<std::mutex> lock(g_host_mu);
+        stages.swap(g_stage);
+    }
+    for (Stage *s : stages) free_stage(s);
 }
 
 }  // namespace accel

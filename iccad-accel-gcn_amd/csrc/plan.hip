@@ -23,7 +23,7 @@
 //
 // Nothing here is sorted: the pass that placed the rows (place_rows in preprocess.hip) knows of
 // every row, in the caller's order, whether it starts a unit, so a scan of the counts per share
-// of rows puts the units in that order (list_units_kernel).  The pieces of a column group are
+// of rows puts the units in that order (list_units in preprocess.h).  The pieces of a column group are
 // ordered by a scan over (class of rows, group, row of the class).  What bounds all of it is
 // the number of dependent launches (2 to 5 us each), not bytes: five launches and no
 // synchronisation before the last, where there were 45 launches and two (110 of 440 us of
@@ -72,64 +72,6 @@ __device__ __forceinline__ int64_t plan_index(int queue, int pos, int n_queues)
 {
     // queue q, position p  ->  slot of wavefront (p % 4) in workgroup (p / 4) * n_queues + q
     return ((int64_t)(pos / kWavesPerGroup) * n_queues + queue) * kWavesPerGroup + pos % kWavesPerGroup;
-}
-
-// One wavefront per share of the caller's rows: writes the units of whole rows that start in
-// it, the running cost and the number of heavy units before each, and the rank of each split row
-// of 8 column groups among those rows, all in the caller's order.
-__global__ __launch_bounds__(kThreads) void list_units_kernel(
-    SortedRows sr, int share, int n_shares, const int *__restrict__ sums, int pitch, UnitRule rule, int first_split,
-    int4 *__restrict__ units, int *__restrict__ running, int *__restrict__ heavy_before, int *__restrict__ rank8)
-{
-    __shared__ int run_row[kBins + 1], run_nz[kBins];
-    for (int i = threadIdx.x; i <= kBins; i += kThreads) run_row[i] = sr.run_row[i];
-    for (int i = threadIdx.x; i < kBins; i += kThreads) run_nz[i] = sr.run_nz[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, c = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
-    if (c == 0 && lane == 0) {
-        const int n = sums[kSumUnits * pitch + n_shares];
-        running[n] = sums[kSumCost * pitch + n_shares];
-        heavy_before[n] = sums[kSumHeavy * pitch + n_shares];
-    }
-    if (c >= n_shares) return;
-    int n_units = sums[kSumUnits * pitch + c], cost0 = sums[kSumCost * pitch + c];
-    int heavy0 = sums[kSumHeavy * pitch + c], rows8 = sums[kSumRows8 * pitch + c];
-    const int64_t r_end = min(sr.rows, (int64_t)(c + 1) * share);
-    for (int64_t r0 = (int64_t)c * share; r0 < r_end; r0 += 64) {
-        const int64_t r = r0 + lane;
-        const bool ok = r < r_end;
-        const int d = ok ? sr.indptr[r + 1] - sr.indptr[r] : 0;
-        const int p = ok ? (int)sr.place[r] : 0;
-        int n = 0, in_run = 0;
-        if (d > 0 && d <= rule.split) {
-            in_run = p - run_row[d];
-            n = unit_rows(d, in_run, run_row[d + 1] - run_row[d], rule);
-        }
-        const int nz = d * n;
-        const int cost = n > 0 ? unit_cost(nz, n, rule.cost_shift) : 0;
-        const unsigned long long heads = __ballot(n > 0), heavies = __ballot(n > 0 && nz > rule.light_nz);
-        int inc = cost;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(inc, off);
-            if (lane >= off) inc += t;
-        }
-        if (n > 0) {
-            int w, rpb;
-            slice_rule(d, w, rpb);
-            const int at = n_units + lanes_below(heads, lane);
-            units[at] = make_int4(d, p, run_nz[d] + in_run * d, (w << 16) + n);
-            running[at] = cost0 + inc - cost;
-            heavy_before[at] = heavy0 + lanes_below(heavies, lane);
-        }
-        const bool is8 = d > rule.split && row_groups(d, rule.groups) == kXcds;
-        const unsigned long long eights = __ballot(is8);
-        if (is8) rank8[p - first_split] = rows8 + lanes_below(eights, lane);
-        n_units += __popcll(heads);
-        cost0 += __shfl(inc, 63);
-        heavy0 += __popcll(heavies);
-        rows8 += __popcll(eights);
-    }
 }
 
 // A split row's place in its class: rows of 8 groups follow the caller's row ids, the longer
@@ -402,9 +344,10 @@ int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups)
 }
 
 int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
-                    const int *share_sums, const int *gcount, const Mail *stats, int64_t n_short_units, int *zeroed,
-                    Mail *mail, hipStream_t s)
+                    const PlanUnits &pu, const int *gcount, int64_t n_short_units, int *zeroed, Mail *mail, hipStream_t s)
 {
+    const Mail *stats = mail;
+    const int *share_sums = pu.sums;
     // pieces of split rows hold up to piece_nz non-zeros, units of several whole rows up to unit_nz
     const int piece_nz = std::max(h->plan_unit, h->plan_split), forced = rule.groups;
     const int nq = h->plan_queues;                     // 8 interleaved queues, or 1 (plain order)
@@ -413,24 +356,19 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
     const ClassLayout cl = class_layout(n_split, stats, forced);
     const int pitch = sh.pitch + kWaves4;
     int rc;
-    int4 *units;
-    int *running, *heavy, *rank8 = nullptr, *row_units = nullptr, *bins = nullptr;
+    const int4 *units = pu.units;
+    const int *running = pu.running, *heavy = pu.heavy_before, *rank8 = pu.rank8;
+    int *row_units = nullptr, *bins = nullptr;
     PlanHead *head;
-    if ((rc = tmp->alloc(&units, (size_t)n_short_units))) return rc;
-    if ((rc = tmp->alloc(&running, (size_t)n_short_units + 1))) return rc;
-    if ((rc = tmp->alloc(&heavy, (size_t)n_short_units + 1))) return rc;
     if ((rc = tmp->alloc(&head, 1))) return rc;
     // the slots of each split row, and behind them one counter per split row (zero between launches)
     DevBuf dslot;
     if ((rc = dslot.alloc(sizeof(int) * (size_t)(2 * (int64_t)n_split + 1)))) return rc;
     int *slot = dslot.as<int>(), *row_done = slot + n_split + 1;
     if (n_split > 0) {
-        if ((rc = tmp->alloc(&rank8, (size_t)n_split))) return rc;
         if ((rc = tmp->alloc(&row_units, (size_t)n_split))) return rc;
         if ((rc = tmp->alloc(&bins, (size_t)cl.total + 1))) return rc;
     }
-    list_units_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(sr, sh.share, sh.n, share_sums, pitch, rule,
-                                                                  (int)first_split, units, running, heavy, rank8);
     if (n_split > 0) {
         // (each workgroup ends on eight atomics to the same eight words)
         const unsigned groups = std::min(grid_for((int64_t)n_split * 64), 1024u);

@@ -52,6 +52,25 @@ struct MailHolder {
     MailHolder &operator=(const MailHolder &) = delete;
 };
 
+// Pinned memory that transfers go through (transfer.hip), with events for its pieces.
+constexpr size_t kStageBytes = (size_t)16 << 20, kStagePiece = (size_t)2 << 20;
+struct Stage {
+    void *p = nullptr;
+    size_t bytes = 0;
+    hipEvent_t event[kStageBytes / kStagePiece] = {}, last = nullptr;
+    int device = 0;
+    bool busy = false;            // `last` stands behind the last copy out of it
+};
+Stage *take_stage(size_t bytes);      // memory.hip: min(bytes, kStageBytes) or more; null when there is none
+void give_stage(Stage *s);
+struct StageHolder {
+    Stage *s;
+    explicit StageHolder(size_t bytes) : s(take_stage(bytes)) {}
+    ~StageHolder() { give_stage(s); }
+    StageHolder(const StageHolder &) = delete;
+    StageHolder &operator=(const StageHolder &) = delete;
+};
+
 // Temporaries of one preprocessing call come out of a few large pieces of device memory (there
 // are some twenty of them).  The pieces are given back when the arena goes out of scope; what
 // is still queued then is queued on the null stream.
@@ -339,10 +358,79 @@ struct SortedRows {
     const int *run_nz = nullptr;              // [kBins] first non-zero of each bin
 };
 
+// The units of whole rows in the caller's order, and what the plan needs to know of them.
+struct PlanUnits {
+    int *sums = nullptr;                      // [kSums][pitch + kWaves4], scanned
+    int4 *units = nullptr;
+    int *running = nullptr;                   // [n + 1] cost of the units before each
+    int *heavy_before = nullptr;              // [n + 1] units before each that are not light
+    int *rank8 = nullptr;                     // split row of 8 column groups -> its rank among them in the caller's order
+};
+
+// A wavefront writes the units of whole rows that start in share c of the caller's rows, the running
+// cost and the number of heavy units before each, and the rank of each split row of 8 column groups
+// among those rows, all in the caller's order.
+__device__ __forceinline__ void list_units(const SortedRows &sr, const UnitRule &rule, const PlanUnits &pu, int share,
+                                           int n_shares, int pitch, int first_split, const int *run_row /* LDS */,
+                                           const int *run_nz /* LDS */, int c)
+{
+    const int lane = threadIdx.x & 63;
+    if (c == 0 && lane == 0) {
+        const int n = pu.sums[kSumUnits * pitch + n_shares];
+        pu.running[n] = pu.sums[kSumCost * pitch + n_shares];
+        pu.heavy_before[n] = pu.sums[kSumHeavy * pitch + n_shares];
+    }
+    if (c >= n_shares) return;
+    int n_units = pu.sums[kSumUnits * pitch + c], cost0 = pu.sums[kSumCost * pitch + c];
+    int heavy0 = pu.sums[kSumHeavy * pitch + c], rows8 = pu.sums[kSumRows8 * pitch + c];
+    const int64_t r_end = min(sr.rows, (int64_t)(c + 1) * share);
+    for (int64_t r1 = (int64_t)c * share; r1 < r_end; r1 += 4 * 64) {
+        int deg[4], plc[4];                              // four rounds' rows are on their way at once
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t r = r1 + j * 64 + lane;
+            deg[j] = r < r_end ? sr.indptr[r + 1] - sr.indptr[r] : 0;
+            plc[j] = r < r_end ? (int)sr.place[r] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int d = deg[j], p = plc[j];
+            int n = 0, in_run = 0;
+            if (d > 0 && d <= rule.split) {
+                in_run = p - run_row[d];
+                n = unit_rows(d, in_run, run_row[d + 1] - run_row[d], rule);
+            }
+            const int nz = d * n;
+            const int cost = n > 0 ? unit_cost(nz, n, rule.cost_shift) : 0;
+            const unsigned long long heads = __ballot(n > 0), heavies = __ballot(n > 0 && nz > rule.light_nz);
+            int inc = cost;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int t = __shfl_up(inc, off);
+                if (lane >= off) inc += t;
+            }
+            if (n > 0) {
+                int w, rpb;
+                slice_rule(d, w, rpb);
+                const int at = n_units + lanes_below(heads, lane);
+                pu.units[at] = make_int4(d, p, run_nz[d] + in_run * d, (w << 16) + n);
+                pu.running[at] = cost0 + inc - cost;
+                pu.heavy_before[at] = heavy0 + lanes_below(heavies, lane);
+            }
+            const bool is8 = d > rule.split && row_groups(d, rule.groups) == kXcds;
+            const unsigned long long eights = __ballot(is8);
+            if (is8) pu.rank8[p - first_split] = rows8 + lanes_below(eights, lane);
+            n_units += __popcll(heads);
+            cost0 += __shfl(inc, 63);
+            heavy0 += __popcll(heavies);
+            rows8 += __popcll(eights);
+        }
+    }
+}
+
 // plan.hip
 int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
-                    const int *share_sums, const int *gcount, const Mail *stats, int64_t n_short_units, int *zeroed,
-                    Mail *mail, hipStream_t s);
+                    const PlanUnits &pu, const int *gcount, int64_t n_short_units, int *zeroed, Mail *mail, hipStream_t s);
 // ints that must be zero when build_work_list is called (place_rows clears them)
 int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups);
 

@@ -61,54 +61,61 @@ __global__ __launch_bounds__(kThreads) void degree_kernel(DegreeArgs a, int *__r
 #pragma unroll
     for (int k = 0; k < kStatCount; k++) st[k] = 0;
     const int64_t r_end = min(a.rows, (int64_t)(c + 1) * a.share);
-    const int64_t r_first = (int64_t)c * a.share + lane;
-    int lo_next = r_first < r_end ? a.indptr[r_first] : 0, hi_next = r_first < r_end ? a.indptr[r_first + 1] : 0;
-    for (int64_t r0 = (int64_t)c * a.share; r0 < r_end; r0 += 64) {
-        const int64_t r = r0 + lane;
-        const bool ok = r < r_end;
-        const int lo = lo_next, hi = hi_next;                // the next round's are on their way
-        if (r + 64 < r_end) {
-            lo_next = a.indptr[r + 64];
-            hi_next = a.indptr[r + 65];
-        } else {
-            lo_next = hi_next = 0;
+    for (int64_t r1 = (int64_t)c * a.share; r1 < r_end; r1 += 4 * 64) {
+        int los[4], his[4], befores[4];                      // four rounds' rows are on their way at once
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t r = r1 + j * 64 + lane;
+            los[j] = r < r_end ? a.indptr[r] : 0;
+            his[j] = r < r_end ? a.indptr[r + 1] : 0;
+            befores[j] = r < r_end && r > 0 && lane == 0 ? a.indptr[r - 1] : 0;
         }
-        int before = __shfl_up(lo, 1);
-        if (lane == 0) before = r > 0 ? a.indptr[r - 1] : lo;
-        int d = hi - lo;
-        bool bad = false;
-        if (ok) {
-            bad = hi < lo || (r == 0 && lo != 0) || (r == a.rows - 1 && (int64_t)hi != a.nnz);
-            if (hi < lo) d = 0;
-            if (r > 0 && d < lo - before) st[kStatUnsorted] = 1;
-            st[kStatBadIndptr] |= bad;
-            st[kStatMaxDegree] = max(st[kStatMaxDegree], d);
-            if (d > kDegBound) st[kStatLongBlocks] += (d + kDegBound - 1) / kDegBound;
-            if (d > kWideRow) {
-                st[kStatWideRows]++;
-                st[kStatWideChunks] += (d + kWideChunk - 1) / kWideChunk;
-                const int ng = row_groups(d, 0);
-                st[kStatRows16] += ng == 16;
-                st[kStatRows32] += ng == 32;
-                st[kStatRows64] += ng == 64;
+        int sample[4];                                       // position of this lane's sampled non-zero, or -1
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t r = r1 + j * 64 + lane;
+            const bool ok = r < r_end;
+            const int lo = los[j], hi = his[j];
+            int before = __shfl_up(lo, 1);
+            if (lane == 0) before = befores[j];
+            int d = hi - lo;
+            if (ok) {
+                const bool bad = hi < lo || (r == 0 && lo != 0) || (r == a.rows - 1 && (int64_t)hi != a.nnz);
+                if (hi < lo) d = 0;
+                if (r > 0 && d < lo - before) st[kStatUnsorted] = 1;
+                st[kStatBadIndptr] |= bad;
+                st[kStatMaxDegree] = max(st[kStatMaxDegree], d);
+                if (d > kDegBound) st[kStatLongBlocks] += (d + kDegBound - 1) / kDegBound;
+                if (d > kWideRow) {
+                    st[kStatWideRows]++;
+                    st[kStatWideChunks] += (d + kWideChunk - 1) / kWideChunk;
+                    const int ng = row_groups(d, 0);
+                    st[kStatRows16] += ng == 16;
+                    st[kStatRows32] += ng == 32;
+                    st[kStatRows64] += ng == 64;
+                }
+                st[kStatBig] += d > 32 * a.split;
+                st[kStatBigAlt] += d > 32 * a.alt_split;
+                atomicAdd(&cnt[w][min(d, kLongBin)], 1);
             }
-            st[kStatBig] += d > 32 * a.split;
-            st[kStatBigAlt] += d > 32 * a.alt_split;
-            atomicAdd(&cnt[w][min(d, kLongBin)], 1);
-        }
-        if (a.idx) {
-            // four of the 64 rows are sampled, by 16 lanes each
+            // four of the 64 rows are sampled, by 16 lanes each, spread over the row whatever its order
             const int from = lane / kLocalitySample * kLocalityStride, i = lane % kLocalitySample;
             const int ra = __shfl(lo, from);
             int rd = __shfl(ok ? hi - lo : 0, from);
             if (ra < 0 || rd < 0 || (int64_t)ra + rd > a.nnz) rd = 0;
             const int n = min(rd, kLocalitySample);
-            if (i < n) {                                 // spread over the row, whatever its order
-                const int64_t place = a.rows > 1 ? (r0 + from) * (a.cols - 1) / (a.rows - 1) : 0;
-                const int64_t off = (int64_t)a.idx[ra + (int)((int64_t)i * rd / n)] - place;
-                st[kStatSampled]++;
-                st[kStatLocal] += (off < 0 ? -off : off) <= a.band;
-            }
+            sample[j] = a.idx && i < n ? ra + (int)((int64_t)i * rd / n) : -1;
+        }
+        int col[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) col[j] = sample[j] >= 0 ? a.idx[sample[j]] : 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (sample[j] < 0) continue;
+            const int64_t r = r1 + j * 64 + lane / kLocalitySample * kLocalityStride;
+            const int64_t off = (int64_t)col[j] - (a.rows > 1 ? r * (a.cols - 1) / (a.rows - 1) : 0);
+            st[kStatSampled]++;
+            st[kStatLocal] += (off < 0 ? -off : off) <= a.band;
         }
     }
     static_assert(kLocalityStride == 16 && kLocalitySample == 16, "the lanes of a round are dealt out for these");
@@ -221,6 +228,22 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
     __shared__ int next[kWaves4][kBins];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     static_assert(kBins <= 2 * kThreads, "two bins per thread");
+    // this wavefront's counters and its first rows are on their way while the tables are made
+    const int c = (int)blockIdx.x * kWaves4 + w;
+    const int64_t r_end = c < a.n_shares ? min(a.rows, (int64_t)(c + 1) * a.share) : 0;
+    constexpr int kCounters = (kBins + 63) / 64;
+    int before[kCounters], deg[4];
+#pragma unroll
+    for (int j = 0; j < kCounters; j++)
+        before[j] = c < a.n_shares && j * 64 + lane < kBins ? a.bins[(int64_t)(j * 64 + lane) * a.pitch + c] : 0;
+    auto load_rows = [&](int64_t r1) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t r = r1 + j * 64 + lane;
+            deg[j] = r < r_end ? a.indptr[r + 1] - a.indptr[r] : 0;
+        }
+    };
+    load_rows((int64_t)c * a.share);
     {
         int cnt[2], nz[2], blk[2], t;
 #pragma unroll
@@ -280,43 +303,47 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
     if (a.s_indptr && me == 0) a.s_indptr[a.rows] = a.indptr[a.rows];
 
     // the rows of this wavefront's share
-    const int c = (int)blockIdx.x * kWaves4 + w;
     if (c >= a.n_shares) return;
-    for (int b = lane; b < kBins; b += 64) next[w][b] = run_row[b] + a.bins[(int64_t)b * a.pitch + c];
+#pragma unroll
+    for (int j = 0; j < kCounters; j++)
+        if (j * 64 + lane < kBins) next[w][j * 64 + lane] = run_row[j * 64 + lane] + before[j];
     __builtin_amdgcn_wave_barrier();
     int n_units = 0, cost = 0, n_heavy = 0, n_rows8 = 0;
-    const int64_t r_end = min(a.rows, (int64_t)(c + 1) * a.share);
-    const int64_t r_first = (int64_t)c * a.share + lane;
-    int d_next = r_first < r_end ? a.indptr[r_first + 1] - a.indptr[r_first] : 0;
-    for (int64_t r0 = (int64_t)c * a.share; r0 < r_end; r0 += 64) {
-        const int64_t r = r0 + lane;
-        const bool ok = r < r_end;
-        const int d = d_next;                                // the next round's is on its way
-        d_next = r + 64 < r_end ? a.indptr[r + 65] - a.indptr[r + 64] : 0;
-        const int bin = min(d, kLongBin);
-        const unsigned long long peers = wave_match(bin, 9, ok);
-        const int rank = lanes_below(peers, lane);
-        const int p = next[w][bin] + rank;
-        __builtin_amdgcn_wave_barrier();
-        if (ok && rank == 0) next[w][bin] = p + __popcll(peers);
-        __builtin_amdgcn_wave_barrier();
-        if (ok) {
-            if (d > kDegBound) {
-                a.long_deg[p - n_binned] = d;
-                a.long_row[p - n_binned] = (uint32_t)r;
-            } else {
-                if (a.perm) a.perm[p] = (int32_t)r;
-                if (a.place) a.place[r] = (uint32_t)p;
-            }
-            if (d > 0 && d <= a.rule.split) {
-                const int n = unit_rows(d, p - run_row[d], run_row[d + 1] - run_row[d], a.rule);
-                if (n > 0) {
-                    n_units++;
-                    cost += unit_cost(d * n, n, a.rule.cost_shift);
-                    n_heavy += d * n > a.rule.light_nz;
+    for (int64_t r1 = (int64_t)c * a.share; r1 < r_end; r1 += 4 * 64) {
+        int d4[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) d4[j] = deg[j];
+        load_rows(r1 + 4 * 64);                                // the next four rounds' rows
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t r = r1 + j * 64 + lane;
+            const bool ok = r < r_end;
+            const int d = d4[j];
+            const int bin = min(d, kLongBin);
+            const unsigned long long peers = wave_match(bin, 9, ok);
+            const int rank = lanes_below(peers, lane);
+            const int p = next[w][bin] + rank;
+            __builtin_amdgcn_wave_barrier();
+            if (ok && rank == 0) next[w][bin] = p + __popcll(peers);
+            __builtin_amdgcn_wave_barrier();
+            if (ok) {
+                if (d > kDegBound) {
+                    a.long_deg[p - n_binned] = d;
+                    a.long_row[p - n_binned] = (uint32_t)r;
+                } else {
+                    if (a.perm) a.perm[p] = (int32_t)r;
+                    if (a.place) a.place[r] = (uint32_t)p;
                 }
+                if (d > 0 && d <= a.rule.split) {
+                    const int n = unit_rows(d, p - run_row[d], run_row[d + 1] - run_row[d], a.rule);
+                    if (n > 0) {
+                        n_units++;
+                        cost += unit_cost(d * n, n, a.rule.cost_shift);
+                        n_heavy += d * n > a.rule.light_nz;
+                    }
+                }
+                if (d > a.rule.split) n_rows8 += row_groups(d, a.rule.groups) == kXcds;
             }
-            if (d > a.rule.split) n_rows8 += row_groups(d, a.rule.groups) == kXcds;
         }
     }
     if (!a.sums) return;
@@ -334,14 +361,14 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Rows of more than 384 non-zeros: ranked by (degree, row).  Up to kFewLong of them one workgroup
-// does everything (ranks by comparing each with all, scans, blocks) in one launch, 8 us at 800
-// rows; up to kRankMax they are ranked the same way by many workgroups (8,192 rows: 10 us), more
-// by a stable radix sort, 8 bits a pass, and the rest is scans.
+// Rows of more than 384 non-zeros: ranked by (degree, row), up to kRankMax of them by comparing each
+// with all (rank_long_rows_kernel; one workgroup for 800 rows takes 18 us, thirteen 5), more by a
+// stable radix sort, 8 bits a pass.  Their scans and blocks are one workgroup's work up to kFewLong
+// rows, launches of their own beyond.
 // ---------------------------------------------------------------------------
 constexpr int kFewLong = 2048;
 constexpr int kRankMax = 8192;
-constexpr int kRankRows = 64;                 // rows ranked by a workgroup, by four threads each
+constexpr int kRankRows = 64;                 // rows ranked by sixteen wavefronts, each against a sixteenth
 
 // How many of the n4 * 4 degrees at `tile` (LDS), the first of which is long row `at0`, rank before
 // long row j of degree d.  Equal degrees rank by row, which is the order they are listed in.
@@ -357,26 +384,35 @@ __device__ __forceinline__ int count_before(const int4 *tile, int n4, int at0, i
     return below;
 }
 
-__global__ __launch_bounds__(kThreads) void rank_long_rows_kernel(
+// The first kSums workgroups scan one kind each of the counts per share (sums, null: none), which has
+// nothing to do with the rest but that both come behind place_rows; the others rank the long rows.
+__global__ __launch_bounds__(1024) void rank_long_rows_kernel(
     const int *__restrict__ deg, const uint32_t *__restrict__ row, int n, int64_t first_long,
-    int32_t *__restrict__ perm, uint32_t *__restrict__ place, int *__restrict__ sorted_deg)
+    int32_t *__restrict__ perm, uint32_t *__restrict__ place, int *__restrict__ sorted_deg, int *__restrict__ sums,
+    int sum_pitch, int n_shares)
 {
-    __shared__ __attribute__((aligned(16))) int tile[kThreads * 4];
-    __shared__ int part[4][kRankRows];
-    const int j = (int)blockIdx.x * kRankRows + (threadIdx.x & 63), seg = threadIdx.x >> 6;
-    const int d = j < n ? deg[j] : 0;
-    int below = 0;
-    for (int t0 = 0; t0 < n; t0 += kThreads * 4) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < kThreads * 4; i += kThreads) tile[i] = t0 + i < n ? deg[t0 + i] : INT_MAX;
-        __syncthreads();
-        below += count_before(reinterpret_cast<const int4 *>(tile + seg * kThreads), kThreads / 4, t0 + seg * kThreads, d, j);
+    __shared__ __attribute__((aligned(16))) int tile[4096];
+    __shared__ int part[16][kRankRows];
+    int b = blockIdx.x;
+    if (sums) {
+        if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, tile); return; }
+        b -= kSums;
     }
-    part[seg][threadIdx.x & 63] = below;
+    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
+    const int d = j < n ? deg[j] : 0;
+    const uint32_t r = j < n ? row[j] : 0;
+    int below = 0;
+    for (int t0 = 0; t0 < n; t0 += 4096) {
+        const int here = min(4096, n - t0), per = (here + 63) / 64;       // vectors of four per wavefront
+        __syncthreads();
+        for (int i = threadIdx.x; i < per * 64; i += 1024) tile[i] = i < here ? deg[t0 + i] : INT_MAX;
+        __syncthreads();
+        below += count_before(reinterpret_cast<const int4 *>(tile) + seg * per, per, t0 + seg * per * 4, d, j);
+    }
+    part[seg][lane] = below;
     __syncthreads();
     if (seg == 0 && j < n) {
-        for (int q = 1; q < 4; q++) below += part[q][threadIdx.x];
-        const uint32_t r = row[j];
+        for (int q = 1; q < 16; q++) below += part[q][lane];
         const int64_t p = first_long + below;
         if (perm) perm[p] = (int32_t)r;
         if (place) place[r] = (uint32_t)p;
@@ -400,29 +436,33 @@ struct LongArgs {
     int *first_chunk, *chunk_row;             // of long row i (null: none is wide)
 };
 
-// Workgroup 0: the long rows, when there are few.  The others: one kind each of the counts per share
-// (kSum*), whose scan the launch plan needs and which have nothing to do with it but the launch.
-__global__ __launch_bounds__(1024) void few_long_rows_kernel(LongArgs a, int *__restrict__ sums, int sum_pitch,
-                                                             int n_shares)
+// The units of whole rows, for which everything is known by then.
+struct UnitsArgs {
+    SortedRows sr;
+    UnitRule rule;
+    PlanUnits pu;
+    int share, n_shares, pitch, first_split;
+    int groups;                               // workgroups, 0: not wanted
+};
+
+// Workgroup 0: row pointers, blocks and chunks of the long rows, when there are few.  The others: the
+// units of whole rows, a share of rows per wavefront.
+__global__ __launch_bounds__(1024) void few_long_rows_kernel(LongArgs a, const int *__restrict__ sorted_deg, UnitsArgs u)
 {
     __shared__ int lds[16];
+    __shared__ int sorted[kFewLong], first_block[kFewLong], loc[kFewLong];
+    const int t = threadIdx.x;
     if (blockIdx.x > 0) {
-        scan_shares(sums + (int64_t)(blockIdx.x - 1) * sum_pitch, n_shares, lds);
+        static_assert(kFewLong >= kBins + 1, "the runs' tables fit");
+        for (int i = t; i <= kBins; i += 1024) sorted[i] = u.sr.run_row[i];
+        for (int i = t; i < kBins; i += 1024) loc[i] = u.sr.run_nz[i];
+        __syncthreads();
+        list_units(u.sr, u.rule, u.pu, u.share, u.n_shares, u.pitch, u.first_split, sorted, loc,
+                   ((int)blockIdx.x - 1) * 16 + (t >> 6));
         return;
     }
     if (a.n == 0) return;
-    __shared__ __attribute__((aligned(16))) int deg[kFewLong];
-    __shared__ int sorted[kFewLong], first_block[kFewLong], loc[kFewLong];
-    const int t = threadIdx.x, n4 = (a.n + 3) / 4;
-    for (int i = t; i < n4 * 4; i += 1024) deg[i] = i < a.n ? a.deg[i] : INT_MAX;
-    __syncthreads();
-    for (int j = t; j < a.n; j += 1024) {
-        const int d = deg[j], below = count_before(reinterpret_cast<const int4 *>(deg), n4, 0, d, j);
-        sorted[below] = d;
-        const uint32_t r = a.row[j];
-        if (a.perm) a.perm[a.first_long + below] = (int32_t)r;
-        if (a.place) a.place[r] = (uint32_t)(a.first_long + below);
-    }
+    for (int i = t; i < a.n; i += 1024) sorted[i] = sorted_deg[i];
     __syncthreads();
     {
         const int i = 2 * t, d0 = i < a.n ? sorted[i] : 0, d1 = i + 1 < a.n ? sorted[i + 1] : 0;
@@ -568,15 +608,10 @@ __global__ __launch_bounds__(1024) void small_scan_kernel(int *__restrict__ v, i
     }
 }
 
-// Ranks the n long rows (perm, place and the degrees in sorted order).
+// Sorts many long rows (perm, place and the degrees in sorted order).
 int sort_long_rows(Arena *tmp, const int *deg, const uint32_t *row, int n, int max_degree, int64_t first_long,
                    int32_t *perm, uint32_t *place, int *sorted_deg, hipStream_t s)
 {
-    if (n <= kRankMax) {
-        rank_long_rows_kernel<<<dim3((unsigned)((n + kRankRows - 1) / kRankRows)), dim3(kThreads), 0, s>>>(
-            deg, row, n, first_long, perm, place, sorted_deg);
-        return ACCEL_OK;
-    }
     uint32_t *keys[2], *vals[2];
     int *hist, rc;
     const int64_t tiles = ((int64_t)n + kTile - 1) / kTile;
@@ -618,24 +653,27 @@ __global__ __launch_bounds__(kThreads) void long_blocks_kernel(LongArgs a, const
 // Ints that must be zero for place_long_rows (place_rows clears them).
 int64_t long_zeroed_ints(int64_t n) { return n > kFewLong ? 3 * scan_zeroed(n) : 0; }
 
-// The long rows' places, row pointers, blocks and chunks, and the scan of the counts per share (sums,
-// may be null).  in_order: the rows are sorted already, so they are listed in sorted order.
+// The long rows' places, row pointers, blocks and chunks, and the units of whole rows (u.groups > 0).
+// in_order: the rows are sorted already, so they are listed in sorted order.
 int place_long_rows(Arena *tmp, const LongArgs &a, bool in_order, int max_degree, const int32_t *loc_of, int *zeroed,
-                    int *sums, const Shares &sh, hipStream_t s)
+                    const UnitsArgs &u, hipStream_t s)
 {
-    const bool few = a.n <= kFewLong;
-    if (few || sums) {
-        LongArgs la = a;
-        if (!few) la.n = 0;
-        few_long_rows_kernel<<<dim3(1 + (sums ? kSums : 0)), dim3(1024), 0, s>>>(la, sums, sh.pitch + kWaves4, sh.n);
-    }
-    if (few) return ACCEL_OK;
     int rc, *sorted_deg = const_cast<int *>(a.deg), *blocks, *chunks = nullptr;
-    if (!in_order) {
-        if ((rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
-        if ((rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
-            return rc;
-    }
+    int *sums = u.groups ? u.pu.sums : nullptr;
+    const int ranked = !in_order && a.n <= kRankMax ? a.n : 0;
+    if (!in_order && (rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
+    if (sums || ranked > 0)
+        rank_long_rows_kernel<<<dim3((unsigned)((sums ? kSums : 0) + (ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0,
+                                s>>>(a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, u.pitch,
+                                     u.n_shares);
+    if (!in_order && a.n > kRankMax &&
+        (rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
+        return rc;
+    LongArgs few = a;
+    if (a.n > kFewLong) few.n = 0;
+    if (few.n > 0 || u.groups > 0)
+        few_long_rows_kernel<<<dim3(1u + (unsigned)u.groups), dim3(1024), 0, s>>>(few, sorted_deg, u);
+    if (a.n <= kFewLong) return ACCEL_OK;
     if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
     if (a.first_chunk && (rc = tmp->alloc(&chunks, (size_t)a.n))) return rc;
     long_sizes_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(sorted_deg, a.n, blocks, chunks);
@@ -964,11 +1002,13 @@ __global__ __launch_bounds__(kThreads) void wide_scan_kernel(CopyArgs a, WideArg
     }
 }
 
-__global__ __launch_bounds__(kThreads) void wide_place_kernel(CopyArgs a, WideArgs wa)
+constexpr int kPlaceThreads = 1024;
+__global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, WideArgs wa)
 {
-    constexpr int R = kWideChunk / kThreads;             // rounds of a wavefront, which takes a quarter of the chunk
+    constexpr int kWaves = kPlaceThreads / 64;
+    constexpr int R = kWideChunk / kPlaceThreads;        // rounds of a wavefront, which takes a sixteenth of the chunk
     __shared__ int2 buf[kWideChunk];
-    __shared__ int at[kWaves4][kMaxGroups], off[kMaxGroups];
+    __shared__ int at[kWaves][kMaxGroups], off[kMaxGroups];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const WideChunk ch = wide_chunk(a, wa, (int)blockIdx.x);
     const int bits = 31 - __clz(ch.ng);
@@ -989,8 +1029,9 @@ __global__ __launch_bounds__(kThreads) void wide_place_kernel(CopyArgs a, WideAr
         if ((w * R + j) * 64 + lane < ch.n) atomicAdd(&at[w][col_group(col[j], ch.ng)], 1);
     __syncthreads();
     if (w == 0) {
-        int v[kWaves4], total = 0;
-        for (int q = 0; q < kWaves4; q++) { v[q] = at[q][lane]; total += v[q]; }
+        int v[kWaves], total = 0;
+#pragma unroll
+        for (int q = 0; q < kWaves; q++) { v[q] = at[q][lane]; total += v[q]; }
         int inc = total;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -999,7 +1040,8 @@ __global__ __launch_bounds__(kThreads) void wide_place_kernel(CopyArgs a, WideAr
         }
         int run = inc - total;                           // where the chunk's group `lane` starts in LDS
         off[lane] = wa.chunk_count[(int64_t)blockIdx.x * kMaxGroups + lane] - run;
-        for (int q = 0; q < kWaves4; q++) { at[q][lane] = run; run += v[q]; }
+#pragma unroll
+        for (int q = 0; q < kWaves; q++) { at[q][lane] = run; run += v[q]; }
     }
     __syncthreads();
 #pragma unroll
@@ -1018,7 +1060,7 @@ __global__ __launch_bounds__(kThreads) void wide_place_kernel(CopyArgs a, WideAr
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < ch.n; e += kThreads) {
+    for (int e = threadIdx.x; e < ch.n; e += kPlaceThreads) {
         const int2 v = buf[e];
         const int64_t to = (int64_t)off[col_group(v.x, ch.ng)] + e;
         if (a.idx_out) a.idx_out[to] = v.x;
@@ -1348,7 +1390,7 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
         la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
         la.nz0 = (int)rt.nnz; la.block0 = (int)rt.blocks;
         la.block4 = b4.as<int4>();
-        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, nullptr, sh, s))) return rc;
+        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, UnitsArgs{}, s))) return rc;
     }
     ACCEL_HIP(hipGetLastError());
     *block4_dev = static_cast<int32_t *>(b4.release());
@@ -1426,7 +1468,7 @@ static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, i
     if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp);
     if (n_wide > 0) {
         wide_scan_kernel<<<dim3((unsigned)n_wide), dim3(kThreads), 0, s>>>(a, wa, n_split - n_wide, counts);
-        wide_place_kernel<<<dim3((unsigned)h->n_chunks), dim3(kThreads), 0, s>>>(a, wa);
+        wide_place_kernel<<<dim3((unsigned)h->n_chunks), dim3(kPlaceThreads), 0, s>>>(a, wa);
     }
     ACCEL_HIP(hipGetLastError());
     return ACCEL_OK;
@@ -1619,9 +1661,14 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
                      (size_t)plan_zeroed * kScanTile / 2 * 4 + (size_t)h->n_chunks * 260 + (size_t)whole.units * 24 +
                      (1 << 16);
     uint32_t *place, *long_row;
-    int *sums, *zeroed, *long_deg, *gcount = nullptr;
+    int *zeroed, *long_deg, *gcount = nullptr;
+    PlanUnits pu;
     if ((rc = tmp.alloc(&place, (size_t)rows))) return rc;
-    if ((rc = tmp.alloc(&sums, (size_t)kSums * (sh.pitch + kWaves4)))) return rc;
+    if ((rc = tmp.alloc(&pu.sums, (size_t)kSums * (sh.pitch + kWaves4)))) return rc;
+    if ((rc = tmp.alloc(&pu.units, (size_t)whole.units))) return rc;
+    if ((rc = tmp.alloc(&pu.running, (size_t)whole.units + 1))) return rc;
+    if ((rc = tmp.alloc(&pu.heavy_before, (size_t)whole.units + 1))) return rc;
+    if (n_split > 0 && (rc = tmp.alloc(&pu.rank8, (size_t)n_split))) return rc;
     if ((rc = tmp.alloc(&zeroed, (size_t)n_zeroed))) return rc;
     if ((rc = tmp.alloc(&long_deg, (size_t)n_long))) return rc;
     if ((rc = tmp.alloc(&long_row, (size_t)n_long))) return rc;
@@ -1660,7 +1707,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     pa.block4 = b4.as<int4>();
     pa.run_row = h->runs; pa.run_nz = h->runs + kBins + 1;
     pa.long_deg = long_deg; pa.long_row = long_row;
-    pa.sums = sums; pa.zero = zeroed; pa.n_zero = n_zeroed;
+    pa.sums = pu.sums; pa.zero = zeroed; pa.n_zero = n_zeroed;
     place_rows_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(pa);
     LongArgs la{};
     la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
@@ -1668,7 +1715,13 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     la.perm = h->perm; la.place = place; la.s_indptr = h->s_indptr;
     la.block4 = b4.as<int4>();
     la.first_chunk = h->first_chunk; la.chunk_row = h->chunk_row;
-    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, sums, sh, s))) return rc;
+    UnitsArgs ua{};
+    ua.sr = sorted_rows(h);
+    ua.sr.place = place;
+    ua.rule = rule; ua.pu = pu;
+    ua.share = sh.share; ua.n_shares = sh.n; ua.pitch = sh.pitch + kWaves4; ua.first_split = (int)(rows - n_split);
+    ua.groups = (sh.n + 15) / 16;
+    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, ua, s))) return rc;
     if (given && !h->identity_perm)
         compare_order_kernel<<<dim3(grid_for(rows)), dim3(kThreads), 0, s>>>(
             reinterpret_cast<const uint32_t *>(h->perm), given->perm_dev, rows, mail);
@@ -1686,9 +1739,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
 
     // ---- work list (ends on the second synchronisation) -----------------------------------
     h->nnz_short = whole.nnz;
-    SortedRows sr = sorted_rows(h);
-    sr.place = place;
-    if ((rc = build_work_list(&tmp, h, sr, rule, sh, sums, gcount, mail, whole.units, zeroed, mail, s))) return rc;
+    if ((rc = build_work_list(&tmp, h, ua.sr, rule, sh, pu, gcount, whole.units, zeroed, mail, s))) return rc;
     if (mail->bad_index) {
         set_error("a column index lies outside [0, cols)");
         return ACCEL_ERR_CSR;

@@ -97,3 +97,15 @@ def test_memory_is_kept_for_the_next_handle_and_given_back(gpu):
                     np.ones((60_000, 8), np.float32)) <= so.TOL
     dX.close()
     dY.close()
+
+
+@pytest.mark.parametrize("rows", [524_287, 524_288, 4_194_303, 4_300_000])
+def test_partition_stage_at_the_transfers_pieces(gpu, rows):
+    """Row pointers that end at a piece of the transfer buffer (2 MiB), at the buffer itself
+    (16 MiB) and beyond; the metadata of the last is longer than the buffer too."""
+    deg = np.sort(np.random.default_rng(rows).integers(0, 40, rows))
+    deg[-3:] = (400, 5000, 384 * 7)
+    deg.sort()
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    got = gpu.block_level_partition.partition(indptr, backend="gpu")
+    assert np.array_equal(got, gpu.block_level_partition.partition(indptr, backend="host"))
