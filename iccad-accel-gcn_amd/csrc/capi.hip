@@ -27,7 +27,7 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
                           int32_t **block4_dev, int64_t *n_blocks);
 bool stream_is_capturing(hipStream_t s);
 int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int K, int N, int64_t ldx, int64_t ldz,
-                    hipStream_t stream);      // dense.hip
+                    hipStream_t stream, bool may_prepare);      // dense.hip
 
 // Work that is queued on the null stream alone orders itself before whoever takes the memory
 // next (memory.hip); for a handle that other streams, or graphs, have used, the device is
@@ -1047,7 +1047,8 @@ int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32
     if (rows == 0) return ACCEL_OK;
     if (!X || !W || !Z) { set_error("%s: null operand", fn); return ACCEL_ERR_ARG; }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!stream_is_capturing(s)) {              // see check_operand
+    const bool capturing = stream_is_capturing(s);
+    if (!capturing) {                           // see check_operand
         const size_t x_bytes = ((size_t)(rows - 1) * (size_t)ldx + (size_t)K) * sizeof(float);
         const size_t z_bytes = ((size_t)(rows - 1) * (size_t)ldz + (size_t)N) * sizeof(float);
         if (int rc = check_operand(X, x_bytes, fn, "X")) return rc;
@@ -1061,7 +1062,7 @@ int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32
             return ACCEL_ERR_ARG;
         }
     }
-    return dense_xw_launch(X, W, Z, rows, K, N, ldx, ldz, s);
+    return dense_xw_launch(X, W, Z, rows, K, N, ldx, ldz, s, !capturing);
 }
 
 }  // extern "C"

@@ -1,46 +1,104 @@
-// Z = X * W in fp32 on the matrix cores: the dense half of a GCN layer, whose result is the
+// Z = X * W in fp32 on the bf16 matrix cores: the dense half of a GCN layer, whose result is the
 // dense operand of the sparse product (upstream's operator stops at A * X, spmm_accel.cu:16-102;
 // a layer around it multiplies the features by a weight matrix first).
 //
+// The fp32 matrix instructions run at a sixteenth of the bf16 rate (157 TFLOP/s against 2.5
+// PFLOP/s), so an fp32 value is taken apart into three bf16 values that add up to it exactly,
+// x = x1 + x2 + x3 (each the nearest bf16 to what is left: 8 bits each of the 24), and the product
+// x w is the sum of the six products x1 w1, x1 w2, x2 w1, x1 w3, x2 w2, x3 w1.  Products of bf16
+// values are exact in the matrix unit and are added up in fp32.  What is left out, x2 w3 + x3 w2 + x3 w3,
+// is below 2^-25 |x w|, half of what rounding one fp32 product may cost, and the accumulator is
+// rounded 0.4 times per k instead of 0.5; measured against fp64 on K = 16 .. 602 the error is the
+// smaller than that of v_mfma_f32_32x32x2_f32 on the same operands (2-norm of the difference over that of
+// the product, K = 602: 3.7e-7 against 4.4e-7; K = 128: 1.6e-7 against 2.0e-7).  Values that bf16 cannot carry this way (infinities, magnitudes of 2^127
+// and more, which would round up to one, and magnitudes below 2^-100, whose third part would
+// be too small for bf16) are multiplied by ordinary fp32 instructions instead, tile by tile where
+// they occur.
+//
 // X is rows x K with rows in the millions and K, N in the tens to hundreds, so the product
-// streams X once, writes Z once and keeps W on chip: 2 K N / (4 (K + N)) flops per byte, about
-// the ratio of the fp32 matrix rate to the memory rate at K = 128, N = 64.  A workgroup of four
-// wavefronts owns 128 rows of X and up to 128 columns of Z; each wavefront keeps a 32-row
-// band of that as 32 x 32 accumulator tiles of v_mfma_f32_32x32x2_f32.  K is walked in steps
-// of 32: the workgroup reads a step's 128 x 32 block of X (full 128-byte lines, eight lanes
-// per row) into registers two steps ahead and its 32 x (32 NT) block of W one step ahead,
-// while the matrix cores work on the steps before, then hands them over through LDS, where a
-// lane finds its row's 16 values of the step as four 16-byte reads.
+// streams X once, writes Z once and keeps W on chip.  A wavefront owns 32 rows of X and up to 128
+// columns of Z (32 x 32 accumulator tiles of v_mfma_f32_32x32x16_bf16), a workgroup four of them.  K is
+// walked in steps of 32.  A lane reads 64 consecutive bytes of its own row per step, two steps ahead,
+// and takes them apart in registers between the matrix instructions of the step before: nobody else
+// needs them, so X does not pass through LDS.  W's 32 x 128 block of the step goes through LDS, two
+// blocks deep, so that one barrier per step is enough; it is taken apart by the workgroup on the
+// way, or, for products large enough to pay for a launch, once beforehand (dense_prepare_kernel).
+//
+// Measured at 1 M x 602 times 602 x 128 (154 Gflop, 2.9 GB): 1.53 ms with the fp32 matrix instructions,
+// 0.96 ms taken apart on the way, 0.93 prepared; at 2.45 M x 128 times 128 x 64: 0.44 and 0.38 ms.
+// What bounds the first is the power the matrix cores may draw: their work alone takes 0.46 ms at the
+// 1.9 GHz the clock settles at under it (65 % of the launch), reading X under it takes the clock lower.
 #include <atomic>
 
-#include "internal.h"
+#include "preprocess.h"
 
 namespace accel {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef v4f v4f_unaligned __attribute__((aligned(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDenseWaves = 4;                          // wavefronts per workgroup
 constexpr int kDenseThreads = kDenseWaves * 64;
-constexpr int kDenseRows = 32;                          // rows per wavefront (one MFMA tile high)
+constexpr int kDenseRows = 32;                          // rows per wavefront (one tile high)
 constexpr int kDenseBlockRows = kDenseWaves * kDenseRows;
-constexpr int kDenseStep = 32;                          // columns of X (rows of W) per round: 16 MFMAs per tile
-// Row stride of the X block in LDS, in floats: 16-byte reads of 16 lanes whose rows are 36
-// floats apart fall into 16 different groups of four banks.
-constexpr int kDenseXStride = kDenseStep + 4;
-constexpr int kDenseXLoads = kDenseBlockRows * kDenseStep / 4 / kDenseThreads;     // 16-byte loads per thread and step: 4
+constexpr int kDenseStep = 32;                          // columns of X (rows of W) per step: two instructions deep
+constexpr int kDenseHalf = kDenseStep / 2;              // of which a lane holds one half
+constexpr int kParts = 3;                               // bf16 values per fp32 value
+// Row stride of a column's 32 bf16 values in LDS, in bytes: 16-byte reads of 16 lanes whose columns
+// are 80 bytes apart fall into 16 different groups of four banks.
+constexpr int kWStride = 2 * kDenseStep + 16;
 
-// Operand layout of v_mfma_f32_32x32x2_f32 (one block): lane l holds A[l % 32][l / 32] and
-// B[l / 32][l % 32]; accumulator register v of lane l is D[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].
-// The two k of one instruction need not be neighbours, only the same for A and B: lanes 0..31
-// carry k0 + j, lanes 32..63 carry k0 + 16 + j, so that a lane's 16 values of A are 64
-// consecutive bytes of its row.
-//
-// The grid is sized to what the GPU holds at once and every workgroup walks blocks of 128
-// rows, gridDim.x apart, as one sequence of steps: the reads of a block's first step are
-// issued while the matrix cores work on the last step of the block before, and that block's
-// rows of Z are stored behind them, so the memory latency is paid once per workgroup, not
-// once per block.  The column tiles of one block of rows (N > 128) follow each other in the
-// same workgroup: the block of X they share comes from L2 for all but the first.
+// Operand layout of v_mfma_f32_32x32x16_bf16: lane l holds A[l % 32][8 (l / 32) + j] and
+// B[8 (l / 32) + j][l % 32], j = 0..7; accumulator register v of lane l is
+// D[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].  The order of the sixteen k of one instruction is free,
+// only the same for A and B: lanes 0..31 carry the first half of the step's k, lanes 32..63 the second,
+// 8 i .. 8 i + 7 of them in instruction i, so that a lane's 16 values are 64 consecutive bytes of its row.
+
+// The k a half of the step starts at.  Where the row ends inside the half, the half is moved back
+// to end with the row (nothing is read past it), and W is zero for the k that belong to the half or
+// the step before.  (K < 16: the loads are clamped one by one instead.)
+__device__ __forceinline__ int half_start(int k0, int half, int K)
+{
+    const int k = k0 + kDenseHalf * half;
+    return K < kDenseHalf ? k : min(k, K - kDenseHalf);
+}
+
+// Takes two values apart: the three parts of each, packed in pairs.
+__device__ __forceinline__ void take_apart(float a, float b, uint32_t (&part)[kParts])
+{
+#pragma unroll
+    for (int p = 0; p < kParts; p++) {
+        part[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+        if (p + 1 < kParts) {                           // exact: what is left has fewer bits
+            a -= __uint_as_float(part[p] << 16);
+            b -= __uint_as_float(part[p] & 0xFFFF0000u);
+        }
+    }
+}
+
+// Magnitudes below 2^-100 are looked for value by value (zero is not one).  The large ones need no
+// look: a value that rounds up to infinity leaves infinity minus infinity in its second part, so
+// every sum it takes part in comes out as NaN, which is looked for before a tile is stored.
+struct Seen {
+    uint32_t least = 0xFFFFFFFFu;                       // smallest magnitude's bits, twice, minus one (zero: the largest value)
+    __device__ __forceinline__ void add(float a, float b)
+    {
+        least = min(least, min((__float_as_uint(a) << 1) - 1u, (__float_as_uint(b) << 1) - 1u));
+    }
+    __device__ __forceinline__ bool bad() const { return least < ((uint32_t)(127 - 100) << 24) - 1u; }
+};
+
+// W(k, col) of a step's half, or zero where the half does not own k (see half_start).
+__device__ __forceinline__ float w_at(const float *__restrict__ W, int K, int N, int k0, int half, int j, int col)
+{
+    const int owned = k0 + kDenseHalf * half, k = half_start(k0, half, K) + j;
+    return k >= owned && k < K && col < N ? W[(int64_t)k * N + col] : 0.f;
+}
 
 // A step of a workgroup's walk: rows [128 row_block, +128), columns [32 NT tile, +32 NT), k in [k0, k0 + 32).
 struct DenseStepAt {
@@ -56,78 +114,187 @@ struct DenseStepAt {
     }
 };
 
-template <int NT, bool kVec>
-__global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kernel(
-    const float *__restrict__ X, const float *__restrict__ W, float *__restrict__ Z, int64_t rows, int K, int N,
-    int64_t ldx, int64_t ldz, int64_t n_row_blocks, int n_col_tiles)
+struct DenseArgs {
+    const float *X, *W;
+    float *Z;
+    int64_t rows, ldx, ldz, n_row_blocks;
+    int K, N, n_col_tiles, n_steps;
+    const u32x4 *image;          // W taken apart (dense_prepare_kernel)
+    const int *bad;              // per column tile and step of the image: holds values below 2^-100
+};
+
+// One workgroup per (column tile, step): the block of W taken apart, as [part][column][32 bf16].
+template <int NT>
+__global__ __launch_bounds__(kDenseThreads) void dense_prepare_kernel(DenseArgs a, u32x4 *__restrict__ image,
+                                                                      int *__restrict__ bad)
+{
+    constexpr int kCols = NT * 32, kVecs = kCols * kParts * 4;
+    __shared__ int any_bad;
+    const int tile = (int)blockIdx.x / a.n_steps, k0 = (int)blockIdx.x % a.n_steps * kDenseStep;
+    if (threadIdx.x == 0) any_bad = 0;
+    __syncthreads();
+    u32x4 *to = image + (int64_t)blockIdx.x * kVecs;
+    for (int i = threadIdx.x; i < kCols * 4; i += kDenseThreads) {
+        const int c = i % kCols, v = i / kCols;             // vector v: 8 k of half v / 2
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) w[j] = w_at(a.W, a.K, a.N, k0, v / 2, v % 2 * 8 + j, tile * kCols + c);
+        Seen seen;
+        uint32_t part[4][kParts];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            seen.add(w[2 * j], w[2 * j + 1]);
+            take_apart(w[2 * j], w[2 * j + 1], part[j]);
+        }
+#pragma unroll
+        for (int p = 0; p < kParts; p++)
+            to[(p * kCols + c) * 4 + v] = u32x4{part[0][p], part[1][p], part[2][p], part[3][p]};
+        if (seen.bad()) any_bad = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) bad[blockIdx.x] = any_bad;
+}
+
+// How the product gets its block of W per step.
+enum DenseW {
+    kWPrepared,                  // from the image
+    kWOnTheWay,                  // taken apart by the workgroup
+    kWShort                      // the same, K < 16
+};
+
+// A workgroup's block of W of a step on its way through registers into LDS.
+template <int NT, DenseW kHow> struct WStage;
+template <int NT> struct WStage<NT, kWPrepared> {
+    static constexpr int kCols = NT * 32, kVecs = kCols * kParts * 4;
+    static constexpr int kMine = (kVecs + kDenseThreads - 1) / kDenseThreads;
+    u32x4 v[kMine];
+    __device__ __forceinline__ void fetch(const DenseArgs &a, const DenseStepAt &at)
+    {
+        const u32x4 *from = a.image + ((int64_t)at.tile * a.n_steps + at.k0 / kDenseStep) * kVecs + threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < kMine; i++)
+            if (kVecs % kDenseThreads == 0 || i * kDenseThreads + (int)threadIdx.x < kVecs) v[i] = from[i * kDenseThreads];
+    }
+    __device__ __forceinline__ void store(const DenseArgs &, const DenseStepAt &, char *lds, int *, int)
+    {
+#pragma unroll
+        for (int i = 0; i < kMine; i++) {
+            const int at = i * kDenseThreads + (int)threadIdx.x;
+            if (kVecs % kDenseThreads == 0 || at < kVecs) *reinterpret_cast<u32x4 *>(lds + at / 4 * kWStride + at % 4 * 16) = v[i];
+        }
+    }
+};
+template <int NT, DenseW kHow> struct WStage {
+    static constexpr int kCols = NT * 32;
+    static constexpr int kRun = kDenseStep * kCols / kDenseThreads;      // consecutive k of a thread: 16, 8, 4
+    float v[kRun];
+    __device__ __forceinline__ void fetch(const DenseArgs &a, const DenseStepAt &at)
+    {
+        // the same loads on every path; what the block does not own is replaced by zero in store()
+        const int c = (int)threadIdx.x % kCols, k = (int)threadIdx.x / kCols * kRun;
+        const int col = min(at.tile * kCols + c, a.N - 1);
+        if (at.k0 + kDenseStep <= a.K) {
+            const float *wb = a.W + (int64_t)(at.k0 + k) * a.N + col;
+#pragma unroll
+            for (int i = 0; i < kRun; i++) v[i] = wb[(int64_t)i * a.N];
+        } else {
+            const int k1 = half_start(at.k0, k / kDenseHalf, a.K) + k % kDenseHalf;
+#pragma unroll
+            for (int i = 0; i < kRun; i++) v[i] = a.W[(int64_t)min(k1 + i, a.K - 1) * a.N + col];
+        }
+    }
+    // bad: the step whose block is not to be used, per LDS buffer
+    __device__ __forceinline__ void store(const DenseArgs &a, const DenseStepAt &at, char *lds, int *bad, int step)
+    {
+        const int c = (int)threadIdx.x % kCols, k = (int)threadIdx.x / kCols * kRun;
+        if (at.k0 + kDenseStep > a.K || (at.tile + 1) * kCols > a.N) {
+            const bool col_ok = at.tile * kCols + c < a.N;
+            const int owned = at.k0 + k - k % kDenseHalf, k1 = half_start(at.k0, k / kDenseHalf, a.K) + k % kDenseHalf;
+#pragma unroll
+            for (int i = 0; i < kRun; i++) v[i] = col_ok && k1 + i >= owned && k1 + i < a.K ? v[i] : 0.f;
+        }
+        Seen seen;
+        uint32_t part[kRun / 2][kParts];
+#pragma unroll
+        for (int i = 0; i < kRun; i += 2) {
+            seen.add(v[i], v[i + 1]);
+            take_apart(v[i], v[i + 1], part[i / 2]);
+        }
+#pragma unroll
+        for (int p = 0; p < kParts; p++) {
+            char *to = lds + (p * kCols + c) * kWStride + 2 * k;
+            if constexpr (kRun >= 8) {
+#pragma unroll
+                for (int i = 0; i < kRun / 2; i += 4)
+                    *reinterpret_cast<u32x4 *>(to + 4 * i) = u32x4{part[i][p], part[i + 1][p], part[i + 2][p], part[i + 3][p]};
+            } else {
+                *reinterpret_cast<uint2 *>(to) = make_uint2(part[0][p], part[1][p]);
+            }
+        }
+        if (seen.bad()) *bad = step;
+    }
+};
+
+// The grid is sized to what the GPU holds at once and every workgroup walks blocks of 128
+// rows, gridDim.x apart, as one sequence of steps: the reads of a block's first steps are
+// issued while the matrix cores work on the last steps of the block before, and that block's
+// rows of Z are stored behind them, so the memory latency is paid once per workgroup, not
+// once per block.  The column tiles of one block of rows (N > 128) follow each other in the
+// same workgroup: the rows of X they share come from L2 for all but the first.
+// Loads are the same in number on every path (clamped, not branched around), which keeps the
+// compiler's waits for them exact.
+template <int NT, DenseW kHow>
+__global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kernel(DenseArgs a)
 {
     constexpr int kCols = NT * 32;
-    // two floats of padding put the rows k and k + 16, read together by the two halves of a
-    // wavefront, 32 banks apart
-    constexpr int kWStride = kCols + 2;
-    constexpr int kWLoads = kDenseStep * kCols / kDenseThreads;             // 4 NT
-    __shared__ __attribute__((aligned(16))) float x_lds[kDenseBlockRows * kDenseXStride];
-    __shared__ float w_lds[kDenseStep * kWStride];
+    __shared__ __attribute__((aligned(16))) char w_lds[2][kParts * kCols * kWStride];
+    __shared__ int w_bad[2];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int half = lane >> 5, l32 = lane & 31;
-    const int xc = (tid & 7) * 4;              // this thread reads 16 bytes of row tid / 8 + 32 q, q = 0..3, per step
 
-    // Registers for the blocks of X of the next two steps and the block of W of the next one:
-    // a read from memory takes several steps' worth of matrix work under load, and what is in
-    // flight per compute unit bounds the rate at which X streams in.
-    float4 xreg[2][kDenseXLoads];
-    float wreg[kWLoads];
-    // Loads only, so that nothing waits for them here, and the same number of loads on every
-    // path, which keeps the waits for them exact: with kVec (rows of X start on 16-byte
-    // boundaries and K is a multiple of 4) four 16-byte loads, otherwise sixteen 4-byte loads,
-    // from addresses clamped into the row.  What lies past K or N is replaced by zero when the
-    // registers are handed to LDS.  Rows past the end of X read the last row (their results are
-    // not stored), and so does a step past the end of the walk.
-    // Each has a short form for the usual case, decided for the whole workgroup: a step that
-    // lies inside K, rows inside X, a tile inside N need no clamping, and then the addresses
-    // of a thread's loads are one base and constant strides (a few integer instructions per
-    // step instead of a hundred, which would otherwise compete with the matrix instructions
-    // for the issue slots of the SIMD).
-    constexpr int kWRowsPerLoad = kDenseThreads / kCols;      // rows of W between a thread's loads
-    auto fetch_x = [&](float4 (&dst)[kDenseXLoads], const DenseStepAt &at) {
-        const int k = at.k0 + xc;
-        const int64_t r0 = at.row_block * kDenseBlockRows + (tid >> 3);
-        if (kVec && at.k0 + kDenseStep <= K && (at.row_block + 1) * kDenseBlockRows <= rows) {
-            const float *xb = X + r0 * ldx + k;
+    // This lane's 16 values of X of a step; rows past the end of X read the last row (their results
+    // are not stored), and so does a step past the end of the walk.  Narrow outputs, whose product
+    // is bound by streaming X, read eight lanes to a row (whole lines per instruction) and turn the
+    // values in LDS, within the wavefront (2.45 M x 100 x 32: 298 -> 275 us; with more columns the
+    // detour costs as much as it gives: 128 x 64 382 -> 375 us at 2.45 M rows, 28 -> 32 at 170 k).
+    constexpr bool kTurn = NT == 1 && kHow != kWShort;
+    __shared__ v4f x_lds[kTurn ? kDenseWaves : 1][kTurn ? kDenseRows * 8 : 1];
+    auto turned = [&](const v4f (&x)[4], v4f (&y)[4]) {
+        if constexpr (kTurn) {
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int q = 0; q < kDenseXLoads; q++)
-                dst[q] = *reinterpret_cast<const float4 *>(xb + (int64_t)q * (kDenseThreads / 8) * ldx);
-            return;
-        }
-#pragma unroll
-        for (int q = 0; q < kDenseXLoads; q++) {
-            const int64_t r = r0 + (kDenseThreads / 8) * q;
-            const float *xr = X + (r < rows ? r : rows - 1) * ldx;
-            if (kVec) {
-                dst[q] = *reinterpret_cast<const float4 *>(xr + (k < K ? k : K - 4));
-            } else {
-                const int last = K - 1;
-                dst[q].x = xr[k < last ? k : last];
-                dst[q].y = xr[k + 1 < last ? k + 1 : last];
-                dst[q].z = xr[k + 2 < last ? k + 2 : last];
-                dst[q].w = xr[k + 3 < last ? k + 3 : last];
+            for (int q = 0; q < 4; q++) {
+                const int row = 8 * q + (lane >> 3);
+                x_lds[wave][row * 8 + ((lane & 7) ^ (row & 7))] = x[q];
             }
+            __builtin_amdgcn_wave_barrier();
         }
-    };
-    auto fetch_w = [&](const DenseStepAt &at) {
-        const int k = at.k0 + tid / kCols, col = at.tile * kCols + tid % kCols;
-        if (at.k0 + kDenseStep <= K && (at.tile + 1) * kCols <= N) {
-            const float *wb = W + (int64_t)k * N + col;
 #pragma unroll
-            for (int i = 0; i < kWLoads; i++) wreg[i] = wb[(int64_t)i * kWRowsPerLoad * N];
+        for (int q = 0; q < 4; q++) y[q] = kTurn ? x_lds[wave][l32 * 8 + ((4 * half + q) ^ (l32 & 7))] : x[q];
+    };
+    auto fetch_x = [&](v4f (&x)[4], const DenseStepAt &at) {
+        if constexpr (kTurn) {
+            const int64_t r0 = at.row_block * kDenseBlockRows + wave * kDenseRows + (lane >> 3);
+            const int k = half_start(at.k0, (lane >> 2) & 1, a.K) + 4 * (lane & 3);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int64_t r = r0 + 8 * q;
+                x[q] = *reinterpret_cast<const v4f_unaligned *>(a.X + (r < a.rows ? r : a.rows - 1) * a.ldx + k);
+            }
             return;
         }
-        const int cc = col < N ? col : N - 1;
+        const int64_t r = at.row_block * kDenseBlockRows + wave * kDenseRows + l32;
+        const float *xr = a.X + (r < a.rows ? r : a.rows - 1) * a.ldx;
+        const int k = half_start(at.k0, half, a.K);
+        if constexpr (kHow == kWShort) {
 #pragma unroll
-        for (int i = 0; i < kWLoads; i++) {
-            const int ki = k + kWRowsPerLoad * i;
-            wreg[i] = W[(int64_t)(ki < K ? ki : K - 1) * N + cc];
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[q][i] = xr[min(k + 4 * q + i, a.K - 1)];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const v4f_unaligned *>(xr + k + 4 * q);
         }
     };
 
@@ -138,77 +305,127 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
         for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
 
     const int64_t stride = gridDim.x;          // gridDim.x <= n_row_blocks: every workgroup has work
-    DenseStepAt now{(int64_t)blockIdx.x, 0, 0}, next = now, after = now;
-    next.advance(K, n_col_tiles, stride);
+    DenseStepAt now{(int64_t)blockIdx.x, 0, 0}, next = now, after;
+    next.advance(a.K, a.n_col_tiles, stride);
     after = next;
-    after.advance(K, n_col_tiles, stride);
-    fetch_x(xreg[0], now);
-    fetch_w(now);
-    fetch_x(xreg[1], next);
+    after.advance(a.K, a.n_col_tiles, stride);
+    v4f x0[4], x1[4];
+    WStage<NT, kHow> w;
+    bf16x8 apart[2][kParts];                   // this step's values of X, taken apart
+    Seen seen;
+    auto take_pair = [&](const v4f (&x)[4], int q, uint32_t (&pair)[kParts]) {
+        const float u = x[q / 2][2 * (q & 1)], v = x[q / 2][2 * (q & 1) + 1];
+        seen.add(u, v);
+        take_apart(u, v, pair);
+        // (keeps the work here, between the matrix instructions, where the compiler would move it
+        // to the next step)
+        asm volatile("" : "+v"(pair[0]), "+v"(pair[1]), "+v"(pair[2]));
+    };
+    auto gather_pairs = [&](const uint32_t (&pair)[8][kParts]) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int p = 0; p < kParts; p++)
+                apart[i][p] = __builtin_bit_cast(bf16x8, u32x4{pair[4 * i][p], pair[4 * i + 1][p], pair[4 * i + 2][p],
+                                                               pair[4 * i + 3][p]});
+    };
 
-    // one step; `mine` is the half of xreg that holds its block of X
-    auto step = [&](float4 (&mine)[kDenseXLoads]) {
-        __syncthreads();                       // the previous step's reads of LDS are done
-        float *xs = &x_lds[(tid >> 3) * kDenseXStride + xc];
-        float *ws = &w_lds[(tid / kCols) * kWStride + tid % kCols];
-        if (now.k0 + kDenseStep <= K && (now.tile + 1) * kCols <= N) {         // nothing to mask
+    if (tid < 2) w_bad[tid] = -1;
+    w.fetch(a, now);
+    fetch_x(x0, now);
+    fetch_x(x1, next);
+    if constexpr (kHow != kWPrepared) __syncthreads();
+    {
+        uint32_t pair[8][kParts];
+        v4f y[4];
+        turned(x0, y);
 #pragma unroll
-            for (int q = 0; q < kDenseXLoads; q++)
-                *reinterpret_cast<float4 *>(xs + q * (kDenseThreads / 8) * kDenseXStride) = mine[q];
-#pragma unroll
-            for (int i = 0; i < kWLoads; i++) ws[i * kWRowsPerLoad * kWStride] = wreg[i];
-        } else {
-            const int kx = now.k0 + xc;
-            const int kw = now.k0 + tid / kCols;
-            const bool col_inside = now.tile * kCols + tid % kCols < N;
-#pragma unroll
-            for (int q = 0; q < kDenseXLoads; q++) {
-                float4 x = mine[q];
-                x.x = kx < K ? x.x : 0.f; x.y = kx + 1 < K ? x.y : 0.f;
-                x.z = kx + 2 < K ? x.z : 0.f; x.w = kx + 3 < K ? x.w : 0.f;
-                *reinterpret_cast<float4 *>(xs + q * (kDenseThreads / 8) * kDenseXStride) = x;
-            }
-#pragma unroll
-            for (int i = 0; i < kWLoads; i++)
-                ws[i * kWRowsPerLoad * kWStride] = (col_inside && kw + kWRowsPerLoad * i < K) ? wreg[i] : 0.f;
-        }
-        __syncthreads();
-        // in flight while the matrix cores work: W of the next step, X of the one after it
-        fetch_w(next);
-        fetch_x(mine, after);
-        // the loads go out here, ahead of the matrix work that hides them, not behind it
-        __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < 8; q++) take_pair(y, q, pair[q]);
+        gather_pairs(pair);
+    }
+    bool tile_ok = true, x_ok = !__any(seen.bad());
+    w.store(a, now, w_lds[0], &w_bad[0], 0);
+    int step = 0;
+    // xf: free registers, for the step after the next; xn: the next step's X
+    auto one = [&](v4f (&xf)[4], v4f (&xn)[4]) {
+        const int buf = step & 1;
+        __syncthreads();                       // this step's block of W is in place; the other one's readers are done
+        if constexpr (kHow == kWPrepared) tile_ok &= x_ok && !a.bad[now.tile * a.n_steps + now.k0 / kDenseStep];
+        else tile_ok &= x_ok && w_bad[buf] != step;
+        w.fetch(a, next);
+        fetch_x(xf, after);
+        __builtin_amdgcn_sched_barrier(0);     // the loads go out here, ahead of the matrix work that hides them
 
-        float a[16];
-        const float4 *ap = reinterpret_cast<const float4 *>(&x_lds[(wave * kDenseRows + l32) * kDenseXStride + half * 16]);
+        // The step's 12 NT matrix instructions in groups of one or two tiles' six; the reads of the
+        // next group's W and a share of taking the next step's X apart go between them.
+        constexpr int P = NT < 2 ? NT : 2, kGroups = 2 * NT / P;
+        bf16x8 b[2][P][kParts];
+        auto read_b = [&](bf16x8 (&to)[P][kParts], int g) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const float4 x = ap[q];
-            a[4 * q] = x.x; a[4 * q + 1] = x.y; a[4 * q + 2] = x.z; a[4 * q + 3] = x.w;
+            for (int u = 0; u < P; u++)
+#pragma unroll
+                for (int p = 0; p < kParts; p++)
+                    to[u][p] = *reinterpret_cast<const bf16x8 *>(
+                        &w_lds[buf][(p * kCols + 32 * (g * P % NT + u) + l32) * kWStride + 32 * half + 16 * (g * P / NT)]);
+        };
+        uint32_t pair[8][kParts];
+        seen = Seen();
+        read_b(b[0], 0);
+        v4f y[4];
+        turned(xn, y);
+#pragma unroll
+        for (int g = 0; g < kGroups; g++) {
+            if (g + 1 < kGroups) read_b(b[(g + 1) & 1], g + 1);
+            constexpr int ap[6] = {2, 0, 1, 1, 0, 0}, bp[6] = {0, 2, 1, 0, 1, 0};     // the small products first
+#pragma unroll
+            for (int q = 0; q < 6; q++)
+#pragma unroll
+                for (int u = 0; u < P; u++)
+                    acc[g * P % NT + u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(apart[g * P / NT][ap[q]], b[g & 1][u][bp[q]],
+                                                                                  acc[g * P % NT + u], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (q * kGroups / 8 == g) take_pair(y, q, pair[q]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int j = 0; j < 16; j++)
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], w_lds[(half * 16 + j) * kWStride + t * 32 + l32],
-                                                              acc[t], 0, 0, 0);
+        gather_pairs(pair);
+        x_ok = !__any(seen.bad());
+        w.store(a, next, w_lds[buf ^ 1], &w_bad[buf ^ 1], step + 1);      // its readers were done at this step's barrier
 
         if (next.k0 == 0) {                    // that was the last step of this tile: store it, start the next at zero
             const int64_t row0 = now.row_block * kDenseBlockRows + wave * kDenseRows;
             const int col = now.tile * kCols + l32;
-            float *z = Z + (row0 + 4 * half) * ldz + col;
-            if (row0 + kDenseRows <= rows && now.tile * kCols + kCols <= N) {      // the usual case: nothing to mask
+            float *z = a.Z + (row0 + 4 * half) * a.ldz + col;
+            bool finite = true;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) finite &= __builtin_isfinite(acc[t][v]);
+            if (!tile_ok || __any(!finite)) {
+                // values out of range among the operands: ordinary fp32, from memory
+#pragma unroll 1
+                for (int i = 0; i < 16 * NT; i++) {
+                    const int64_t row = row0 + 2 * (i % 16) + half;
+                    const int c = col + 32 * (i / 16);
+                    if (row >= a.rows || c >= a.N) continue;
+                    float sum = 0.f;
+#pragma unroll 1
+                    for (int k = 0; k < a.K; k++) sum = fmaf(a.X[row * a.ldx + k], a.W[(int64_t)k * a.N + c], sum);
+                    a.Z[row * a.ldz + c] = sum;
+                }
+                tile_ok = true;
+            } else if (row0 + kDenseRows <= a.rows && now.tile * kCols + kCols <= a.N) {      // nothing to mask
 #pragma unroll
                 for (int t = 0; t < NT; t++)
 #pragma unroll
-                    for (int v = 0; v < 16; v++) z[(8 * (v / 4) + v % 4) * ldz + t * 32] = acc[t][v];
+                    for (int v = 0; v < 16; v++) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v];
             } else {
 #pragma unroll
                 for (int t = 0; t < NT; t++)
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
                         const int64_t row = row0 + 8 * (v / 4) + 4 * half + (v % 4);
-                        if (col + t * 32 < N && row < rows) z[(8 * (v / 4) + v % 4) * ldz + t * 32] = acc[t][v];
+                        if (col + t * 32 < a.N && row < a.rows) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v];
                     }
             }
 #pragma unroll
@@ -218,59 +435,88 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
         }
         now = next;
         next = after;
-        after.advance(K, n_col_tiles, stride);
+        after.advance(a.K, a.n_col_tiles, stride);
+        step++;
     };
-    while (now.row_block < n_row_blocks) {
-        step(xreg[0]);
-        if (now.row_block >= n_row_blocks) break;
-        step(xreg[1]);
+    while (now.row_block < a.n_row_blocks) {
+        one(x0, x1);
+        if (now.row_block >= a.n_row_blocks) break;
+        one(x1, x0);
     }
 }
 
 // The grid: as many workgroups as the GPU holds at once (asked of the runtime for the kernel
 // that runs, once per device and kernel), or one per block of rows when there are fewer.
 constexpr int kDenseDevices = 64;
-static std::atomic<int> g_resident[kDenseDevices][6];     // [device][kernel]: workgroups the device holds, 0 = not asked yet
+static std::atomic<int> g_resident[kDenseDevices][9];     // [device][kernel]: workgroups the device holds, 0 = not asked yet
 
-template <int NT, bool kVec>
-static int dense_launch(hipStream_t s, const float *X, const float *W, float *Z, int64_t rows, int K, int N, int64_t ldx,
-                        int64_t ldz, int64_t n_row_blocks, int n_col_tiles)
+template <int NT, DenseW kHow>
+static int dense_launch(const DenseArgs &a, hipStream_t s)
 {
-    constexpr int which = (NT == 1 ? 0 : NT == 2 ? 2 : 4) + (kVec ? 1 : 0);
+    constexpr int which = (NT == 1 ? 0 : NT == 2 ? 3 : 6) + (int)kHow;
     int dev = 0;
     ACCEL_HIP(hipGetDevice(&dev));
     int resident = dev >= 0 && dev < kDenseDevices ? g_resident[dev][which].load(std::memory_order_relaxed) : 0;
     if (resident == 0) {
         int cus = 0, per_cu = 0;
         ACCEL_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        ACCEL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, dense_xw_kernel<NT, kVec>, kDenseThreads, 0));
+        ACCEL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, dense_xw_kernel<NT, kHow>, kDenseThreads, 0));
         resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);
         if (dev >= 0 && dev < kDenseDevices) g_resident[dev][which].store(resident, std::memory_order_relaxed);
     }
-    const unsigned grid = (unsigned)(n_row_blocks < resident ? n_row_blocks : resident);
-    dense_xw_kernel<NT, kVec><<<grid, kDenseThreads, 0, s>>>(X, W, Z, rows, K, N, ldx, ldz, n_row_blocks, n_col_tiles);
+    const unsigned grid = (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
+    dense_xw_kernel<NT, kHow><<<grid, kDenseThreads, 0, s>>>(a);
     return ACCEL_OK;
 }
 
+// Wide products (128 columns to a workgroup) of this many multiplications and more take W apart
+// beforehand: a launch more (5 us) and half the integer work inside (1 M rows: 300 x 100 548 -> 502 us,
+// 602 x 128 964 -> 926, 512 x 256 1527 -> 1466).  Narrow ones are bound by memory and gain nothing
+// (2.45 M x 128 x 64: 382 -> 394 us).
+constexpr double kPrepareFrom = 1e10;
+
+template <int NT>
+static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
+{
+    if (a.K < kDenseHalf) return dense_launch<NT, kWShort>(a, s);
+    if constexpr (NT == 4) {
+        const size_t blocks = (size_t)a.n_col_tiles * (size_t)a.n_steps;
+        const size_t image_bytes = blocks * (NT * 32 * kParts * 4) * sizeof(u32x4);
+        char *mem = nullptr;
+        if (may_prepare && (double)a.rows * a.K * a.N >= kPrepareFrom)
+            mem = static_cast<char *>(take_stream_memory(image_bytes + blocks * sizeof(int), s));
+        if (mem) {
+            u32x4 *image = reinterpret_cast<u32x4 *>(mem);
+            int *bad = reinterpret_cast<int *>(mem + image_bytes);
+            dense_prepare_kernel<NT><<<dim3((unsigned)blocks), kDenseThreads, 0, s>>>(a, image, bad);
+            a.image = image;
+            a.bad = bad;
+            const int rc = dense_launch<NT, kWPrepared>(a, s);
+            give_stream_memory(mem, s);
+            return rc;
+        }
+    }
+    return dense_launch<NT, kWOnTheWay>(a, s);
+}
+
 // Arguments have been checked by the caller (accel_dense_xw): rows >= 1, K, N >= 1,
-// ldx >= K, ldz >= N, operands readable and large enough.
+// ldx >= K, ldz >= N, operands readable and large enough.  may_prepare: s is not capturing (a graph's
+// memory would have to live as long as the graph).
 int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int K, int N, int64_t ldx, int64_t ldz,
-                    hipStream_t stream)
+                    hipStream_t s, bool may_prepare)
 {
     (void)hipGetLastError();
     const int nt = N <= 32 ? 1 : N <= 64 ? 2 : 4;
-    const int n_col_tiles = (N + nt * 32 - 1) / (nt * 32);
-    const int64_t n_row_blocks = (rows + kDenseBlockRows - 1) / kDenseBlockRows;
-    // 16-byte reads of X need every row to start on a 16-byte boundary and to end on one
-    const bool vec = (reinterpret_cast<uintptr_t>(X) % 16 == 0) && (ldx % 4 == 0) && (K % 4 == 0);
-    int rc;
-#define DENSE_CASE(NT_)                                                                                  \
-    rc = vec ? dense_launch<NT_, true>(stream, X, W, Z, rows, K, N, ldx, ldz, n_row_blocks, n_col_tiles)  \
-             : dense_launch<NT_, false>(stream, X, W, Z, rows, K, N, ldx, ldz, n_row_blocks, n_col_tiles)
-    if (nt == 1) DENSE_CASE(1);
-    else if (nt == 2) DENSE_CASE(2);
-    else DENSE_CASE(4);
-#undef DENSE_CASE
+    DenseArgs a{};
+    a.X = X; a.W = W; a.Z = Z;
+    a.rows = rows; a.ldx = ldx; a.ldz = ldz;
+    a.n_row_blocks = (rows + kDenseBlockRows - 1) / kDenseBlockRows;
+    a.K = K; a.N = N;
+    a.n_col_tiles = (N + nt * 32 - 1) / (nt * 32);
+    a.n_steps = (K + kDenseStep - 1) / kDenseStep;
+    const int rc = nt == 1   ? dense_product<1>(a, s, may_prepare)
+                   : nt == 2 ? dense_product<2>(a, s, may_prepare)
+                             : dense_product<4>(a, s, may_prepare);
     if (rc) return rc;
     ACCEL_HIP(hipGetLastError());
     return ACCEL_OK;

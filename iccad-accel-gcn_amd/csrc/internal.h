@@ -165,6 +165,9 @@ namespace accel {
 void *take_memory(size_t bytes, bool any_stream);
 void give_memory(void *p, bool settled);
 void release_idle_memory();
+// The same for memory that work queued on s will use, from now on and until it is given back.
+void *take_stream_memory(size_t bytes, hipStream_t s);
+void give_stream_memory(void *p, hipStream_t s);
 // transfer.hip: ordinary host memory to and from the device, queued on s; upload returns when src has
 // been read, download when dst has been written
 int upload(void *dst, const void *src, size_t bytes, hipStream_t s);

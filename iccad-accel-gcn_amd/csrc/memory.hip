@@ -19,11 +19,12 @@
 // four fifths of it, so that subgraphs of about the same size find each other's memory.
 //
 // Order on the device.  hipFree waits for the device; giving memory back here does not.  A
-// block may therefore still be in use by kernels queued on the null stream (and by nothing
-// else: whoever has used other streams waits for the device before it gives memory back).
-// The preprocessing, which takes nearly all of it, works on the null stream and is ordered
-// behind those kernels by the stream; a taker that will use the memory on another stream says
-// so (`any_stream`) and the null stream is waited for if the block needs it.
+// block may therefore still be in use by kernels queued on the null stream, or on one other
+// stream, behind which it carries an event (a handle that has used several streams waits for the
+// device before it gives its memory back).  The preprocessing, which takes nearly all of it,
+// works on the null stream and is ordered behind the former by the stream; every other
+// combination of the last use and the next waits for the event on the device, or on the host
+// where the next stream is not known (`any_stream`) or the last one was the null stream.
 #include <chrono>
 #include <mutex>
 #include <unordered_map>
@@ -42,7 +43,8 @@ struct Idle {
     void *p;
     size_t bytes;
     int device;
-    bool settled;                                 // no kernel uses it any more
+    bool settled;                                 // no kernel on the null stream uses it any more
+    hipEvent_t after;                             // stands behind its last use on another stream, or null
     Clock::time_point since;
 };
 
@@ -72,7 +74,8 @@ void free_block(const Idle &b)
     int now = 0;
     (void)hipGetDevice(&now);
     if (now != b.device) (void)hipSetDevice(b.device);
-    if (hipFree(b.p) != hipSuccess) (void)hipGetLastError();
+    if (hipFree(b.p) != hipSuccess) (void)hipGetLastError();          // waits for the device
+    if (b.after) (void)hipEventDestroy(b.after);
     if (now != b.device) (void)hipSetDevice(now);
 }
 
@@ -116,14 +119,14 @@ void release_idle_device_memory()
 
 }  // namespace
 
-void *take_memory(size_t bytes, bool any_stream)
+// s: the stream the memory will be used on first; null: the null stream, or (any) one not known yet.
+static void *take(size_t bytes, hipStream_t s, bool any)
 {
     Pool &pl = pool();
     const size_t want = size_class(bytes);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    void *p = nullptr;
-    bool settled = true;
+    Idle got{};
     std::vector<Idle> gone;
     {
         std::lock_guard<std::mutex> lock(pl.mu);
@@ -134,18 +137,29 @@ void *take_memory(size_t bytes, bool any_stream)
             if (best == pl.idle.size() || b.bytes <= pl.idle[best].bytes) best = i;
         }
         if (best < pl.idle.size()) {
-            p = pl.idle[best].p;
-            settled = pl.idle[best].settled;
-            pl.live[p] = {pl.idle[best].bytes, dev};
+            got = pl.idle[best];
+            pl.live[got.p] = {got.bytes, dev};
             pl.idle.erase(pl.idle.begin() + (long)best);
         }
         expire(pl, gone);
     }
     free_idle(gone);
-    if (p) {
-        if (any_stream && !settled && hipStreamSynchronize(nullptr) != hipSuccess) (void)hipGetLastError();
-        return p;
+    if (got.p) {
+        hipError_t e = hipSuccess;
+        if (got.after) {                                          // last used on another stream than the null stream
+            e = any ? hipEventSynchronize(got.after) : hipStreamWaitEvent(s, got.after, 0);
+            (void)hipEventDestroy(got.after);
+        } else if (!got.settled && (any || s)) {
+            e = hipStreamSynchronize(nullptr);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipDeviceSynchronize();
+            (void)hipGetLastError();
+        }
+        return got.p;
     }
+    void *p = nullptr;
     if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
         release_idle_device_memory();
@@ -164,7 +178,7 @@ void *take_memory(size_t bytes, bool any_stream)
     return p;
 }
 
-void give_memory(void *p, bool settled)
+static void give(void *p, bool settled, hipEvent_t after)
 {
     if (!p) return;
     Pool &pl = pool();
@@ -173,11 +187,30 @@ void give_memory(void *p, bool settled)
         std::lock_guard<std::mutex> lock(pl.mu);
         const auto it = pl.live.find(p);
         if (it == pl.live.end()) return;
-        pl.idle.push_back({p, it->second.first, it->second.second, settled, Clock::now()});
+        pl.idle.push_back({p, it->second.first, it->second.second, settled, after, Clock::now()});
         pl.live.erase(it);
         expire(pl, gone);
     }
     free_idle(gone);
+}
+
+void *take_memory(size_t bytes, bool any_stream) { return take(bytes, nullptr, any_stream); }
+void give_memory(void *p, bool settled) { give(p, settled, nullptr); }
+void *take_stream_memory(size_t bytes, hipStream_t s) { return take(bytes, s, false); }
+
+void give_stream_memory(void *p, hipStream_t s)
+{
+    if (!s) { give(p, false, nullptr); return; }
+    hipEvent_t after = nullptr;
+    if (hipEventCreateWithFlags(&after, hipEventDisableTiming) == hipSuccess && hipEventRecord(after, s) == hipSuccess) {
+        give(p, true, after);
+        return;
+    }
+    (void)hipGetLastError();
+    if (after) (void)hipEventDestroy(after);
+    (void)hipStreamSynchronize(s);
+    (void)hipGetLastError();
+    give(p, true, nullptr);
 }
 
 // Pinned blocks for the preprocessing's results, one per call that is under way; kept (a few KB

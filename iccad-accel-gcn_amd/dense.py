@@ -1,4 +1,4 @@
-"""The dense side of a GCN layer around the sparse product: Z = X W on the GPU's fp32
+"""The dense side of a GCN layer around the sparse product: Z = X W in fp32 on the GPU's
 matrix cores (accel_dense_xw), and the layer Y = act(A (X W) + bias) as two launches.
 
 Upstream's operator takes the dense operand as given (spmm_accel.cu:16-102 computes

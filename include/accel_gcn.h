@@ -379,12 +379,12 @@ int accel_time_ex(accel_handle *h, const accel_run_args *args, int warmup, int i
  * at A X).  X: rows x K floats, rows ldx floats apart (0 = K); W: K x N floats, packed
  * row-major; Z: rows x N floats, rows ldz apart (0 = N; the columns N .. ldz-1 are not
  * written); all three on the device, Z overlapping neither input.  Any rows >= 0, K >= 1,
- * N >= 1; rows of X that start and end on 16-byte boundaries (X aligned, ldx and K multiples
- * of 4) are read as 16-byte vectors.  Needs no handle; asynchronous on `stream`; allocates nothing.
- * Computed on the fp32 matrix cores: sums of K products in fp32, whose order differs from a
- * sequential loop (compare against a higher-precision product, as for accel_run).  Built for
- * the shapes of a layer: many rows and N up to 128, where the product is bound by streaming
- * X; for wider outputs (N = 256 and more) a BLAS is the better tool. */
+ * N >= 1.  Needs no handle; asynchronous on `stream`.  Products of more than 64 columns and 1e10
+ * multiplications take a workspace of 6 bytes per element of W from the memory the library keeps
+ * (accel_release_memory); the others, and all of them while the stream is capturing, take none.
+ * Computed on the matrix cores, each fp32 value as three bf16 values that add up to it: sums of K
+ * products in fp32 (error as of fp32 instructions, or smaller), whose order differs from a
+ * sequential loop (compare against a higher-precision product, as for accel_run). */
 int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32_t K, int32_t N,
                    int32_t ldx, int32_t ldz, void *stream);
 
