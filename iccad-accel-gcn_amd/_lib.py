@@ -79,6 +79,8 @@ SIGNATURES = {
     "accel_set_plan_groups": (C.c_int, [vp, C.c_int]),
     "accel_set_plan_split": (C.c_int, [vp, C.c_int]),
     "accel_set_plan_team": (C.c_int, [vp, C.c_int]),
+    "accel_row_stride": (C.c_int, [vp, C.c_int32]),
+    "accel_run_rows": (C.c_int, [vp, C.POINTER(RunArgs), C.c_int32]),
     "accel_set_plan_panel": (C.c_int, [vp, C.c_int]),
     "accel_set_plan_queues": (C.c_int, [vp, C.c_int]),
     "accel_set_plan_reduce": (C.c_int, [vp, C.c_int]),

@@ -48,6 +48,7 @@ void release_products(accel_handle *h)
     give_memory(h->long_slot, settled);
     give_memory(h->block4, settled);
     give_memory(h->partial, settled);
+    give_memory(h->x_rows, settled);
     give_memory(h->src_pos, settled);
     h->src_pos = nullptr;
     h->val_stale = false;
@@ -65,6 +66,8 @@ void release_products(accel_handle *h)
     h->work = nullptr; h->long_slot = nullptr; h->row_done = nullptr; h->block4 = nullptr; h->partial = nullptr;
     h->runs = h->first_chunk = h->chunk_row = nullptr;
     h->n_units = h->n_long_units = 0;
+    h->x_rows = nullptr;
+    h->x_rows_floats = 0; h->reserved_N = 0;
     h->partial_floats = 0; h->owns_sorted = false; h->ready = false;
 }
 
@@ -143,7 +146,7 @@ static int check_device(const accel_handle *h, const char *fn)
 
 // argument checks shared by the run entry points
 static int check_run(accel_handle *h, const float *X, float *Y, int32_t N, const float *bias, const char *fn,
-                     hipStream_t stream, int32_t ld = 0)
+                     hipStream_t stream, int32_t ld = 0, int32_t ldx = 0)
 {
     if (!h) { set_error("%s: null handle", fn); return ACCEL_ERR_ARG; }
     if (!h->ready) { set_error("%s: call accel_preprocess first", fn); return ACCEL_ERR_STATE; }
@@ -153,8 +156,9 @@ static int check_run(accel_handle *h, const float *X, float *Y, int32_t N, const
     if (h->rows == 0) return ACCEL_OK;
     if (stream_is_capturing(stream)) return ACCEL_OK;    // see check_operand
     if (ld <= 0) ld = N;
+    if (ldx <= 0) ldx = ld;
     // the last row only has to hold N floats
-    const size_t x_floats = h->cols > 0 ? (size_t)(h->cols - 1) * (size_t)ld + (size_t)N : 0;
+    const size_t x_floats = h->cols > 0 ? (size_t)(h->cols - 1) * (size_t)ldx + (size_t)N : 0;
     const size_t y_floats = (size_t)(h->rows - 1) * (size_t)ld + (size_t)N;
     if (int rc = check_operand(X, x_floats * sizeof(float), fn, "X")) return rc;
     if (int rc = check_operand(Y, y_floats * sizeof(float), fn, "Y")) return rc;
@@ -938,13 +942,38 @@ int accel_run_ex(accel_handle *h, const accel_run_args *a)
                        (a->flags & ACCEL_EPILOGUE_RELU) ? 1 : 0, false, ld);
 }
 
+int accel_row_stride(const accel_handle *h, int32_t N)
+{
+    clear_error();
+    if (!h) { set_error("accel_row_stride: null handle"); return 0; }
+    if (N <= 0) { set_error("accel_row_stride: N must be positive, got %d", N); return 0; }
+    return h->ready ? row_stride(h, N) : N;
+}
+
+int accel_run_rows(accel_handle *h, const accel_run_args *a, int32_t ldx)
+{
+    clear_error();
+    const char *fn = "accel_run_rows";
+    if (!a) { set_error("%s: null arguments", fn); return ACCEL_ERR_ARG; }
+    const int32_t ld = a->ld == 0 ? a->N : a->ld;
+    if (ldx == 0) ldx = a->N;
+    if (ld < a->N || ldx < a->N) {
+        set_error("%s: the row strides (%d, %d) must be 0 or at least N (%d)", fn, ldx, a->ld, a->N);
+        return ACCEL_ERR_ARG;
+    }
+    if (a->flags & ~ACCEL_EPILOGUE_RELU) { set_error("%s: unknown flags %d", fn, a->flags); return ACCEL_ERR_ARG; }
+    if (int rc = check_run(h, a->X, a->Y, a->N, a->bias, fn, static_cast<hipStream_t>(a->stream), ld, ldx)) return rc;
+    return spmm_launch(h, a->X, a->Y, a->N, static_cast<hipStream_t>(a->stream), nullptr, nullptr, a->bias,
+                       (a->flags & ACCEL_EPILOGUE_RELU) ? 1 : 0, false, ld, ldx);
+}
+
 int accel_reserve(accel_handle *h, int32_t max_N)
 {
     clear_error();
     if (!h) { set_error("accel_reserve: null handle"); return ACCEL_ERR_ARG; }
     if (!h->ready) { set_error("accel_reserve: call accel_preprocess first"); return ACCEL_ERR_STATE; }
     if (max_N <= 0) { set_error("accel_reserve: N must be positive, got %d", max_N); return ACCEL_ERR_ARG; }
-    return reserve_partial(h, (size_t)h->n_long_units * (size_t)max_N, true);
+    return reserve_run(h, max_N);
 }
 
 int accel_run_static(accel_handle *h, const float *X, float *Y, int32_t N, void *stream)

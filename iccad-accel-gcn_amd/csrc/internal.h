@@ -128,6 +128,10 @@ struct accel_handle {
     // scratch for the partial sums of long-row segments: [n_long_blocks * N]
     float *partial = nullptr;
     size_t partial_floats = 0;
+    // X copied to padded rows, by runs for which that pays (see pads_x in spmm.hip)
+    float *x_rows = nullptr;
+    size_t x_rows_floats = 0;
+    int reserved_N = 0;               // runs with up to so many columns allocate nothing (accel_reserve)
     // sorted position -> position in the caller's arrays, built by the first value update
     int32_t *src_pos = nullptr;
     // the handle's own copy of the caller's values (owns_input) is behind the sorted copy: a value
@@ -191,8 +195,9 @@ int note_update(accel_handle *h, hipStream_t s, bool capturing);
 // spmm.hip
 int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t stream,
                 hipEvent_t main_start = nullptr, hipEvent_t main_stop = nullptr, const float *bias = nullptr,
-                int relu = 0, bool static_partial = false, int ld = 0);
-int reserve_partial(accel_handle *h, size_t floats, bool any_stream);
+                int relu = 0, bool static_partial = false, int ld = 0, int ldx = 0);
+int reserve_run(accel_handle *h, int max_N);
+int row_stride(const accel_handle *h, int N);
 int fill_u32(void *dst, uint32_t v, size_t n, hipStream_t s);
 int copy_u32(void *dst, const void *src, size_t n, hipStream_t s);
 }  // namespace accel

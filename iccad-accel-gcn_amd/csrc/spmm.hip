@@ -59,6 +59,9 @@ constexpr int kUnroll = 4;                // gathers in flight per lane in the m
 constexpr int kTeamUnroll = 4;            // the same with workgroup units (8: 5-10 % slower)
 constexpr int kPanel = 64;                // column-panel width for wide operands on large matrices
 constexpr int kPanelMinNnz = 4000000;     // smaller matrices are not worth several launches
+constexpr int kPadRows = 64;              // rows that a workgroup of pad_rows_kernel copies
+constexpr int kPadMaxN = 512;             // wider rows: what padding saves is less than one line in 17
+constexpr size_t kPadMaxFloats = ((size_t)1 << 30) - 1;   // copies below 4 GiB, a 64th of the memory (and 32-bit offsets)
 constexpr int kStreamingMinBytes = 64;    // rows of Y of at least this many bytes are stored streaming
                                           // (64-byte rows: L2-resident X -18 %, elsewhere within 1 %)
 
@@ -194,14 +197,14 @@ __device__ __forceinline__ void finish_split_row(const float *__restrict__ src, 
 // uniform base; otherwise the column, and the address is formed with 64-bit arithmetic.
 template <int VEC, int U, bool kWide, bool kShift>
 __device__ __forceinline__ void gather_row(const int2 *__restrict__ row_st, int d, int k, int gp,
-                                           const float *__restrict__ X, int col, int ld,
+                                           const float *__restrict__ X, int col, int ldx,
                                            float (&acc)[VEC])
 {
     const char *xb = reinterpret_cast<const char *>(X);
     const uint32_t lane_off = (uint32_t)col * 4u;
     auto fetch = [&](int where, float (&x)[VEC]) {
         if constexpr (kWide)
-            load_vec<VEC, kShift>(X + col + (int64_t)where * ld, x);
+            load_vec<VEC, kShift>(X + col + (int64_t)where * ldx, x);
         else
             load_vec<VEC, kShift>(reinterpret_cast<const float *>(xb + ((uint32_t)where + lane_off)), x);
     };
@@ -274,12 +277,12 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
     const int4 *__restrict__ work, int n_units,
     const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
     const int32_t *__restrict__ perm, const float *__restrict__ X, float *__restrict__ Y,
-    float *__restrict__ partial, int N, int ld, int n_zero_rows, int n_zero_groups,
+    float *__restrict__ partial, int N, int ldx, int ld, int n_zero_rows, int n_zero_groups,
     const float *__restrict__ bias, int relu, const int32_t *__restrict__ long_slot, int first_split_row,
     int *__restrict__ row_done)
 {
-    // N columns are computed; rows of X, Y and the partial sums are ld floats apart
-    // (ld > N when the launch covers one column panel of a wider operand)
+    // N columns are computed; rows of X are ldx floats apart, those of Y and the partial sums ld
+    // (more than N when the launch covers one column panel of a wider operand)
     constexpr int G = 64 / L;        // lane groups per wavefront
     constexpr int CW = L * VEC;      // columns covered per pass
     __shared__ int2 stage[kWaves][kDegBound];
@@ -323,7 +326,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
 #pragma unroll
         for (int j = 0; j < kRounds; j++) {
             const int i = lane + 64 * j;
-            if (i < total_nz) st[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ld * 4u)), __float_as_int(cv[j]));
+            if (i < total_nz) st[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ldx * 4u)), __float_as_int(cv[j]));
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -356,7 +359,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
             float acc[VEC];
 #pragma unroll
             for (int v = 0; v < VEC; v++) acc[v] = 0.0f;
-            if (live) gather_row<VEC, kUnroll, kWide, kShift>(st + r * d, d, k, gp, X, col, ld, acc);
+            if (live) gather_row<VEC, kUnroll, kWide, kShift>(st + r * d, d, k, gp, X, col, ldx, acc);
             // add the gp partial sums of each row (all lanes take part)
             for (int m = L; m < (L << lg); m <<= 1) {
 #pragma unroll
@@ -406,7 +409,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
     const int4 *__restrict__ work, int n_units,
     const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
     const int32_t *__restrict__ perm, const float *__restrict__ X, float *__restrict__ Y,
-    float *__restrict__ partial, int N, int ld, int n_zero_rows, int n_zero_groups,
+    float *__restrict__ partial, int N, int ldx, int ld, int n_zero_rows, int n_zero_groups,
     const float *__restrict__ bias, int relu, const int32_t *__restrict__ long_slot, int first_split_row,
     int *__restrict__ row_done)
 {
@@ -450,7 +453,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
 #pragma unroll
         for (int j = 0; j < kRounds; j++) {
             const int i = (int)threadIdx.x + kWgThreads * j;
-            if (i < total_nz) stage[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ld * 4u)), __float_as_int(cv[j]));
+            if (i < total_nz) stage[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ldx * 4u)), __float_as_int(cv[j]));
         }
     }
     __syncthreads();
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
             float acc[VEC];
 #pragma unroll
             for (int v = 0; v < VEC; v++) acc[v] = 0.0f;
-            if (live) gather_row<VEC, kTeamUnroll, kWide, kShift>(stage + r * d, d, k, gp, X, col, ld, acc);
+            if (live) gather_row<VEC, kTeamUnroll, kWide, kShift>(stage + r * d, d, k, gp, X, col, ldx, acc);
             // the row's groups inside this wavefront (all lanes take part)
             for (int m = L; m < L * in_wave; m <<= 1) {
 #pragma unroll
@@ -630,6 +633,41 @@ __global__ __launch_bounds__(256) void copy_u32_kernel(uint32_t *__restrict__ ds
         dst[i] = src[i];
 }
 
+// Copies rows of N floats, ld apart, to rows ldx apart (a multiple of 16, with zeros behind the N):
+// 64 rows per workgroup, four 16-byte vectors per thread on their way.  Bound by memory: 5.8 to 6.7
+// TB/s of reads and writes on 2.45 M rows of 25 to 127 floats (4.5 at 14).  The copy is written with
+// ordinary stores, since the gather that follows reads it.
+__global__ __launch_bounds__(kWgThreads) void pad_rows_kernel(const float *__restrict__ X, int64_t rows, int N, int64_t ld,
+                                                              float *__restrict__ out, int ldx)
+{
+    const int64_t row0 = (int64_t)blockIdx.x * kPadRows;
+    const int n_rows = (int)min((int64_t)kPadRows, rows - row0);
+    const int per_row = ldx / 4, n = n_rows * per_row;
+    const float *src = X + row0 * ld;
+    v4f *dst = reinterpret_cast<v4f *>(out + row0 * ldx);
+    const uint32_t inverse = 0xFFFFFFFFu / (uint32_t)per_row + 1;     // exact for i < 2^16, per_row <= 128
+    constexpr int U = 4;
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * kWgThreads) {
+        v4f t[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + u * kWgThreads, r = (int)__umulhi((uint32_t)i, inverse), c = (i - r * per_row) * 4;
+            const bool on = i < n && c < N;
+            // a row's last vector is taken from where it ends with the row, and moved down
+            const int back = on ? max(c + 4 - N, 0) : 0;
+            const v4f q = __builtin_nontemporal_load(
+                reinterpret_cast<const v4f_unaligned *>(src + (on ? r * ld + c - back : 0)));
+            t[u].x = !on ? 0.0f : back == 0 ? q.x : back == 1 ? q.y : back == 2 ? q.z : q.w;
+            t[u].y = !on || back == 3 ? 0.0f : back == 0 ? q.y : back == 1 ? q.z : q.w;
+            t[u].z = !on || back >= 2 ? 0.0f : back == 0 ? q.z : q.w;
+            t[u].w = !on || back >= 1 ? 0.0f : q.w;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * kWgThreads < n) dst[i0 + u * kWgThreads] = t[u];
+    }
+}
+
 struct LaunchArgs {
     bool team;
     dim3 grid;
@@ -642,7 +680,7 @@ struct LaunchArgs {
     const float *X;
     float *Y;
     float *partial;
-    int N, ld, n_zero_rows, n_zero_groups;
+    int N, ldx, ld, n_zero_rows, n_zero_groups;
     const float *bias;
     int relu;
     const int32_t *long_slot;
@@ -660,22 +698,22 @@ void launch_one(const LaunchArgs &a)
         if (a.team)
             hipExtLaunchKernelGGL((spmm_team_kernel<L, VEC, kWide, kShift>), a.grid, dim3(kWgThreads), 0, a.stream,
                                   a.start_ev, a.stop_ev, 0, a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y,
-                                  a.partial, a.N, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
+                                  a.partial, a.N, a.ldx, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
                                   a.first_split_row, a.row_done);
         else
             hipExtLaunchKernelGGL((spmm_gather_kernel<L, VEC, kWide, kShift>), a.grid, dim3(kWgThreads), 0, a.stream,
                                   a.start_ev, a.stop_ev, 0, a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y,
-                                  a.partial, a.N, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
+                                  a.partial, a.N, a.ldx, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
                                   a.first_split_row, a.row_done);
         return;
     }
     if (a.team)
         spmm_team_kernel<L, VEC, kWide, kShift><<<a.grid, dim3(kWgThreads), 0, a.stream>>>(
-            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ld, a.n_zero_rows,
+            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ldx, a.ld, a.n_zero_rows,
             a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done);
     else
         spmm_gather_kernel<L, VEC, kWide, kShift><<<a.grid, dim3(kWgThreads), 0, a.stream>>>(
-            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ld, a.n_zero_rows,
+            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ldx, a.ld, a.n_zero_rows,
             a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done);
 }
 
@@ -775,24 +813,96 @@ int reserve_partial(accel_handle *h, size_t floats, bool any_stream)
     return ACCEL_OK;
 }
 
+// 128-byte lines that a row of N floats touches on average, rows ld floats apart from address x on.
+static double lines_per_row(uintptr_t x, int N, int64_t ld)
+{
+    const unsigned stride = (unsigned)(ld * 4 % 128);
+    unsigned step = 128;                              // the rows' places in a line are x, x + step, ...
+    while (stride % step) step /= 2;
+    int lines = 0, n = 0;
+    for (unsigned at = (unsigned)(x % step); at < 128; at += step, n++) lines += (int)((at + 4u * (unsigned)N + 127) / 128);
+    return (double)lines / n;
+}
+
+// Row stride, in floats, at which a gathered row touches as few lines as it can.
+static int whole_lines(int N) { return N <= 16 ? 16 : (N + 31) / 32 * 32; }
+
+// Seconds that a run saves when every row of X starts on a line instead of at x + i * ld.
+//
+// A gather is bound by the lines it pulls through the L2s, so what counts is how many of them are
+// saved: Gathered * lines / 7.2 TB/s if all of them missed.  Measured share of that (rows padded by
+// the caller against packed ones, power-law graphs of 8 to 125 M non-zeros): 0.4 at N = 14, 0.55 at
+// 25, 0.6 at 50, 0.8 at 90, 1.0 at 127; less when X nearly fits the L2s (X of 10 MB: a third);
+// 0.1 to 0.16 for a matrix whose non-zeros lie near the diagonal, where the rows share their lines.
+static double saved_by_padding(const accel_handle *h, uintptr_t x, int N, int64_t ld)
+{
+    if (N <= 8) return 0.0;                           // a padded row would take up twice the cache and more
+    const double lines = lines_per_row(x, N, ld) - lines_per_row(0, N, whole_lines(N));
+    const double mb = 4e-6 * (double)h->cols * N;
+    const double share = h->local ? 0.1 : std::min(1.0, 0.4 + 0.005 * N) * std::min(1.0, mb / 32);
+    return (double)h->nnz * lines * 128 / 7.2e12 * share;
+}
+
+// Stride at which a run with N columns wants the rows of an X that nobody has laid out yet: padded
+// to whole lines if that saves more than writing and fetching the padding costs.
+int row_stride(const accel_handle *h, int N)
+{
+    const double more = 8.0 * (double)h->cols * (whole_lines(N) - N) / 5e12;
+    return saved_by_padding(h, 0, N, N) > more ? whole_lines(N) : N;
+}
+
+// Whether a run copies X to padded rows first: it has to save more than the copy (one pass over X
+// at 5 TB/s, and a launch), with a fifth to spare.  That is graphs of some ten or more non-zeros per
+// row and column counts that packed rows suit badly.  Measured, whole runs, 2.45 M rows and 125 M
+// non-zeros: N = 25: 2.77 -> 1.92 ms (copy 0.09),
+// N = 50: 4.29 -> 3.67 (0.17), N = 127: 9.40 -> 7.54 (0.43); 8 M non-zeros in 400 k rows, N = 25: 181
+// -> 143 us, N = 50: 278 -> 275.
+static bool pads_x(const accel_handle *h, uintptr_t x, int N, int64_t ld)
+{
+    const double saved = saved_by_padding(h, x, N, ld);
+    return saved > 5e-6 && saved > 1.2 * (4e-6 + 4.0 * (double)h->cols * (N + whole_lines(N)) / 5e12);
+}
+
+// Room for X in padded rows, kept by the handle.  Not had: no error, the run takes X as it lies.
+static bool room_for_rows(accel_handle *h, size_t floats, bool any_stream)
+{
+    if (h->x_rows_floats >= floats) return true;
+    if (h->x_rows) {
+        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();     // nobody reads the old one
+        give_memory(h->x_rows, true);
+    }
+    h->x_rows_floats = 0;
+    h->x_rows = static_cast<float *>(take_memory(floats * sizeof(float), any_stream));
+    if (!h->x_rows) {
+        (void)hipGetLastError();
+        return false;
+    }
+    h->x_rows_floats = floats;
+    return true;
+}
+
+// All that a run with up to max_N columns allocates.
+int reserve_run(accel_handle *h, int max_N)
+{
+    if (int rc = reserve_partial(h, (size_t)h->n_long_units * (size_t)max_N, true)) return rc;
+    h->reserved_N = std::max(h->reserved_N, max_N);
+    size_t floats = 0;
+    for (int N = std::min(max_N, kPadMaxN); N > 0 && floats == 0; N--)
+        if (pads_x(h, 0, N, N)) floats = (size_t)h->cols * (size_t)whole_lines(N);
+    if (floats > 0 && floats <= kPadMaxFloats) (void)room_for_rows(h, floats, true);
+    return ACCEL_OK;
+}
+
 // main_start / main_stop: events bound to the gather kernel (to the first and the last launch
 // when the run is done in column panels), for timing it alone.
 int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t stream,
                 hipEvent_t main_start, hipEvent_t main_stop, const float *bias, int relu, bool static_partial,
-                int ld)
+                int ld, int ldx)
 {
     if (h->rows == 0) return ACCEL_OK;
     (void)hipGetLastError();                         // launch errors are read back below: start from a clean slate
-    if (ld <= 0) ld = N;                             // rows of X and Y are ld floats apart
-    // 16-byte vectors whenever a row holds one.  When N is not a multiple of 4, or X or Y
-    // is not 16-byte aligned, rows start at odd multiples of 4 bytes: the vectors are then
-    // loaded and stored at 4-byte aligned addresses, and a row's last vector is moved back
-    // so that it ends with the row (it overlaps the one before; both lanes hold the same
-    // sums for the shared columns).  Scalar lanes are left for N < 4.
-    const uintptr_t align = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y);
-    const int mode = N < 4 ? 2 : (N % 4 == 0 && ld % 4 == 0 && align % 16 == 0) ? 0 : 1;
-    const int vec = mode == 2 ? 1 : 4;
-
+    if (ld <= 0) ld = N;                             // rows of Y are ld floats apart
+    if (ldx <= 0) ldx = ld;                          // those of X ldx
     // partial sums of the pieces of split rows: the handle's buffer (allocated here when a
     // run needs more than it holds), or this GPU's static array, which is never allocated
     float *partial = h->partial;
@@ -800,7 +910,8 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // the capture status is only asked for where something depends on it: a buffer that would
     // have to grow, or a stream the handle would have to order against another
     const bool must_grow = uses_handle_partial && h->partial_floats < (size_t)h->n_long_units * (size_t)ld;
-    const bool capturing = (must_grow || needs_capture_status(h, stream)) && stream_is_capturing(stream);
+    bool pad = !static_partial && N <= kPadMaxN && pads_x(h, reinterpret_cast<uintptr_t>(X), N, ldx);
+    const bool capturing = (must_grow || pad || needs_capture_status(h, stream)) && stream_is_capturing(stream);
     if (static_partial) {
         partial = nullptr;
         const size_t need = (size_t)h->n_long_units * (size_t)ld;
@@ -824,11 +935,35 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
         }
         partial = h->partial;
     }
+    // X copied to padded rows.  Not while capturing: the graph would keep the address of a buffer
+    // that a later run may replace.
+    if (pad) {
+        const size_t need = (size_t)h->cols * (size_t)whole_lines(N);
+        pad = !capturing && need <= kPadMaxFloats &&
+              (h->x_rows_floats >= need || (N > h->reserved_N && room_for_rows(h, need, stream != nullptr)));
+    }
     // The buffer is shared by all runs of this handle, and a value update may still be
     // rewriting what this run reads: a run on another stream than the one that used them
     // last waits for that stream on the device (runs queued on one stream are ordered anyway).
     hipEvent_t run_done = nullptr;                  // to be bound to the run's last kernel
-    if (int rc = order_run(h, stream, uses_handle_partial, capturing, &run_done)) return rc;
+    if (int rc = order_run(h, stream, uses_handle_partial || pad, capturing, &run_done)) return rc;
+    if (pad) {
+        const int to = whole_lines(N);
+        const dim3 grid((unsigned)((h->cols + kPadRows - 1) / kPadRows));
+        hipExtLaunchKernelGGL(pad_rows_kernel, grid, dim3(kWgThreads), 0, stream, main_start, nullptr, 0, X, (int64_t)h->cols,
+                              N, (int64_t)ldx, h->x_rows, to);
+        main_start = nullptr;
+        X = h->x_rows;
+        ldx = to;
+    }
+    // 16-byte vectors whenever a row holds one.  When N is not a multiple of 4, or X or Y
+    // is not 16-byte aligned, rows start at odd multiples of 4 bytes: the vectors are then
+    // loaded and stored at 4-byte aligned addresses, and a row's last vector is moved back
+    // so that it ends with the row (it overlaps the one before; both lanes hold the same
+    // sums for the shared columns).  Scalar lanes are left for N < 4.
+    const uintptr_t align = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y);
+    const int mode = N < 4 ? 2 : (N % 4 == 0 && ld % 4 == 0 && ldx % 4 == 0 && align % 16 == 0) ? 0 : 1;
+    const int vec = mode == 2 ? 1 : 4;
     // split rows are added up by the gather kernel itself (the wavefront that stores a row's
     // last piece), or, when the handle has no counters for that, by a second kernel
     int *row_done = h->fused_reduce ? h->row_done : nullptr;
@@ -839,15 +974,18 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // Measured (panel 64 against one pass): N = 256 on the hub graph -12 %, N = 128 on the
     // dense and the power-law 100 M-non-zero graphs -7 % and -4 %; no gain when the
     // columns have no popularity skew or the rows are very short, and a loss when N is
-    // not a multiple of the panel (N = 100: 64 + 36 leaves lanes idle).
+    // not a multiple of the panel (N = 100: 64 + 36 leaves lanes idle).  Rows that lie on whole
+    // lines count as wide as their lines: N = 127 at a stride of 128, 125 M non-zeros: -5 %.
     int panel = N;
     const int want = h->plan_panel_option > 0 ? h->plan_panel_option : kPanel;
     const bool forced = h->plan_panel_option > 0;
-    if (mode == 0 && N > want &&
-        (forced || (N % want == 0 && h->nnz >= kPanelMinNnz && h->nnz >= 16 * h->rows)))
+    const bool even = (mode == 0 && N % want == 0) ||                       // panels of whole lines
+                      (mode != 2 && ldx % 32 == 0 && whole_lines(N) % want == 0);
+    if (N > want &&
+        ((forced && mode == 0) || (!forced && even && h->nnz >= kPanelMinNnz && h->nnz >= 16 * h->rows)))
         panel = want;
     // operands below 4 GiB are addressed with 32-bit byte offsets (see gather_row)
-    const bool wide = (uint64_t)h->cols * (uint64_t)ld * 4u > 0xFFFFFFFFull;
+    const bool wide = (uint64_t)h->cols * (uint64_t)ldx * 4u > 0xFFFFFFFFull;
     const int4 *wk = reinterpret_cast<const int4 *>(h->work);
     const int64_t entry_groups = h->plan_team ? h->n_units : h->n_units / kWaves;
     for (int c0 = 0; c0 < N; c0 += panel) {
@@ -873,7 +1011,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
         hipEvent_t stop = last ? main_stop : nullptr;
         if (last && !stop && !has_reduce) stop = run_done;      // the run ends with this launch
         const LaunchArgs la{h->plan_team, grid, stream, wk, (int)h->n_units, h->s_idx, h->s_val, h->perm,
-                            Xp, Yp, Pp, n, ld, (int)h->n_zero_rows, (int)zero_groups, bp, relu,
+                            Xp, Yp, Pp, n, ldx, ld, (int)h->n_zero_rows, (int)zero_groups, bp, relu,
                             h->long_slot, (int)(h->rows - h->n_split_rows), row_done,
                             first ? main_start : nullptr, stop};
         const int rc = launch_for_mode(mode, wide, L, la);

@@ -63,12 +63,14 @@ class GcnLayer:
             if b.shape != (self.N,):
                 raise AccelError(_lib.ERR_ARG, f"bias must hold {self.N} floats")
             self._b = DeviceBuffer.from_numpy(b)
-        self._z = DeviceBuffer(max(op.n_cols * self.N * 4, 4))      # X W: the sparse product's dense operand
+        # X W, the sparse product's dense operand, in the layout that gathers best
+        self._ldz = op.row_stride(self.N)
+        self._z = DeviceBuffer(max(op.n_cols * self._ldz * 4, 4))
 
     def forward(self, X, Y, stream=None) -> None:
         """X: ``n_cols x K`` on the device, Y: ``n_rows x N`` on the device."""
-        dense_xw(X, self._w, self._z, self.op.n_cols, self.K, self.N, stream=stream)
-        self.op.run_epilogue(self._z, Y, self.N, bias=self._b, relu=self.relu, stream=stream)
+        dense_xw(X, self._w, self._z, self.op.n_cols, self.K, self.N, ldz=self._ldz, stream=stream)
+        self.op.run_ex(self._z, Y, self.N, bias=self._b, relu=self.relu, stream=stream, ldx=self._ldz)
 
     def forward_numpy(self, X: np.ndarray) -> np.ndarray:
         X = _lib.as_f32(X)

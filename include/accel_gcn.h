@@ -333,12 +333,27 @@ typedef struct accel_run_args {
 } accel_run_args;
 int accel_run_ex(accel_handle *h, const accel_run_args *args);
 
-/* accel_run keeps the partial sums of split rows (pieces x N floats) in a buffer of the
+/* accel_run_ex with rows of X `ldx` floats apart (0 = packed) and rows of Y args->ld apart, for a
+ * caller that lays X out itself but not Y (GcnLayer: its X is the dense product's output).
+ * accel_row_stride names the stride at which this matrix gathers rows of N floats best: N, or N
+ * rounded up to whole cache lines where that pays (N before accel_preprocess; 0 and an error message
+ * for bad arguments).
+ * Floats between the rows are never read. */
+int accel_row_stride(const accel_handle *h, int32_t N);
+int accel_run_rows(accel_handle *h, const accel_run_args *args, int32_t ldx);
+
+/* Where packed rows of X touch many more cache lines than whole ones would, the columns are not
+ * near the diagonal and the matrix has enough non-zeros per row, a run first copies X to padded
+ * rows in a buffer that the handle keeps (below 4 GiB; one pass over X).
+ * Not while its stream captures, and not for accel_run_static.
+ *
+ * accel_run keeps the partial sums of split rows (pieces x N floats) in a buffer of the
  * handle.  It is allocated by the first accel_run with a given N and replaced by a larger
  * one when a later run brings a larger N; a HIP graph captured with the old buffer must
  * then be captured again.  accel_reserve allocates it for every N up to max_N at once, so
  * that no later accel_run with N <= max_N allocates or frees: call it before capturing a
- * graph or entering a loop that must not allocate (a run that would have to grow the
+ * graph or entering a loop that must not allocate; it allocates the buffer for padded
+ * rows too, if any of these N would use it (a run that would have to grow the
  * buffer while its stream is capturing fails with ACCEL_ERR_STATE).  No counterpart
  * upstream, whose kernel adds split rows up with atomicAdd (spmm_accel.cu:84,97). */
 int accel_reserve(accel_handle *h, int32_t max_N);
