@@ -96,7 +96,7 @@ struct accel_handle {
     int64_t n_units = 0;              // multiple of 4 * plan_queues
     int64_t n_long_units = 0;         // units that write a partial sum
     int32_t *long_slot = nullptr;     // [n_split_rows+1] partial-sum slots of each split row
-    int32_t *row_done = nullptr;      // [n_split_rows] pieces of each split row stored so far in the running
+    int32_t *row_done = nullptr;      // [2 * n_split_rows] pieces of each split row stored so far in the running
                                       // launch; zero between launches (part of the long_slot allocation)
     int plan_reduce_option = 0;       // 0: choose (in the gather kernel); 1: in the gather kernel; 2: second kernel
     bool fused_reduce = true;         // split rows are added up by the gather kernel itself

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(
         const int total = wave_sum(u);
         if (lane == 0) {
             row_units[lr] = total;
-            row_done[lr] = 0;
+            row_done[lr] = row_done[n_split + lr] = 0;
         }
     }
     cost += __shfl_xor(cost, 8);
@@ -361,9 +361,9 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
     int *row_units = nullptr, *bins = nullptr;
     PlanHead *head;
     if ((rc = tmp->alloc(&head, 1))) return rc;
-    // the slots of each split row, and behind them one counter per split row (zero between launches)
+    // the slots of each split row, and behind them two counters per split row (zero between launches)
     DevBuf dslot;
-    if ((rc = dslot.alloc(sizeof(int) * (size_t)(2 * (int64_t)n_split + 1)))) return rc;
+    if ((rc = dslot.alloc(sizeof(int) * (size_t)(3 * (int64_t)n_split + 1)))) return rc;
     int *slot = dslot.as<int>(), *row_done = slot + n_split + 1;
     if (n_split > 0) {
         if ((rc = tmp->alloc(&row_units, (size_t)n_split))) return rc;

@@ -272,6 +272,28 @@ __device__ __forceinline__ void zero_fill_rows(const int32_t *__restrict__ perm,
     }
 }
 
+// A launch over two column halves (see spmm_launch): the even dies compute columns 0 .. half-1, the
+// odd ones the others, and two neighbours go through the workgroups of both their queues in the
+// same order.  wg, of n in one half: workgroup of the launch in, workgroup of the plan out.
+__device__ __forceinline__ void take_half(int n, int half, int n_split, int &wg, const float *__restrict__ &X,
+                                          float *__restrict__ &Y, float *__restrict__ &partial, int &N,
+                                          const float *__restrict__ &bias, int *__restrict__ &row_done)
+{
+    const int die = wg % kXcds, i = wg / kXcds, per_queue = n / kXcds;
+    const int second = i >= per_queue;
+    wg = (i - (second ? per_queue : 0)) * kXcds + (die & ~1) + second;
+    if (die & 1) {
+        X += half;
+        Y += half;
+        partial += half;
+        if (row_done) row_done += n_split;           // a counter per row and half
+        if (bias) bias += half;
+        N -= half;
+    } else {
+        N = half;
+    }
+}
+
 template <int L, int VEC, bool kWide, bool kShift>
 __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
     const int4 *__restrict__ work, int n_units,
@@ -279,7 +301,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
     const int32_t *__restrict__ perm, const float *__restrict__ X, float *__restrict__ Y,
     float *__restrict__ partial, int N, int ldx, int ld, int n_zero_rows, int n_zero_groups,
     const float *__restrict__ bias, int relu, const int32_t *__restrict__ long_slot, int first_split_row,
-    int *__restrict__ row_done)
+    int *__restrict__ row_done, int half, int n_split)
 {
     // N columns are computed; rows of X are ldx floats apart, those of Y and the partial sums ld
     // (more than N when the launch covers one column panel of a wider operand)
@@ -294,7 +316,9 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
 
     const int lane = threadIdx.x & 63;
     const int wv = uniform(threadIdx.x >> 6);
-    const int e = ((int)blockIdx.x - n_zero_groups) * kWaves + wv;
+    int wg = (int)blockIdx.x - n_zero_groups;
+    if (half > 0) take_half(n_units / kWaves, half, n_split, wg, X, Y, partial, N, bias, row_done);
+    const int e = wg * kWaves + wv;
     if (e >= n_units) return;
 
     const int4 b = work[e];
@@ -686,6 +710,7 @@ struct LaunchArgs {
     const int32_t *long_slot;
     int first_split_row;
     int *row_done;
+    int half, n_split;
     // events bound to this launch itself (its start and its end), or null: unlike an event
     // recorded behind the launch they put no packet of their own into the queue
     hipEvent_t start_ev, stop_ev;
@@ -704,7 +729,7 @@ void launch_one(const LaunchArgs &a)
             hipExtLaunchKernelGGL((spmm_gather_kernel<L, VEC, kWide, kShift>), a.grid, dim3(kWgThreads), 0, a.stream,
                                   a.start_ev, a.stop_ev, 0, a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y,
                                   a.partial, a.N, a.ldx, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
-                                  a.first_split_row, a.row_done);
+                                  a.first_split_row, a.row_done, a.half, a.n_split);
         return;
     }
     if (a.team)
@@ -714,7 +739,7 @@ void launch_one(const LaunchArgs &a)
     else
         spmm_gather_kernel<L, VEC, kWide, kShift><<<a.grid, dim3(kWgThreads), 0, a.stream>>>(
             a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ldx, a.ld, a.n_zero_rows,
-            a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done);
+            a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done, a.half, a.n_split);
 }
 
 // Lane-group widths: 1..64 lanes of one 16-byte vector each; scalar lanes only serve N < 4.
@@ -837,8 +862,12 @@ static int whole_lines(int N) { return N <= 16 ? 16 : (N + 31) / 32 * 32; }
 static double saved_by_padding(const accel_handle *h, uintptr_t x, int N, int64_t ld)
 {
     if (N <= 8) return 0.0;                           // a padded row would take up twice the cache and more
-    const double lines = lines_per_row(x, N, ld) - lines_per_row(0, N, whole_lines(N));
+    double lines = lines_per_row(x, N, ld) - lines_per_row(0, N, whole_lines(N));
     const double mb = 4e-6 * (double)h->cols * N;
+    // rows of whole lines can also be computed in column panels (see spmm_launch): a twelfth less
+    // where X is not many times what the L2s hold
+    if (N > kPanel && N % kPanel != 0 && whole_lines(N) % kPanel == 0)
+        lines += whole_lines(N) / (32 * 12.0) * std::min(1.0, 100 / mb);
     const double share = h->local ? 0.1 : std::min(1.0, 0.4 + 0.005 * N) * std::min(1.0, mb / 32);
     return (double)h->nnz * lines * 128 / 7.2e12 * share;
 }
@@ -984,20 +1013,31 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     if (N > want &&
         ((forced && mode == 0) || (!forced && even && h->nnz >= kPanelMinNnz && h->nnz >= 16 * h->rows)))
         panel = want;
+    // With more than one panel, two neighbouring panels are computed in one launch, each by every
+    // other die: a die then sees twice the units but half of every row of X, so that what it fetches
+    // into its L2 serves twice the gathers.  Also where several launches would not pay.  Measured at
+    // N = 128 / 256: 1.5 M non-zeros in 50 k rows 77 -> 62 / 172 -> 126 us, 2.4 M in 170 k 139 -> 126 /
+    // 302 -> 258, 10 M in 1 M 724 -> 695 / 1471 -> 1400, 114 M in 233 k 3.46 -> 3.32 / 6.94 -> 6.60 ms,
+    // 125 M in 2.45 M 7.00 -> 6.92 / 14.4 -> 13.8; five per row 389 -> 391 / 808.  Halves of 32 columns
+    // at N = 64 lose (3.40 -> 3.57 ms on the last): as much staging for half the lines.  So do workgroup
+    // units (208 k non-zeros: 12.2 -> 15.1 us), which are bound by latency.  Both dies go through the
+    // same queue at the same time: through different ones is 5 to 10 % slower.
+    const bool halves = even && !forced && N > want && !h->plan_team && h->plan_queues == kXcds;
     // operands below 4 GiB are addressed with 32-bit byte offsets (see gather_row)
     const bool wide = (uint64_t)h->cols * (uint64_t)ldx * 4u > 0xFFFFFFFFull;
     const int4 *wk = reinterpret_cast<const int4 *>(h->work);
     const int64_t entry_groups = h->plan_team ? h->n_units : h->n_units / kWaves;
-    for (int c0 = 0; c0 < N; c0 += panel) {
-        const int n = std::min(panel, N - c0);
+    for (int c0 = 0, n; c0 < N; c0 += n) {
+        const int half = halves && N - c0 > want ? want : 0;
+        n = half ? std::min(2 * half, N - c0) : std::min(panel, N - c0);
         int L = 1;                                   // lanes per row: one per vector, a power of two
-        while (L * vec < n && L < 64) L <<= 1;
+        while (L * vec < (half ? half : n) && L < 64) L <<= 1;
         // zero-fill workgroups come first; their count is rounded up to a multiple of the
         // queue count so that entry group i still lands on die i % 8 (surplus ones exit at once)
         const int zr = zero_rows_per_group(n);
         int64_t zero_groups = (h->n_zero_rows + zr - 1) / zr;
         zero_groups = (zero_groups + h->plan_queues - 1) / h->plan_queues * h->plan_queues;
-        const int64_t groups = entry_groups + zero_groups;
+        const int64_t groups = entry_groups * (half ? 2 : 1) + zero_groups;
         if (groups > 0x7fffffffLL) {
             set_error("launch of %lld workgroups exceeds the grid limit", (long long)groups);
             return ACCEL_ERR_ARG;
@@ -1007,12 +1047,12 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
         const float *Xp = X ? X + c0 : X;
         float *Yp = Y + c0, *Pp = partial ? partial + c0 : nullptr;
         const float *bp = bias ? bias + c0 : nullptr;
-        const bool first = c0 == 0, last = c0 + panel >= N;
+        const bool first = c0 == 0, last = c0 + n >= N;
         hipEvent_t stop = last ? main_stop : nullptr;
         if (last && !stop && !has_reduce) stop = run_done;      // the run ends with this launch
         const LaunchArgs la{h->plan_team, grid, stream, wk, (int)h->n_units, h->s_idx, h->s_val, h->perm,
                             Xp, Yp, Pp, n, ldx, ld, (int)h->n_zero_rows, (int)zero_groups, bp, relu,
-                            h->long_slot, (int)(h->rows - h->n_split_rows), row_done,
+                            h->long_slot, (int)(h->rows - h->n_split_rows), row_done, half, (int)h->n_split_rows,
                             first ? main_start : nullptr, stop};
         const int rc = launch_for_mode(mode, wide, L, la);
         if (rc) return rc;
