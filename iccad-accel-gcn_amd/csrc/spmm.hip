@@ -294,14 +294,15 @@ __device__ __forceinline__ void take_half(int n, int half, int n_split, int &wg,
     }
 }
 
+// The first 14 words of arguments are in registers when a wavefront starts (see build.py); what the
+// way to the first load needs comes first.
 template <int L, int VEC, bool kWide, bool kShift>
 __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
-    const int4 *__restrict__ work, int n_units,
-    const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
-    const int32_t *__restrict__ perm, const float *__restrict__ X, float *__restrict__ Y,
-    float *__restrict__ partial, int N, int ldx, int ld, int n_zero_rows, int n_zero_groups,
+    const int4 *__restrict__ work, const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
+    const int32_t *__restrict__ perm, int n_units, int n_zero_groups, int half, int N, int ldx, int ld,
+    const float *__restrict__ X, float *__restrict__ Y, float *__restrict__ partial, int n_zero_rows,
     const float *__restrict__ bias, int relu, const int32_t *__restrict__ long_slot, int first_split_row,
-    int *__restrict__ row_done, int half, int n_split)
+    int *__restrict__ row_done, int n_split)
 {
     // N columns are computed; rows of X are ldx floats apart, those of Y and the partial sums ld
     // (more than N when the launch covers one column panel of a wider operand)
@@ -430,10 +431,9 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
 // times shorter and rows of up to one unit need no partial sums.
 template <int L, int VEC, bool kWide, bool kShift>
 __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
-    const int4 *__restrict__ work, int n_units,
-    const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
-    const int32_t *__restrict__ perm, const float *__restrict__ X, float *__restrict__ Y,
-    float *__restrict__ partial, int N, int ldx, int ld, int n_zero_rows, int n_zero_groups,
+    const int4 *__restrict__ work, const int32_t *__restrict__ s_idx, const float *__restrict__ s_val,
+    const int32_t *__restrict__ perm, int n_units, int n_zero_groups, int N, int ldx, const float *__restrict__ X,
+    float *__restrict__ Y, int ld, float *__restrict__ partial, int n_zero_rows,
     const float *__restrict__ bias, int relu, const int32_t *__restrict__ long_slot, int first_split_row,
     int *__restrict__ row_done)
 {
@@ -719,27 +719,21 @@ struct LaunchArgs {
 template <int L, int VEC, bool kWide, bool kShift>
 void launch_one(const LaunchArgs &a)
 {
-    if (a.start_ev || a.stop_ev) {
-        if (a.team)
-            hipExtLaunchKernelGGL((spmm_team_kernel<L, VEC, kWide, kShift>), a.grid, dim3(kWgThreads), 0, a.stream,
-                                  a.start_ev, a.stop_ev, 0, a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y,
-                                  a.partial, a.N, a.ldx, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
-                                  a.first_split_row, a.row_done);
+    // (a launch with events costs the host more than one without)
+    auto launch = [&](auto kernel, auto... args) {
+        if (a.start_ev || a.stop_ev)
+            hipExtLaunchKernelGGL(kernel, a.grid, dim3(kWgThreads), 0, a.stream, a.start_ev, a.stop_ev, 0, args...);
         else
-            hipExtLaunchKernelGGL((spmm_gather_kernel<L, VEC, kWide, kShift>), a.grid, dim3(kWgThreads), 0, a.stream,
-                                  a.start_ev, a.stop_ev, 0, a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y,
-                                  a.partial, a.N, a.ldx, a.ld, a.n_zero_rows, a.n_zero_groups, a.bias, a.relu, a.long_slot,
-                                  a.first_split_row, a.row_done, a.half, a.n_split);
-        return;
-    }
+            kernel<<<a.grid, dim3(kWgThreads), 0, a.stream>>>(args...);
+    };
     if (a.team)
-        spmm_team_kernel<L, VEC, kWide, kShift><<<a.grid, dim3(kWgThreads), 0, a.stream>>>(
-            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ldx, a.ld, a.n_zero_rows,
-            a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done);
+        launch(spmm_team_kernel<L, VEC, kWide, kShift>, a.work, a.s_idx, a.s_val, a.perm, a.n_units, a.n_zero_groups, a.N,
+               a.ldx, a.X, a.Y, a.ld, a.partial, a.n_zero_rows, a.bias, a.relu, a.long_slot, a.first_split_row,
+               a.row_done);
     else
-        spmm_gather_kernel<L, VEC, kWide, kShift><<<a.grid, dim3(kWgThreads), 0, a.stream>>>(
-            a.work, a.n_units, a.s_idx, a.s_val, a.perm, a.X, a.Y, a.partial, a.N, a.ldx, a.ld, a.n_zero_rows,
-            a.n_zero_groups, a.bias, a.relu, a.long_slot, a.first_split_row, a.row_done, a.half, a.n_split);
+        launch(spmm_gather_kernel<L, VEC, kWide, kShift>, a.work, a.s_idx, a.s_val, a.perm, a.n_units, a.n_zero_groups,
+               a.half, a.N, a.ldx, a.ld, a.X, a.Y, a.partial, a.n_zero_rows, a.bias, a.relu, a.long_slot,
+               a.first_split_row, a.row_done, a.n_split);
 }
 
 // Lane-group widths: 1..64 lanes of one 16-byte vector each; scalar lanes only serve N < 4.
