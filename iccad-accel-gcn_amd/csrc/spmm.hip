@@ -56,7 +56,6 @@ constexpr int kReduceThreads = 256;       // workgroup of the partial-sum reduct
 __host__ __device__ inline int zero_rows_per_group(int N) { return N >= kZeroFloats ? 1 : kZeroFloats / N; }
 
 constexpr int kUnroll = 4;                // gathers in flight per lane in the main loop (2 and 8 measured within 2 %)
-constexpr int kTeamUnroll = 4;            // the same with workgroup units (8: 5-10 % slower)
 constexpr int kPanel = 64;                // column-panel width for wide operands on large matrices
 constexpr int kPanelMinNnz = 4000000;     // smaller matrices are not worth several launches
 constexpr int kPadRows = 64;              // rows that a workgroup of pad_rows_kernel copies
@@ -189,63 +188,100 @@ __device__ __forceinline__ void finish_split_row(const float *__restrict__ src, 
     }
 }
 
-// One lane group's share of one row: non-zeros k, k + gp, ... of the d pairs at row_st are
-// multiplied with their rows of X and added into acc.  U gathers are issued back to back;
-// full batches carry no masks, only the last batch of a row is predicated.
-// The staged pair holds the value and, when the operand is smaller than 4 GiB (kWide ==
-// false), the byte offset of the row of X, so that the address is one 32-bit add to a
-// uniform base; otherwise the column, and the address is formed with 64-bit arithmetic.
-template <int VEC, int U, bool kWide, bool kShift>
-__device__ __forceinline__ void gather_row(const int2 *__restrict__ row_st, int d, int k, int gp,
-                                           const float *__restrict__ X, int col, int ldx,
-                                           float (&acc)[VEC])
+// Stages the n pairs at idx, val in LDS, R rounds of T threads (T * (R - 1) < n <= T * R).  All loads are
+// issued before the first is waited for: nothing depends on the thread but the last round's index, which
+// is clamped.  (Loads under a condition per round make the compiler wait for one round before it issues
+// the next.)  st has room for what the last round writes behind the n-th pair.
+template <int R, int T, bool kWide>
+__device__ __forceinline__ void stage_rounds(const int32_t *__restrict__ idx, const float *__restrict__ val, int n, int tid,
+                                             int ldx, int2 *st)
 {
-    const char *xb = reinterpret_cast<const char *>(X);
-    const uint32_t lane_off = (uint32_t)col * 4u;
-    auto fetch = [&](int where, float (&x)[VEC]) {
-        if constexpr (kWide)
-            load_vec<VEC, kShift>(X + col + (int64_t)where * ldx, x);
-        else
-            load_vec<VEC, kShift>(reinterpret_cast<const float *>(xb + ((uint32_t)where + lane_off)), x);
-    };
+    int c[R];
+    float v[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const uint32_t i = (uint32_t)(j < R - 1 ? tid + T * j : min(tid + T * j, n - 1));
+        c[j] = idx[i];
+        v[j] = val[i];
+    }
+#pragma unroll
+    for (int j = 0; j < R; j++)
+        st[tid + T * j] = make_int2(kWide ? c[j] : (int)((uint32_t)c[j] * ((uint32_t)ldx * 4u)), __float_as_int(v[j]));
+}
+
+// The vector of row `where` of X at column col.  The staged pair holds the value and, when the operand is
+// smaller than 4 GiB (kWide == false), the byte offset of the row, so that the address is one 32-bit add
+// to a uniform base; otherwise the column, and the address is formed with 64-bit arithmetic.
+template <int VEC, bool kWide, bool kShift>
+__device__ __forceinline__ void fetch_row(const float *__restrict__ X, int where, int col, int ldx, float (&x)[VEC])
+{
+    if constexpr (kWide)
+        load_vec<VEC, kShift>(X + col + (int64_t)where * ldx, x);
+    else
+        load_vec<VEC, kShift>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(X) +
+                                                              ((uint32_t)where + (uint32_t)col * 4u)), x);
+}
+
+// S non-zeros (o, o + gp, ...) of a row, all gathers issued back to back, added in order into acc; the
+// last of them may lie behind the row's end (d).
+template <int S, int VEC, bool kWide, bool kShift>
+__device__ __forceinline__ void gather_steps(const int2 *row_st, int o, int gp, int d, const float *__restrict__ X, int col,
+                                             int ldx, float (&acc)[VEC])
+{
+    const int last = o + (S - 1) * gp;
+    const bool on = last < d;
+    int2 p[S];
+    float x[S][VEC];
+#pragma unroll
+    for (int s = 0; s < S; s++) p[s] = row_st[s < S - 1 ? o + s * gp : min(last, d - 1)];
+#pragma unroll
+    for (int s = 0; s < S; s++) fetch_row<VEC, kWide, kShift>(X, p[s].x, col, ldx, x[s]);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        const bool use = s < S - 1 || on;
+        const float a = use ? __int_as_float(p[s].y) : 0.0f;
+#pragma unroll
+        for (int v = 0; v < VEC; v++) acc[v] = fmaf(a, use ? x[s][v] : 0.0f, acc[v]);
+    }
+}
+
+// One lane group's share of one row: non-zeros k, k + gp, ... of its d pairs, in full batches of four, and
+// the rest in as many steps as there are (a gather under a condition of its own per step took as long to
+// issue as four).  d and gp are the same for the whole wavefront: the branches are scalar ones.
+// Together with the staging above: 114 M non-zeros, N = 64: 1748 -> 1704 us; 4 M next to the diagonal,
+// N = 64: 205 -> 192; 8 M, N = 32: 104 -> 91; 208 k, N = 32: 7.9 -> 7.6.  Several row sets at a time
+// (gathers of up to three rows per lane group together) need 64 and more registers: 203 and 103 us.
+template <int VEC, bool kWide, bool kShift>
+__device__ __forceinline__ void gather_row(const int2 *row_st, int d, int k, int lg, const float *__restrict__ X, int col,
+                                           int ldx, float (&acc)[VEC])
+{
+    static_assert(kUnroll == 4, "the steps of a rest are dealt with one by one");
+    const int gp = 1 << lg, full = d >> (lg + 2);
     int o = k;
-    for (; o + (U - 1) * gp < d; o += U * gp) {          // full batches
-        int2 p[U];
-        float x[U][VEC];
+    for (int i = 0; i < full; i++, o += kUnroll * gp) {
+        int2 p[kUnroll];
+        float x[kUnroll][VEC];
 #pragma unroll
-        for (int u = 0; u < U; u++) p[u] = row_st[o + u * gp];
+        for (int u = 0; u < kUnroll; u++) p[u] = row_st[o + u * gp];
 #pragma unroll
-        for (int u = 0; u < U; u++) fetch(p[u].x, x[u]);
+        for (int u = 0; u < kUnroll; u++) fetch_row<VEC, kWide, kShift>(X, p[u].x, col, ldx, x[u]);
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const float a = __int_as_float(p[u].y);
+        for (int u = 0; u < kUnroll; u++)
 #pragma unroll
-            for (int v = 0; v < VEC; v++) acc[v] = fmaf(a, x[u][v], acc[v]);
-        }
+            for (int v = 0; v < VEC; v++) acc[v] = fmaf(__int_as_float(p[u].y), x[u][v], acc[v]);
     }
-    if (o < d) {                                         // the row's last, partial batch
-        int2 p[U];
-        float x[U][VEC];
-        bool ok[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ou = o + u * gp;
-            ok[u] = ou < d;
-            p[u] = row_st[ok[u] ? ou : k];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-#pragma unroll
-            for (int v = 0; v < VEC; v++) x[u][v] = 0.0f;
-            if (ok[u]) fetch(p[u].x, x[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const float a = ok[u] ? __int_as_float(p[u].y) : 0.0f;
-#pragma unroll
-            for (int v = 0; v < VEC; v++) acc[v] = fmaf(a, x[u][v], acc[v]);
-        }
+    switch ((d - full * kUnroll * gp + gp - 1) >> lg) {
+    case 1: gather_steps<1, VEC, kWide, kShift>(row_st, o, gp, d, X, col, ldx, acc); break;
+    case 2: gather_steps<2, VEC, kWide, kShift>(row_st, o, gp, d, X, col, ldx, acc); break;
+    case 3: gather_steps<3, VEC, kWide, kShift>(row_st, o, gp, d, X, col, ldx, acc); break;
+    case 4: gather_steps<4, VEC, kWide, kShift>(row_st, o, gp, d, X, col, ldx, acc); break;
     }
+}
+
+// v of the lane whose number differs in bit m.
+__device__ __forceinline__ float from_lane_xor(float v, int lane, int m)
+{
+    return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ m) << 2, __float_as_int(v)));
 }
 
 // Zero-degree rows are the first n_zero_rows rows of the sorted order; the workgroups at
@@ -332,27 +368,19 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
 
     // output row of each of the unit's rows, fetched up front (lane r holds row r)
     int my_out = row0 + lane;
-    if (!is_long && perm && lane < n_rows) my_out = perm[row0 + lane];
+    if (!is_long && perm) my_out = perm[row0 + min(lane, n_rows - 1)];
 
-    // stage the entry's (column, value) pairs: all loads are issued before the first LDS write
     int2 *st = stage[wv];
     {
-        constexpr int kRounds = kDegBound / 64;
-        int ci[kRounds];
-        float cv[kRounds];
-#pragma unroll
-        for (int j = 0; j < kRounds; j++) {
-            const int i = lane + 64 * j;
-            if (i < total_nz) {
-                ci[j] = s_idx[loc + i];
-                cv[j] = s_val[loc + i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kRounds; j++) {
-            const int i = lane + 64 * j;
-            if (i < total_nz) st[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ldx * 4u)), __float_as_int(cv[j]));
-        }
+        const int32_t *idx = s_idx + loc;
+        const float *val = s_val + loc;
+        static_assert(kDegBound == 6 * 64, "rounds of staging");
+        if (total_nz <= 64) stage_rounds<1, 64, kWide>(idx, val, total_nz, lane, ldx, st);
+        else if (total_nz <= 128) stage_rounds<2, 64, kWide>(idx, val, total_nz, lane, ldx, st);
+        else if (total_nz <= 192) stage_rounds<3, 64, kWide>(idx, val, total_nz, lane, ldx, st);
+        else if (total_nz <= 256) stage_rounds<4, 64, kWide>(idx, val, total_nz, lane, ldx, st);
+        else if (total_nz <= 320) stage_rounds<5, 64, kWide>(idx, val, total_nz, lane, ldx, st);
+        else stage_rounds<6, 64, kWide>(idx, val, total_nz, lane, ldx, st);
     }
     __builtin_amdgcn_wave_barrier();
 
@@ -384,11 +412,11 @@ __global__ __launch_bounds__(kWgThreads) void spmm_gather_kernel(
             float acc[VEC];
 #pragma unroll
             for (int v = 0; v < VEC; v++) acc[v] = 0.0f;
-            if (live) gather_row<VEC, kUnroll, kWide, kShift>(st + r * d, d, k, gp, X, col, ldx, acc);
+            if (live) gather_row<VEC, kWide, kShift>(st + r * d, d, k, lg, X, col, ldx, acc);
             // add the gp partial sums of each row (all lanes take part)
             for (int m = L; m < (L << lg); m <<= 1) {
 #pragma unroll
-                for (int v = 0; v < VEC; v++) acc[v] += __shfl_xor(acc[v], m);
+                for (int v = 0; v < VEC; v++) acc[v] += from_lane_xor(acc[v], lane, m);
             }
             const int64_t out_row = __shfl(my_out, r < n_rows ? r : 0);
             if (live && k == 0) {
@@ -440,7 +468,7 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
     constexpr int G = 64 / L;        // lane groups per wavefront
     constexpr int TG = G * kWaves;   // lane groups per workgroup
     constexpr int CW = L * VEC;      // columns covered per pass
-    __shared__ int2 stage[kDegBound];
+    __shared__ int2 stage[2 * kWgThreads];
     __shared__ float meet[kWaves][CW];
 
     if ((int)blockIdx.x < n_zero_groups) {
@@ -462,24 +490,12 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
     int my_out = row0 + lane;
     if (!is_long && perm && lane < n_rows) my_out = perm[row0 + lane];
 
-    {   // stage the unit's (column, value) pairs: 256 threads, at most two rounds
-        constexpr int kRounds = (kDegBound + kWgThreads - 1) / kWgThreads;
-        int ci[kRounds];
-        float cv[kRounds];
-#pragma unroll
-        for (int j = 0; j < kRounds; j++) {
-            const int i = (int)threadIdx.x + kWgThreads * j;
-            if (i < total_nz) {
-                ci[j] = s_idx[loc + i];
-                cv[j] = s_val[loc + i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kRounds; j++) {
-            const int i = (int)threadIdx.x + kWgThreads * j;
-            if (i < total_nz) stage[i] = make_int2(kWide ? ci[j] : (int)((uint32_t)ci[j] * ((uint32_t)ldx * 4u)), __float_as_int(cv[j]));
-        }
-    }
+    // stage the unit's (column, value) pairs: one round of the workgroup, or two
+    static_assert(kDegBound <= 2 * kWgThreads, "rounds of staging");
+    if (total_nz > kWgThreads)
+        stage_rounds<2, kWgThreads, kWide>(s_idx + loc, s_val + loc, total_nz, (int)threadIdx.x, ldx, stage);
+    else if ((int)threadIdx.x < total_nz)
+        stage_rounds<1, kWgThreads, kWide>(s_idx + loc, s_val + loc, total_nz, (int)threadIdx.x, ldx, stage);
     __syncthreads();
 
     // groups per row: power of two that minimises ceil(n_rows / (TG/gp)) * ceil(d / gp)
@@ -512,11 +528,11 @@ __global__ __launch_bounds__(kWgThreads) void spmm_team_kernel(
             float acc[VEC];
 #pragma unroll
             for (int v = 0; v < VEC; v++) acc[v] = 0.0f;
-            if (live) gather_row<VEC, kTeamUnroll, kWide, kShift>(stage + r * d, d, k, gp, X, col, ldx, acc);
+            if (live) gather_row<VEC, kWide, kShift>(stage + r * d, d, k, lg, X, col, ldx, acc);
             // the row's groups inside this wavefront (all lanes take part)
             for (int m = L; m < L * in_wave; m <<= 1) {
 #pragma unroll
-                for (int v = 0; v < VEC; v++) acc[v] += __shfl_xor(acc[v], m);
+                for (int v = 0; v < VEC; v++) acc[v] += from_lane_xor(acc[v], lane, m);
             }
             if (waves_per_row > 1) {                 // workgroup-uniform
                 if (g == 0) {
