@@ -1400,48 +1400,43 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
 // Small matrices are latency-bound: the time of a launch is the longest chain of
 // dependent memory round trips in one wavefront, not the traffic.  For them a unit is
 // given to a whole workgroup (four wavefronts share its rows, or its row's non-zeros),
-// which shortens that chain, and rows of up to 384 non-zeros stay whole, so that most
-// such matrices need no partial sums and no second launch.
-// Measured (everything one call launches, N = 16 / 64 / 128, wavefront units with their
-// best unit size against workgroup units of 96 with whole rows up to 384):
-//   99 k non-zeros, longest row 171:   10.1 / 11.2 / 16.3 us  ->  7.3 /  9.4 / 11.4 us
-//   208 k non-zeros, power law:        11.8 / 12.4 / 19.8 us  ->  7.9 / 10.5 / 12.6 us
-//   1.2 M, 1.6 M and 2.4 M non-zeros:  wavefront units are faster (26 / 53 / 99 us against
-//                                      34 / 55 / 102 us on the 1.2 M one).
-constexpr int64_t kTeamMaxNnz = 512 * 1024;
+// which shortens that chain, as long as the launch's workgroups are few: 2,048 of them are
+// on the GPU at once, and from about twice as many on wavefront units are faster (four
+// times fewer workgroups).  Units are about rows / 12 + nnz / 96, from the rows of a block4
+// entry and the unit size.  Measured (three matrices in turn, N = 12 / 32 / 64 / 128,
+// workgroup units, then wavefront units of up to 384):
+//   100 k non-zeros in 10 k rows, power law (1,900):   4.9 / 5.9 / 7.7 / 9.3 us,     8.0 / 7.6 / 11.8 / 12.4
+//   208 k in 10 k rows, power law (3,000):             6.1 / 8.5 / 10.3 / 12.7,      6.3 / 8.1 / 12.1 / 12.1
+//   300 k in 3 k rows, lognormal (3,400):              6.0 / 7.0 / 7.4 / 11.4,       6.0 / 6.5 / 8.7 / 10.8
+//   300 k in 15 k rows, power law (4,400):             8.0 / 10.7 / 12.5 / 17.6,     6.9 / 8.8 / 12.7 / 14.9
+//   150 k in 38 k rows, near the diagonal (4,700):     7.0 / 8.0 / 9.0 / 13.5,       5.0 / 5.1 / 8.7 / 10.9
+//   450 k in 27 k rows, hub rows (6,900):              14.6 / 15.7 / 18.4 / 24.8,    12.1 / 12.4 / 17.3 / 22.0
+//   300 k in 75 k rows, near the diagonal (9,400):     11.8 / 12.3 / 14.5 / 23.4,    5.7 / 7.2 / 10.7 / 16.8
+constexpr int64_t kTeamMaxUnits = 4096, kSmallNnz = 512 * 1024;
 static bool choose_plan_team(int64_t rows, int64_t nnz)
 {
-    (void)rows;
-    return nnz < kTeamMaxNnz;
+    return nnz < kSmallNnz && rows / 12 + nnz / 96 < kTeamMaxUnits;
 }
 
 // Unit size of the launch plan: the most non-zeros of a unit of several whole rows (and,
-// with wavefront units, of a piece of a split row).  Large matrices keep the block4
-// granularity (384: fewest descriptors and partial sums, and the launch is bandwidth-bound
-// anyway).  Small ones want short chains: workgroup units of 96 non-zeros (48 below 64 k
-// non-zeros: 10.0 against 11.2 us at N = 64 on a 35 k one).  With wavefront units on a
-// small matrix (only when asked for) 48 / 96 are best too: a 99 k-non-zero matrix 11 us
-// with units of 48 against 17 us with 384; from about 1 M non-zeros on 384 is best or within 2 %.
-static int choose_plan_unit(int64_t rows, int64_t nnz, bool team)
+// with wavefront units, of a piece of a split row).  Wavefront units keep the block4
+// granularity (384: fewest descriptors and partial sums); 48 below 128 k non-zeros, where they
+// are taken only when asked for.  Workgroup units want short chains: 96 non-zeros, 48 below
+// 64 k non-zeros (10.0 against 11.2 us at N = 64 on a 35 k one).
+static int choose_plan_unit(int64_t nnz, bool team)
 {
-    (void)rows;
     if (team) return nnz < (int64_t)64 * 1024 ? 48 : 96;
-    if (nnz < (int64_t)128 * 1024) return 48;
-    if (nnz < (int64_t)512 * 1024) return 96;
-    return kDegBound;
+    return nnz < (int64_t)128 * 1024 ? 48 : kDegBound;
 }
 
-// Rows above this many non-zeros are stored by column group and cut into pieces.
+// Rows above this many non-zeros are stored by column group and cut into pieces, which
+// a small matrix does not need for its balance and whose partial sums it waits for:
+// 450 k non-zeros, N = 32: 4.4 us with 384, 6.3 with 192.
 // Measured with 384, 256, 192, 128 and 96 (N = 64): 192 is 8 % faster than 384 on the
 // dense 115 M-non-zero matrix, 2 % on the 125 M power-law one, neutral elsewhere;
 // below 192 the extra partial sums start to cost at N = 16.
 constexpr int kPlanSplit = 192;
-static int choose_plan_split(int64_t rows, int64_t nnz, bool team)
-{
-    (void)rows;
-    (void)nnz;
-    return team ? kDegBound : kPlanSplit;        // workgroup units: rows up to one unit stay whole
-}
+static int choose_plan_split(int64_t nnz, bool team) { return team || nnz < kSmallNnz ? kDegBound : kPlanSplit; }
 
 // Launches that fill the sorted copy (see CopyArgs).  Needs perm (or none), s_indptr, the bins' runs,
 // n_split_rows and, for wide rows, the chunk tables, as the preprocessing leaves them on the handle.
@@ -1588,8 +1583,8 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     h->n_units = h->n_long_units = 0;
     h->n_split_rows = h->n_big_rows = h->n_wide_rows = h->n_chunks = 0;
     h->plan_team = h->plan_team_option == 2 || (h->plan_team_option == 0 && choose_plan_team(rows, nnz));
-    h->plan_unit = h->plan_unit_option > 0 ? h->plan_unit_option : choose_plan_unit(rows, nnz, h->plan_team);
-    h->plan_split = h->plan_split_option > 0 ? h->plan_split_option : choose_plan_split(rows, nnz, h->plan_team);
+    h->plan_unit = h->plan_unit_option > 0 ? h->plan_unit_option : choose_plan_unit(nnz, h->plan_team);
+    h->plan_split = h->plan_split_option > 0 ? h->plan_split_option : choose_plan_split(nnz, h->plan_team);
     // a wavefront never takes more than plan_unit non-zeros; a workgroup takes a whole row of
     // up to plan_split even when units of several rows are kept smaller
     if (!h->plan_team) h->plan_split = std::min(h->plan_split, h->plan_unit);
