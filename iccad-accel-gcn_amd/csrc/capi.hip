@@ -30,11 +30,13 @@ int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int 
                     hipStream_t stream, bool may_prepare);      // dense.hip
 
 // Work that is queued on the null stream alone orders itself before whoever takes the memory
-// next (memory.hip); for a handle that other streams, or graphs, have used, the device is
-// waited for first.  Returns whether nothing uses the handle's memory any more.
+// next (memory.hip); for a handle that other streams, or graphs, have used, its device (which
+// need not be the current one) is waited for first.  Returns whether nothing uses the handle's
+// memory any more.
 static bool settle(const accel_handle *h)
 {
     if (!h->multi_stream && !h->captured && !(h->has_home && h->home)) return !h->has_home;
+    OnDevice on(h->device);
     if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
     return true;
 }
@@ -973,6 +975,7 @@ int accel_reserve(accel_handle *h, int32_t max_N)
     if (!h) { set_error("accel_reserve: null handle"); return ACCEL_ERR_ARG; }
     if (!h->ready) { set_error("accel_reserve: call accel_preprocess first"); return ACCEL_ERR_STATE; }
     if (max_N <= 0) { set_error("accel_reserve: N must be positive, got %d", max_N); return ACCEL_ERR_ARG; }
+    OnDevice on(h->device);
     return reserve_run(h, max_N);
 }
 

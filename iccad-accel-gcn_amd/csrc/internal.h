@@ -68,6 +68,22 @@ __host__ __device__ inline void slice_rule(int d, int &w_nz, int &rows_per_block
     rows_per_block = kSlices / split;
 }
 
+// Makes a GPU current for a scope: the handle's, where the caller's current one may be another.
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device)
+    {
+        int now = device;
+        if (hipGetDevice(&now) != hipSuccess) (void)hipGetLastError();
+        if (now == device) return;
+        if (hipSetDevice(device) == hipSuccess) before = now;
+        else (void)hipGetLastError();
+    }
+    ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+};
+
 }  // namespace accel
 
 // The operator state behind the opaque C handle.

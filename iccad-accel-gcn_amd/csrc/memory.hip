@@ -71,12 +71,9 @@ size_t size_class(size_t bytes)
 
 void free_block(const Idle &b)
 {
-    int now = 0;
-    (void)hipGetDevice(&now);
-    if (now != b.device) (void)hipSetDevice(b.device);
+    OnDevice on(b.device);
     if (hipFree(b.p) != hipSuccess) (void)hipGetLastError();          // waits for the device
     if (b.after) (void)hipEventDestroy(b.after);
-    if (now != b.device) (void)hipSetDevice(now);
 }
 
 void free_idle(std::vector<Idle> &gone)

@@ -137,6 +137,7 @@ int accel_load_state(accel_handle *h, const char *path)
     clear_error();
     if (!h || !path) { set_error("accel_load_state: null argument"); return ACCEL_ERR_ARG; }
     if (int rc = check_borrowed_csr(h, "accel_load_state")) return rc;
+    OnDevice on(h->device);
     const auto t0 = std::chrono::steady_clock::now();
     File in;
     in.f = fopen(path, "rb");
