@@ -31,31 +31,30 @@ int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int 
 
 // Work that is queued on the null stream alone orders itself before whoever takes the memory
 // next (memory.hip); for a handle that other streams, or graphs, have used, its device (which
-// need not be the current one) is waited for first.  Returns whether nothing uses the handle's
-// memory any more.
-static bool settle(const accel_handle *h)
+// need not be the current one) is waited for first.  Returns what may still use the handle's
+// memory.
+static InUse settle(const accel_handle *h)
 {
-    if (!h->multi_stream && !h->captured && !(h->has_home && h->home)) return !h->has_home;
+    if (!h->multi_stream && !h->captured && !(h->has_home && h->home))
+        return h->has_home ? InUse::null_stream : InUse::no;
     OnDevice on(h->device);
-    if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
-    return true;
+    return wait_for_device();
 }
 
-void release_products(accel_handle *h)
+static void release_products(accel_handle *h, InUse use)
 {
-    const bool settled = settle(h);
-    give_memory(h->slab, settled);                     // perm, s_indptr and the sorted copy live in here
+    give_memory(h->slab, use);                         // perm, s_indptr and the sorted copy live in here
     h->slab = nullptr;
-    give_memory(h->work, settled);
-    give_memory(h->long_slot, settled);
-    give_memory(h->block4, settled);
-    give_memory(h->partial, settled);
-    give_memory(h->x_rows, settled);
-    give_memory(h->src_pos, settled);
+    give_memory(h->work, use);
+    give_memory(h->long_slot, use);
+    give_memory(h->block4, use);
+    give_memory(h->partial, use);
+    give_memory(h->x_rows, use);
+    give_memory(h->src_pos, use);
     h->src_pos = nullptr;
     h->val_stale = false;
-    // what other streams still held was queued against the memory given back above and has
-    // finished, so the bookkeeping starts afresh
+    // what other streams still held was queued against the memory given back above, which nobody
+    // gets before it has finished, so the bookkeeping starts afresh
     if (h->writer_done) (void)hipEventDestroy(h->writer_done);
     for (auto &sl : h->slot) {
         if (sl.done) (void)hipEventDestroy(sl.done);
@@ -72,6 +71,8 @@ void release_products(accel_handle *h)
     h->x_rows_floats = 0; h->reserved_N = 0;
     h->partial_floats = 0; h->owns_sorted = false; h->ready = false;
 }
+
+void release_products(accel_handle *h) { release_products(h, settle(h)); }
 
 static int need_gpu()
 {
@@ -550,9 +551,9 @@ int accel_create(const int32_t *indptr, const int32_t *idx, const float *val, in
         const size_t sb = sizeof(int32_t) * (size_t)nnz, sc = sizeof(float) * (size_t)nnz;
         void *a = take_memory(sa, false), *b = take_memory(sb, false), *c = take_memory(sc, false);
         if (!a || !b || !c) {
-            give_memory(a, true);
-            give_memory(b, true);
-            give_memory(c, true);
+            give_memory(a, InUse::null_stream);        // as they may have been taken
+            give_memory(b, InUse::null_stream);
+            give_memory(c, InUse::null_stream);
             delete h;
             set_error("device allocation for the CSR (%zu bytes) failed", sa + sb + sc);
             return ACCEL_ERR_ALLOC;
@@ -577,12 +578,12 @@ int accel_create(const int32_t *indptr, const int32_t *idx, const float *val, in
 int accel_destroy(accel_handle *h)
 {
     if (!h) return ACCEL_OK;
-    const bool settled = settle(h);                    // the kernels may read the CSR in place
-    release_products(h);
+    const InUse use = settle(h);                       // the kernels may read the CSR in place
+    release_products(h, use);
     if (h->owns_input) {
-        give_memory(const_cast<int32_t *>(h->indptr), settled);
-        give_memory(const_cast<int32_t *>(h->idx), settled);
-        give_memory(const_cast<float *>(h->val), settled);
+        give_memory(const_cast<int32_t *>(h->indptr), use);
+        give_memory(const_cast<int32_t *>(h->idx), use);
+        give_memory(const_cast<float *>(h->val), use);
     }
     delete h;
     return ACCEL_OK;
@@ -682,7 +683,7 @@ int accel_preprocess(accel_handle *h)
     if (int rc = check_device(h, "accel_preprocess")) return rc;
     if (int rc = check_borrowed_csr(h, "accel_preprocess")) return rc;     // still there, still large enough
     if (h->val_stale) {                     // value updates since: the handle's copy of the values first
-        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
+        ACCEL_HIP(hipDeviceSynchronize());
         if (int rc = restore_own_values(h, nullptr)) return rc;
     }
     release_products(h);
@@ -912,8 +913,8 @@ int accel_partition_gpu(const int32_t *indptr, int64_t rows, int32_t *block4_out
         const int64_t take = std::min(nb, cap);
         if (take > 0) rc = download(block4_out, b4, sizeof(int32_t) * 4 * (size_t)take, nullptr);
     }
-    give_memory(b4, false);
-    give_memory(dptr, false);
+    give_memory(b4, InUse::null_stream);
+    give_memory(dptr, InUse::null_stream);
     return rc;
 }
 

@@ -180,10 +180,15 @@ struct accel_handle {
 namespace accel {
 // memory.hip: device memory that outlives a handle.  take_memory returns null when there is
 // none; any_stream: the memory will first be used on another stream than the null stream.
-// give_memory returns it; settled: no kernel uses it any more (else: only kernels queued on the
-// null stream may).
+// give_memory returns it, with what may still use it.
+enum class InUse {
+    no,
+    null_stream,              // kernels queued on the null stream
+    unknown                   // kernels anywhere: a wait for them has failed
+};
 void *take_memory(size_t bytes, bool any_stream);
-void give_memory(void *p, bool settled);
+void give_memory(void *p, InUse use);
+InUse wait_for_device();      // the current one: no, or unknown if the wait failed
 void release_idle_memory();
 // The same for memory that work queued on s will use, from now on and until it is given back.
 void *take_stream_memory(size_t bytes, hipStream_t s);

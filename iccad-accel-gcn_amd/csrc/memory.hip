@@ -25,6 +25,10 @@
 // works on the null stream and is ordered behind the former by the stream; every other
 // combination of the last use and the next waits for the event on the device, or on the host
 // where the next stream is not known (`any_stream`) or the last one was the null stream.
+//
+// A wait may be refused (most are while any stream of the process captures).  A block whose last
+// use could not be waited for is marked so, stays on the list, and is handed out or freed only
+// once a wait for its whole device has succeeded; until then requests get other memory.
 #include <chrono>
 #include <mutex>
 #include <unordered_map>
@@ -33,6 +37,14 @@
 #include "preprocess.h"
 
 namespace accel {
+
+InUse wait_for_device()
+{
+    if (hipDeviceSynchronize() == hipSuccess) return InUse::no;
+    (void)hipGetLastError();
+    return InUse::unknown;
+}
+
 namespace {
 
 using Clock = std::chrono::steady_clock;
@@ -43,8 +55,8 @@ struct Idle {
     void *p;
     size_t bytes;
     int device;
-    bool settled;                                 // no kernel on the null stream uses it any more
-    hipEvent_t after;                             // stands behind its last use on another stream, or null
+    InUse use;                                    // what may still use it, apart from
+    hipEvent_t after;                             // ... what this event stands behind (or null)
     Clock::time_point since;
 };
 
@@ -69,17 +81,40 @@ size_t size_class(size_t bytes)
     return (bytes + step - 1) / step * step;
 }
 
-void free_block(const Idle &b)
+// A block goes (back) on the list: one that could not be waited for, or could not be freed.
+void keep_in_doubt(Idle b)
 {
-    OnDevice on(b.device);
-    if (hipFree(b.p) != hipSuccess) (void)hipGetLastError();          // waits for the device
-    if (b.after) (void)hipEventDestroy(b.after);
+    b.use = InUse::unknown;
+    b.since = Clock::now();
+    Pool &pl = pool();
+    std::lock_guard<std::mutex> lock(pl.mu);
+    pl.idle.push_back(b);
 }
 
 void free_idle(std::vector<Idle> &gone)
 {
-    for (const Idle &b : gone) free_block(b);
+    for (const Idle &b : gone) {
+        OnDevice on(b.device);
+        if (hipFree(b.p) != hipSuccess) {                             // waits for the device
+            (void)hipGetLastError();
+            keep_in_doubt(b);
+        } else if (b.after) {
+            (void)hipEventDestroy(b.after);
+        }
+    }
     gone.clear();
+}
+
+// Whether the next use of b, on s (with `any`: on a stream not known yet), comes behind its last one.
+bool order_behind(const Idle &b, hipStream_t s, bool any)
+{
+    hipError_t e = hipSuccess;
+    if (b.use == InUse::unknown) e = hipDeviceSynchronize();
+    else if (b.after) e = any ? hipEventSynchronize(b.after) : hipStreamWaitEvent(s, b.after, 0);
+    else if (b.use == InUse::null_stream && (any || s)) e = hipStreamSynchronize(nullptr);
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();
+    return wait_for_device() == InUse::no;
 }
 
 // Takes the blocks idle for longer than kIdleSeconds, and the oldest beyond the bound, off the
@@ -135,27 +170,18 @@ static void *take(size_t bytes, hipStream_t s, bool any)
         }
         if (best < pl.idle.size()) {
             got = pl.idle[best];
-            pl.live[got.p] = {got.bytes, dev};
             pl.idle.erase(pl.idle.begin() + (long)best);
         }
         expire(pl, gone);
     }
     free_idle(gone);
-    if (got.p) {
-        hipError_t e = hipSuccess;
-        if (got.after) {                                          // last used on another stream than the null stream
-            e = any ? hipEventSynchronize(got.after) : hipStreamWaitEvent(s, got.after, 0);
-            (void)hipEventDestroy(got.after);
-        } else if (!got.settled && (any || s)) {
-            e = hipStreamSynchronize(nullptr);
-        }
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipDeviceSynchronize();
-            (void)hipGetLastError();
-        }
+    if (got.p && order_behind(got, s, any)) {
+        if (got.after) (void)hipEventDestroy(got.after);
+        std::lock_guard<std::mutex> lock(pl.mu);
+        pl.live[got.p] = {got.bytes, dev};
         return got.p;
     }
+    if (got.p) keep_in_doubt(got);
     void *p = nullptr;
     if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
@@ -175,7 +201,7 @@ static void *take(size_t bytes, hipStream_t s, bool any)
     return p;
 }
 
-static void give(void *p, bool settled, hipEvent_t after)
+static void give(void *p, InUse use, hipEvent_t after)
 {
     if (!p) return;
     Pool &pl = pool();
@@ -184,7 +210,7 @@ static void give(void *p, bool settled, hipEvent_t after)
         std::lock_guard<std::mutex> lock(pl.mu);
         const auto it = pl.live.find(p);
         if (it == pl.live.end()) return;
-        pl.idle.push_back({p, it->second.first, it->second.second, settled, after, Clock::now()});
+        pl.idle.push_back({p, it->second.first, it->second.second, use, after, Clock::now()});
         pl.live.erase(it);
         expire(pl, gone);
     }
@@ -192,22 +218,22 @@ static void give(void *p, bool settled, hipEvent_t after)
 }
 
 void *take_memory(size_t bytes, bool any_stream) { return take(bytes, nullptr, any_stream); }
-void give_memory(void *p, bool settled) { give(p, settled, nullptr); }
+void give_memory(void *p, InUse use) { give(p, use, nullptr); }
 void *take_stream_memory(size_t bytes, hipStream_t s) { return take(bytes, s, false); }
 
 void give_stream_memory(void *p, hipStream_t s)
 {
-    if (!s) { give(p, false, nullptr); return; }
+    if (!s) { give(p, InUse::null_stream, nullptr); return; }
     hipEvent_t after = nullptr;
     if (hipEventCreateWithFlags(&after, hipEventDisableTiming) == hipSuccess && hipEventRecord(after, s) == hipSuccess) {
-        give(p, true, after);
+        give(p, InUse::no, after);
         return;
     }
     (void)hipGetLastError();
     if (after) (void)hipEventDestroy(after);
-    (void)hipStreamSynchronize(s);
-    (void)hipGetLastError();
-    give(p, true, nullptr);
+    const bool done = hipStreamSynchronize(s) == hipSuccess;
+    if (!done) (void)hipGetLastError();
+    give(p, done ? InUse::no : InUse::unknown, nullptr);
 }
 
 // Pinned blocks for the preprocessing's results, one per call that is under way; kept (a few KB

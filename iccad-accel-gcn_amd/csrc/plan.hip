@@ -407,7 +407,7 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
             return ACCEL_ERR_STATE;
         }
         room = mail->per_queue;
-        give_memory(dwork.release(), true);
+        give_memory(dwork.release(), InUse::no);
     }
     if (mail->n_units != (int)n_short_units) {
         set_error("internal: %d units of whole rows, %lld were expected from the degree histogram", mail->n_units,

@@ -73,7 +73,7 @@ struct StageHolder {
 
 // Temporaries of one preprocessing call come out of a few large pieces of device memory (there
 // are some twenty of them).  The pieces are given back when the arena goes out of scope; what
-// is still queued then is queued on the null stream.
+// is still queued then is queued on the null stream, unless `use` says otherwise.
 struct Arena {
     static constexpr int kMaxChunks = 32;
     char *chunk[kMaxChunks] = {};
@@ -81,12 +81,13 @@ struct Arena {
     int n_chunks = 0;
     size_t next_chunk = 0;         // size hint for the next chunk
     bool any_stream = false;       // will be used on another stream than the null stream
+    InUse use = InUse::null_stream;
     Arena() = default;
     Arena(const Arena &) = delete;
     Arena &operator=(const Arena &) = delete;
     ~Arena()
     {
-        for (int i = 0; i < n_chunks; i++) give_memory(chunk[i], any_stream);
+        for (int i = 0; i < n_chunks; i++) give_memory(chunk[i], use);
     }
     void *take(size_t bytes)
     {
@@ -116,10 +117,11 @@ struct Arena {
 
 struct DevBuf {  // device memory that is given back on scope exit unless it is released
     void *p = nullptr;
+    InUse use = InUse::null_stream;
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { give_memory(p, false); }
+    ~DevBuf() { give_memory(p, use); }
     int alloc(size_t bytes, bool any_stream = false)
     {
         p = take_memory(bytes, any_stream);

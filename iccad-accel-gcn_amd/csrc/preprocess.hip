@@ -1495,8 +1495,10 @@ int build_source_positions(accel_handle *h, hipStream_t s)
     if (int rc = map.alloc(sizeof(int32_t) * (size_t)h->nnz, s != nullptr)) return rc;
     const CopyArgs ca{sorted_rows(h), h->idx, nullptr, (uint32_t)h->cols, nullptr, map.as<int32_t>(), 1, nullptr};
     const int rc = copy_nonzeros(&tmp, h, ca, h->nnz_short, nullptr, s);
-    ACCEL_HIP(hipStreamSynchronize(s));       // the temporaries are given back on return
+    const hipError_t e = hipStreamSynchronize(s);      // the temporaries are given back on return
+    tmp.use = map.use = e == hipSuccess ? InUse::no : InUse::unknown;
     if (rc) return rc;
+    ACCEL_HIP(e);
     h->src_pos = static_cast<int32_t *>(map.release());
     return ACCEL_OK;
 }

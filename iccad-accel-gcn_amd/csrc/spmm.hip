@@ -834,10 +834,7 @@ static int static_scratch_address(float **out)
 int reserve_partial(accel_handle *h, size_t floats, bool any_stream)
 {
     if (h->partial_floats >= floats) return ACCEL_OK;
-    if (h->partial) {
-        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();     // nobody reads the old one
-        give_memory(h->partial, true);
-    }
+    if (h->partial) give_memory(h->partial, wait_for_device());      // nobody reads the old one
     h->partial_floats = 0;
     h->partial = static_cast<float *>(take_memory(floats * sizeof(float), any_stream));
     if (!h->partial) {
@@ -906,10 +903,7 @@ static bool pads_x(const accel_handle *h, uintptr_t x, int N, int64_t ld)
 static bool room_for_rows(accel_handle *h, size_t floats, bool any_stream)
 {
     if (h->x_rows_floats >= floats) return true;
-    if (h->x_rows) {
-        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();     // nobody reads the old one
-        give_memory(h->x_rows, true);
-    }
+    if (h->x_rows) give_memory(h->x_rows, wait_for_device());      // nobody reads the old one
     h->x_rows_floats = 0;
     h->x_rows = static_cast<float *>(take_memory(floats * sizeof(float), any_stream));
     if (!h->x_rows) {

@@ -57,7 +57,12 @@ struct File {
 
 struct PinnedBuf {   // host memory the GPU copies from and to directly
     void *p = nullptr;
-    ~PinnedBuf() { if (p) (void)hipHostFree(p); }
+    bool queued = false;                               // by a copy on the null stream
+    ~PinnedBuf()
+    {
+        // (left alone where the copy cannot be waited for)
+        if (p && (!queued || hipStreamSynchronize(nullptr) == hipSuccess)) (void)hipHostFree(p);
+    }
     int alloc(size_t bytes)
     {
         if (hipHostMalloc(&p, bytes ? bytes : 4, hipHostMallocDefault) != hipSuccess) {
@@ -72,7 +77,7 @@ struct PinnedBuf {   // host memory the GPU copies from and to directly
 
 struct DevMem {
     void *p = nullptr;
-    ~DevMem() { give_memory(p, false); }
+    ~DevMem() { give_memory(p, InUse::null_stream); }
 };
 
 }  // namespace
@@ -196,11 +201,12 @@ int accel_load_state(accel_handle *h, const char *path)
             set_error("device allocation of %zu bytes failed", bytes);
             return ACCEL_ERR_ALLOC;
         }
+        host.queued = true;
         ACCEL_HIP(hipMemcpyAsync(dev.p, host.p, bytes, hipMemcpyHostToDevice, nullptr));
         order.perm_dev = static_cast<const uint32_t *>(dev.p);
     }
     if (h->val_stale) {                     // value updates since: the handle's copy of the values first
-        if (hipDeviceSynchronize() != hipSuccess) (void)hipGetLastError();
+        ACCEL_HIP(hipDeviceSynchronize());
         if (int rc = restore_own_values(h, nullptr)) return rc;
     }
     release_products(h);
@@ -213,7 +219,6 @@ int accel_load_state(accel_handle *h, const char *path)
     h->plan_queues_option = hd.plan_queues_option;
     h->plan_reduce_option = hd.plan_reduce_option;
     const int rc = preprocess_device(h, &order);
-    (void)hipStreamSynchronize(nullptr);            // the staging buffers go away with this scope
     if (rc) {
         release_products(h);
         h->plan_unit_option = keep[0]; h->plan_split_option = keep[1]; h->plan_groups = keep[2];

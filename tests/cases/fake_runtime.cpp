@@ -263,6 +263,136 @@ static void reserved_with_another_gpu_current()
     CHECK(g_side[0].done == g_side[0].queued);             // the old buffer's users
 }
 
+// The wait in accel_destroy is refused (another stream of the process captures).
+static void wait_refused_on_close()
+{
+    Used u(g_side[0]);
+    g_refuse_host_waits = true;
+    CHECK(accel_destroy(u.h) == ACCEL_OK);
+    void *p = take_memory(kBlock, true);
+    CHECK(p && u.safe(p, nullptr));                        // still refused: other memory
+    g_refuse_host_waits = false;
+    void *q = take_memory(kBlock, true);
+    CHECK(q && u.safe(q, nullptr));
+    CHECK(q == u.block);                                   // not lost
+}
+
+// Expired memory whose hipFree is refused is neither lost nor handed out unordered.
+static void free_refused()
+{
+    Used u(g_side[0]);
+    g_refuse_host_waits = true;
+    CHECK(accel_destroy(u.h) == ACCEL_OK);
+    CHECK(accel_release_memory() == ACCEL_OK);
+    CHECK(g_frees == 0);
+    g_refuse_host_waits = false;
+    CHECK(accel_release_memory() == ACCEL_OK);
+    CHECK(g_frees > 0 && find_memory(u.block) == g_memory.end());
+}
+
+// The waits of the next user are refused: for a block behind an event, and for one of the null stream.
+static void wait_refused_on_take()
+{
+    void *p = take_stream_memory(kBlock, handle_of(g_side[0]));
+    g_side[0].queued++;
+    give_stream_memory(p, handle_of(g_side[0]));
+    g_refuse_host_waits = true;
+    CHECK(take_memory(kBlock, true) != p);
+    g_refuse_events = true;
+    CHECK(take_stream_memory(kBlock, handle_of(g_side[1])) != p);
+    g_refuse_host_waits = g_refuse_events = false;
+    CHECK(take_memory(kBlock, true) == p && g_side[0].done == g_side[0].queued);
+
+    void *q;
+    {
+        DevBuf b;                                          // given back behind work on the null stream
+        CHECK(b.alloc(4 * kBlock) == ACCEL_OK);
+        q = b.p;
+        g_null[0].queued++;
+    }
+    g_refuse_host_waits = true;
+    CHECK(take_memory(4 * kBlock, true) != q);
+    g_refuse_host_waits = false;
+    CHECK(take_memory(4 * kBlock, true) == q && g_null[0].done == g_null[0].queued);
+}
+
+// Neither an event nor a wait can be had when memory is given back behind a stream.
+static void nothing_to_be_had_on_give()
+{
+    void *p = take_stream_memory(kBlock, handle_of(g_side[0]));
+    g_side[0].queued++;
+    g_refuse_host_waits = g_refuse_events = true;
+    give_stream_memory(p, handle_of(g_side[0]));
+    CHECK(take_memory(kBlock, false) != p);
+    g_refuse_host_waits = g_refuse_events = false;
+    CHECK(take_memory(kBlock, false) == p && g_side[0].done == g_side[0].queued);
+}
+
+// accel_create that runs out of memory gives back what it took as it took it: behind the null stream.
+static void create_runs_out_of_memory()
+{
+    void *q;
+    {
+        DevBuf b;
+        CHECK(b.alloc(kBlock) == ACCEL_OK);
+        q = b.p;
+        g_null[0].queued++;
+    }
+    std::vector<int32_t> indptr(kBlock / 4, 0), idx(kBlock);
+    std::vector<float> val(kBlock);
+    indptr.back() = (int32_t)kBlock;
+    g_mallocs_left = 0;
+    accel_handle *h = nullptr;
+    CHECK(accel_create(indptr.data(), idx.data(), val.data(), (int64_t)indptr.size() - 1, 1, (int64_t)kBlock,
+                       ACCEL_PTR_HOST, &h) == ACCEL_ERR_ALLOC);
+    g_mallocs_left = -1;
+    void *p = take_memory(kBlock, true);
+    CHECK(p != q || g_null[0].done == g_null[0].queued);
+}
+
+// A buffer that grows while the wait for its last users is refused.
+static void wait_refused_on_growth()
+{
+    Used u(g_side[0]);
+    void *old = u.h->partial = static_cast<float *>(take_memory(2 * kBlock, false));
+    u.h->partial_floats = 2 * kBlock / 4;
+    u.h->n_long_units = (int64_t)kBlock / 64;
+    g_refuse_host_waits = true;
+    (void)accel_reserve(u.h, 128);
+    CHECK(take_memory(2 * kBlock, true) != old);
+    g_refuse_host_waits = false;
+    CHECK(take_memory(2 * kBlock, true) == old);
+}
+
+// The position map of a value update: its temporaries are in use until its wait has succeeded.
+static void wait_refused_in_a_value_update()
+{
+    Used u(g_side[0]);
+    u.h->nnz = u.h->nnz_short = (int64_t)kBlock;
+    u.h->owns_sorted = true;
+    void *val = nullptr;
+    CHECK(hipMalloc(&val, 4 * kBlock) == hipSuccess);
+    g_refuse_host_waits = true;
+    CHECK(accel_update_values_async(u.h, static_cast<float *>(val), handle_of(g_side[0])) != ACCEL_OK);
+    std::set<void *> before;
+    for (auto &m : g_memory) before.insert(m.first);
+    void *p = take_memory(4 * kBlock, false);              // the map's size
+    CHECK(p && !before.count(p));
+}
+
+// Values are restored from a sorted copy that an update may still be writing: not without the wait for it.
+static void wait_refused_before_values_are_restored()
+{
+    Used u(g_side[0]);
+    u.h->owns_sorted = u.h->val_stale = true;
+    u.h->src_pos = static_cast<int32_t *>(u.block);
+    u.h->s_val = static_cast<float *>(u.block);
+    const long queued = g_null[0].queued;
+    g_refuse_host_waits = true;
+    CHECK(accel_preprocess(u.h) == ACCEL_ERR_HIP);
+    CHECK(g_null[0].queued == queued && u.h->val_stale);
+}
+
 int main(int argc, char **argv)
 {
     g_null[1].device = 1;
@@ -271,6 +401,14 @@ int main(int argc, char **argv)
 #define SCENARIO(name) {#name, name}
         SCENARIO(closed_with_another_gpu_current),
         SCENARIO(reserved_with_another_gpu_current),
+        SCENARIO(wait_refused_on_close),
+        SCENARIO(free_refused),
+        SCENARIO(wait_refused_on_take),
+        SCENARIO(nothing_to_be_had_on_give),
+        SCENARIO(create_runs_out_of_memory),
+        SCENARIO(wait_refused_on_growth),
+        SCENARIO(wait_refused_in_a_value_update),
+        SCENARIO(wait_refused_before_values_are_restored),
     };
     if (argc != 2 || !all.count(argv[1])) {
         for (auto &s : all) std::printf("%s\n", s.first.c_str());
