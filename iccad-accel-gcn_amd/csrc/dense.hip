@@ -10,10 +10,12 @@
 // is below 2^-25 |x w|, half of what rounding one fp32 product may cost, and the accumulator is
 // rounded 0.4 times per k instead of 0.5; measured against fp64 on K = 16 .. 602 the error is the
 // smaller than that of v_mfma_f32_32x32x2_f32 on the same operands (2-norm of the difference over that of
-// the product, K = 602: 3.7e-7 against 4.4e-7; K = 128: 1.6e-7 against 2.0e-7).  Values that bf16 cannot carry this way (infinities, magnitudes of 2^127
-// and more, which would round up to one, and magnitudes below 2^-100, whose third part would
-// be too small for bf16) are multiplied by ordinary fp32 instructions instead, tile by tile where
-// they occur.
+// the product, K = 602: 3.7e-7 against 4.4e-7; K = 128: 1.6e-7 against 2.0e-7).  Both operands are
+// multiplied by 2^24 on the way, so that the last bit of the smallest denormal is still a bf16 value, and
+// the sums by 2^-48 when they are stored: small magnitudes need no other path.  Infinities, NaN, operands of
+// 2^103 and more and sums of 2^79 and more leave a tile with sums that are not finite; it is computed
+// again on the fp32 matrix instructions.  20,000 x 602 times 602 x 128: 40 us whatever the small
+// values among the operands, 113 to 132 us with an infinity in some tiles or in all.
 //
 // X is rows x K with rows in the millions and K, N in the tens to hundreds, so the product
 // streams X once, writes Z once and keeps W on chip.  A wavefront owns 32 rows of X and up to 128
@@ -68,9 +70,12 @@ __device__ __forceinline__ int half_start(int k0, int half, int K)
     return K < kDenseHalf ? k : min(k, K - kDenseHalf);
 }
 
-// Takes two values apart: the three parts of each, packed in pairs.
+// Takes two values apart, times kScale: the three parts of each, packed in pairs.
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
 __device__ __forceinline__ void take_apart(float a, float b, uint32_t (&part)[kParts])
 {
+    a *= kScale;
+    b *= kScale;
 #pragma unroll
     for (int p = 0; p < kParts; p++) {
         part[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
@@ -80,18 +85,6 @@ __device__ __forceinline__ void take_apart(float a, float b, uint32_t (&part)[kP
         }
     }
 }
-
-// Magnitudes below 2^-100 are looked for value by value (zero is not one).  The large ones need no
-// look: a value that rounds up to infinity leaves infinity minus infinity in its second part, so
-// every sum it takes part in comes out as NaN, which is looked for before a tile is stored.
-struct Seen {
-    uint32_t least = 0xFFFFFFFFu;                       // smallest magnitude's bits, twice, minus one (zero: the largest value)
-    __device__ __forceinline__ void add(float a, float b)
-    {
-        least = min(least, min((__float_as_uint(a) << 1) - 1u, (__float_as_uint(b) << 1) - 1u));
-    }
-    __device__ __forceinline__ bool bad() const { return least < ((uint32_t)(127 - 100) << 24) - 1u; }
-};
 
 // W(k, col) of a step's half, or zero where the half does not own k (see half_start).
 __device__ __forceinline__ float w_at(const float *__restrict__ W, int K, int N, int k0, int half, int j, int col)
@@ -120,39 +113,27 @@ struct DenseArgs {
     int64_t rows, ldx, ldz, n_row_blocks;
     int K, N, n_col_tiles, n_steps;
     const u32x4 *image;          // W taken apart (dense_prepare_kernel)
-    const int *bad;              // per column tile and step of the image: holds values below 2^-100
 };
 
 // One workgroup per (column tile, step): the block of W taken apart, as [part][column][32 bf16].
 template <int NT>
-__global__ __launch_bounds__(kDenseThreads) void dense_prepare_kernel(DenseArgs a, u32x4 *__restrict__ image,
-                                                                      int *__restrict__ bad)
+__global__ __launch_bounds__(kDenseThreads) void dense_prepare_kernel(DenseArgs a, u32x4 *__restrict__ image)
 {
     constexpr int kCols = NT * 32, kVecs = kCols * kParts * 4;
-    __shared__ int any_bad;
     const int tile = (int)blockIdx.x / a.n_steps, k0 = (int)blockIdx.x % a.n_steps * kDenseStep;
-    if (threadIdx.x == 0) any_bad = 0;
-    __syncthreads();
     u32x4 *to = image + (int64_t)blockIdx.x * kVecs;
     for (int i = threadIdx.x; i < kCols * 4; i += kDenseThreads) {
         const int c = i % kCols, v = i / kCols;             // vector v: 8 k of half v / 2
         float w[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) w[j] = w_at(a.W, a.K, a.N, k0, v / 2, v % 2 * 8 + j, tile * kCols + c);
-        Seen seen;
         uint32_t part[4][kParts];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            seen.add(w[2 * j], w[2 * j + 1]);
-            take_apart(w[2 * j], w[2 * j + 1], part[j]);
-        }
+        for (int j = 0; j < 4; j++) take_apart(w[2 * j], w[2 * j + 1], part[j]);
 #pragma unroll
         for (int p = 0; p < kParts; p++)
             to[(p * kCols + c) * 4 + v] = u32x4{part[0][p], part[1][p], part[2][p], part[3][p]};
-        if (seen.bad()) any_bad = 1;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) bad[blockIdx.x] = any_bad;
 }
 
 // How the product gets its block of W per step.
@@ -175,7 +156,7 @@ template <int NT> struct WStage<NT, kWPrepared> {
         for (int i = 0; i < kMine; i++)
             if (kVecs % kDenseThreads == 0 || i * kDenseThreads + (int)threadIdx.x < kVecs) v[i] = from[i * kDenseThreads];
     }
-    __device__ __forceinline__ void store(const DenseArgs &, const DenseStepAt &, char *lds, int *, int)
+    __device__ __forceinline__ void store(const DenseArgs &, const DenseStepAt &, char *lds)
     {
 #pragma unroll
         for (int i = 0; i < kMine; i++) {
@@ -203,8 +184,7 @@ template <int NT, DenseW kHow> struct WStage {
             for (int i = 0; i < kRun; i++) v[i] = a.W[(int64_t)min(k1 + i, a.K - 1) * a.N + col];
         }
     }
-    // bad: the step whose block is not to be used, per LDS buffer
-    __device__ __forceinline__ void store(const DenseArgs &a, const DenseStepAt &at, char *lds, int *bad, int step)
+    __device__ __forceinline__ void store(const DenseArgs &a, const DenseStepAt &at, char *lds)
     {
         const int c = (int)threadIdx.x % kCols, k = (int)threadIdx.x / kCols * kRun;
         if (at.k0 + kDenseStep > a.K || (at.tile + 1) * kCols > a.N) {
@@ -213,13 +193,9 @@ template <int NT, DenseW kHow> struct WStage {
 #pragma unroll
             for (int i = 0; i < kRun; i++) v[i] = col_ok && k1 + i >= owned && k1 + i < a.K ? v[i] : 0.f;
         }
-        Seen seen;
         uint32_t part[kRun / 2][kParts];
 #pragma unroll
-        for (int i = 0; i < kRun; i += 2) {
-            seen.add(v[i], v[i + 1]);
-            take_apart(v[i], v[i + 1], part[i / 2]);
-        }
+        for (int i = 0; i < kRun; i += 2) take_apart(v[i], v[i + 1], part[i / 2]);
 #pragma unroll
         for (int p = 0; p < kParts; p++) {
             char *to = lds + (p * kCols + c) * kWStride + 2 * k;
@@ -231,9 +207,39 @@ template <int NT, DenseW kHow> struct WStage {
                 *reinterpret_cast<uint2 *>(to) = make_uint2(part[0][p], part[1][p]);
             }
         }
-        if (seen.bad()) *bad = step;
     }
 };
+
+// Adds the products of k in [0, K) to a wavefront's tile by the fp32 matrix instructions, from memory.
+// v_mfma_f32_32x32x2_f32: lane l holds A[l % 32][l / 32] and B[l / 32][l % 32], the accumulators as above.  Rows and
+// columns past the end repeat the last one (their sums are not stored); a k past the end is zero on both
+// sides (an infinity times zero would be a NaN).
+template <int NT>
+__device__ __forceinline__ void add_in_fp32(const DenseArgs &a, int64_t row0, int col0, f32x16 (&acc)[NT])
+{
+    const int half = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+    const int64_t r = row0 + l32;
+    const float *xr = a.X + (r < a.rows ? r : a.rows - 1) * a.ldx;
+    constexpr int U = 4;                                    // instructions whose operands are on their way together
+#pragma unroll 1
+    for (int k = 0; k < a.K; k += 2 * U) {
+        float x[U], w[U][NT];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int at = min(k + 2 * u + half, a.K - 1);
+            x[u] = xr[at];
+#pragma unroll
+            for (int t = 0; t < NT; t++) w[u][t] = a.W[(int64_t)at * a.N + min(col0 + 32 * t + l32, a.N - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool in = k + 2 * u + half < a.K;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x[u] : 0.f, in ? w[u][t] : 0.f, acc[t], 0, 0, 0);
+        }
+    }
+}
 
 // The grid is sized to what the GPU holds at once and every workgroup walks blocks of 128
 // rows, gridDim.x apart, as one sequence of steps: the reads of a block's first steps are
@@ -248,7 +254,6 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
 {
     constexpr int kCols = NT * 32;
     __shared__ __attribute__((aligned(16))) char w_lds[2][kParts * kCols * kWStride];
-    __shared__ int w_bad[2];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int half = lane >> 5, l32 = lane & 31;
@@ -312,11 +317,8 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
     v4f x0[4], x1[4];
     WStage<NT, kHow> w;
     bf16x8 apart[2][kParts];                   // this step's values of X, taken apart
-    Seen seen;
     auto take_pair = [&](const v4f (&x)[4], int q, uint32_t (&pair)[kParts]) {
-        const float u = x[q / 2][2 * (q & 1)], v = x[q / 2][2 * (q & 1) + 1];
-        seen.add(u, v);
-        take_apart(u, v, pair);
+        take_apart(x[q / 2][2 * (q & 1)], x[q / 2][2 * (q & 1) + 1], pair);
         // (keeps the work here, between the matrix instructions, where the compiler would move it
         // to the next step)
         asm volatile("" : "+v"(pair[0]), "+v"(pair[1]), "+v"(pair[2]));
@@ -330,11 +332,9 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
                                                                pair[4 * i + 3][p]});
     };
 
-    if (tid < 2) w_bad[tid] = -1;
     w.fetch(a, now);
     fetch_x(x0, now);
     fetch_x(x1, next);
-    if constexpr (kHow != kWPrepared) __syncthreads();
     {
         uint32_t pair[8][kParts];
         v4f y[4];
@@ -343,15 +343,12 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
         for (int q = 0; q < 8; q++) take_pair(y, q, pair[q]);
         gather_pairs(pair);
     }
-    bool tile_ok = true, x_ok = !__any(seen.bad());
-    w.store(a, now, w_lds[0], &w_bad[0], 0);
+    w.store(a, now, w_lds[0]);
     int step = 0;
     // xf: free registers, for the step after the next; xn: the next step's X
     auto one = [&](v4f (&xf)[4], v4f (&xn)[4]) {
         const int buf = step & 1;
         __syncthreads();                       // this step's block of W is in place; the other one's readers are done
-        if constexpr (kHow == kWPrepared) tile_ok &= x_ok && !a.bad[now.tile * a.n_steps + now.k0 / kDenseStep];
-        else tile_ok &= x_ok && w_bad[buf] != step;
         w.fetch(a, next);
         fetch_x(xf, after);
         __builtin_amdgcn_sched_barrier(0);     // the loads go out here, ahead of the matrix work that hides them
@@ -369,7 +366,6 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
                         &w_lds[buf][(p * kCols + 32 * (g * P % NT + u) + l32) * kWStride + 32 * half + 16 * (g * P / NT)]);
         };
         uint32_t pair[8][kParts];
-        seen = Seen();
         read_b(b[0], 0);
         v4f y[4];
         turned(xn, y);
@@ -389,8 +385,7 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
             __builtin_amdgcn_sched_barrier(0);
         }
         gather_pairs(pair);
-        x_ok = !__any(seen.bad());
-        w.store(a, next, w_lds[buf ^ 1], &w_bad[buf ^ 1], step + 1);      // its readers were done at this step's barrier
+        w.store(a, next, w_lds[buf ^ 1]);      // its readers were done at this step's barrier
 
         if (next.k0 == 0) {                    // that was the last step of this tile: store it, start the next at zero
             const int64_t row0 = now.row_block * kDenseBlockRows + wave * kDenseRows;
@@ -401,31 +396,27 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
             for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) finite &= __builtin_isfinite(acc[t][v]);
-            if (!tile_ok || __any(!finite)) {
-                // values out of range among the operands: ordinary fp32, from memory
-#pragma unroll 1
-                for (int i = 0; i < 16 * NT; i++) {
-                    const int64_t row = row0 + 2 * (i % 16) + half;
-                    const int c = col + 32 * (i / 16);
-                    if (row >= a.rows || c >= a.N) continue;
-                    float sum = 0.f;
-#pragma unroll 1
-                    for (int k = 0; k < a.K; k++) sum = fmaf(a.X[row * a.ldx + k], a.W[(int64_t)k * a.N + c], sum);
-                    a.Z[row * a.ldz + c] = sum;
-                }
-                tile_ok = true;
-            } else if (row0 + kDenseRows <= a.rows && now.tile * kCols + kCols <= a.N) {      // nothing to mask
+            float unscale = kUnscale;
+            if (__any(!finite)) {
+                unscale = 1;
 #pragma unroll
                 for (int t = 0; t < NT; t++)
 #pragma unroll
-                    for (int v = 0; v < 16; v++) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v];
+                    for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+                add_in_fp32<NT>(a, row0, now.tile * kCols, acc);
+            }
+            if (row0 + kDenseRows <= a.rows && now.tile * kCols + kCols <= a.N) {      // nothing to mask
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v] * unscale;
             } else {
 #pragma unroll
                 for (int t = 0; t < NT; t++)
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
                         const int64_t row = row0 + 8 * (v / 4) + 4 * half + (v % 4);
-                        if (col + t * 32 < a.N && row < a.rows) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v];
+                        if (col + t * 32 < a.N && row < a.rows) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v] * unscale;
                     }
             }
 #pragma unroll
@@ -482,15 +473,13 @@ static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
     if constexpr (NT == 4) {
         const size_t blocks = (size_t)a.n_col_tiles * (size_t)a.n_steps;
         const size_t image_bytes = blocks * (NT * 32 * kParts * 4) * sizeof(u32x4);
-        char *mem = nullptr;
+        void *mem = nullptr;
         if (may_prepare && (double)a.rows * a.K * a.N >= kPrepareFrom)
-            mem = static_cast<char *>(take_stream_memory(image_bytes + blocks * sizeof(int), s));
+            mem = take_stream_memory(image_bytes, s);
         if (mem) {
-            u32x4 *image = reinterpret_cast<u32x4 *>(mem);
-            int *bad = reinterpret_cast<int *>(mem + image_bytes);
-            dense_prepare_kernel<NT><<<dim3((unsigned)blocks), kDenseThreads, 0, s>>>(a, image, bad);
+            u32x4 *image = static_cast<u32x4 *>(mem);
+            dense_prepare_kernel<NT><<<dim3((unsigned)blocks), kDenseThreads, 0, s>>>(a, image);
             a.image = image;
-            a.bad = bad;
             const int rc = dense_launch<NT, kWPrepared>(a, s);
             give_stream_memory(mem, s);
             return rc;

@@ -399,7 +399,9 @@ int accel_time_ex(accel_handle *h, const accel_run_args *args, int warmup, int i
  * (accel_release_memory); the others, and all of them while the stream is capturing, take none.
  * Computed on the matrix cores, each fp32 value as three bf16 values that add up to it: sums of K
  * products in fp32 (error as of fp32 instructions, or smaller), whose order differs from a
- * sequential loop (compare against a higher-precision product, as for accel_run). */
+ * sequential loop (compare against a higher-precision product, as for accel_run).  Tiles of 32 rows and
+ * up to 128 columns with infinities, NaN, operands of 2^103 and more or sums of 2^79 and more are computed
+ * a second time by fp32 instructions (some three times the time where that is every tile). */
 int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32_t K, int32_t N,
                    int32_t ldx, int32_t ldz, void *stream);
 

@@ -89,3 +89,74 @@ def test_prepared_weights_on_two_streams(gpu):
         z.close(); dW[i].close()
     dX.close()
     assert hip.hipStreamDestroy(stream) == 0
+
+
+@pytest.mark.parametrize("where", ["X", "W", "both"])
+@pytest.mark.parametrize("K,N", [(9, 40), (33, 20), (100, 50), (160, 128), (67, 130)])
+def test_small_magnitudes_among_ordinary_values(gpu, where, K, N):
+    """Values below 2^-100 (denormals among them) next to ordinary ones, in a few places or everywhere, also where
+    whole rows hold nothing else: every element as exact as fp32 sums are."""
+    rng = np.random.default_rng(K + N)
+    rows = 300
+    X = rng.standard_normal((rows, K)).astype(np.float32)
+    W = rng.standard_normal((K, N)).astype(np.float32)
+    if where != "W":
+        X[rng.random(X.shape) < 0.02] = 3e-38
+        X[40:80] *= np.float32(2.0 ** -110)
+        X[81, K // 2] = 1e-42
+    if where != "X":
+        W[K // 3] *= np.float32(2.0 ** -104)
+        W[:, N // 2] *= np.float32(2.0 ** -101) if where == "W" else np.float32(1)
+    Z = gpu.dense_xw_numpy(X, W)
+    want = X.astype(np.float64) @ W.astype(np.float64)
+    scale = np.abs(X).astype(np.float64) @ np.abs(W).astype(np.float64)
+    # K additions, each rounded to 24 bits or to a multiple of the smallest number
+    assert (np.abs(Z - want) <= (K + 1) * (2.0 ** -24 * scale + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("value", [2.0 ** 78, 2.0 ** 80, 2.0 ** 103])
+def test_large_magnitudes_among_ordinary_values(gpu, value):
+    """Where an operand or a sum leaves the range of the scaled values, the tile is computed again."""
+    rng = np.random.default_rng(3)
+    X = rng.standard_normal((200, 70)).astype(np.float32)
+    W = rng.standard_normal((70, 100)).astype(np.float32)
+    X[100, 60] = value
+    W[4, 99] = -value
+    Z = gpu.dense_xw_numpy(X, W)
+    assert so.check_dense(Z, X, W) <= 71 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("where,value,limit", [("W", 1e-38, 2), ("X", 1e-38, 2), ("X", np.inf, 8)])
+def test_speed_does_not_hang_on_single_values(gpu, where, value, limit):
+    """Small values cost nothing; an infinity makes its tile be computed again, by fp32 instructions (in every
+    tile that is some three times the time)."""
+    hip = C.CDLL("libamdhip64.so.7")
+    rows, K, N = 60_000, 256, 128
+    rng = np.random.default_rng(1)
+    X = rng.uniform(-1, 1, (rows, K)).astype(np.float32)
+    W = rng.standard_normal((K, N)).astype(np.float32)
+
+    def milliseconds():
+        dX, dW, dZ = gpu.DeviceBuffer.from_numpy(X), gpu.DeviceBuffer.from_numpy(W), gpu.DeviceBuffer(rows * N * 4)
+        ev = [C.c_void_p() for _ in range(2)]
+        for e in ev:
+            assert hip.hipEventCreate(C.byref(e)) == 0
+        for _ in range(3):
+            gpu.dense_xw(dX, dW, dZ, rows, K, N)
+        assert hip.hipEventRecord(ev[0], None) == 0
+        for _ in range(5):
+            gpu.dense_xw(dX, dW, dZ, rows, K, N)
+        assert hip.hipEventRecord(ev[1], None) == 0 and hip.hipEventSynchronize(ev[1]) == 0
+        t = C.c_float()
+        assert hip.hipEventElapsedTime(C.byref(t), *ev) == 0
+        for e in ev:
+            assert hip.hipEventDestroy(e) == 0
+        for b in (dX, dW, dZ):
+            b.close()
+        return t.value / 5
+
+    plain = milliseconds()
+    (W if where == "W" else X)[K // 2, 5] = value
+    if where == "X":
+        X[rng.integers(0, rows, 200), rng.integers(0, K, 200)] = value
+    assert milliseconds() <= limit * plain
