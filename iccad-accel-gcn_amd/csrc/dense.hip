@@ -63,12 +63,8 @@ constexpr int kWStride = 2 * kDenseStep + 16;
 
 // The k a half of the step starts at.  Where the row ends inside the half, the half is moved back
 // to end with the row (nothing is read past it), and W is zero for the k that belong to the half or
-// the step before.  (K < 16: the loads are clamped one by one instead.)
-__device__ __forceinline__ int half_start(int k0, int half, int K)
-{
-    const int k = k0 + kDenseHalf * half;
-    return K < kDenseHalf ? k : min(k, K - kDenseHalf);
-}
+// the step before.
+__device__ __forceinline__ int half_start(int k0, int half, int K) { return min(k0 + kDenseHalf * half, K - kDenseHalf); }
 
 // Takes two values apart, times kScale: the three parts of each, packed in pairs.
 constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
@@ -139,8 +135,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_prepare_kernel(DenseArgs 
 // How the product gets its block of W per step.
 enum DenseW {
     kWPrepared,                  // from the image
-    kWOnTheWay,                  // taken apart by the workgroup
-    kWShort                      // the same, K < 16
+    kWOnTheWay                   // taken apart by the workgroup
 };
 
 // A workgroup's block of W of a step on its way through registers into LDS.
@@ -263,7 +258,7 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
     // is bound by streaming X, read eight lanes to a row (whole lines per instruction) and turn the
     // values in LDS, within the wavefront (2.45 M x 100 x 32: 298 -> 275 us; with more columns the
     // detour costs as much as it gives: 128 x 64 382 -> 375 us at 2.45 M rows, 28 -> 32 at 170 k).
-    constexpr bool kTurn = NT == 1 && kHow != kWShort;
+    constexpr bool kTurn = NT == 1;
     __shared__ v4f x_lds[kTurn ? kDenseWaves : 1][kTurn ? kDenseRows * 8 : 1];
     auto turned = [&](const v4f (&x)[4], v4f (&y)[4]) {
         if constexpr (kTurn) {
@@ -292,15 +287,8 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
         const int64_t r = at.row_block * kDenseBlockRows + wave * kDenseRows + l32;
         const float *xr = a.X + (r < a.rows ? r : a.rows - 1) * a.ldx;
         const int k = half_start(at.k0, half, a.K);
-        if constexpr (kHow == kWShort) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) x[q][i] = xr[min(k + 4 * q + i, a.K - 1)];
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const v4f_unaligned *>(xr + k + 4 * q);
-        }
+        for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const v4f_unaligned *>(xr + k + 4 * q);
     };
 
     f32x16 acc[NT];
@@ -436,27 +424,143 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kerne
     }
 }
 
+// K < 16: one instruction deep, so that W's columns stay in registers while a wavefront walks tiles of 32
+// rows, the next tile's X ahead of the products; bound by storing Z.  kInFp32 (K = 1 and 2): by the fp32
+// instructions, whose error is the smaller one there (each product is exact before it is added: one
+// rounding per sum at K = 1.  2-norm of the difference over that of the product, normal operands: 2.5e-8
+// against 3.5e-8 in three parts; K = 2: 3.1e-8, 3.4e-8; K = 3: 3.6e-8, 3.3e-8; K = 8: 5.3e-8, 3.1e-8).
+// With several column tiles (N > 128) W is fetched again for every one of them; by workgroups of their own,
+// which store the lines that two tiles meet in at different times, 10 x 300 takes 1.32 to 1.48 ms.
+// 2.45 M rows, in the kernel above (W through LDS, 32 k per step) and here: 1 x 64 131 -> 117 us, 2 x 128
+// 261 -> 246, 4 x 16 101 -> 53, 8 x 64 239 -> 179, 12 x 32 138 -> 93, 15 x 128 290 -> 256, 10 x 300 1093 -> 1049.
+template <int NT, bool kInFp32>
+__global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_short_kernel(DenseArgs a)
+{
+    constexpr int J = kInFp32 ? 1 : 8;         // k that a lane holds of the one instruction: J half ...
+    const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t n_row_tiles = (a.rows + kDenseRows - 1) / kDenseRows;
+    const int64_t stride = (int64_t)gridDim.x * kDenseWaves;
+    // those behind K read the last one and count as zero
+    auto fetch_x = [&](float (&x)[J], int64_t row_tile) {
+        const int64_t r = row_tile * kDenseRows + l32;
+        const float *xr = a.X + (r < a.rows ? r : a.rows - 1) * a.ldx;
+#pragma unroll
+        for (int j = 0; j < J; j++) x[j] = xr[min(J * half + j, a.K - 1)];
+    };
+    auto or_zero = [&](const float (&x)[J], int j) { return J * half + j < a.K ? x[j] : 0.f; };
+    struct Operand {
+        bf16x8 part[kParts];
+        float whole;
+    };
+    auto operand = [&](const float (&x)[J], Operand &to) {
+        if constexpr (kInFp32) {
+            to.whole = or_zero(x, 0);
+        } else {
+            uint32_t pair[4][kParts];
+#pragma unroll
+            for (int j = 0; j < 4; j++) take_apart(or_zero(x, 2 * j), or_zero(x, 2 * j + 1), pair[j]);
+#pragma unroll
+            for (int p = 0; p < kParts; p++)
+                to.part[p] = __builtin_bit_cast(bf16x8, u32x4{pair[0][p], pair[1][p], pair[2][p], pair[3][p]});
+        }
+    };
+    Operand w[NT];
+    auto fetch_w = [&](int col0) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            float v[J];
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                v[j] = a.W[(int64_t)min(J * half + j, a.K - 1) * a.N + min(col0 + 32 * t + l32, a.N - 1)];
+            operand(v, w[t]);
+        }
+    };
+    fetch_w(0);
+    float x[J], next[J];
+    int64_t row_tile = (int64_t)blockIdx.x * kDenseWaves + wave;
+    fetch_x(x, row_tile);
+    for (; row_tile < n_row_tiles; row_tile += stride) {
+        fetch_x(next, row_tile + stride);
+        const int64_t row0 = row_tile * kDenseRows;
+        Operand xt;
+        operand(x, xt);
+        for (int tile = 0; tile < (NT == 4 ? a.n_col_tiles : 1); tile++) {
+            const int col0 = tile * NT * 32;
+            if (NT == 4 && a.n_col_tiles > 1) fetch_w(col0);
+            f32x16 acc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+            float unscale = 1;
+            if constexpr (kInFp32) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(xt.whole, w[t].whole, acc[t], 0, 0, 0);
+            } else {
+                constexpr int ap[6] = {2, 0, 1, 1, 0, 0}, bp[6] = {0, 2, 1, 0, 1, 0};         // the small products first
+#pragma unroll
+                for (int q = 0; q < 6; q++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xt.part[ap[q]], w[t].part[bp[q]], acc[t], 0, 0, 0);
+                bool finite = true;
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) finite &= __builtin_isfinite(acc[t][v]);
+                unscale = kUnscale;
+                if (__any(!finite)) {
+                    unscale = 1;
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
+                    add_in_fp32<NT>(a, row0, col0, acc);
+                }
+            }
+            const int64_t rows = a.rows - row0 - 4 * half;
+            const int col = col0 + l32;
+            float *z = a.Z + (row0 + 4 * half) * a.ldz + col;
+            asm volatile("" : "+v"(z));            // (the stores' addresses are formed here, not kept from tile to tile)
+            if (row0 + kDenseRows <= a.rows && col0 + NT * 32 <= a.N) {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v] * unscale;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        if (col + t * 32 < a.N && 8 * (v / 4) + v % 4 < rows)
+                            z[(8 * (v / 4) + v % 4) * a.ldz + t * 32] = acc[t][v] * unscale;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++) x[j] = next[j];
+    }
+}
+
 // The grid: as many workgroups as the GPU holds at once (asked of the runtime for the kernel
 // that runs, once per device and kernel), or one per block of rows when there are fewer.
 constexpr int kDenseDevices = 64;
-static std::atomic<int> g_resident[kDenseDevices][9];     // [device][kernel]: workgroups the device holds, 0 = not asked yet
+static std::atomic<int> g_resident[kDenseDevices][12];    // [device][kernel]: workgroups the device holds, 0 = not asked yet
 
-template <int NT, DenseW kHow>
-static int dense_launch(const DenseArgs &a, hipStream_t s)
+static int dense_launch(void (*kernel)(DenseArgs), int which, const DenseArgs &a, hipStream_t s)
 {
-    constexpr int which = (NT == 1 ? 0 : NT == 2 ? 3 : 6) + (int)kHow;
     int dev = 0;
     ACCEL_HIP(hipGetDevice(&dev));
     int resident = dev >= 0 && dev < kDenseDevices ? g_resident[dev][which].load(std::memory_order_relaxed) : 0;
     if (resident == 0) {
         int cus = 0, per_cu = 0;
         ACCEL_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        ACCEL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, dense_xw_kernel<NT, kHow>, kDenseThreads, 0));
+        ACCEL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kDenseThreads, 0));
         resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);
         if (dev >= 0 && dev < kDenseDevices) g_resident[dev][which].store(resident, std::memory_order_relaxed);
     }
     const unsigned grid = (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
-    dense_xw_kernel<NT, kHow><<<grid, kDenseThreads, 0, s>>>(a);
+    kernel<<<grid, kDenseThreads, 0, s>>>(a);
     return ACCEL_OK;
 }
 
@@ -469,7 +573,9 @@ constexpr double kPrepareFrom = 1e10;
 template <int NT>
 static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
 {
-    if (a.K < kDenseHalf) return dense_launch<NT, kWShort>(a, s);
+    constexpr int which = NT == 1 ? 0 : NT == 2 ? 4 : 8;
+    if (a.K <= 2) return dense_launch(dense_short_kernel<NT, true>, which, a, s);
+    if (a.K < kDenseHalf) return dense_launch(dense_short_kernel<NT, false>, which + 1, a, s);
     if constexpr (NT == 4) {
         const size_t blocks = (size_t)a.n_col_tiles * (size_t)a.n_steps;
         const size_t image_bytes = blocks * (NT * 32 * kParts * 4) * sizeof(u32x4);
@@ -480,12 +586,12 @@ static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
             u32x4 *image = static_cast<u32x4 *>(mem);
             dense_prepare_kernel<NT><<<dim3((unsigned)blocks), kDenseThreads, 0, s>>>(a, image);
             a.image = image;
-            const int rc = dense_launch<NT, kWPrepared>(a, s);
+            const int rc = dense_launch(dense_xw_kernel<NT, kWPrepared>, which + 2, a, s);
             give_stream_memory(mem, s);
             return rc;
         }
     }
-    return dense_launch<NT, kWOnTheWay>(a, s);
+    return dense_launch(dense_xw_kernel<NT, kWOnTheWay>, which + 3, a, s);
 }
 
 // Arguments have been checked by the caller (accel_dense_xw): rows >= 1, K, N >= 1,

@@ -160,3 +160,41 @@ def test_speed_does_not_hang_on_single_values(gpu, where, value, limit):
     if where == "X":
         X[rng.integers(0, rows, 200), rng.integers(0, K, 200)] = value
     assert milliseconds() <= limit * plain
+
+
+@pytest.mark.parametrize("rows,N", [(1, 1), (31, 33), (300, 20), (1000, 100), (129, 300)])
+def test_one_product_per_sum_is_rounded_once(gpu, rows, N):
+    """K = 1: every element is one fp32 product, correctly rounded."""
+    rng = np.random.default_rng(rows + N)
+    X = rng.standard_normal((rows, 1)).astype(np.float32)
+    W = rng.standard_normal((1, N)).astype(np.float32)
+    assert np.array_equal(gpu.dense_xw_numpy(X, W).view(np.uint32), (X * W).view(np.uint32))
+
+
+@pytest.mark.parametrize("K", [2, 3, 7, 8, 14, 15])
+@pytest.mark.parametrize("N", [5, 33, 100, 260])
+def test_short_k(gpu, K, N):
+    """Below half a step of the walk: sums of K rounded additions, infinities where they belong, and in rows that
+    are further apart than K nothing between them is read."""
+    rng = np.random.default_rng(K + N)
+    X = rng.standard_normal((1000, K)).astype(np.float32)
+    W = rng.standard_normal((K, N)).astype(np.float32)
+    assert so.check_dense(gpu.dense_xw_numpy(X, W), X, W) <= (K + 1) * 2.0 ** -24
+    ld = K + 3
+    wide = np.full((1000, ld), np.nan, np.float32)
+    wide[:, :K] = X
+    wide[70, K - 1] = np.inf
+    W[0, 3] = np.inf
+    dX, dW, dZ = gpu.DeviceBuffer.from_numpy(wide), gpu.DeviceBuffer.from_numpy(W), gpu.DeviceBuffer(1000 * (N + 5) * 4)
+    dZ.fill_u32(0x7FC00000)
+    gpu.dense_xw(dX, dW, dZ, 1000, K, N, ldx=ld, ldz=N + 5)
+    gpu._lib.check(gpu.lib().accel_stream_sync(None))
+    Z = dZ.to_numpy(np.float32, (1000, N + 5))
+    for b in (dX, dW, dZ):
+        b.close()
+    X[70, K - 1] = np.inf
+    with np.errstate(all="ignore"):
+        want = X.astype(np.float64) @ W.astype(np.float64)
+    assert np.isnan(Z[:, N:]).all()
+    assert np.array_equal(np.isfinite(Z[:, :N]), np.isfinite(want))
+    assert np.array_equal(np.isnan(Z[:, :N]), np.isnan(want))
