@@ -12,7 +12,8 @@
 //   - it holds at most 1/64 of the device's memory (4.5 GB here); beyond that the memory that
 //     has been idle longest is freed;
 //   - what nobody has asked for within kIdleSeconds is freed by the next call that takes or
-//     gives memory;
+//     gives memory (not by take_stream_memory and give_stream_memory, whose callers are not to
+//     wait for the device: they free only what is beyond the bound);
 //   - when an allocation fails, everything idle is freed and the allocation is tried again;
 //   - accel_release_memory() frees everything idle.
 // Sizes are rounded up to an eighth of a power of two and a block serves requests of down to
@@ -23,8 +24,8 @@
 // stream, behind which it carries an event (a handle that has used several streams waits for the
 // device before it gives its memory back).  The preprocessing, which takes nearly all of it,
 // works on the null stream and is ordered behind the former by the stream; every other
-// combination of the last use and the next waits for the event on the device, or on the host
-// where the next stream is not known (`any_stream`) or the last one was the null stream.
+// combination of the last use and the next waits on the device, for the event or for what the null
+// stream holds now, or on the host where the next stream is not known (`any_stream`).
 //
 // A wait may be refused (most are while any stream of the process captures).  A block whose last
 // use could not be waited for is marked so, stays on the list, and is handed out or freed only
@@ -105,21 +106,33 @@ void free_idle(std::vector<Idle> &gone)
     gone.clear();
 }
 
+// What is queued on s from now on comes behind what the null stream holds now.
+hipError_t wait_for_null_stream(hipStream_t s)
+{
+    hipEvent_t now = nullptr;
+    hipError_t e = hipEventCreateWithFlags(&now, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+    e = hipEventRecord(now, nullptr);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, now, 0);
+    (void)hipEventDestroy(now);
+    return e;
+}
+
 // Whether the next use of b, on s (with `any`: on a stream not known yet), comes behind its last one.
 bool order_behind(const Idle &b, hipStream_t s, bool any)
 {
     hipError_t e = hipSuccess;
     if (b.use == InUse::unknown) e = hipDeviceSynchronize();
     else if (b.after) e = any ? hipEventSynchronize(b.after) : hipStreamWaitEvent(s, b.after, 0);
-    else if (b.use == InUse::null_stream && (any || s)) e = hipStreamSynchronize(nullptr);
+    else if (b.use == InUse::null_stream && (any || s)) e = any ? hipStreamSynchronize(nullptr) : wait_for_null_stream(s);
     if (e == hipSuccess) return true;
     (void)hipGetLastError();
     return wait_for_device() == InUse::no;
 }
 
-// Takes the blocks idle for longer than kIdleSeconds, and the oldest beyond the bound, off the
-// list (the caller frees them, without the lock).
-void expire(Pool &pl, std::vector<Idle> &gone)
+// Takes the oldest blocks beyond the bound and (by_age) those idle for longer than kIdleSeconds off
+// the list (the caller frees them, without the lock).
+void expire(Pool &pl, std::vector<Idle> &gone, bool by_age)
 {
     const Clock::time_point now = Clock::now();
     std::unordered_map<int, size_t> held;
@@ -127,7 +140,7 @@ void expire(Pool &pl, std::vector<Idle> &gone)
     size_t keep = 0;
     for (size_t i = 0; i < pl.idle.size(); i++) {
         const Idle &b = pl.idle[i];
-        const bool old = std::chrono::duration<double>(now - b.since).count() > kIdleSeconds;
+        const bool old = by_age && std::chrono::duration<double>(now - b.since).count() > kIdleSeconds;
         if (old || held[b.device] > pl.most_idle[b.device]) {
             held[b.device] -= b.bytes;
             gone.push_back(b);
@@ -152,7 +165,7 @@ void release_idle_device_memory()
 }  // namespace
 
 // s: the stream the memory will be used on first; null: the null stream, or (any) one not known yet.
-static void *take(size_t bytes, hipStream_t s, bool any)
+static void *take(size_t bytes, hipStream_t s, bool any, bool by_age)
 {
     Pool &pl = pool();
     const size_t want = size_class(bytes);
@@ -172,7 +185,7 @@ static void *take(size_t bytes, hipStream_t s, bool any)
             got = pl.idle[best];
             pl.idle.erase(pl.idle.begin() + (long)best);
         }
-        expire(pl, gone);
+        expire(pl, gone, by_age);
     }
     free_idle(gone);
     if (got.p && order_behind(got, s, any)) {
@@ -201,7 +214,7 @@ static void *take(size_t bytes, hipStream_t s, bool any)
     return p;
 }
 
-static void give(void *p, InUse use, hipEvent_t after)
+static void give(void *p, InUse use, hipEvent_t after, bool by_age)
 {
     if (!p) return;
     Pool &pl = pool();
@@ -212,28 +225,28 @@ static void give(void *p, InUse use, hipEvent_t after)
         if (it == pl.live.end()) return;
         pl.idle.push_back({p, it->second.first, it->second.second, use, after, Clock::now()});
         pl.live.erase(it);
-        expire(pl, gone);
+        expire(pl, gone, by_age);
     }
     free_idle(gone);
 }
 
-void *take_memory(size_t bytes, bool any_stream) { return take(bytes, nullptr, any_stream); }
-void give_memory(void *p, InUse use) { give(p, use, nullptr); }
-void *take_stream_memory(size_t bytes, hipStream_t s) { return take(bytes, s, false); }
+void *take_memory(size_t bytes, bool any_stream) { return take(bytes, nullptr, any_stream, true); }
+void give_memory(void *p, InUse use) { give(p, use, nullptr, true); }
+void *take_stream_memory(size_t bytes, hipStream_t s) { return take(bytes, s, false, false); }
 
 void give_stream_memory(void *p, hipStream_t s)
 {
-    if (!s) { give(p, InUse::null_stream, nullptr); return; }
+    if (!s) { give(p, InUse::null_stream, nullptr, false); return; }
     hipEvent_t after = nullptr;
     if (hipEventCreateWithFlags(&after, hipEventDisableTiming) == hipSuccess && hipEventRecord(after, s) == hipSuccess) {
-        give(p, InUse::no, after);
+        give(p, InUse::no, after, false);
         return;
     }
     (void)hipGetLastError();
     if (after) (void)hipEventDestroy(after);
     const bool done = hipStreamSynchronize(s) == hipSuccess;
     if (!done) (void)hipGetLastError();
-    give(p, done ? InUse::no : InUse::unknown, nullptr);
+    give(p, done ? InUse::no : InUse::unknown, nullptr, false);
 }
 
 // Pinned blocks for the preprocessing's results, one per call that is under way; kept (a few KB

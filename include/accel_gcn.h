@@ -396,7 +396,9 @@ int accel_time_ex(accel_handle *h, const accel_run_args *args, int warmup, int i
  * written); all three on the device, Z overlapping neither input.  Any rows >= 0, K >= 1,
  * N >= 1.  Needs no handle; asynchronous on `stream`.  Products of more than 64 columns and 1e10
  * multiplications take a workspace of 6 bytes per element of W from the memory the library keeps
- * (accel_release_memory); the others, and all of them while the stream is capturing, take none.
+ * (accel_release_memory): the first one allocates it, a later one on another stream is ordered
+ * behind the last on the device; memory is freed only where what the library keeps exceeds its bound.
+ * The others, and all of them while the stream is capturing, take none.
  * Computed on the matrix cores, each fp32 value as three bf16 values that add up to it: sums of K
  * products in fp32 (error as of fp32 instructions, or smaller), whose order differs from a
  * sequential loop (compare against a higher-precision product, as for accel_run).  Tiles of 32 rows and

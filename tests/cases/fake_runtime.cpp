@@ -393,6 +393,34 @@ static void wait_refused_before_values_are_restored()
     CHECK(g_null[0].queued == queued && u.h->val_stale);
 }
 
+// The dense product waits on the device only, and frees nothing, whichever stream used its workspace last
+// and however long that is ago.
+static void dense_product_never_waits()
+{
+    const int64_t rows = 300000;
+    const int K = 300, N = 128;
+    void *X, *W, *Z;
+    CHECK(hipMalloc(&X, sizeof(float) * (size_t)rows * K) == hipSuccess);
+    CHECK(hipMalloc(&W, sizeof(float) * (size_t)K * N) == hipSuccess);
+    CHECK(hipMalloc(&Z, sizeof(float) * (size_t)rows * N) == hipSuccess);
+    auto product = [&](hipStream_t s) {
+        return accel_dense_xw(static_cast<float *>(X), static_cast<float *>(W), static_cast<float *>(Z), rows, K, N, 0, 0, s);
+    };
+    { DevBuf b; CHECK(b.alloc(kBlock) == ACCEL_OK); }      // idle memory of another size, about to expire
+    CHECK(product(nullptr) == ACCEL_OK);
+    const long tick = g_null[0].queued;
+    std::this_thread::sleep_for(std::chrono::milliseconds(1200));
+    const size_t blocks = g_memory.size();
+    CHECK(product(handle_of(g_side[0])) == ACCEL_OK);
+    CHECK(g_memory.size() == blocks);                      // the same workspace ...
+    CHECK(g_side[0].behind[&g_null[0]] >= tick);           // ... behind the product on the null stream
+    CHECK(product(handle_of(g_side[1])) == ACCEL_OK);
+    CHECK(g_side[1].behind[&g_side[0]] >= g_side[0].queued);
+    CHECK(product(nullptr) == ACCEL_OK);
+    CHECK(g_null[0].behind[&g_side[1]] >= g_side[1].queued);
+    CHECK(g_memory.size() == blocks && g_host_waits == 0 && g_frees == 0);
+}
+
 int main(int argc, char **argv)
 {
     g_null[1].device = 1;
@@ -409,6 +437,7 @@ int main(int argc, char **argv)
         SCENARIO(wait_refused_on_growth),
         SCENARIO(wait_refused_in_a_value_update),
         SCENARIO(wait_refused_before_values_are_restored),
+        SCENARIO(dense_product_never_waits),
     };
     if (argc != 2 || !all.count(argv[1])) {
         for (auto &s : all) std::printf("%s\n", s.first.c_str());
