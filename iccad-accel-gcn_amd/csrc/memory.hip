@@ -283,9 +283,13 @@ void give_mail(Mail *m)
     g_mail.push_back(m);
 }
 
+// One whose copies cannot be waited for is left alone.
 static void free_stage(Stage *s)
 {
-    if (s->busy) (void)hipEventSynchronize(s->last);
+    if (s->in_doubt || (s->busy && hipEventSynchronize(s->last) != hipSuccess)) {
+        (void)hipGetLastError();
+        return;
+    }
     for (hipEvent_t e : s->event)
         if (e) (void)hipEventDestroy(e);
     if (s->last) (void)hipEventDestroy(s->last);
@@ -308,10 +312,13 @@ Stage *take_stage(size_t bytes)
                 g_stage.erase(g_stage.begin() + (long)i);
             }
     }
-    if (s) {
-        if (s->busy && hipEventSynchronize(s->last) != hipSuccess) (void)hipGetLastError();
+    if (s && (!s->busy || hipEventSynchronize(s->last) == hipSuccess)) {
         s->busy = false;
         return s;
+    }
+    if (s) {                      // the wait was refused: another one
+        (void)hipGetLastError();
+        give_stage(s);
     }
     s = new Stage;
     s->bytes = want;
@@ -329,7 +336,7 @@ Stage *take_stage(size_t bytes)
 
 void give_stage(Stage *s)
 {
-    if (!s) return;
+    if (!s || s->in_doubt) return;
     Stage *gone = nullptr;
     {
         std::lock_guard<std::mutex> lock(g_host_mu);

@@ -60,6 +60,7 @@ struct Stage {
     hipEvent_t event[kStageBytes / kStagePiece] = {}, last = nullptr;
     int device = 0;
     bool busy = false;            // `last` stands behind the last copy out of it
+    bool in_doubt = false;        // copies nobody has waited for, with no event behind them
 };
 Stage *take_stage(size_t bytes);      // memory.hip: min(bytes, kStageBytes) or more; null when there is none
 void give_stage(Stage *s);

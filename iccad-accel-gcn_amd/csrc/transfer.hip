@@ -29,11 +29,13 @@ int upload(void *dst, const void *src, size_t bytes, hipStream_t s)
         if (off >= kStageBytes) ACCEL_HIP(hipEventSynchronize(done));
         char *stage = static_cast<char *>(st.s->p) + at;
         memcpy(stage, static_cast<const char *>(src) + off, n);
-        st.s->busy = true;
+        st.s->in_doubt = true;
         ACCEL_HIP(hipMemcpyAsync(static_cast<char *>(dst) + off, stage, n, hipMemcpyHostToDevice, s));
         if (bytes > kStageBytes) ACCEL_HIP(hipEventRecord(done, s));
     }
     ACCEL_HIP(hipEventRecord(st.s->last, s));           // who takes the buffer next waits for its last copy
+    st.s->busy = true;
+    st.s->in_doubt = false;
     return ACCEL_OK;
 }
 
@@ -44,6 +46,7 @@ int download(void *dst, const void *src, size_t bytes, hipStream_t s)
     for (size_t done = 0; done < bytes;) {
         const size_t here = std::min(bytes - done, kStageBytes);
         const int n = (int)((here + kStagePiece - 1) / kStagePiece);
+        st.s->in_doubt = true;
         char *to = static_cast<char *>(dst) + done, *stage = static_cast<char *>(st.s->p);
         for (int i = 0; i < n; i++) {
             const size_t off = (size_t)i * kStagePiece;
@@ -75,6 +78,7 @@ int download(void *dst, const void *src, size_t bytes, hipStream_t s)
         copy_pieces();
         for (int i = 0; i < n_helpers; i++) helper[i].join();
         ACCEL_HIP(e);
+        st.s->in_doubt = false;
         done += here;
     }
     return ACCEL_OK;

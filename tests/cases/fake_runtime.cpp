@@ -421,6 +421,27 @@ static void dense_product_never_waits()
     CHECK(g_memory.size() == blocks && g_host_waits == 0 && g_frees == 0);
 }
 
+// A pinned transfer buffer whose copies could not be waited for is not used again.
+static void wait_refused_in_a_transfer()
+{
+    std::vector<char> host(kStagePiece + 100);
+    void *dev;
+    CHECK(hipMalloc(&dev, host.size()) == hipSuccess);
+    CHECK(upload(dev, host.data(), host.size(), nullptr) == ACCEL_OK);
+    Stage *first = take_stage(host.size());                // waits for the copies out of it
+    void *const pinned = first->p;
+    CHECK(g_null[0].done == g_null[0].queued);
+    give_stage(first);
+    CHECK(upload(dev, host.data(), host.size(), nullptr) == ACCEL_OK);
+    g_refuse_host_waits = true;
+    Stage *other = take_stage(host.size());
+    CHECK(other && other->p != pinned);
+    give_stage(other);
+    CHECK(download(host.data(), dev, host.size(), nullptr) != ACCEL_OK);
+    Stage *third = take_stage(host.size());
+    CHECK(third && third->p != pinned && third->p != other->p);
+}
+
 int main(int argc, char **argv)
 {
     g_null[1].device = 1;
@@ -438,6 +459,7 @@ int main(int argc, char **argv)
         SCENARIO(wait_refused_in_a_value_update),
         SCENARIO(wait_refused_before_values_are_restored),
         SCENARIO(dense_product_never_waits),
+        SCENARIO(wait_refused_in_a_transfer),
     };
     if (argc != 2 || !all.count(argv[1])) {
         for (auto &s : all) std::printf("%s\n", s.first.c_str());
