@@ -46,8 +46,15 @@ Mail *take_mail();            // memory.hip; null when there is none
 void give_mail(Mail *m);
 struct MailHolder {
     Mail *m;
+    bool written = false;         // every kernel that writes it has been waited for
     MailHolder() : m(take_mail()) {}
-    ~MailHolder() { give_mail(m); }
+    // (on an error kernels that write it may be queued on the null stream; left alone where they cannot
+    // be waited for)
+    ~MailHolder()
+    {
+        if (written || hipStreamSynchronize(nullptr) == hipSuccess) give_mail(m);
+        else (void)hipGetLastError();
+    }
     MailHolder(const MailHolder &) = delete;
     MailHolder &operator=(const MailHolder &) = delete;
 };

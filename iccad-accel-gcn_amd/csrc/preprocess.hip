@@ -1363,8 +1363,11 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
         return rc;
     if (mail->stat[kStatUnsorted]) {
         tmp.next_chunk = (size_t)rows * 13 + (1 << 16);
-        return partition_any_order(&tmp, indptr_dev, rows, block4_dev, n_blocks, mail, s);
+        rc = partition_any_order(&tmp, indptr_dev, rows, block4_dev, n_blocks, mail, s);
+        mh.written = rc == ACCEL_OK;
+        return rc;
     }
+    mh.written = true;                        // by the counting pass alone
     const RunTotals rt = run_totals(mail->hist, kDegBound, kDegBound);
     const int n_long = mail->hist[kLongBin];
     const int64_t n_zeroed = long_zeroed_ints(n_long);
@@ -1737,6 +1740,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     // ---- work list (ends on the second synchronisation) -----------------------------------
     h->nnz_short = whole.nnz;
     if ((rc = build_work_list(&tmp, h, ua.sr, rule, sh, pu, gcount, whole.units, zeroed, mail, s))) return rc;
+    mh.written = true;
     if (mail->bad_index) {
         set_error("a column index lies outside [0, cols)");
         return ACCEL_ERR_CSR;

@@ -442,6 +442,32 @@ static void wait_refused_in_a_transfer()
     CHECK(third && third->p != pinned && third->p != other->p);
 }
 
+// Preprocessing that runs out of memory half way: kernels still queued write into the pinned block that
+// its results come through.
+static void preprocessing_runs_out_of_memory()
+{
+    const int rows = 1000;
+    std::vector<int32_t> indptr(rows + 1), idx(rows, 0);
+    std::vector<float> val(rows, 1.0f);
+    for (int i = 0; i <= rows; i++) indptr[i] = i;
+    int failed = 0;
+    for (int n = 0; n < 40; n++) {
+        accel_handle *h = nullptr;
+        CHECK(accel_create(indptr.data(), idx.data(), val.data(), rows, 1, rows, ACCEL_PTR_HOST, &h) == ACCEL_OK);
+        CHECK(accel_release_memory() == ACCEL_OK);
+        g_mallocs_left = n;
+        const int rc = accel_preprocess(h);
+        g_mallocs_left = -1;
+        failed += rc == ACCEL_ERR_ALLOC;
+        Mail *m = take_mail();
+        CHECK(g_null[0].done == g_null[0].queued);
+        give_mail(m);
+        CHECK(accel_destroy(h) == ACCEL_OK);
+        if (rc == ACCEL_OK) { CHECK(failed >= 4); return; }
+    }
+    CHECK(false);
+}
+
 int main(int argc, char **argv)
 {
     g_null[1].device = 1;
@@ -460,6 +486,7 @@ int main(int argc, char **argv)
         SCENARIO(wait_refused_before_values_are_restored),
         SCENARIO(dense_product_never_waits),
         SCENARIO(wait_refused_in_a_transfer),
+        SCENARIO(preprocessing_runs_out_of_memory),
     };
     if (argc != 2 || !all.count(argv[1])) {
         for (auto &s : all) std::printf("%s\n", s.first.c_str());
