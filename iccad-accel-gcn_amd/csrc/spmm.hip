@@ -895,6 +895,7 @@ int row_stride(const accel_handle *h, int N)
 // -> 143 us, N = 50: 278 -> 275.
 static bool pads_x(const accel_handle *h, uintptr_t x, int N, int64_t ld)
 {
+    if (N > kPadMaxN || (size_t)h->cols * (size_t)whole_lines(N) > kPadMaxFloats) return false;
     const double saved = saved_by_padding(h, x, N, ld);
     return saved > 5e-6 && saved > 1.2 * (4e-6 + 4.0 * (double)h->cols * (N + whole_lines(N)) / 5e12);
 }
@@ -922,7 +923,7 @@ int reserve_run(accel_handle *h, int max_N)
     size_t floats = 0;
     for (int N = std::min(max_N, kPadMaxN); N > 0 && floats == 0; N--)
         if (pads_x(h, 0, N, N)) floats = (size_t)h->cols * (size_t)whole_lines(N);
-    if (floats > 0 && floats <= kPadMaxFloats) (void)room_for_rows(h, floats, true);
+    if (floats > 0) (void)room_for_rows(h, floats, true);
     return ACCEL_OK;
 }
 
@@ -943,7 +944,8 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // the capture status is only asked for where something depends on it: a buffer that would
     // have to grow, or a stream the handle would have to order against another
     const bool must_grow = uses_handle_partial && h->partial_floats < (size_t)h->n_long_units * (size_t)ld;
-    bool pad = !static_partial && N <= kPadMaxN && pads_x(h, reinterpret_cast<uintptr_t>(X), N, ldx);
+    const bool best_padded = pads_x(h, reinterpret_cast<uintptr_t>(X), N, ldx);
+    bool pad = best_padded && !static_partial;
     const bool capturing = (must_grow || pad || needs_capture_status(h, stream)) && stream_is_capturing(stream);
     if (static_partial) {
         partial = nullptr;
@@ -972,7 +974,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // that a later run may replace.
     if (pad) {
         const size_t need = (size_t)h->cols * (size_t)whole_lines(N);
-        pad = !capturing && need <= kPadMaxFloats &&
+        pad = !capturing &&
               (h->x_rows_floats >= need || (N > h->reserved_N && room_for_rows(h, need, stream != nullptr)));
     }
     // The buffer is shared by all runs of this handle, and a value update may still be
@@ -980,6 +982,16 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // last waits for that stream on the device (runs queued on one stream are ordered anyway).
     hipEvent_t run_done = nullptr;                  // to be bound to the run's last kernel
     if (int rc = order_run(h, stream, uses_handle_partial || pad, capturing, &run_done)) return rc;
+    // What decides how the sums are grouped (panels and halves below, the vectors of the second kernel)
+    // is the same whether X has been copied or not: a run that could not (capturing, static, no memory) gives
+    // the bits of one that did.  (It pays for that where the copy would have put N = 97..127, 161..191, 225..255
+    // on whole lines: two panels of packed rows both take the line they meet in.  125 M non-zeros, captured, one
+    // pass and two panels: N = 127 9.19 and 10.40 ms, N = 191 12.8 and 15.2; 2.45 M, N = 127: 193 and 202 us.
+    // One pass in lane groups as narrow as a panel's, which adds up in the same order, takes 10.46 and 16.1 ms.)
+    const uintptr_t at_x = reinterpret_cast<uintptr_t>(X), at_y = reinterpret_cast<uintptr_t>(Y);
+    const bool whole_rows = ldx % 32 == 0 || best_padded;
+    const bool y_vectors = N % 4 == 0 && ld % 4 == 0 && at_y % 16 == 0;
+    const bool vectors = y_vectors && ((ldx % 4 == 0 && at_x % 16 == 0) || best_padded);
     if (pad) {
         const int to = whole_lines(N);
         const dim3 grid((unsigned)((h->cols + kPadRows - 1) / kPadRows));
@@ -994,8 +1006,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     // loaded and stored at 4-byte aligned addresses, and a row's last vector is moved back
     // so that it ends with the row (it overlaps the one before; both lanes hold the same
     // sums for the shared columns).  Scalar lanes are left for N < 4.
-    const uintptr_t align = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y);
-    const int mode = N < 4 ? 2 : (N % 4 == 0 && ld % 4 == 0 && ldx % 4 == 0 && align % 16 == 0) ? 0 : 1;
+    const int mode = N < 4 ? 2 : (y_vectors && ldx % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0) ? 0 : 1;
     const int vec = mode == 2 ? 1 : 4;
     // split rows are added up by the gather kernel itself (the wavefront that stores a row's
     // last piece), or, when the handle has no counters for that, by a second kernel
@@ -1012,10 +1023,10 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     int panel = N;
     const int want = h->plan_panel_option > 0 ? h->plan_panel_option : kPanel;
     const bool forced = h->plan_panel_option > 0;
-    const bool even = (mode == 0 && N % want == 0) ||                       // panels of whole lines
-                      (mode != 2 && ldx % 32 == 0 && whole_lines(N) % want == 0);
+    const bool even = (vectors && N % want == 0) ||                         // panels of whole lines
+                      (mode != 2 && whole_rows && whole_lines(N) % want == 0);
     if (N > want &&
-        ((forced && mode == 0) || (!forced && even && h->nnz >= kPanelMinNnz && h->nnz >= 16 * h->rows)))
+        ((forced && vectors) || (!forced && even && h->nnz >= kPanelMinNnz && h->nnz >= 16 * h->rows)))
         panel = want;
     // With more than one panel, two neighbouring panels are computed in one launch, each by every
     // other die: a die then sees twice the units but half of every row of X, so that what it fetches
@@ -1068,7 +1079,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
         // others share one: as many rows per workgroup as leaves a row one thread per vector
         // of columns (16 at least, so that a row's loads stay coalesced)
         const int n_split = (int)h->n_split_rows, n_big = (int)h->n_big_rows, n_shared = n_split - n_big;
-        const int rvec = mode == 0 ? 4 : 1;          // 16-byte accesses need the same as the gather kernel's
+        const int rvec = y_vectors ? 4 : 1;          // 16-byte accesses
         const int nv = (N + rvec - 1) / rvec;
         int threads_per_row = 16;
         while (threads_per_row < nv && threads_per_row < kReduceThreads) threads_per_row <<= 1;

@@ -209,7 +209,8 @@ int accel_set_plan_queues(accel_handle *h, int queues);
 /* Where the partial sums of split rows are added up.  Upstream's run is one launch
  * (spmm_accel.cu:104-108) whose blocks add long rows into vout with atomicAdd (:84,97).
  * Here every piece of a split row stores its sum to a slot of its own and the slots are
- * added in a fixed order (results are the same bits on every run): 1 = by the gather
+ * added in a fixed order (results are the same bits on every run of the same call; how sums are
+ * grouped depends on the plan, on N, and on the stride and alignment of X and Y): 1 = by the gather
  * kernel itself, one launch: each piece counts itself in on a per-row counter and the
  * wavefront that stores the row's last piece adds the row up; 2 = by a second, small
  * kernel behind the gather kernel; 0 (the default) = the library chooses: 1 when the
@@ -345,7 +346,9 @@ int accel_run_rows(accel_handle *h, const accel_run_args *args, int32_t ldx);
 /* Where packed rows of X touch many more cache lines than whole ones would, the columns are not
  * near the diagonal and the matrix has enough non-zeros per row, a run first copies X to padded
  * rows in a buffer that the handle keeps (below 4 GiB; one pass over X).
- * Not while its stream captures, and not for accel_run_static.
+ * Not while its stream captures, not for accel_run_static, and not where the memory cannot be had:
+ * such a run gives the same bits and takes longer.  The buffer is kept until the handle is
+ * preprocessed again or destroyed.
  *
  * accel_run keeps the partial sums of split rows (pieces x N floats) in a buffer of the
  * handle.  It is allocated by the first accel_run with a given N and replaced by a larger

@@ -1,5 +1,7 @@
 """Runs that copy X to rows on whole cache lines first give the packed run's result (accel_run_static never copies),
 whatever the column count, the stride and the alignment of X; the GCN layer lays its own buffer out so."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -53,13 +55,46 @@ def test_padded_run_is_the_packed_one(gpu, graph, N, ld, shift):
         for b in (dX, dP, dY, dS):
             b.close()
     assert np.isnan(Y[:, N:]).all()
-    if N > 96:                                         # two column panels: the sums are grouped otherwise
-        assert np.abs(Y[:, :N] - S).max() <= 2e-5 * np.abs(S).max()
-    else:
-        assert np.array_equal(Y[:, :N].view(np.int32), S.view(np.int32))
+    assert np.array_equal(Y[:, :N].view(np.int32), S.view(np.int32))
     rows = np.concatenate([np.arange(0, ROWS, 997), [ROWS - 1, int(np.argmax(np.diff(graph[0])))]])
     want = expected(graph, X, rows)
     assert np.abs(Y[rows, :N] - want).max() <= 2e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("N,shift", [(25, 0), (97, 0), (97, 3), (100, 0), (100, 1), (112, 2), (127, 0), (127, 2), (128, 0),
+                                     (128, 1), (191, 0), (225, 1), (256, 3)])
+def test_same_bits_where_nothing_can_be_copied(gpu, graph, N, shift):
+    """Packed rows: a run that may copy X, accel_run_static and a captured run, on the same operands."""
+    op = graph[3]
+    hip = C.CDLL("libamdhip64.so.7")
+    X = np.random.default_rng(N).standard_normal(shift + COLS * N).astype(np.float32)
+    dX, dY = gpu.DeviceBuffer.from_numpy(X), gpu.DeviceBuffer(ROWS * N * 4)
+    address = dX.address + 4 * shift
+    stream, graph_, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+
+    def bits(run):
+        dY.fill_u32(0x7FC00000)
+        run()
+        assert hip.hipDeviceSynchronize() == 0
+        return dY.to_numpy(np.uint32, (ROWS, N))
+
+    try:
+        eager = bits(lambda: op.run(address, dY, N))
+        assert np.isfinite(eager.view(np.float32)).all()
+        if op.info.n_plan_pieces * N * 4 <= gpu._lib.STATIC_SCRATCH_BYTES:
+            assert np.array_equal(bits(lambda: op.run_static(address, dY, N)), eager)
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        op.run(address, dY, N, stream=stream.value)
+        assert hip.hipStreamEndCapture(stream, C.byref(graph_)) == 0
+        assert hip.hipGraphInstantiate(C.byref(exe), graph_, None, None, 0) == 0
+        for _ in range(2):
+            assert np.array_equal(bits(lambda: hip.hipGraphLaunch(exe, stream)), eager)
+        assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph_) == 0
+    finally:
+        assert hip.hipStreamDestroy(stream) == 0
+        dX.close()
+        dY.close()
 
 
 def test_layer_on_padded_rows(gpu, graph):
