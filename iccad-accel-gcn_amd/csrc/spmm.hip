@@ -995,9 +995,7 @@ int spmm_launch(accel_handle *h, const float *X, float *Y, int N, hipStream_t st
     if (pad) {
         const int to = whole_lines(N);
         const dim3 grid((unsigned)((h->cols + kPadRows - 1) / kPadRows));
-        hipExtLaunchKernelGGL(pad_rows_kernel, grid, dim3(kWgThreads), 0, stream, main_start, nullptr, 0, X, (int64_t)h->cols,
-                              N, (int64_t)ldx, h->x_rows, to);
-        main_start = nullptr;
+        pad_rows_kernel<<<grid, dim3(kWgThreads), 0, stream>>>(X, (int64_t)h->cols, N, (int64_t)ldx, h->x_rows, to);
         X = h->x_rows;
         ldx = to;
     }

@@ -97,6 +97,17 @@ def test_same_bits_where_nothing_can_be_copied(gpu, graph, N, shift):
         dY.close()
 
 
+def test_main_time_is_the_gather_kernels_alone(gpu, graph):
+    """What a run that copies X first takes beyond its gather kernel holds the copy (204 MB, 12 us at twice the
+    memory's rate), next to the same run on rows that are on whole lines already."""
+    op, N = graph[3], 127
+    dX, dY = gpu.DeviceBuffer.from_numpy(np.ones((COLS, 128), np.float32)), gpu.DeviceBuffer(ROWS * 128 * 4)
+    beyond = [np.median(np.subtract(*op.time_ex(dX, dY, N, ld=ld, warmup=4, iters=20))) for ld in (127, 128)]
+    dX.close()
+    dY.close()
+    assert beyond[0] - beyond[1] >= 0.012, beyond
+
+
 def test_layer_on_padded_rows(gpu, graph):
     op = graph[3]
     K, N = 24, 25
