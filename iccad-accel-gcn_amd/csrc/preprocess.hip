@@ -1406,15 +1406,20 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
 // which shortens that chain, as long as the launch's workgroups are few: 2,048 of them are
 // on the GPU at once, and from about twice as many on wavefront units are faster (four
 // times fewer workgroups).  Units are about rows / 12 + nnz / 96, from the rows of a block4
-// entry and the unit size.  Measured (three matrices in turn, N = 12 / 32 / 64 / 128,
-// workgroup units, then wavefront units of up to 384):
-//   100 k non-zeros in 10 k rows, power law (1,900):   4.9 / 5.9 / 7.7 / 9.3 us,     8.0 / 7.6 / 11.8 / 12.4
-//   208 k in 10 k rows, power law (3,000):             6.1 / 8.5 / 10.3 / 12.7,      6.3 / 8.1 / 12.1 / 12.1
-//   300 k in 3 k rows, lognormal (3,400):              6.0 / 7.0 / 7.4 / 11.4,       6.0 / 6.5 / 8.7 / 10.8
-//   300 k in 15 k rows, power law (4,400):             8.0 / 10.7 / 12.5 / 17.6,     6.9 / 8.8 / 12.7 / 14.9
-//   150 k in 38 k rows, near the diagonal (4,700):     7.0 / 8.0 / 9.0 / 13.5,       5.0 / 5.1 / 8.7 / 10.9
-//   450 k in 27 k rows, hub rows (6,900):              14.6 / 15.7 / 18.4 / 24.8,    12.1 / 12.4 / 17.3 / 22.0
-//   300 k in 75 k rows, near the diagonal (9,400):     11.8 / 12.3 / 14.5 / 23.4,    5.7 / 7.2 / 10.7 / 16.8
+// entry and the unit size.  The choice is made without N, and between some 2,400 and 4,400 units it
+// depends on N which is faster: the line lies at the upper end of that, where workgroup units are still
+// level at N = 64.  Measured (one matrix, runs back to back, N = 12 / 32 / 64 / 128, workgroup
+// units, then wavefront units of up to 384):
+//   100 k non-zeros in 10 k rows, power law (1,900):   4.8 / 5.8 / 6.8 / 11.3 us,    6.8 / 7.4 / 8.1 / 9.6
+//   150 k in 10 k rows, power law (2,400):             5.1 / 6.6 / 7.3 / 9.1,        7.3 / 7.0 / 8.3 / 9.1
+//   80 k in 20 k rows, near the diagonal (2,500):      4.7 / 5.4 / 5.6 / 7.6,        4.7 / 4.8 / 6.5 / 7.9
+//   120 k in 20 k rows, power law (2,900):             5.2 / 6.2 / 7.8 / 9.4,        6.9 / 7.5 / 9.1 / 12.4
+//   208 k in 10 k rows, power law (3,000):             5.9 / 7.6 / 8.6 / 11.0,       5.4 / 8.0 / 9.4 / 10.5
+//   300 k in 3 k rows, lognormal (3,400):              5.8 / 6.8 / 7.2 / 10.1,       5.2 / 6.0 / 9.3 / 10.2
+//   250 k in 10 k rows, power law (3,400):             6.5 / 8.4 / 9.3 / 14.5,       6.2 / 7.9 / 9.4 / 10.5
+//   300 k in 15 k rows, power law (4,400):             7.4 / 9.4 / 11.2 / 14.2,      6.4 / 6.4 / 10.7 / 14.0
+//   150 k in 38 k rows, near the diagonal (4,700):     6.5 / 6.9 / 8.4 / 13.2,       4.7 / 4.8 / 6.5 / 9.1
+//   450 k in 27 k rows, hub rows (6,900):              13.1 / 14.3 / 17.0 / 22.9,    11.0 / 10.8 / 16.9 / 21.2
 constexpr int64_t kTeamMaxUnits = 4096, kSmallNnz = 512 * 1024;
 static bool choose_plan_team(int64_t rows, int64_t nnz)
 {

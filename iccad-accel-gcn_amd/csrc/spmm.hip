@@ -249,7 +249,7 @@ __device__ __forceinline__ void gather_steps(const int2 *row_st, int o, int gp, 
 // the rest in as many steps as there are (a gather under a condition of its own per step took as long to
 // issue as four).  d and gp are the same for the whole wavefront: the branches are scalar ones.
 // Together with the staging above: 114 M non-zeros, N = 64: 1748 -> 1704 us; 4 M next to the diagonal,
-// N = 64: 205 -> 192; 8 M, N = 32: 104 -> 91; 208 k, N = 32: 7.9 -> 7.6.  Several row sets at a time
+// N = 64: 205 -> 192; 8 M, N = 32: 104 -> 91; 208 k, N = 32, back to back: 7.9 -> 7.6.  Several row sets at a time
 // (gathers of up to three rows per lane group together) need 64 and more registers: 203 and 103 us.
 template <int VEC, bool kWide, bool kShift>
 __device__ __forceinline__ void gather_row(const int2 *row_st, int d, int k, int lg, const float *__restrict__ X, int col,

@@ -93,9 +93,11 @@ int accel_dev_fill_u32(void *dst_dev, uint32_t value, size_t n_words, void *stre
 int accel_dev_copy_u32(void *dst_dev, const void *src_dev, size_t n_words, void *stream);
 int accel_stream_sync(void *stream); /* NULL = default stream */
 /* Device memory of destroyed handles and of finished preprocessing is kept for the next handle:
- * at most 1/64 of the device's memory, for a second after its last use (later calls of the
- * library free it), and never at the price of a failed allocation.  This call frees what is
- * kept now. */
+ * at most 1/64 of the device's memory, and never at the price of a failed allocation of this
+ * library (other allocators of the process do not see it).  What has not been used for a second is
+ * freed by the next accel_create, accel_preprocess, accel_partition_gpu, accel_destroy or run that
+ * has to allocate, which pays for it; a program that makes no such call keeps it.  This call
+ * frees what is kept now (but not what a wait was refused for, see accel_destroy). */
 int accel_release_memory(void);
 
 /* ---- the operator ----------------------------------------------------------
@@ -410,8 +412,10 @@ int accel_time_ex(accel_handle *h, const accel_run_args *args, int warmup, int i
 int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32_t K, int32_t N,
                    int32_t ldx, int32_t ldz, void *stream);
 
-/* Waits for the device when the handle has been used on another stream than the null stream or
- * in a graph; work on the null stream may still be running when it returns. */
+/* Waits for the handle's GPU (whichever is current) when the handle has been used on another stream
+ * than the null stream or in a graph; work on the null stream may still be running when it returns.  Where
+ * the wait is refused (a stream of the process is capturing) the memory is kept and neither handed out
+ * nor freed before a later wait has succeeded. */
 int accel_destroy(accel_handle *h);
 
 #ifdef __cplusplus
