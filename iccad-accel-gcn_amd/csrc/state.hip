@@ -8,10 +8,10 @@
 // sorted copy of the non-zeros is as large as the CSR itself.  The state therefore holds
 // the one product that is an input to all the others, the degree-sort permutation, plus
 // the plan options the handle was preprocessed with.  accel_load_state reads it and runs
-// the preprocessing with the sort replaced by the stored order.
+// the preprocessing, the sort included (its bins are needed by everything that follows).
 //
 // Nothing in the file is trusted: the stored order is accepted only if a kernel finds it
-// to be exactly the order the sort would produce for this CSR's indptr (that order is
+// to be exactly the order the sort gives for this CSR's indptr (that order is
 // unique), so a state of another matrix, of another library version or with flipped bits
 // is refused with ACCEL_ERR_META, and everything that indexes memory is computed afresh
 // by the code that is running.

@@ -94,7 +94,7 @@ class AccelSpMM:
         check(lib().accel_save_state(self._h, str(path).encode()))
 
     def load_state(self, path) -> "AccelSpMM":
-        """Take the place of preprocess(): the preprocessing with the sort replaced by the
+        """Take the place of preprocess(): the preprocessing, checked against the
         order saved for the same CSR.  Raises AccelError (ERR_META) if the file belongs to
         another CSR or is damaged."""
         check(lib().accel_load_state(self._h, str(path).encode()))

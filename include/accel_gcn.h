@@ -150,16 +150,15 @@ int accel_set_plan_team(accel_handle *h, int mode);
  * accel_preprocess but one is rebuilt faster than a file of its size can be read, so
  * accel_save_state writes that one, the degree-sort permutation (4 bytes per row), and
  * the plan options of the handle.  accel_load_state takes the place of accel_preprocess
- * on a handle created on the same CSR: it runs the preprocessing with the sort replaced
- * by the stored order.  Nothing in the file is trusted: the order is used only after a
- * kernel has found it to be exactly the degree order of this CSR (ascending degree,
- * ties by row id: there is only one), so a file saved for another matrix, written by
+ * on a handle created on the same CSR: it runs the preprocessing, the sort included, and
+ * compares the stored order with the one the sort gives.  Nothing in the file is trusted:
+ * the degree order of a CSR is unique (ascending degree, ties by row id), so a file saved for another matrix, written by
  * another library version or damaged gives ACCEL_ERR_META and leaves the handle
  * un-preprocessed and its options as they were; a missing or short file gives
  * ACCEL_ERR_IO.  After a successful load the handle is the one that was saved: the same
  * options, and the results of accel_run are the same bits; accel_info.preprocess_ms is
- * the time of the load.  The load is not faster than accel_preprocess (reading the file
- * costs more than the sort it replaces); it exists for callers that want the operator's
+ * the time of the load.  The load is not faster than accel_preprocess (the file is read
+ * on top of it); it exists for callers that want the operator's
  * state to travel with the graph, as upstream's metadata file does. */
 int accel_save_state(const accel_handle *h, const char *path);
 int accel_load_state(accel_handle *h, const char *path);

@@ -258,6 +258,7 @@ static void reserved_with_another_gpu_current()
     u.h->partial_floats = kBlock / 4;
     u.h->n_long_units = (int64_t)kBlock / 64;
     CHECK(hipSetDevice(1) == hipSuccess);
+    CHECK(accel_run(u.h, u.h->partial, u.h->partial, 1, nullptr) == ACCEL_ERR_STATE);
     CHECK(accel_reserve(u.h, 128) == ACCEL_OK);
     CHECK(g_device == 1 && u.h->partial != old && find_memory(u.h->partial)->second.second == 0);
     CHECK(g_side[0].done == g_side[0].queued);             // the old buffer's users
