@@ -283,11 +283,26 @@ void give_mail(Mail *m)
     g_mail.push_back(m);
 }
 
-// One whose copies cannot be waited for is left alone.
+// Whether nothing copies out of the buffer or into it any more.
+static bool settle_stage(Stage *s)
+{
+    if (s->in_doubt) {
+        OnDevice on(s->device);
+        if (wait_for_device() != InUse::no) return false;
+    } else if (s->busy && hipEventSynchronize(s->last) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    s->in_doubt = s->busy = false;
+    return true;
+}
+
+// One whose copies cannot be waited for goes back on the list.
 static void free_stage(Stage *s)
 {
-    if (s->in_doubt || (s->busy && hipEventSynchronize(s->last) != hipSuccess)) {
-        (void)hipGetLastError();
+    if (!settle_stage(s)) {
+        std::lock_guard<std::mutex> lock(g_host_mu);
+        g_stage.insert(g_stage.begin(), s);
         return;
     }
     for (hipEvent_t e : s->event)
@@ -312,14 +327,8 @@ Stage *take_stage(size_t bytes)
                 g_stage.erase(g_stage.begin() + (long)i);
             }
     }
-    if (s && (!s->busy || hipEventSynchronize(s->last) == hipSuccess)) {
-        s->busy = false;
-        return s;
-    }
-    if (s) {                      // the wait was refused: another one
-        (void)hipGetLastError();
-        give_stage(s);
-    }
+    if (s && settle_stage(s)) return s;
+    if (s) give_stage(s);         // the wait was refused: another one
     s = new Stage;
     s->bytes = want;
     s->device = dev;
@@ -336,17 +345,17 @@ Stage *take_stage(size_t bytes)
 
 void give_stage(Stage *s)
 {
-    if (!s || s->in_doubt) return;
-    Stage *gone = nullptr;
+    if (!s) return;
+    std::vector<Stage *> gone;
     {
         std::lock_guard<std::mutex> lock(g_host_mu);
         g_stage.push_back(s);
-        if (g_stage.size() > kIdleStages) {
-            gone = g_stage.front();
+        while (g_stage.size() > kIdleStages) {
+            gone.push_back(g_stage.front());
             g_stage.erase(g_stage.begin());
         }
     }
-    if (gone) free_stage(gone);
+    for (Stage *g : gone) free_stage(g);
 }
 
 void release_idle_memory()

@@ -31,7 +31,7 @@ struct FakeEvent {
 static FakeStream g_null[2];                      // two devices
 static int g_device = 0;
 static bool g_refuse_host_waits = false, g_refuse_events = false;
-static int g_host_waits = 0, g_frees = 0;
+static int g_host_waits = 0, g_frees = 0, g_pinned = 0;
 static long g_mallocs_left = -1;                  // -1: no limit
 static std::map<char *, std::pair<size_t, int>> g_memory;
 static hipError_t g_last = hipSuccess;
@@ -82,8 +82,8 @@ hipError_t hipFree(void *p)
     free(p);
     return hipSuccess;
 }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = calloc(1, n); return hipSuccess; }
-hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = calloc(1, n); g_pinned++; return hipSuccess; }
+hipError_t hipHostFree(void *p) { free(p); g_pinned--; return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
 {
     memset(a, 0, sizeof *a);
@@ -422,7 +422,7 @@ static void dense_product_never_waits()
     CHECK(g_memory.size() == blocks && g_host_waits == 0 && g_frees == 0);
 }
 
-// A pinned transfer buffer whose copies could not be waited for is not used again.
+// A pinned transfer buffer whose copies could not be waited for is not used before they have been, and not lost.
 static void wait_refused_in_a_transfer()
 {
     std::vector<char> host(kStagePiece + 100);
@@ -441,6 +441,11 @@ static void wait_refused_in_a_transfer()
     CHECK(download(host.data(), dev, host.size(), nullptr) != ACCEL_OK);
     Stage *third = take_stage(host.size());
     CHECK(third && third->p != pinned && third->p != other->p);
+    give_stage(third);
+    CHECK(g_pinned == 3);
+    g_refuse_host_waits = false;
+    CHECK(accel_release_memory() == ACCEL_OK);
+    CHECK(g_pinned == 0 && g_null[0].done == g_null[0].queued);
 }
 
 // Preprocessing that runs out of memory half way: kernels still queued write into the pinned block that
