@@ -32,6 +32,7 @@
 // once a wait for its whole device has succeeded; until then requests get other memory.
 #include <chrono>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -329,7 +330,8 @@ Stage *take_stage(size_t bytes)
     }
     if (s && settle_stage(s)) return s;
     if (s) give_stage(s);         // the wait was refused: another one
-    s = new Stage;
+    s = new (std::nothrow) Stage;
+    if (!s) { set_error("host allocation failed"); return nullptr; }
     s->bytes = want;
     s->device = dev;
     bool ok = hipHostMalloc(&s->p, want, hipHostMallocDefault) == hipSuccess;

@@ -10,7 +10,7 @@
 // nothing can start before they have (260 against 280 to 330).
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "preprocess.h"
@@ -68,7 +68,7 @@ int download(void *dst, const void *src, size_t bytes, hipStream_t s)
         int n_helpers = 0;
         try {
             for (; n_helpers < std::min(kHelpers, n - 1); n_helpers++) helper[n_helpers] = std::thread(copy_pieces);
-        } catch (const std::system_error &) {           // fewer, then
+        } catch (const std::exception &) {              // no thread or no memory for one: fewer, then
         }
         hipError_t e = hipSuccess;
         for (int i = 0; i < n; i++) {
