@@ -398,16 +398,18 @@ int accel_time_ex(accel_handle *h, const accel_run_args *args, int warmup, int i
  * at A X).  X: rows x K floats, rows ldx floats apart (0 = K); W: K x N floats, packed
  * row-major; Z: rows x N floats, rows ldz apart (0 = N; the columns N .. ldz-1 are not
  * written); all three on the device, Z overlapping neither input.  Any rows >= 0, K >= 1,
- * N >= 1.  Needs no handle; asynchronous on `stream`.  Products of more than 64 columns and 1e10
- * multiplications take a workspace of 6 bytes per element of W from the memory the library keeps
- * (accel_release_memory): the first one allocates it, a later one on another stream is ordered
- * behind the last on the device; memory is freed only where what the library keeps exceeds its bound.
- * The others, and all of them while the stream is capturing, take none.
- * Computed on the matrix cores, each fp32 value as three bf16 values that add up to it: sums of K
- * products in fp32 (error as of fp32 instructions, or smaller), whose order differs from a
- * sequential loop (compare against a higher-precision product, as for accel_run).  Tiles of 32 rows and
- * up to 128 columns with infinities, NaN, operands of 2^103 and more or sums of 2^79 and more are computed
- * a second time by fp32 instructions (some three times the time where that is every tile). */
+ * N >= 1.  Needs no handle; asynchronous on `stream`.  Products of K >= 64 and 1e9 multiplications
+ * (N > 64; 4e9 for N = 33 .. 64) take a workspace of 4 bytes per element of W (its rows and columns rounded up to whole
+ * steps and tiles) from the memory the library keeps (accel_release_memory): the first one allocates it, a
+ * later one on another stream is ordered behind the last on the device; memory is freed only where what the
+ * library keeps exceeds its bound.  The others, and all of them while the stream is capturing, take none.
+ * Computed on the matrix cores: sums of K products in fp32 (error as of fp32 instructions, or smaller), whose
+ * order differs from a sequential loop (compare against a higher-precision product, as for accel_run).  With a workspace each
+ * fp32 value is two fp16 values (22 bits and more of it; error against fp64 0.7 of that without at K = 64, 0.5 from 256 on, and not the
+ * same bits), without one three bf16 values that add up to it.  Tiles of 32 rows and
+ * up to 128 columns with infinities, NaN or, without a workspace, operands of 2^103 and more or sums of 2^79 and more are computed
+ * a second time by fp32 instructions (some three times the time where that is every tile); with one, magnitudes of X
+ * more than 2^29 apart inside a tile cost extra steps, at worst a sixth of the time, and in W leave the product to three values. */
 int accel_dense_xw(const float *X, const float *W, float *Z, int64_t rows, int32_t K, int32_t N,
                    int32_t ldx, int32_t ldz, void *stream);
 
