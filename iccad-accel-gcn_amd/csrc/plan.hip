@@ -25,24 +25,15 @@
 // every row, in the caller's order, whether it starts a unit, so a scan of the counts per share
 // of rows puts the units in that order (list_units in preprocess.h).  The pieces of a column group are
 // ordered by a scan over (class of rows, group, row of the class).  What bounds all of it is
-// the number of dependent launches (2 to 5 us each), not bytes: five launches and no
-// synchronisation before the last, where there were 45 launches and two (110 of 440 us of
-// kernels at 2.45 M non-zeros, 400 us of 1.79 ms at 125 M).
+// the number of dependent launches (2 to 5 us each), not bytes: three launches and no
+// synchronisation before the last (the units are listed and the split rows counted in launches of
+// preprocess.hip), where there were 45 launches and two.
 #include "preprocess.h"
 
 namespace accel {
 namespace {
 
-constexpr int kClasses = 4;                 // rows stored in 8, 16, 32, 64 column groups
-// The split rows' unit counts per group are laid out [class][group][rank in the class].
-struct ClassLayout {
-    int rows[kClasses];                     // split rows of each class
-    int base[kClasses];                     // where the class's counts start
-    int above[kClasses];                    // rows of the classes with more groups
-    int total;                              // counts in all
-};
-
-ClassLayout class_layout(int64_t n_split, const Mail *stats, int groups)
+static ClassLayout class_layout(int64_t n_split, const Mail *stats, int groups)
 {
     ClassLayout c{};
     if (groups) {
@@ -72,56 +63,6 @@ __device__ __forceinline__ int64_t plan_index(int queue, int pos, int n_queues)
 {
     // queue q, position p  ->  slot of wavefront (p % 4) in workgroup (p / 4) * n_queues + q
     return ((int64_t)(pos / kWavesPerGroup) * n_queues + queue) * kWavesPerGroup + pos % kWavesPerGroup;
-}
-
-// A split row's place in its class: rows of 8 groups follow the caller's row ids, the longer
-// ones come largest first (they touch all of X whatever their id; the hub workload measured
-// 2 % faster that way: 2.31 against 2.36 ms at N = 256).
-struct SplitRow {
-    int d, groups, cls, rank;
-};
-__device__ __forceinline__ SplitRow split_row(const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
-                                              int lr, const int *__restrict__ rank8, const ClassLayout &cl, int forced)
-{
-    SplitRow s;
-    s.d = s_indptr[first_split + lr + 1] - s_indptr[first_split + lr];
-    s.groups = row_groups(s.d, forced);
-    s.cls = 31 - __clz(s.groups / kXcds);
-    s.rank = s.cls == 0 ? rank8[lr] : n_split - cl.above[s.cls] - 1 - lr;
-    return s;
-}
-
-// One wavefront per split row, lane = column group: pieces per group (into `bins`) and per row,
-// and what they cost per queue (column group g belongs to queue g % n_queues).
-__global__ __launch_bounds__(kThreads) void split_rows_kernel(
-    const int *__restrict__ gcount, const int32_t *__restrict__ s_indptr, int64_t first_split, int n_split,
-    const int *__restrict__ rank8, ClassLayout cl, int forced, int piece, int cost_shift, int n_queues,
-    int *__restrict__ bins, int *__restrict__ row_units, int *__restrict__ row_done, int *__restrict__ queue_cost)
-{
-    __shared__ int part[kWaves4][kXcds];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int cost = 0;
-    for (int lr = (int)blockIdx.x * kWaves4 + w; lr < n_split; lr += (int)gridDim.x * kWaves4) {
-        const SplitRow s = split_row(s_indptr, first_split, n_split, lr, rank8, cl, forced);
-        const int c = lane < s.groups ? gcount[(int64_t)lr * kMaxGroups + lane] : 0;
-        const int u = (c + piece - 1) / piece;
-        if (lane < s.groups) bins[cl.base[s.cls] + lane * cl.rows[s.cls] + s.rank] = u;
-        if (c > 0) cost += ((c + 9 * u) >> cost_shift) + u;
-        const int total = wave_sum(u);
-        if (lane == 0) {
-            row_units[lr] = total;
-            row_done[lr] = row_done[n_split + lr] = 0;
-        }
-    }
-    cost += __shfl_xor(cost, 8);
-    cost += __shfl_xor(cost, 16);
-    cost += __shfl_xor(cost, 32);
-    if (lane < kXcds) part[w][lane] = cost;
-    __syncthreads();
-    if ((int)threadIdx.x < kXcds) {
-        for (int q = 1; q < kWaves4; q++) cost += part[q][threadIdx.x];
-        if (cost) atomicAdd(&queue_cost[threadIdx.x % n_queues], cost);
-    }
 }
 
 // Where everything goes in the list: computed by one workgroup, read by the kernels that write it.
@@ -343,40 +284,54 @@ int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups)
     return kZeroQueueLoad + scan_zeroed(n_split) + scan_zeroed(class_layout(n_split, stats, groups).total);
 }
 
-int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
-                    const PlanUnits &pu, const int *gcount, int64_t n_short_units, int *zeroed, Mail *mail, hipStream_t s)
+int prepare_split_rows(Arena *tmp, const accel_handle *h, const SortedRows &sr, const UnitRule &rule, const PlanUnits &pu,
+                       int *zeroed, const Mail *stats, DevBuf *slot, SplitArgs *out)
 {
-    const Mail *stats = mail;
-    const int *share_sums = pu.sums;
-    // pieces of split rows hold up to piece_nz non-zeros, units of several whole rows up to unit_nz
-    const int piece_nz = std::max(h->plan_unit, h->plan_split), forced = rule.groups;
-    const int nq = h->plan_queues;                     // 8 interleaved queues, or 1 (plain order)
     const int n_split = (int)h->n_split_rows;
-    const int64_t first_split = h->rows - n_split;
-    const ClassLayout cl = class_layout(n_split, stats, forced);
+    int rc;
+    SplitArgs a{};
+    a.s_indptr = sr.s_indptr;
+    a.first_split = h->rows - n_split;
+    a.n_split = n_split;
+    a.rank8 = pu.rank8;
+    a.cl = class_layout(n_split, stats, rule.groups);
+    a.forced = rule.groups;
+    // pieces of split rows hold up to this many non-zeros, units of several whole rows up to plan_unit
+    a.piece = std::max(h->plan_unit, h->plan_split);
+    a.cost_shift = rule.cost_shift;
+    a.n_queues = h->plan_queues;                       // 8 interleaved queues, or 1 (plain order)
+    a.queue_cost = zeroed;
+    // the slots of each split row, and behind them two counters per split row (zero between launches)
+    if ((rc = slot->alloc(sizeof(int) * (size_t)(3 * (int64_t)n_split + 1)))) return rc;
+    a.row_done = slot->as<int>() + n_split + 1;
+    if (n_split > 0) {
+        if ((rc = tmp->alloc(&a.row_units, (size_t)n_split))) return rc;
+        if ((rc = tmp->alloc(&a.bins, (size_t)a.cl.total + 1))) return rc;
+    }
+    *out = a;
+    return ACCEL_OK;
+}
+
+int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
+                    const PlanUnits &pu, const SplitArgs &split, DevBuf *dslot, int64_t n_short_units, int *zeroed, Mail *mail,
+                    hipStream_t s)
+{
+    const int *share_sums = pu.sums, *gcount = split.gcount;
+    const int piece_nz = split.piece, forced = rule.groups, nq = split.n_queues;
+    const int n_split = split.n_split;
+    const int64_t first_split = split.first_split;
+    const ClassLayout &cl = split.cl;
     const int pitch = sh.pitch + kWaves4;
     int rc;
     const int4 *units = pu.units;
     const int *running = pu.running, *heavy = pu.heavy_before, *rank8 = pu.rank8;
-    int *row_units = nullptr, *bins = nullptr;
+    int *bins = split.bins;
     PlanHead *head;
     if ((rc = tmp->alloc(&head, 1))) return rc;
-    // the slots of each split row, and behind them two counters per split row (zero between launches)
-    DevBuf dslot;
-    if ((rc = dslot.alloc(sizeof(int) * (size_t)(3 * (int64_t)n_split + 1)))) return rc;
-    int *slot = dslot.as<int>(), *row_done = slot + n_split + 1;
+    int *slot = dslot->as<int>();
     if (n_split > 0) {
-        if ((rc = tmp->alloc(&row_units, (size_t)n_split))) return rc;
-        if ((rc = tmp->alloc(&bins, (size_t)cl.total + 1))) return rc;
-    }
-    if (n_split > 0) {
-        // (each workgroup ends on eight atomics to the same eight words)
-        const unsigned groups = std::min(grid_for((int64_t)n_split * 64), 1024u);
-        split_rows_kernel<<<dim3(groups), dim3(kThreads), 0, s>>>(
-            gcount, sr.s_indptr, first_split, n_split, rank8, cl, forced, piece_nz, rule.cost_shift, nq, bins,
-            row_units, row_done, zeroed);
         int *z = zeroed + kZeroQueueLoad;
-        launch_scans({{{row_units, slot, n_split, 0, z}, {bins, bins, cl.total, 0, z + scan_zeroed(n_split)}}, {}}, 2, s);
+        launch_scans({{{split.row_units, slot, n_split, 0, z}, {bins, bins, cl.total, 0, z + scan_zeroed(n_split)}}, {}}, 2, s);
     }
     plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, zeroed, running, share_sums, pitch, sh.n, nq, head,
                                                   mail);
@@ -417,7 +372,7 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
     h->n_units = (int64_t)mail->per_queue * nq;
     h->n_long_units = n_split > 0 ? mail->n_pieces : 0;
     h->work = static_cast<int32_t *>(dwork.release());
-    h->long_slot = static_cast<int32_t *>(dslot.release());
+    h->long_slot = static_cast<int32_t *>(dslot->release());
     h->row_done = h->long_slot + n_split + 1;
     h->fused_reduce = h->plan_reduce_option == 1 ||
                       (h->plan_reduce_option == 0 && h->n_long_units <= kFusedReduceMaxPieces);

@@ -19,9 +19,9 @@
 // launch plan that it opens.  One pass counts (degree_kernel), one workgroup per bin scans the
 // counts over the shares of rows (bin_scan_kernel), one pass places the rows and writes all of
 // that (place_rows_kernel).  The longer rows, few on most graphs, are ranked by comparison (or
-// by a radix sort when there are many) and scanned by one workgroup.
-// Measured against a radix sort of all rows with scans for every product: 24 launches instead
-// of 100 and two synchronisations instead of four.
+// by a radix sort when there are many).
+// Nine launches on a graph of 2.45 M non-zeros (ten more where thousands of rows are longer than 384) and two
+// synchronisations; a radix sort of all rows with scans for every product took 100 and four.
 #include <chrono>
 #include <climits>
 
@@ -361,10 +361,11 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Rows of more than 384 non-zeros: ranked by (degree, row), up to kRankMax of them by comparing each
-// with all (rank_long_rows_kernel; one workgroup for 800 rows takes 18 us, thirteen 5), more by a
-// stable radix sort, 8 bits a pass.  Their scans and blocks are one workgroup's work up to kFewLong
-// rows, launches of their own beyond.
+// Rows of more than 384 non-zeros, by (degree, row).  Up to kFewLong of them: each is compared with all
+// (place_long_kernel), and the non-zeros, blocks and chunks of the rows before it are added up on the way, which is all
+// there is to know (ranking, then a scan by one workgroup, took a launch and 10 us more on 2.45 M non-zeros).  More
+// are ranked by comparison up to kRankMax (rank_long_rows_kernel; one workgroup for 800 rows takes 18 us, thirteen 5),
+// or by a stable radix sort, 8 bits a pass; their scans and blocks are launches of their own.
 // ---------------------------------------------------------------------------
 constexpr int kFewLong = 2048;
 constexpr int kRankMax = 8192;
@@ -436,65 +437,66 @@ struct LongArgs {
     int *first_chunk, *chunk_row;             // of long row i (null: none is wide)
 };
 
-// The units of whole rows, for which everything is known by then.
-struct UnitsArgs {
-    SortedRows sr;
-    UnitRule rule;
-    PlanUnits pu;
-    int share, n_shares, pitch, first_split;
-    int groups;                               // workgroups, 0: not wanted
-};
-
-// Workgroup 0: row pointers, blocks and chunks of the long rows, when there are few.  The others: the
-// units of whole rows, a share of rows per wavefront.
-__global__ __launch_bounds__(1024) void few_long_rows_kernel(LongArgs a, const int *__restrict__ sorted_deg, UnitsArgs u)
+// Up to kFewLong long rows, completely: places, row pointers, blocks and chunks, 64 rows per workgroup.  The first kSums
+// workgroups scan the counts per share, as in rank_long_rows_kernel.
+__global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__restrict__ sums, int sum_pitch, int n_shares)
 {
-    __shared__ int lds[16];
-    __shared__ int sorted[kFewLong], first_block[kFewLong], loc[kFewLong];
-    const int t = threadIdx.x;
-    if (blockIdx.x > 0) {
-        static_assert(kFewLong >= kBins + 1, "the runs' tables fit");
-        for (int i = t; i <= kBins; i += 1024) sorted[i] = u.sr.run_row[i];
-        for (int i = t; i < kBins; i += 1024) loc[i] = u.sr.run_nz[i];
-        __syncthreads();
-        list_units(u.sr, u.rule, u.pu, u.share, u.n_shares, u.pitch, u.first_split, sorted, loc,
-                   ((int)blockIdx.x - 1) * 16 + (t >> 6));
-        return;
+    __shared__ __attribute__((aligned(16))) int deg[kFewLong + 64];
+    __shared__ int part[16][4][kRankRows];
+    __shared__ int4 mine[kRankRows];                     // rank, first non-zero, first block, first chunk
+    int b = blockIdx.x;
+    if (sums) {
+        if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, deg); return; }
+        b -= kSums;
     }
-    if (a.n == 0) return;
-    for (int i = t; i < a.n; i += 1024) sorted[i] = sorted_deg[i];
+    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
+    const uint32_t r = j < a.n ? a.row[j] : 0;
+    const int per = (a.n + 15) / 16;                     // of a wavefront
+    for (int i = threadIdx.x; i < a.n; i += 1024) deg[i] = a.deg[i];
     __syncthreads();
-    {
-        const int i = 2 * t, d0 = i < a.n ? sorted[i] : 0, d1 = i + 1 < a.n ? sorted[i + 1] : 0;
-        int tot;
-        const int nz = a.nz0 + block_exclusive_sum<1024>(d0 + d1, lds, tot);
-        const int blk = a.block0 + block_exclusive_sum<1024>(blocks_of(d0) + blocks_of(d1), lds, tot);
-        const int chk = block_exclusive_sum<1024>(chunks_of(d0) + chunks_of(d1), lds, tot);
-        if (i < a.n) {
-            loc[i] = nz;
-            first_block[i] = blk;
-            if (a.s_indptr) a.s_indptr[a.first_long + i] = nz;
-            if (a.first_chunk) a.first_chunk[i] = chk;
+    const int d = j < a.n ? deg[j] : 0;
+    int below = 0, nz = 0, blk = 0, chk = 0;
+    const int to = min(a.n, (seg + 1) * per);
+#pragma unroll 4
+    for (int i = seg * per; i < to; i++) {
+        const int e = deg[i];                            // equal degrees rank by row, which is the order they are listed in
+        if (e < d + (i < j)) {
+            below++;
+            nz += e;
+            blk += blocks_of(e);
+            chk += chunks_of(e);
         }
-        if (i + 1 < a.n) {
-            loc[i + 1] = nz + d0;
-            first_block[i + 1] = blk + blocks_of(d0);
-            if (a.s_indptr) a.s_indptr[a.first_long + i + 1] = nz + d0;
-            if (a.first_chunk) a.first_chunk[i + 1] = chk + chunks_of(d0);
-        }
-        if (a.first_chunk && t == 0) a.first_chunk[a.n] = tot;
     }
-    __syncthreads();                                     // (global stores of this workgroup are read back below)
-    const int lane = t & 63;
-    for (int i = t >> 6; i < a.n; i += 16) {
-        const int d = sorted[i];
-        for (int k = lane; k < blocks_of(d); k += 64)
-            a.block4[first_block[i] + k] =
-                make_int4(d, (int)a.first_long + i, loc[i] + k * kDegBound, min(kDegBound, d - k * kDegBound));
-        if (a.first_chunk && chunks_of(d) > 0) {
-            const int c0 = a.first_chunk[i];
-            for (int k = lane; k < chunks_of(d); k += 64) a.chunk_row[c0 + k] = i;
+    part[seg][0][lane] = below;
+    part[seg][1][lane] = nz;
+    part[seg][2][lane] = blk;
+    part[seg][3][lane] = chk;
+    __syncthreads();
+    if (seg == 0 && j < a.n) {
+        for (int q = 1; q < 16; q++) {
+            below += part[q][0][lane];
+            nz += part[q][1][lane];
+            blk += part[q][2][lane];
+            chk += part[q][3][lane];
         }
+        const int64_t p = a.first_long + below;
+        if (a.perm) a.perm[p] = (int32_t)r;
+        if (a.place) a.place[r] = (uint32_t)p;
+        if (a.s_indptr) a.s_indptr[p] = a.nz0 + nz;
+        if (a.first_chunk) {
+            a.first_chunk[below] = chk;
+            if (below == a.n - 1) a.first_chunk[a.n] = chk + chunks_of(d);
+        }
+        mine[lane] = make_int4(below, a.nz0 + nz, a.block0 + blk, chk);
+    }
+    __syncthreads();
+    for (int i = seg; i < kRankRows && b * kRankRows + i < a.n; i += 16) {
+        const int di = deg[b * kRankRows + i];
+        const int4 m = mine[i];
+        for (int k = lane; k < blocks_of(di); k += 64)
+            a.block4[m.z + k] = make_int4(di, (int)a.first_long + m.x, m.y + k * kDegBound, min(kDegBound, di - k * kDegBound));
+        if (a.first_chunk)
+            for (int k = lane; k < chunks_of(di); k += 64) a.chunk_row[m.w + k] = m.x;
     }
 }
 
@@ -653,27 +655,26 @@ __global__ __launch_bounds__(kThreads) void long_blocks_kernel(LongArgs a, const
 // Ints that must be zero for place_long_rows (place_rows clears them).
 int64_t long_zeroed_ints(int64_t n) { return n > kFewLong ? 3 * scan_zeroed(n) : 0; }
 
-// The long rows' places, row pointers, blocks and chunks, and the units of whole rows (u.groups > 0).
+// The long rows' places, row pointers, blocks and chunks, and the scan of the counts per share of rows (sums, null: none).
 // in_order: the rows are sorted already, so they are listed in sorted order.
 int place_long_rows(Arena *tmp, const LongArgs &a, bool in_order, int max_degree, const int32_t *loc_of, int *zeroed,
-                    const UnitsArgs &u, hipStream_t s)
+                    int *sums, int pitch, int n_shares, hipStream_t s)
 {
     int rc, *sorted_deg = const_cast<int *>(a.deg), *blocks, *chunks = nullptr;
-    int *sums = u.groups ? u.pu.sums : nullptr;
+    const unsigned scans = sums ? kSums : 0;
+    if (a.n <= kFewLong) {
+        const unsigned groups = scans + (unsigned)((a.n + kRankRows - 1) / kRankRows);
+        if (groups > 0) place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
+        return ACCEL_OK;
+    }
     const int ranked = !in_order && a.n <= kRankMax ? a.n : 0;
     if (!in_order && (rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
     if (sums || ranked > 0)
-        rank_long_rows_kernel<<<dim3((unsigned)((sums ? kSums : 0) + (ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0,
-                                s>>>(a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, u.pitch,
-                                     u.n_shares);
+        rank_long_rows_kernel<<<dim3(scans + (unsigned)((ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0, s>>>(
+            a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, pitch, n_shares);
     if (!in_order && a.n > kRankMax &&
         (rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
         return rc;
-    LongArgs few = a;
-    if (a.n > kFewLong) few.n = 0;
-    if (few.n > 0 || u.groups > 0)
-        few_long_rows_kernel<<<dim3(1u + (unsigned)u.groups), dim3(1024), 0, s>>>(few, sorted_deg, u);
-    if (a.n <= kFewLong) return ACCEL_OK;
     if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
     if (a.first_chunk && (rc = tmp->alloc(&chunks, (size_t)a.n))) return rc;
     long_sizes_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(sorted_deg, a.n, blocks, chunks);
@@ -884,15 +885,14 @@ __device__ __forceinline__ void group_row(const CopyArgs &a, GroupLds<R> &l, int
 }
 
 // Longer rows ("wide") in chunks of kWideChunk non-zeros, a workgroup per chunk, so that a row of
-// 200,000 is 49 workgroups and not a chain of 200 rounds in one: count the chunk's groups, scan the
-// counts of each row's chunks, place.  chunk_row[c] = the long row of chunk c, first_chunk[i] = the
+// 200,000 is 49 workgroups and not a chain of 200 rounds in one: count the chunk's groups, place.  chunk_row[c] = the long row of chunk c, first_chunk[i] = the
 // first chunk of long row i.
 struct WideArgs {
     const int *chunk_row, *first_chunk;
     int64_t first_long;                       // sorted row of the first long row
     int n_narrow;                             // long rows before the first wide one
     int forced_groups;
-    int *chunk_count;                         // [chunks][64]: counts, then destinations
+    int *chunk_count;                         // [chunks][64]: non-zeros of each group
 };
 struct WideChunk {
     int64_t src;
@@ -931,9 +931,22 @@ __device__ __forceinline__ void wide_count(const CopyArgs &a, const WideArgs &wa
     if ((int)threadIdx.x < kMaxGroups) wa.chunk_count[(int64_t)c * kMaxGroups + threadIdx.x] = cnt[threadIdx.x];
 }
 
+// The units of whole rows, for which everything is known when the rows are placed.
+struct UnitsArgs {
+    SortedRows sr;
+    UnitRule rule;
+    PlanUnits pu;
+    int share, n_shares, pitch, first_split;
+    int groups;                               // workgroups: a share of rows per wavefront
+};
+struct UnitsLds {
+    int run_row[kBins + 1], run_nz[kBins];
+};
+
 // All of the above in one launch (on a small matrix each would take its few microseconds after the
-// other): workgroups take, in this order, chunks of wide rows to count, split rows of up to 1,024 and
-// of up to 384 non-zeros (four each), tiles of whole rows.
+// other): workgroups take, in this order, shares of rows whose units are listed, chunks of wide rows to count, split rows
+// of up to 1,024 and of up to 384 non-zeros (four each), tiles of whole rows.  The units have nothing to do with the rest
+// but that both come behind the placing of the rows; a launch of their own took 8 to 10 us.
 constexpr int kSmallRounds = kDegBound / 64, kMidRounds = kWideRow / 64;
 struct CopyPlan {
     int n_chunks, n_mid, n_small;             // chunks; split rows
@@ -942,9 +955,10 @@ struct CopyPlan {
     int n_take;                               // non-zeros of whole rows
     int *counts;                              // [split row][64], or null
 };
-__global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArgs wa, CopyPlan cp)
+__global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArgs wa, CopyPlan cp, UnitsArgs u)
 {
     union Lds {
+        UnitsLds units;
         PermuteLds permute;
         GroupLds<kMidRounds> mid;
         GroupLds<kSmallRounds> small;
@@ -953,6 +967,15 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
     __shared__ __attribute__((aligned(16))) char raw[sizeof(Lds)];
     Lds &l = *reinterpret_cast<Lds *>(raw);
     int b = blockIdx.x;
+    if (b < u.groups) {
+        for (int i = threadIdx.x; i <= kBins; i += kThreads) l.units.run_row[i] = u.sr.run_row[i];
+        for (int i = threadIdx.x; i < kBins; i += kThreads) l.units.run_nz[i] = u.sr.run_nz[i];
+        __syncthreads();
+        list_units(u.sr, u.rule, u.pu, u.share, u.n_shares, u.pitch, u.first_split, l.units.run_row, l.units.run_nz,
+                   b * kWaves4 + (int)(threadIdx.x >> 6));
+        return;
+    }
+    b -= u.groups;
     if (b < cp.n_chunks) { wide_count(a, wa, l.cnt, b); return; }
     b -= cp.n_chunks;
     if (b < cp.mid_groups) {                  // a wavefront without a row leaves; no barriers inside
@@ -969,51 +992,39 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
     permute_rows(a, l.permute, b - cp.small_groups, cp.n_take);
 }
 
-// A workgroup per wide row turns the counts of its chunks into destinations in the sorted arrays
-// (thread: group threadIdx % 64, a quarter of the chunks).
-__global__ __launch_bounds__(kThreads) void wide_scan_kernel(CopyArgs a, WideArgs wa, int lr0, int *__restrict__ counts)
-{
-    __shared__ int part[kWaves4][kMaxGroups];
-    const int w = blockIdx.x, g = threadIdx.x & 63, q = threadIdx.x >> 6, i = wa.n_narrow + w;
-    const int c0 = wa.first_chunk[i], n = wa.first_chunk[i + 1] - c0;
-    const int per = (n + kWaves4 - 1) / kWaves4, from = c0 + min(n, q * per), to = c0 + min(n, (q + 1) * per);
-    int sum = 0;
-    for (int c = from; c < to; c++) sum += wa.chunk_count[(int64_t)c * kMaxGroups + g];
-    part[q][g] = sum;
-    __syncthreads();
-    int total = 0, before = 0;
-    for (int k = 0; k < kWaves4; k++) {
-        if (k < q) before += part[k][g];
-        total += part[k][g];
-    }
-    if (q == 0 && counts) counts[(int64_t)(lr0 + w) * kMaxGroups + g] = total;
-    int inc = total;                                     // every wavefront scans the 64 totals
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int t = __shfl_up(inc, off);
-        if (g >= off) inc += t;
-    }
-    int run = a.sr.s_indptr[wa.first_long + i] + inc - total + before;
-    for (int c = from; c < to; c++) {
-        int *p = wa.chunk_count + (int64_t)c * kMaxGroups + g;
-        const int v = *p;
-        *p = run;
-        run += v;
-    }
-}
-
+// Counts the split rows for the plan and, in the workgroups behind, places the chunks of wide rows, one each (both
+// come behind the counts of the chunks and nothing else: as launches of their own, with another that added up the
+// chunks' counts, they took 12 us more on 2.45 M non-zeros).
 constexpr int kPlaceThreads = 1024;
-__global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, WideArgs wa)
+__global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, WideArgs wa, int split_groups, SplitArgs split)
 {
     constexpr int kWaves = kPlaceThreads / 64;
     constexpr int R = kWideChunk / kPlaceThreads;        // rounds of a wavefront, which takes a sixteenth of the chunk
     __shared__ int2 buf[kWideChunk];
-    __shared__ int at[kWaves][kMaxGroups], off[kMaxGroups];
+    __shared__ int at[kWaves][kMaxGroups], off[kMaxGroups], sum[2][kWaves][kMaxGroups];
+    if ((int)blockIdx.x < split_groups) {
+        count_split_rows<kPlaceThreads>(split, (int)blockIdx.x, split_groups, reinterpret_cast<int (*)[kXcds]>(&sum[0][0][0]));
+        return;
+    }
+    const int chunk = (int)blockIdx.x - split_groups;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const WideChunk ch = wide_chunk(a, wa, (int)blockIdx.x);
+    const WideChunk ch = wide_chunk(a, wa, chunk);
     const int bits = 31 - __clz(ch.ng);
     at[w][lane] = 0;
     __builtin_amdgcn_wave_barrier();
+    // the row's non-zeros of each group, and those of the chunks before this one
+    {
+        const int i = wa.chunk_row[chunk], c0 = wa.first_chunk[i], c1 = wa.first_chunk[i + 1];
+        int all = 0, before = 0;
+#pragma unroll 4
+        for (int c = c0 + w; c < c1; c += kWaves) {
+            const int v = wa.chunk_count[(int64_t)c * kMaxGroups + lane];
+            all += v;
+            before += c < chunk ? v : 0;
+        }
+        sum[0][w][lane] = all;
+        sum[1][w][lane] = before;
+    }
     int col[R], pay[R];
 #pragma unroll
     for (int j = 0; j < R; j++) {
@@ -1039,7 +1050,19 @@ __global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, W
             if (lane >= o) inc += t;
         }
         int run = inc - total;                           // where the chunk's group `lane` starts in LDS
-        off[lane] = wa.chunk_count[(int64_t)blockIdx.x * kMaxGroups + lane] - run;
+        int all = 0, before = 0;
+#pragma unroll
+        for (int q = 0; q < kWaves; q++) {
+            all += sum[0][q][lane];
+            before += sum[1][q][lane];
+        }
+        int upto = all;                                  // the row's non-zeros of the groups up to this one
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(upto, o);
+            if (lane >= o) upto += t;
+        }
+        off[lane] = a.sr.s_indptr[wa.first_long + wa.chunk_row[chunk]] + upto - all + before - run;
 #pragma unroll
         for (int q = 0; q < kWaves; q++) { at[q][lane] = run; run += v[q]; }
     }
@@ -1393,7 +1416,7 @@ int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
         la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
         la.nz0 = (int)rt.nnz; la.block0 = (int)rt.blocks;
         la.block4 = b4.as<int4>();
-        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, UnitsArgs{}, s))) return rc;
+        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, nullptr, 0, 0, s))) return rc;
     }
     ACCEL_HIP(hipGetLastError());
     *block4_dev = static_cast<int32_t *>(b4.release());
@@ -1447,9 +1470,10 @@ constexpr int kPlanSplit = 192;
 static int choose_plan_split(int64_t nnz, bool team) { return team || nnz < kSmallNnz ? kDegBound : kPlanSplit; }
 
 // Launches that fill the sorted copy (see CopyArgs).  Needs perm (or none), s_indptr, the bins' runs,
-// n_split_rows and, for wide rows, the chunk tables, as the preprocessing leaves them on the handle.
-static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, int64_t nnz_short, int *counts,
-                         hipStream_t s)
+// n_split_rows and, for wide rows, the chunk tables, as the preprocessing leaves them on the handle.  The units of
+// whole rows are listed (u.groups > 0) and the split rows counted for the plan (split.n_split > 0) on the way.
+static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, int64_t nnz_short, const UnitsArgs &u,
+                         SplitArgs split, hipStream_t s)
 {
     const int64_t rows = h->rows;
     const int n_split = (int)h->n_split_rows, n_long = (int)h->n_long_rows, n_wide = (int)h->n_wide_rows;
@@ -1465,14 +1489,18 @@ static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, i
     cp.first_mid = rows - n_long;
     cp.first_small = rows - n_split;
     cp.n_take = (int)nnz_short;
-    cp.counts = counts;
-    const int64_t groups = (int64_t)cp.n_chunks + cp.mid_groups + cp.small_groups +
+    cp.counts = split.gcount;
+    const int64_t groups = (int64_t)u.groups + cp.n_chunks + cp.mid_groups + cp.small_groups +
                            (nnz_short + kPermuteTile - 1) / kPermuteTile;
-    if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp);
-    if (n_wide > 0) {
-        wide_scan_kernel<<<dim3((unsigned)n_wide), dim3(kThreads), 0, s>>>(a, wa, n_split - n_wide, counts);
-        wide_place_kernel<<<dim3((unsigned)h->n_chunks), dim3(kPlaceThreads), 0, s>>>(a, wa);
-    }
+    if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp, u);
+    split.n_wide = n_wide;
+    split.first_chunk = wa.first_chunk ? wa.first_chunk + wa.n_narrow : nullptr;
+    split.chunk_count = wa.chunk_count;
+    // (each workgroup of split rows ends on eight atomics to the same eight words)
+    constexpr unsigned kSplitGroups = 1024;
+    const unsigned split_groups = std::min((unsigned)((split.n_split + kPlaceThreads / 64 - 1) / (kPlaceThreads / 64)), kSplitGroups);
+    if (cp.n_chunks + split_groups > 0)
+        wide_place_kernel<<<dim3((unsigned)cp.n_chunks + split_groups), dim3(kPlaceThreads), 0, s>>>(a, wa, (int)split_groups, split);
     ACCEL_HIP(hipGetLastError());
     return ACCEL_OK;
 }
@@ -1502,7 +1530,7 @@ int build_source_positions(accel_handle *h, hipStream_t s)
     tmp.any_stream = s != nullptr;
     if (int rc = map.alloc(sizeof(int32_t) * (size_t)h->nnz, s != nullptr)) return rc;
     const CopyArgs ca{sorted_rows(h), h->idx, nullptr, (uint32_t)h->cols, nullptr, map.as<int32_t>(), 1, nullptr};
-    const int rc = copy_nonzeros(&tmp, h, ca, h->nnz_short, nullptr, s);
+    const int rc = copy_nonzeros(&tmp, h, ca, h->nnz_short, UnitsArgs{}, SplitArgs{}, s);
     const hipError_t e = hipStreamSynchronize(s);      // the temporaries are given back on return
     tmp.use = map.use = e == hipSuccess ? InUse::no : InUse::unknown;
     if (rc) return rc;
@@ -1725,26 +1753,34 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     ua.sr.place = place;
     ua.rule = rule; ua.pu = pu;
     ua.share = sh.share; ua.n_shares = sh.n; ua.pitch = sh.pitch + kWaves4; ua.first_split = (int)(rows - n_split);
-    ua.groups = (sh.n + 15) / 16;
-    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, ua, s))) return rc;
+    ua.groups = (int)sh.groups();
+    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, pu.sums, ua.pitch, sh.n, s)))
+        return rc;
     if (given && !h->identity_perm)
         compare_order_kernel<<<dim3(grid_for(rows)), dim3(kThreads), 0, s>>>(
             reinterpret_cast<const uint32_t *>(h->perm), given->perm_dev, rows, mail);
     ACCEL_HIP(hipGetLastError());
 
     // ---- sorted CSR; every column is looked at once on the way -------------------------
+    DevBuf slot;
+    SplitArgs split;
+    if ((rc = prepare_split_rows(&tmp, h, ua.sr, rule, pu, zeroed, mail, &slot, &split))) return rc;
+    split.gcount = gcount;
     if (own_copy) {
         const CopyArgs ca{sorted_rows(h), h->idx, h->val, (uint32_t)h->cols, s_idx, reinterpret_cast<int32_t *>(s_val), 0,
                           mail};
-        if ((rc = copy_nonzeros(&tmp, h, ca, whole.nnz, gcount, s))) return rc;
-    } else if (nnz > 0) {
-        const unsigned g = (unsigned)std::min<int64_t>((nnz / 4 + kThreads - 1) / kThreads + 1, 16384);
-        index_check_kernel<<<dim3(g), dim3(kThreads), 0, s>>>(h->idx, nnz, h->cols, mail);
+        if ((rc = copy_nonzeros(&tmp, h, ca, whole.nnz, ua, split, s))) return rc;
+    } else {
+        copy_rows_kernel<<<dim3((unsigned)ua.groups), dim3(kThreads), 0, s>>>(CopyArgs{}, WideArgs{}, CopyPlan{}, ua);
+        if (nnz > 0) {
+            const unsigned g = (unsigned)std::min<int64_t>((nnz / 4 + kThreads - 1) / kThreads + 1, 16384);
+            index_check_kernel<<<dim3(g), dim3(kThreads), 0, s>>>(h->idx, nnz, h->cols, mail);
+        }
     }
 
     // ---- work list (ends on the second synchronisation) -----------------------------------
     h->nnz_short = whole.nnz;
-    if ((rc = build_work_list(&tmp, h, ua.sr, rule, sh, pu, gcount, whole.units, zeroed, mail, s))) return rc;
+    if ((rc = build_work_list(&tmp, h, ua.sr, rule, sh, pu, split, &slot, whole.units, zeroed, mail, s))) return rc;
     mh.written = true;
     if (mail->bad_index) {
         set_error("a column index lies outside [0, cols)");
