@@ -23,8 +23,8 @@ void set_error(const char *fmt, ...)
 const char *get_error() { return g_error.c_str(); }
 void clear_error() { g_error.clear(); }
 
-int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
-                          int32_t **block4_dev, int64_t *n_blocks);
+int partition_to_host(const int32_t *indptr_dev, int64_t rows, int64_t nnz, int32_t *block4_out, int64_t cap,
+                      int64_t *n_blocks);
 bool stream_is_capturing(hipStream_t s);
 int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int K, int N, int64_t ldx, int64_t ldz,
                     hipStream_t stream, bool may_prepare);      // dense.hip
@@ -904,16 +904,8 @@ int accel_partition_gpu(const int32_t *indptr, int64_t rows, int32_t *block4_out
         set_error("device allocation failed");
         return ACCEL_ERR_ALLOC;
     }
-    int32_t *b4 = nullptr;
-    int64_t nb = 0;
     int rc = upload(dptr, indptr, bytes, nullptr);
-    if (!rc) rc = partition_only_device(static_cast<int32_t *>(dptr), rows, indptr[rows], &b4, &nb);
-    if (!rc) {
-        *n_blocks = nb;
-        const int64_t take = std::min(nb, cap);
-        if (take > 0) rc = download(block4_out, b4, sizeof(int32_t) * 4 * (size_t)take, nullptr);
-    }
-    give_memory(b4, InUse::null_stream);
+    if (!rc) rc = partition_to_host(static_cast<int32_t *>(dptr), rows, indptr[rows], block4_out, cap, n_blocks);
     give_memory(dptr, InUse::null_stream);
     return rc;
 }

@@ -197,6 +197,10 @@ void give_stream_memory(void *p, hipStream_t s);
 // been read, download when dst has been written
 int upload(void *dst, const void *src, size_t bytes, hipStream_t s);
 int download(void *dst, const void *src, size_t bytes, hipStream_t s);
+// The same for results that kernels write straight over the link: make(context, pinned memory, offset, bytes, s) queues what
+// writes bytes [offset, offset + bytes) there, a piece of 2 MiB at a time.
+using MakePiece = int (*)(const void *context, void *stage, size_t offset, size_t bytes, hipStream_t s);
+int download_made(void *dst, size_t bytes, hipStream_t s, MakePiece make, const void *context);
 // preprocess.hip
 struct SavedOrder {               // a degree-sort order read from a saved state
     bool identity;                // the rows were already in order: no permutation stored

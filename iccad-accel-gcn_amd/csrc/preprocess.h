@@ -20,6 +20,8 @@ constexpr int kLongBin = kDegBound + 1;
 constexpr int kWideRow = 1024;
 constexpr int kWideChunk = 4096;
 
+constexpr int kRunParts = 1024;
+
 // A small block of pinned host memory that kernels write their results for the host into: the
 // host reads it after a synchronisation, with no copy queued in between.
 struct Mail {
@@ -33,6 +35,8 @@ struct Mail {
     int n_pieces;             // pieces of split rows
     int n_units;              // units of whole rows
     int n_blocks;             // entries of the partition (only for rows in any order)
+    // the partition of rows in order: hist holds the first row of each bin then, or -1
+    int part[kRunParts];      // entries of rows longer than 384, summed up per workgroup of run_bounds_kernel
 };
 enum {
     kStatBadIndptr, kStatUnsorted, kStatMaxDegree,        // these three: the largest value over all rows

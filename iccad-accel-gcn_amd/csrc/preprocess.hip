@@ -208,13 +208,13 @@ struct PlaceArgs {
     UnitRule rule;
     // outputs
     int32_t *perm;                            // null: the rows are in order already
-    uint32_t *place;                          // caller's row -> sorted row (null: not wanted); long rows come later
-    int32_t *s_indptr;                        // null: not wanted
+    uint32_t *place;                          // caller's row -> sorted row; long rows come later
+    int32_t *s_indptr;
     int4 *block4;
-    int *run_row, *run_nz;                    // [kBins + 1], [kBins] (null: not wanted)
+    int *run_row, *run_nz;                    // [kBins + 1], [kBins]
     int *long_deg;                            // degrees and ids of the long rows, in the caller's order
     uint32_t *long_row;
-    int *sums;                                // [kSums][pitch + kWaves4] (null: not wanted)
+    int *sums;                                // [kSums][pitch + kWaves4]
     int *zero;                                // n_zero ints to clear
     int64_t n_zero;
 };
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
         }
         __syncthreads();
     }
-    if (blockIdx.x == 0 && a.run_row) {
+    if (blockIdx.x == 0) {
         for (int i = tid; i <= kBins; i += kThreads) a.run_row[i] = run_row[i];
         for (int i = tid; i < kBins; i += kThreads) a.run_nz[i] = run_nz[i];
     }
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
             if (run_row[mid] <= p) lo = mid; else hi = mid - 1;
         }
         const int d = lo, i = (int)p - run_row[d], loc = run_nz[d] + i * d;
-        if (a.s_indptr) a.s_indptr[p] = loc;
+        a.s_indptr[p] = loc;
         if (d > 0) {
             int wn, rpb;
             slice_rule(d, wn, rpb);
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
                     make_int4(d, (int)p, loc, (wn << 16) + min(rpb, run_row[d + 1] - run_row[d] - i));
         }
     }
-    if (a.s_indptr && me == 0) a.s_indptr[a.rows] = a.indptr[a.rows];
+    if (me == 0) a.s_indptr[a.rows] = a.indptr[a.rows];
 
     // the rows of this wavefront's share
     if (c >= a.n_shares) return;
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
                     a.long_row[p - n_binned] = (uint32_t)r;
                 } else {
                     if (a.perm) a.perm[p] = (int32_t)r;
-                    if (a.place) a.place[r] = (uint32_t)p;
+                    a.place[r] = (uint32_t)p;
                 }
                 if (d > 0 && d <= a.rule.split) {
                     const int n = unit_rows(d, p - run_row[d], run_row[d + 1] - run_row[d], a.rule);
@@ -346,7 +346,6 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
             }
         }
     }
-    if (!a.sums) return;
     n_units = wave_sum(n_units);
     cost = wave_sum(cost);
     n_heavy = wave_sum(n_heavy);
@@ -385,7 +384,7 @@ __device__ __forceinline__ int count_before(const int4 *tile, int n4, int at0, i
     return below;
 }
 
-// The first kSums workgroups scan one kind each of the counts per share (sums, null: none), which has
+// The first kSums workgroups scan one kind each of the counts per share (sums), which has
 // nothing to do with the rest but that both come behind place_rows; the others rank the long rows.
 __global__ __launch_bounds__(1024) void rank_long_rows_kernel(
     const int *__restrict__ deg, const uint32_t *__restrict__ row, int n, int64_t first_long,
@@ -395,10 +394,8 @@ __global__ __launch_bounds__(1024) void rank_long_rows_kernel(
     __shared__ __attribute__((aligned(16))) int tile[4096];
     __shared__ int part[16][kRankRows];
     int b = blockIdx.x;
-    if (sums) {
-        if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, tile); return; }
-        b -= kSums;
-    }
+    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, tile); return; }
+    b -= kSums;
     const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
     const int d = j < n ? deg[j] : 0;
     const uint32_t r = j < n ? row[j] : 0;
@@ -416,7 +413,7 @@ __global__ __launch_bounds__(1024) void rank_long_rows_kernel(
         for (int q = 1; q < 16; q++) below += part[q][lane];
         const int64_t p = first_long + below;
         if (perm) perm[p] = (int32_t)r;
-        if (place) place[r] = (uint32_t)p;
+        place[r] = (uint32_t)p;
         sorted_deg[below] = d;
     }
 }
@@ -432,7 +429,7 @@ struct LongArgs {
     int nz0, block0;                          // non-zeros and blocks before them
     int32_t *perm;                            // null: in order already
     uint32_t *place;
-    int32_t *s_indptr;                        // null: not wanted
+    int32_t *s_indptr;
     int4 *block4;
     int *first_chunk, *chunk_row;             // of long row i (null: none is wide)
 };
@@ -445,10 +442,8 @@ __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__res
     __shared__ int part[16][4][kRankRows];
     __shared__ int4 mine[kRankRows];                     // rank, first non-zero, first block, first chunk
     int b = blockIdx.x;
-    if (sums) {
-        if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, deg); return; }
-        b -= kSums;
-    }
+    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, deg); return; }
+    b -= kSums;
     const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
     const uint32_t r = j < a.n ? a.row[j] : 0;
     const int per = (a.n + 15) / 16;                     // of a wavefront
@@ -481,8 +476,8 @@ __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__res
         }
         const int64_t p = a.first_long + below;
         if (a.perm) a.perm[p] = (int32_t)r;
-        if (a.place) a.place[r] = (uint32_t)p;
-        if (a.s_indptr) a.s_indptr[p] = a.nz0 + nz;
+        a.place[r] = (uint32_t)p;
+        a.s_indptr[p] = a.nz0 + nz;
         if (a.first_chunk) {
             a.first_chunk[below] = chk;
             if (below == a.n - 1) a.first_chunk[a.n] = chk + chunks_of(d);
@@ -573,7 +568,7 @@ __global__ __launch_bounds__(kThreads) void apply_long_order_kernel(
     if (i >= n) return;
     const uint32_t r = row[order[i]];
     if (perm) perm[first_long + i] = (int32_t)r;
-    if (place) place[r] = (uint32_t)(first_long + i);
+    place[r] = (uint32_t)(first_long + i);
     sorted_deg[i] = (int)sorted_key[i];
 }
 
@@ -655,24 +650,21 @@ __global__ __launch_bounds__(kThreads) void long_blocks_kernel(LongArgs a, const
 // Ints that must be zero for place_long_rows (place_rows clears them).
 int64_t long_zeroed_ints(int64_t n) { return n > kFewLong ? 3 * scan_zeroed(n) : 0; }
 
-// The long rows' places, row pointers, blocks and chunks, and the scan of the counts per share of rows (sums, null: none).
-// in_order: the rows are sorted already, so they are listed in sorted order.
-int place_long_rows(Arena *tmp, const LongArgs &a, bool in_order, int max_degree, const int32_t *loc_of, int *zeroed,
+// The long rows' places, row pointers, blocks and chunks, and the scan of the counts per share of rows (sums).
+int place_long_rows(Arena *tmp, const LongArgs &a, int max_degree, const int32_t *loc_of, int *zeroed,
                     int *sums, int pitch, int n_shares, hipStream_t s)
 {
-    int rc, *sorted_deg = const_cast<int *>(a.deg), *blocks, *chunks = nullptr;
-    const unsigned scans = sums ? kSums : 0;
+    int rc, *sorted_deg, *blocks, *chunks = nullptr;
     if (a.n <= kFewLong) {
-        const unsigned groups = scans + (unsigned)((a.n + kRankRows - 1) / kRankRows);
-        if (groups > 0) place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
+        const unsigned groups = kSums + (unsigned)((a.n + kRankRows - 1) / kRankRows);
+        place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
         return ACCEL_OK;
     }
-    const int ranked = !in_order && a.n <= kRankMax ? a.n : 0;
-    if (!in_order && (rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
-    if (sums || ranked > 0)
-        rank_long_rows_kernel<<<dim3(scans + (unsigned)((ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0, s>>>(
-            a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, pitch, n_shares);
-    if (!in_order && a.n > kRankMax &&
+    const int ranked = a.n <= kRankMax ? a.n : 0;
+    if ((rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
+    rank_long_rows_kernel<<<dim3(kSums + (unsigned)((ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0, s>>>(
+        a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, pitch, n_shares);
+    if (a.n > kRankMax &&
         (rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
         return rc;
     if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
@@ -685,7 +677,7 @@ int place_long_rows(Arena *tmp, const LongArgs &a, bool in_order, int max_degree
         n_jobs++;
     };
     add(blocks, blocks, a.block0);
-    if (a.s_indptr) add(sorted_deg, a.s_indptr + a.first_long, a.nz0);
+    add(sorted_deg, a.s_indptr + a.first_long, a.nz0);
     if (chunks) add(chunks, a.first_chunk, 0);
     launch_scans(jobs, n_jobs, s);
     long_blocks_kernel<<<dim3(grid_for((int64_t)a.n * 64)), dim3(kThreads), 0, s>>>(a, sorted_deg, loc_of, blocks);
@@ -1298,6 +1290,113 @@ __global__ __launch_bounds__(1) void report_blocks_kernel(const int *__restrict_
 }
 
 // Rows in any order: block4 from scans over the rows.  *block4_out is the caller's to give back.
+// Rows in ascending degree order: the first row of every degree up to 384 and of the longer ones, into mail->hist (-1
+// where there is none), the entries of the longer ones per workgroup, and whether anything is wrong or out of order.  Four
+// rows per thread.
+__global__ __launch_bounds__(kThreads) void run_bounds_kernel(const int32_t *__restrict__ indptr, int64_t rows, int64_t nnz,
+                                                              Mail *__restrict__ mail)
+{
+    __shared__ int sum[kWaves4];
+    const int lane = threadIdx.x & 63;
+    int long_blocks = 0;
+    bool bad = false, unsorted = false;
+    for (int64_t r0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x - lane) * 4; r0 < rows; r0 += (int64_t)gridDim.x * kThreads * 4) {
+        const int64_t r = r0 + lane * 4;                     // of this lane; the wavefront stays together
+        int at[6];                                           // indptr[r - 1 .. r + 4], as far as there are
+        if (r + 3 <= rows) {
+            const int4 v = *reinterpret_cast<const int4 *>(indptr + r);
+            at[1] = v.x; at[2] = v.y; at[3] = v.z; at[4] = v.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) at[1 + j] = r + j <= rows ? indptr[r + j] : 0;
+        }
+        at[0] = __shfl_up(at[4], 1);
+        at[5] = __shfl_down(at[1], 1);
+        if (lane == 0 && r > 0) at[0] = indptr[r - 1];
+        if (lane == 63 && r + 4 <= rows) at[5] = indptr[r + 4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (r + j >= rows) break;
+            const int d = at[j + 2] - at[j + 1], before = r + j > 0 ? at[j + 1] - at[j] : -1;
+            bad |= d < 0 || (r + j == 0 && at[j + 1] != 0) || (r + j == rows - 1 && (int64_t)at[j + 2] != nnz);
+            unsorted |= d < before;
+            const int bin = min(max(d, 0), kLongBin);
+            if (before < 0 || bin != min(before, kLongBin)) mail->hist[bin] = (int)(r + j);
+            if (d > kDegBound) long_blocks += blocks_of(d);
+        }
+    }
+    if (bad) mail->stat[kStatBadIndptr] = 1;
+    if (unsorted) mail->stat[kStatUnsorted] = 1;
+    long_blocks = wave_sum(long_blocks);
+    if (lane == 0) sum[threadIdx.x >> 6] = long_blocks;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kWaves4; q++) long_blocks += sum[q];
+        if (long_blocks > 0) mail->part[blockIdx.x] = long_blocks;
+    }
+}
+
+// Entries of each of the n rows from `indptr` on, and zeroed words for the scan.
+__global__ __launch_bounds__(kThreads) void run_sizes_kernel(const int32_t *__restrict__ indptr, int n, int *__restrict__ blocks,
+                                                             int *__restrict__ zeroed, int n_zeroed)
+{
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < n_zeroed) zeroed[i] = 0;                         // (fewer than the rows, but for the first few)
+    if (i < n) blocks[i] = blocks_of(indptr[i + 1] - indptr[i]);
+}
+
+struct EmitRunsArgs {
+    int run_row[kBins + 1], run_blk[kBins];   // first row and first entry of each degree
+    const int32_t *indptr;
+    const int *first_block;                   // of the rows longer than 384, scanned (null: none is wanted)
+    int4 *out;
+    int64_t b0;                               // entries b0 .. b0 + n - 1 go to out[0 .. n - 1]
+    int n;
+};
+static_assert(sizeof(EmitRunsArgs) <= 4096, "kernel arguments");
+__global__ __launch_bounds__(kThreads) void emit_runs_kernel(EmitRunsArgs a)
+{
+    __shared__ int run_row[kBins + 1], run_blk[kBins];
+    for (int i = threadIdx.x; i <= kBins; i += kThreads) run_row[i] = a.run_row[i];
+    for (int i = threadIdx.x; i < kBins; i += kThreads) run_blk[i] = a.run_blk[i];
+    __syncthreads();
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= a.n) return;
+    const int b = (int)(a.b0 + i);
+    int4 e;
+    if (b < run_blk[kLongBin]) {
+        int lo = 1, hi = kDegBound;                          // the last degree whose entries start at or before b
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (run_blk[mid] <= b) lo = mid; else hi = mid - 1;
+        }
+        int w, rpb;
+        slice_rule(lo, w, rpb);
+        const int p = run_row[lo] + (b - run_blk[lo]) * rpb;
+        e = make_int4(lo, p, a.indptr[p], (w << 16) + min(rpb, run_row[lo + 1] - p));
+    } else {
+        int lo = 0, hi = run_row[kBins] - run_row[kLongBin] - 1;     // the last row whose entries start at or before b
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (a.first_block[mid] <= b) lo = mid; else hi = mid - 1;
+        }
+        const int p = run_row[kLongBin] + lo, from = a.indptr[p], d = a.indptr[p + 1] - from, off = (b - a.first_block[lo]) * kDegBound;
+        e = make_int4(d, p, from + off, min(kDegBound, d - off));
+    }
+    a.out[i] = e;
+}
+
+static int emit_runs_piece(const void *args, void *stage, size_t offset, size_t bytes, hipStream_t s)
+{
+    EmitRunsArgs a = *static_cast<const EmitRunsArgs *>(args);
+    a.out = static_cast<int4 *>(stage);
+    a.b0 = (int64_t)(offset / sizeof(int4));
+    a.n = (int)(bytes / sizeof(int4));
+    emit_runs_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(a);
+    ACCEL_HIP(hipGetLastError());
+    return ACCEL_OK;
+}
+
 int partition_any_order(Arena *tmp, const int32_t *indptr, int64_t rows, int32_t **block4_out, int64_t *n_blocks,
                         Mail *mail, hipStream_t s)
 {
@@ -1370,57 +1469,74 @@ static RunTotals run_totals(const int *hist, int most, int unit_nz)
 }
 
 // Partition a row order as given (no sort): the GPU counterpart of running
-// block_level_partition.py on one *.new_indptr file.
-int partition_only_device(const int32_t *indptr_dev, int64_t rows, int64_t nnz,
-                          int32_t **block4_dev, int64_t *n_blocks)
+// block_level_partition.py on one *.new_indptr file.  At most `cap` entries go to block4_out.
+//
+// Rows in ascending degree order, which is what those files hold: one pass finds where each degree's run starts, and an
+// entry is a closed form of its number (of the rows longer than 384, after a scan).  The entries are written straight into the
+// pinned memory they leave the device through.  2.45 M rows: the passes of the sort took 96 us and copies from device memory
+// 190; so 16 and 165, bound by the link (the whole call 645 -> 566 us).
+int partition_to_host(const int32_t *indptr_dev, int64_t rows, int64_t nnz, int32_t *block4_out, int64_t cap,
+                      int64_t *n_blocks)
 {
     hipStream_t s = nullptr;
     MailHolder mh;
     if (!mh.m) return ACCEL_ERR_ALLOC;
     Mail *mail = mh.m;
     Arena tmp;
-    const Shares sh(rows);
-    int *bins, *bin_total, rc;
-    tmp.next_chunk = (size_t)kBins * sh.pitch * 4 + (size_t)sh.groups() * 64 + (1 << 16);
-    if ((rc = count_rows(&tmp, indptr_dev, nullptr, rows, 0, nnz, kDegBound, kDegBound, sh, &bins, &bin_total, mail, s)))
-        return rc;
+    int rc;
+    for (int &first : mail->hist) first = -1;
+    for (int &v : mail->stat) v = 0;
+    for (int &v : mail->part) v = 0;
+    const int64_t tiles = (rows + 4 * kThreads - 1) / (4 * kThreads);
+    run_bounds_kernel<<<dim3((unsigned)std::min<int64_t>(tiles, kRunParts)), dim3(kThreads), 0, s>>>(indptr_dev, rows, nnz, mail);
+    ACCEL_HIP(hipGetLastError());
+    ACCEL_HIP(hipStreamSynchronize(s));
+    if (mail->stat[kStatBadIndptr]) {
+        set_error("indptr must start at 0, be non-decreasing and end at nnz");
+        return ACCEL_ERR_CSR;
+    }
     if (mail->stat[kStatUnsorted]) {
         tmp.next_chunk = (size_t)rows * 13 + (1 << 16);
-        rc = partition_any_order(&tmp, indptr_dev, rows, block4_dev, n_blocks, mail, s);
+        int32_t *b4 = nullptr;
+        rc = partition_any_order(&tmp, indptr_dev, rows, &b4, n_blocks, mail, s);
         mh.written = rc == ACCEL_OK;
+        const int64_t take = std::min(*n_blocks, cap);
+        if (!rc && take > 0) rc = download(block4_out, b4, sizeof(int4) * (size_t)take, s);
+        give_memory(b4, InUse::null_stream);
         return rc;
     }
-    mh.written = true;                        // by the counting pass alone
-    const RunTotals rt = run_totals(mail->hist, kDegBound, kDegBound);
-    const int n_long = mail->hist[kLongBin];
-    const int64_t n_zeroed = long_zeroed_ints(n_long);
-    tmp.next_chunk = (size_t)n_long * 12 + (size_t)n_zeroed * 4 + (1 << 12);
-    int *long_deg, *zeroed;
-    uint32_t *long_row;
-    if ((rc = tmp.alloc(&long_deg, (size_t)n_long))) return rc;
-    if ((rc = tmp.alloc(&long_row, (size_t)n_long))) return rc;
-    if ((rc = tmp.alloc(&zeroed, (size_t)n_zeroed))) return rc;
-    *n_blocks = rt.blocks + mail->stat[kStatLongBlocks];
-    DevBuf b4;
-    if ((rc = b4.alloc(sizeof(int4) * (size_t)*n_blocks))) return rc;
-    PlaceArgs pa{};
-    pa.indptr = indptr_dev; pa.rows = rows; pa.share = sh.share; pa.n_shares = sh.n; pa.pitch = sh.pitch;
-    pa.bins = bins; pa.bin_total = bin_total;
-    pa.rule = UnitRule{kDegBound, kDegBound, 0, 2, 0};
-    pa.block4 = b4.as<int4>();
-    pa.long_deg = long_deg; pa.long_row = long_row;
-    pa.zero = zeroed; pa.n_zero = n_zeroed;
-    place_rows_kernel<<<dim3(sh.groups()), dim3(kThreads), 0, s>>>(pa);
-    if (n_long > 0) {
-        LongArgs la{};
-        la.deg = long_deg; la.row = long_row; la.n = n_long; la.first_long = rows - n_long;
-        la.nz0 = (int)rt.nnz; la.block0 = (int)rt.blocks;
-        la.block4 = b4.as<int4>();
-        if ((rc = place_long_rows(&tmp, la, true, 0, indptr_dev, zeroed, nullptr, 0, 0, s))) return rc;
+    mh.written = true;
+    EmitRunsArgs ea{};
+    ea.indptr = indptr_dev;
+    ea.run_row[kBins] = (int)rows;
+    int64_t n_short = 0;
+    for (int d = kLongBin; d >= 0; d--) ea.run_row[d] = mail->hist[d] >= 0 ? mail->hist[d] : ea.run_row[d + 1];
+    for (int d = 0; d < kLongBin; d++) {
+        ea.run_blk[d] = (int)n_short;
+        if (d == 0) continue;
+        int w, rpb;
+        slice_rule(d, w, rpb);
+        n_short += (ea.run_row[d + 1] - ea.run_row[d] + rpb - 1) / rpb;
     }
-    ACCEL_HIP(hipGetLastError());
-    *block4_dev = static_cast<int32_t *>(b4.release());
-    return ACCEL_OK;
+    ea.run_blk[kLongBin] = (int)n_short;
+    int64_t nb = n_short;
+    for (const int v : mail->part) nb += v;
+    const int n_long = (int)rows - ea.run_row[kLongBin];
+    *n_blocks = nb;
+    const int64_t take = std::min(nb, cap);
+    if (n_long > 0 && take > n_short) {
+        int *first_block, *zeroed;
+        const int64_t n_zeroed = scan_zeroed(n_long);
+        tmp.next_chunk = (size_t)n_long * 4 + (size_t)n_zeroed * 4 + (1 << 12);
+        if ((rc = tmp.alloc(&first_block, (size_t)n_long + 1))) return rc;
+        if ((rc = tmp.alloc(&zeroed, (size_t)n_zeroed))) return rc;
+        run_sizes_kernel<<<dim3(grid_for(n_long)), dim3(kThreads), 0, s>>>(indptr_dev + ea.run_row[kLongBin], n_long, first_block,
+                                                                           zeroed, (int)n_zeroed);
+        launch_scans({{{first_block, first_block, n_long, (int)n_short, zeroed}}, {}}, 1, s);
+        ea.first_block = first_block;
+    }
+    if (take == 0) return ACCEL_OK;
+    return download_made(block4_out, sizeof(int4) * (size_t)take, s, emit_runs_piece, &ea);
 }
 
 // Small matrices are latency-bound: the time of a launch is the longest chain of
@@ -1754,7 +1870,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     ua.rule = rule; ua.pu = pu;
     ua.share = sh.share; ua.n_shares = sh.n; ua.pitch = sh.pitch + kWaves4; ua.first_split = (int)(rows - n_split);
     ua.groups = (int)sh.groups();
-    if ((rc = place_long_rows(&tmp, la, false, h->max_degree, h->s_indptr, zeroed + plan_zeroed, pu.sums, ua.pitch, sh.n, s)))
+    if ((rc = place_long_rows(&tmp, la, h->max_degree, h->s_indptr, zeroed + plan_zeroed, pu.sums, ua.pitch, sh.n, s)))
         return rc;
     if (given && !h->identity_perm)
         compare_order_kernel<<<dim3(grid_for(rows)), dim3(kThreads), 0, s>>>(

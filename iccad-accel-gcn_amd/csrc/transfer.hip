@@ -17,8 +17,8 @@
 
 namespace accel {
 
-// Both queue on s and return when the host's side is done: upload when src has been read (the copy
-// to dst is ordered on s), download when dst has been written.
+// All queue on s and return when the host's side is done: upload when src has been read (the copy
+// to dst is ordered on s), download and download_made when dst has been written.
 int upload(void *dst, const void *src, size_t bytes, hipStream_t s)
 {
     StageHolder st(bytes);
@@ -39,7 +39,18 @@ int upload(void *dst, const void *src, size_t bytes, hipStream_t s)
     return ACCEL_OK;
 }
 
+static int copy_piece(const void *src, void *stage, size_t offset, size_t bytes, hipStream_t s)
+{
+    ACCEL_HIP(hipMemcpyAsync(stage, static_cast<const char *>(src) + offset, bytes, hipMemcpyDeviceToHost, s));
+    return ACCEL_OK;
+}
+
 int download(void *dst, const void *src, size_t bytes, hipStream_t s)
+{
+    return download_made(dst, bytes, s, copy_piece, src);
+}
+
+int download_made(void *dst, size_t bytes, hipStream_t s, MakePiece make, const void *context)
 {
     StageHolder st(bytes);
     if (!st.s) return ACCEL_ERR_ALLOC;
@@ -50,8 +61,7 @@ int download(void *dst, const void *src, size_t bytes, hipStream_t s)
         char *to = static_cast<char *>(dst) + done, *stage = static_cast<char *>(st.s->p);
         for (int i = 0; i < n; i++) {
             const size_t off = (size_t)i * kStagePiece;
-            ACCEL_HIP(hipMemcpyAsync(stage + off, static_cast<const char *>(src) + done + off,
-                                     std::min(kStagePiece, here - off), hipMemcpyDeviceToHost, s));
+            if (int rc = make(context, stage + off, done + off, std::min(kStagePiece, here - off), s)) return rc;
             ACCEL_HIP(hipEventRecord(st.s->event[i], s));
         }
         std::atomic<int> next{0}, arrived{0};
