@@ -113,12 +113,12 @@ __device__ __forceinline__ float w_at(const float *__restrict__ W, int K, int N,
 struct DenseStepAt {
     int64_t row_block;
     int tile, k0;
-    __device__ void advance(int K, int n_col_tiles, int64_t stride)
+    __device__ void advance(int K, int last_tile, int64_t stride)
     {
         k0 += kDenseStep;
         if (k0 >= K) {
             k0 = 0;
-            if (++tile == n_col_tiles) { tile = 0; row_block += stride; }
+            if (tile == last_tile) { tile = 0; row_block += stride; } else { tile++; }
         }
     }
 };
@@ -128,9 +128,17 @@ struct DenseArgs {
     float *Z;
     int64_t rows, ldx, ldz, n_row_blocks;
     int K, N, n_col_tiles, n_steps;
+    int apart;                   // the column tiles of a block of rows are workgroups of their own
     const u32x4 *image;          // walk_fp16: W taken apart (dense_prepare_kernel), and what is in front of that
     const int *head;
 };
+
+// Where a workgroup starts.
+__device__ __forceinline__ DenseStepAt first_step(const DenseArgs &a)
+{
+    const int64_t b = blockIdx.x;
+    return a.apart ? DenseStepAt{b % a.n_row_blocks, (int)(b / a.n_row_blocks), 0} : DenseStepAt{b, 0, 0};
+}
 
 // A workgroup's block of W of a step on its way through registers, taken apart, into LDS.
 template <int NT> struct WStage {
@@ -269,11 +277,13 @@ __device__ __forceinline__ void walk_bf16(const DenseArgs &a, char (*w_lds)[kPar
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
 
-    const int64_t stride = gridDim.x;          // gridDim.x <= n_row_blocks: every workgroup has work
+    // gridDim.x is at most the number of blocks of rows (or of their tiles): every workgroup has work
+    const int64_t stride = a.apart ? a.n_row_blocks : gridDim.x;
+    const int last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
     DenseStepAt next = now, after;
-    next.advance(a.K, a.n_col_tiles, stride);
+    next.advance(a.K, last_tile, stride);
     after = next;
-    after.advance(a.K, a.n_col_tiles, stride);
+    after.advance(a.K, last_tile, stride);
     v4f x0[4], x1[4];
     WStage<NT> w;
     bf16x8 apart[2][kParts];                   // this step's values of X, taken apart
@@ -386,7 +396,7 @@ __device__ __forceinline__ void walk_bf16(const DenseArgs &a, char (*w_lds)[kPar
         }
         now = next;
         next = after;
-        after.advance(a.K, a.n_col_tiles, stride);
+        after.advance(a.K, last_tile, stride);
         step++;
     };
     while (now.row_block < a.n_row_blocks) {
@@ -400,7 +410,7 @@ template <int NT>
 __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kernel(DenseArgs a)
 {
     __shared__ __attribute__((aligned(16))) char w_lds[2][kParts * NT * 32 * kWStride];
-    walk_bf16<NT>(a, w_lds, DenseStepAt{(int64_t)blockIdx.x, 0, 0});
+    walk_bf16<NT>(a, w_lds, first_step(a));
 }
 
 // ---- two fp16 values per fp32 value -----------------------------------------------------------------------------
@@ -604,7 +614,8 @@ __device__ __forceinline__ void add_lost(const DenseArgs &a, int64_t row0, int c
 // written only between barriers where nobody reads it: bad behind a tile's last step and read at its first (K is more than
 // one step), early in a tile's second step of four and read in the fourth.
 template <int NT>
-__device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_lds)[kParts16 * NT * 32 * 64], int *bad, int *early)
+__device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_lds)[kParts16 * NT * 32 * 64], DenseStepAt now,
+                                                 int *bad, int *early)
 {
     constexpr int kCols = NT * 32, kVecs = kCols * kParts16 * 4, kMine = kVecs / kDenseThreads;
     static_assert(kVecs % kDenseThreads == 0, "whole rounds of W");
@@ -651,11 +662,12 @@ __device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_ld
 #pragma unroll
         for (int t = 0; t < kTiles; t++) high[r][t] = low[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int64_t stride = gridDim.x;          // gridDim.x <= n_row_blocks: every workgroup has work
-    DenseStepAt now{(int64_t)blockIdx.x, 0, 0}, next = now, after;
-    next.advance(a.K, a.n_col_tiles, stride);
+    const int64_t stride = a.apart ? a.n_row_blocks : gridDim.x;       // (as in the other walk)
+    const int last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
+    DenseStepAt next = now, after;
+    next.advance(a.K, last_tile, stride);
     after = next;
-    after.advance(a.K, a.n_col_tiles, stride);
+    after.advance(a.K, last_tile, stride);
     v4f x0[4], x1[4];
     f16x8 apart[2][kParts16];                  // this step's values of X, taken apart
     int scale = 0, scale_next = 0;             // X is multiplied by 2^scale: in this step's tile, in the next step's
@@ -820,7 +832,7 @@ __device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_ld
         scale = scale_next;
         now = next;
         next = after;
-        after.advance(a.K, a.n_col_tiles, stride);
+        after.advance(a.K, last_tile, stride);
         step++;
     };
     // At a barrier: this step's block of W is in place, the other one's readers are done, and what was counted is there.
@@ -851,10 +863,10 @@ __global__ __launch_bounds__(kDenseThreads, 2) void dense_xw_fp16_kernel(DenseAr
 {
     __shared__ __attribute__((aligned(16))) char w_lds[2 * kParts * NT * 32 * kWStride];
     __shared__ int bad, early;
-    DenseStepAt at{(int64_t)blockIdx.x, 0, 0};
+    DenseStepAt at = first_step(a);
     if (!a.head[0]) {
         if (threadIdx.x == 0) bad = early = 0;
-        at = walk_fp16<NT>(a, reinterpret_cast<char (*)[kParts16 * NT * 32 * 64]>(w_lds), &bad, &early);
+        at = walk_fp16<NT>(a, reinterpret_cast<char (*)[kParts16 * NT * 32 * 64]>(w_lds), at, &bad, &early);
     }
     if (at.row_block < a.n_row_blocks)
         walk_bf16<NT>(a, reinterpret_cast<char (*)[kParts * NT * 32 * kWStride]>(w_lds), at);
@@ -995,7 +1007,8 @@ static int dense_launch(void (*kernel)(DenseArgs), int which, const DenseArgs &a
         resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);
         if (dev >= 0 && dev < kDenseDevices) g_resident[dev][which].store(resident, std::memory_order_relaxed);
     }
-    const unsigned grid = (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
+    const unsigned grid = a.apart ? (unsigned)(a.n_row_blocks * a.n_col_tiles)
+                                  : (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
     kernel<<<grid, kDenseThreads, 0, s>>>(a);
     return ACCEL_OK;
 }
@@ -1037,6 +1050,11 @@ static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
     return dense_launch(dense_xw_kernel<NT>, which + 3, a, s);
 }
 
+// Few rows: a workgroup takes one column tile, and a narrower one, as long as there is a compute unit for each (with
+// one tile each, two).  A step takes a microsecond whatever its width.  Rows x K x N, 128 columns and all tiles to a workgroup
+// and so: 2,000 x 250 x 256 31.0 -> 9.4 us, 10,000 x 602 x 128 32.7 -> 21.3, 10,000 x 602 x 256 48.4 -> 29.9, 20,000 x
+// 602 x 256 48.7 -> 39.3.  Beyond the line: 20,000 x 602 x 64 in halves (314 workgroups) 21.4 -> 25.6.
+constexpr int64_t kFewGroups = 256;
 // Arguments have been checked by the caller (accel_dense_xw): rows >= 1, K, N >= 1,
 // ldx >= K, ldz >= N, operands readable and large enough.  may_prepare: s is not capturing (a graph's
 // memory would have to live as long as the graph).
@@ -1044,14 +1062,19 @@ int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int 
                     hipStream_t s, bool may_prepare)
 {
     (void)hipGetLastError();
-    const int nt = N <= 32 ? 1 : N <= 64 ? 2 : 4;
+    int nt = N <= 32 ? 1 : N <= 64 ? 2 : 4;
     DenseArgs a{};
     a.X = X; a.W = W; a.Z = Z;
     a.rows = rows; a.ldx = ldx; a.ldz = ldz;
     a.n_row_blocks = (rows + kDenseBlockRows - 1) / kDenseBlockRows;
     a.K = K; a.N = N;
-    a.n_col_tiles = (N + nt * 32 - 1) / (nt * 32);
     a.n_steps = (K + kDenseStep - 1) / kDenseStep;
+    auto groups = [&](int of) { return a.n_row_blocks * ((N + of * 32 - 1) / (of * 32)); };
+    if (K >= kDenseHalf) {
+        while (nt > 1 && groups(nt / 2) <= kFewGroups) nt /= 2;
+        a.apart = groups(nt) > a.n_row_blocks && groups(nt) <= 2 * kFewGroups;
+    }
+    a.n_col_tiles = (N + nt * 32 - 1) / (nt * 32);
     const int rc = nt == 1   ? dense_product<1>(a, s, may_prepare)
                    : nt == 2 ? dense_product<2>(a, s, may_prepare)
                              : dense_product<4>(a, s, may_prepare);
