@@ -136,6 +136,7 @@ struct accel_handle {
     int64_t nnz_short = 0;            // non-zeros of the rows that are not split
     int64_t n_wide_rows = 0;          // rows with more than 1,024 non-zeros, regrouped in chunks
     int64_t n_chunks = 0;             // ... of 4,096 non-zeros
+    int64_t n_lone_chunks = 0;        // of those, the first ones, that are all there is of their row
     int *runs = nullptr;              // first sorted row and first non-zero of each degree's run (SortedRows)
     int *first_chunk = nullptr, *chunk_row = nullptr;     // first chunk of each long row, long row of each chunk
     int64_t n_blocks = 0, n_long_blocks = 0, n_long_rows = 0, n_zero_rows = 0;

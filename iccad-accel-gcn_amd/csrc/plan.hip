@@ -56,9 +56,6 @@ static ClassLayout class_layout(int64_t n_split, const Mail *stats, int groups)
     return c;
 }
 
-// Zeroed memory: the queue loads, then the two scans' part.
-constexpr int kZeroQueueLoad = 8;
-
 __device__ __forceinline__ int64_t plan_index(int queue, int pos, int n_queues)
 {
     // queue q, position p  ->  slot of wavefront (p % 4) in workgroup (p / 4) * n_queues + q
@@ -85,14 +82,18 @@ __device__ __forceinline__ int queue_of(int running_cost, const int *cut)
 // Queue q takes max(0, level - its pieces' cost) of the whole-row units' cost, level being the
 // smallest common level that takes all of it.
 __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ bins, ClassLayout cl, int n_split,
-                                                        const int *__restrict__ queue_cost,
+                                                        const int *__restrict__ group_cost, int n_groups,
                                                         const int *__restrict__ running, const int *__restrict__ sums,
                                                         int pitch, int n_shares, int n_queues,
                                                         PlanHead *__restrict__ head, Mail *__restrict__ mail)
 {
     static_assert(kXcds * 64 == 512, "one wavefront per queue");
     __shared__ int at[kPlanBins + 1], off[kPlanBins], queue_long[kXcds], cut[kXcds + 1], first[kXcds + 1];
+    __shared__ int part[kXcds][kXcds];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    int cost = 0;                                                  // of the split rows' pieces for die t % 8
+#pragma unroll 4
+    for (int i = t; i < n_groups * kXcds; i += 512) cost += group_cost[i];
     const int n = sums[kSumUnits * pitch + n_shares];
     if (t <= kPlanBins) {
         int v = 0;
@@ -107,6 +108,10 @@ __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ 
         }
         at[t] = v;
     }
+    cost += __shfl_xor(cost, 8);
+    cost += __shfl_xor(cost, 16);
+    cost += __shfl_xor(cost, 32);
+    if (lane < kXcds) part[w][lane] = cost;
     __syncthreads();
     if (t < n_queues) {
         // a die first takes the pieces of the rows with the most groups (the longest rows), one
@@ -123,10 +128,18 @@ __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ 
     if (w == 1) {
         // the smallest level that takes all of it, 64 candidates at a time
         const long long short_cost = sums[kSumCost * pitch + n_shares];
+        int queue_cost[kXcds] = {};
+#pragma unroll
+        for (int q = 0; q < kXcds; q++) {
+            int c = 0;
+#pragma unroll
+            for (int v = 0; v < kXcds; v++) c += part[v][q];
+            if (n_queues == kXcds) queue_cost[q] = c; else queue_cost[0] += c;
+        }
         long long lc[kXcds], lo = 0, hi = short_cost;      // the level lies in [lo, hi]
 #pragma unroll
         for (int q = 0; q < kXcds; q++) {
-            lc[q] = q < n_queues ? (n_split > 0 ? queue_cost[q] : 0) : 0x7fffffffffffffffLL;
+            lc[q] = q < n_queues ? queue_cost[q] : 0x7fffffffffffffffLL;
             if (q < n_queues && lc[q] + short_cost > hi) hi = lc[q] + short_cost;
         }
         while (lo < hi) {
@@ -280,12 +293,12 @@ constexpr int64_t kFusedReduceMaxPieces = 16384;
 
 int64_t plan_zeroed_ints(int64_t n_split, const Mail *stats, int groups)
 {
-    if (n_split == 0) return kZeroQueueLoad;
-    return kZeroQueueLoad + scan_zeroed(n_split) + scan_zeroed(class_layout(n_split, stats, groups).total);
+    if (n_split == 0) return 0;
+    return scan_zeroed(n_split) + scan_zeroed(class_layout(n_split, stats, groups).total);
 }
 
 int prepare_split_rows(Arena *tmp, const accel_handle *h, const SortedRows &sr, const UnitRule &rule, const PlanUnits &pu,
-                       int *zeroed, const Mail *stats, DevBuf *slot, SplitArgs *out)
+                       const Mail *stats, DevBuf *slot, SplitArgs *out)
 {
     const int n_split = (int)h->n_split_rows;
     int rc;
@@ -300,12 +313,13 @@ int prepare_split_rows(Arena *tmp, const accel_handle *h, const SortedRows &sr, 
     a.piece = std::max(h->plan_unit, h->plan_split);
     a.cost_shift = rule.cost_shift;
     a.n_queues = h->plan_queues;                       // 8 interleaved queues, or 1 (plain order)
-    a.queue_cost = zeroed;
+    a.n_groups = split_groups(n_split, place_threads(h->n_chunks - h->n_lone_chunks));
     // the slots of each split row, and behind them two counters per split row (zero between launches)
     if ((rc = slot->alloc(sizeof(int) * (size_t)(3 * (int64_t)n_split + 1)))) return rc;
     a.row_done = slot->as<int>() + n_split + 1;
     if (n_split > 0) {
         if ((rc = tmp->alloc(&a.row_units, (size_t)n_split))) return rc;
+        if ((rc = tmp->alloc(&a.group_cost, (size_t)a.n_groups * kXcds))) return rc;
         if ((rc = tmp->alloc(&a.bins, (size_t)a.cl.total + 1))) return rc;
     }
     *out = a;
@@ -330,10 +344,9 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
     if ((rc = tmp->alloc(&head, 1))) return rc;
     int *slot = dslot->as<int>();
     if (n_split > 0) {
-        int *z = zeroed + kZeroQueueLoad;
-        launch_scans({{{split.row_units, slot, n_split, 0, z}, {bins, bins, cl.total, 0, z + scan_zeroed(n_split)}}, {}}, 2, s);
+        launch_scans({{{split.row_units, slot, n_split, 0, zeroed}, {bins, bins, cl.total, 0, zeroed + scan_zeroed(n_split)}}, {}}, 2, s);
     }
-    plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, zeroed, running, share_sums, pitch, sh.n, nq, head,
+    plan_head_kernel<<<dim3(1), dim3(512), 0, s>>>(bins, cl, n_split, split.group_cost, split.n_groups, running, share_sums, pitch, sh.n, nq, head,
                                                   mail);
     // Room for the list, before its length is known: the queues are level in cost, not in units,
     // so each gets half as much again as its share of the units.  Where that is not enough

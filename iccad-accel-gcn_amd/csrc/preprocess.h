@@ -44,6 +44,7 @@ enum {
     kStatRows16, kStatRows32, kStatRows64,                // rows stored in 16, 32, 64 column groups by row_groups' own rule
     kStatBig, kStatBigAlt,                                // rows with more than 32 times a split threshold
     kStatSampled, kStatLocal,                             // of the locality sample
+    kStatLoneChunks,                                      // wide rows of one chunk
     kStatCount
 };
 Mail *take_mail();            // memory.hip; null when there is none
@@ -172,6 +173,18 @@ __device__ __forceinline__ int block_exclusive_sum(int v, int *lds, int &total)
     return prefix + inc - v;
 }
 
+__device__ __forceinline__ int wave_exclusive_sum(int v)
+{
+    const int lane = threadIdx.x & 63;
+    int inc = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(inc, off);
+        if (lane >= off) inc += t;
+    }
+    return inc - v;
+}
+
 __device__ __forceinline__ int wave_sum(int v)
 {
 #pragma unroll
@@ -189,6 +202,20 @@ __device__ __forceinline__ unsigned long long wave_match(int v, int bits, bool v
         peers &= bit ? bal : ~bal;
     }
     return peers;
+}
+// The same of a column group of ng (8 to 64): four instructions a bit (seven by the loop above).
+__device__ __forceinline__ unsigned long long match_group(int g, int ng, bool valid)
+{
+    const unsigned long long all = __ballot(valid);
+    uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
+    auto bit = [&](int b) {
+        const int m = (g << (31 - b)) >> 31;
+        const unsigned long long bal = __ballot(m != 0);
+        lo &= ~((uint32_t)bal ^ (uint32_t)m);
+        hi &= ~((uint32_t)(bal >> 32) ^ (uint32_t)m);
+    };
+    bit(0); bit(1); bit(2); bit(3); bit(4); bit(5);
+    return (unsigned long long)hi << 32 | lo;
 }
 __device__ __forceinline__ int lanes_below(unsigned long long m, int lane)
 {
@@ -481,17 +508,29 @@ struct SplitArgs {
     const int *rank8;
     ClassLayout cl;
     int forced, piece, cost_shift, n_queues;
-    int *bins, *row_units, *row_done, *queue_cost;
+    int *bins, *row_units, *row_done;
+    int n_groups;                             // workgroups that count
+    int *group_cost;                          // [workgroup][8]
     int n_wide;                               // the last of them are wide rows: row i's chunks are first_chunk[i] to [i + 1]
     const int *first_chunk, *chunk_count;     // of those; [chunk][64]
 };
+// Threads of the workgroups that place chunks of wide rows and count split rows.  A chunk is a chain of 16 rounds by four
+// wavefronts and of four by sixteen, but seven chunks are under way on a compute unit with the former and two with the
+// latter: 2.45 M non-zeros (35 chunks) 10.4 us with 256 threads, 6.8 with 1,024; 30 M (4,200) 62 and 76; 125 M (5,100) 90
+// and 101.  The line lies where the large workgroups stop being on the card all at once, twice over.
+inline int place_threads(int64_t chunks) { return chunks > 1024 ? 256 : 1024; }
+// Workgroups that count n rows: a row per wavefront, a few rows where there are very many.
+constexpr int kSplitGroups = 1024;
+inline int split_groups(int64_t n, int threads) { return (int)std::min<int64_t>((n + threads / 64 - 1) / (threads / 64), kSplitGroups); }
+// (What the rows cost is added up by plan_head_kernel: eight atomics per workgroup, all of them to the same eight words,
+// took 14 of 22 us for 29 k rows.)
 template <int T>
-__device__ __forceinline__ void count_split_rows(const SplitArgs &a, int workgroup, int n_workgroups, int (*part)[kXcds])
+__device__ __forceinline__ void count_split_rows(const SplitArgs &a, int workgroup, int (*part)[kXcds])
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     constexpr int kWaves = T / 64;
     int cost = 0;
-    for (int lr = workgroup * kWaves + w; lr < a.n_split; lr += n_workgroups * kWaves) {
+    for (int lr = workgroup * kWaves + w; lr < a.n_split; lr += a.n_groups * kWaves) {
         const SplitRow s = split_row(a.s_indptr, a.first_split, a.n_split, lr, a.rank8, a.cl, a.forced);
         const int wide = lr - (a.n_split - a.n_wide);
         int c = 0;
@@ -519,7 +558,7 @@ __device__ __forceinline__ void count_split_rows(const SplitArgs &a, int workgro
     __syncthreads();
     if ((int)threadIdx.x < kXcds) {
         for (int q = 1; q < kWaves; q++) cost += part[q][threadIdx.x];
-        if (cost) atomicAdd(&a.queue_cost[threadIdx.x % a.n_queues], cost);
+        a.group_cost[workgroup * kXcds + threadIdx.x] = cost;
     }
 }
 
@@ -527,7 +566,7 @@ __device__ __forceinline__ void count_split_rows(const SplitArgs &a, int workgro
 // The split rows' counters, and the kernel arguments that say where they are (gcount, first_chunk, chunk_count and n_wide left to
 // the caller).  slot: what becomes the handle's long_slot, with its counters behind.
 int prepare_split_rows(Arena *tmp, const accel_handle *h, const SortedRows &sr, const UnitRule &rule, const PlanUnits &pu,
-                       int *zeroed, const Mail *stats, DevBuf *slot, SplitArgs *out);
+                       const Mail *stats, DevBuf *slot, SplitArgs *out);
 // The rest of the plan, behind the counting of the split rows.
 int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const UnitRule &rule, const Shares &sh,
                     const PlanUnits &pu, const SplitArgs &split, DevBuf *slot, int64_t n_short_units, int *zeroed, Mail *mail,

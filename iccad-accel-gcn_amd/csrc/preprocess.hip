@@ -88,6 +88,7 @@ __global__ __launch_bounds__(kThreads) void degree_kernel(DegreeArgs a, int *__r
                 if (d > kDegBound) st[kStatLongBlocks] += (d + kDegBound - 1) / kDegBound;
                 if (d > kWideRow) {
                     st[kStatWideRows]++;
+                    st[kStatLoneChunks] += d <= kWideChunk;
                     st[kStatWideChunks] += (d + kWideChunk - 1) / kWideChunk;
                     const int ng = row_groups(d, 0);
                     st[kStatRows16] += ng == 16;
@@ -712,9 +713,11 @@ __device__ __forceinline__ void report_bad(const CopyArgs &a, bool bad)
 // Rows that stay whole (up to 384 non-zeros): a workgroup copies kPermuteTile consecutive non-zeros
 // of the sorted matrix.  Which rows those are is a closed form of the position (runs of equal
 // degree); their source offsets are put in LDS, and where the tile lies inside one run, as nearly
-// all do on a large matrix, each thread finds the row of its non-zeros by a multiplication.  Bound
-// by reading row segments of some hundred bytes at arbitrary addresses (about twice their bytes in
-// 128-byte lines).
+// all do on a large matrix, each thread finds the row of its non-zeros by a multiplication, elsewhere by
+// a search without branches.  Bound by reading row segments of some hundred bytes at arbitrary addresses (about twice
+// their bytes in 128-byte lines; 64 M non-zeros: 290 us) on a large matrix, by the chain of a tile on a small one: all of
+// a thread's searches and row pointers are under way together (one after the other this kernel took 13.1 us instead of
+// 8.4 on 60 k non-zeros, 22.3 instead of 17.3 on 2.45 M).
 constexpr int kPermuteNz = 8;                        // non-zeros per thread
 constexpr int kPermuteTile = kThreads * kPermuteNz;  // non-zeros per workgroup
 struct PermuteLds {
@@ -746,38 +749,54 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, i
     const int row1 = l.run_row[d_last] + (p1 - 1 - l.run_nz[d_last]) / d_last;
     const int n_here = row1 - row0 + 1;              // at most kPermuteTile: every row holds a non-zero of the tile
     const bool one_run = d_first == d_last;
-    for (int j = threadIdx.x; j < n_here; j += kThreads) {
-        const int row = row0 + j;
-        int lo = d_first, hi = d_last;               // the last bin that starts at or before the row
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (l.run_row[mid] <= row) lo = mid; else hi = mid - 1;
+    constexpr int kRows = 4;                         // rows of a thread under way at once
+    const int bin_step = one_run ? 0 : 1 << (31 - __clz(d_last - d_first));
+    for (int j0 = threadIdx.x; j0 < n_here; j0 += kRows * kThreads) {
+        int bin[kRows], src[kRows];
+#pragma unroll
+        for (int k = 0; k < kRows; k++) {
+            const int row = row0 + min(j0 + k * kThreads, n_here - 1);
+            bin[k] = d_first;
+            src[k] = a.sr.perm ? a.sr.perm[row] : row;
         }
-        const int start = l.run_nz[lo] + (row - l.run_row[lo]) * lo;
-        l.row_end[j] = start + lo;
-        l.shift[j] = a.sr.indptr[a.sr.perm ? a.sr.perm[row] : row] - start;
+        for (int step = bin_step; step > 0; step >>= 1)      // the last bin that starts at or before the row
+#pragma unroll
+            for (int k = 0; k < kRows; k++) {
+                const bool on = l.run_row[min(bin[k] + step, kBins)] <= row0 + j0 + k * kThreads;
+                bin[k] += on & (bin[k] + step <= d_last) ? step : 0;
+            }
+#pragma unroll
+        for (int k = 0; k < kRows; k++) src[k] = a.sr.indptr[src[k]];
+#pragma unroll
+        for (int k = 0; k < kRows; k++) {
+            const int j = j0 + k * kThreads;
+            if (j >= n_here) continue;
+            const int start = l.run_nz[bin[k]] + (row0 + j - l.run_row[bin[k]]) * bin[k];
+            l.row_end[j] = start + bin[k];
+            l.shift[j] = src[k] - start;
+        }
     }
     __syncthreads();
     const int start0 = l.row_end[0] - d_first;       // first non-zero of the tile's first row
     const float inv = 1.0f / (float)d_first;
     int src[kPermuteNz], col[kPermuteNz], pay[kPermuteNz];
     bool bad = false;
+    auto position = [&](int q) { return min(p0 + q * kThreads + (int)threadIdx.x, p1 - 1); };
+    if (one_run) {
 #pragma unroll
-    for (int q = 0; q < kPermuteNz; q++) {
-        const int p = min(p0 + q * kThreads + (int)threadIdx.x, p1 - 1);
-        int j;
-        if (one_run) {
-            j = (int)(((float)(p - start0) + 0.5f) * inv);       // exact: p - start0 < 2,432
-        } else {
-            int lo = 0, hi = n_here - 1;             // first j with row_end[j] > p
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (l.row_end[mid] > p) hi = mid; else lo = mid + 1;
+        for (int q = 0; q < kPermuteNz; q++) src[q] = (int)(((float)(position(q) - start0) + 0.5f) * inv);    // exact: below 2,432
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPermuteNz; q++) src[q] = 0;
+        for (int step = 1 << (31 - __clz(n_here)); step > 0; step >>= 1)     // rows that end at or before the position
+#pragma unroll
+            for (int q = 0; q < kPermuteNz; q++) {
+                const bool on = l.row_end[min(src[q] + step, n_here) - 1] <= position(q);
+                src[q] += on & (src[q] + step <= n_here) ? step : 0;
             }
-            j = lo;
-        }
-        src[q] = p + l.shift[j];
     }
+#pragma unroll
+    for (int q = 0; q < kPermuteNz; q++) src[q] = position(q) + l.shift[src[q]];
 #pragma unroll
     for (int q = 0; q < kPermuteNz; q++) {
         col[q] = a.idx[src[q]];
@@ -798,86 +817,109 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, i
 // stably inside each group, so that a work unit of such a row touches rows of X that belong to one
 // column group.  counts[lr * 64 + g] receives the size of each group (counts may be null).
 // Rows of up to R * 64 non-zeros: a wavefront per row.  The whole row is loaded at once, put in
-// order in LDS and written out in one piece per array: with stores straight from the ranks (up to
-// 64 groups under the same store instruction) and a second read of the columns regrouping 62 M
-// non-zeros took 0.49 ms (0.33 ms so).
+// order in LDS, the columns first and then the payload, and written out in one piece per array.  Bound by memory as
+// long as enough of them are under way: columns and payload together in LDS (33 KB a workgroup instead of 17) let four
+// workgroups on a compute unit instead of seven, the tiles of whole rows in the same launch among them.  With that, with
+// the ranks kept in registers instead of groups counted by atomics first, and with rows of one chunk placed here
+// (place_chunk), the copying of 125 M non-zeros of a power-law matrix takes 548 us where it took 683, that of 30 M with hub
+// rows 155 where it took 202 (with wide_place_kernel).
 template <int R> struct GroupLds {
-    int2 buf[kWaves4][R * 64];
+    int buf[kWaves4][R * 64];
     int cnt[kWaves4][kMaxGroups];
 };
+// Non-zeros e0, e0 + 64, ... of the n at src, the last one again behind the end: their columns, their payloads.
+template <int R>
+__device__ __forceinline__ void load_columns(const CopyArgs &a, int src, int n, int e0, int (&col)[R])
+{
+    const int32_t *idx = a.idx + src;
+#pragma unroll
+    for (int j = 0; j < R; j++) col[j] = idx[min(e0 + j * 64, n - 1)];
+}
+template <int R>
+__device__ __forceinline__ void load_payloads(const CopyArgs &a, int src, int n, int e0, int (&pay)[R])
+{
+    if (a.src_pos) {
+#pragma unroll
+        for (int j = 0; j < R; j++) pay[j] = src + e0 + j * 64;
+    } else {
+        const float *val = a.val + src;
+        asm("" : "+v"(e0));                              // (or the positions of the columns are kept in registers for this)
+#pragma unroll
+        for (int j = 0; j < R; j++) pay[j] = __float_as_int(val[min(e0 + j * 64, n - 1)]);
+    }
+}
+// The place of this lane's non-zero among those of its group that the wavefront has met, R rounds in a row.
+// cnt (64 ints of this wavefront, cleared): the sizes of the groups on return.
+template <int R>
+__device__ __forceinline__ void rank_in_groups(const int (&col)[R], int n, int ng, int *cnt, int (&where)[R])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        if (j * 64 >= n) break;                          // uniform
+        const bool valid = lane < n - j * 64;
+        const int g = col_group(col[j], ng);
+        const unsigned long long peers = match_group(g, ng, valid);
+        const int rank = lanes_below(peers, lane);
+        where[j] = cnt[g] + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) cnt[g] = where[j] + __popcll(peers);     // one lane per group present
+        __builtin_amdgcn_wave_barrier();
+    }
+}
 template <int R>
 __device__ __forceinline__ void group_row(const CopyArgs &a, GroupLds<R> &l, int64_t r, int lr, int forced_groups,
                                           int *__restrict__ counts)
 {
     static_assert(kMaxGroups == 64, "one lane per column group");
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t src0 = a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r];
-    const int64_t dst0 = a.sr.s_indptr[r];
-    const int d = a.sr.s_indptr[r + 1] - (int)dst0;
-    const int ng = row_groups(d, forced_groups), bits = 31 - __clz(ng);
-    int *my = l.cnt[w];
-    int2 *st = l.buf[w];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int src0 = __builtin_amdgcn_readfirstlane(a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r]);
+    const int dst0 = __builtin_amdgcn_readfirstlane(a.sr.s_indptr[r]);
+    const int d = __builtin_amdgcn_readfirstlane(a.sr.s_indptr[r + 1]) - dst0;
+    const int ng = row_groups(d, forced_groups);
+    int *my = l.cnt[w], *st = l.buf[w];
     my[lane] = 0;
     __builtin_amdgcn_wave_barrier();
-    int col[R], pay[R];
+    int col[R], where[R];
     bool bad = false;
+    load_columns<R>(a, src0, d, lane, col);
+    rank_in_groups<R>(col, d, ng, my, where);
+    const int c = my[lane];                              // lane g holds the size of group g
+    if (counts) counts[(int64_t)lr * kMaxGroups + lane] = c;
+    const int start = wave_exclusive_sum(c);
+    __builtin_amdgcn_wave_barrier();
+    my[lane] = start;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int j = 0; j < R; j++) {
-        const int e = j * 64 + lane;
-        col[j] = pay[j] = 0;
-        if (e < d) {
-            col[j] = a.idx[src0 + e];
-            pay[j] = payload(a, src0 + e);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        if (j * 64 + lane < d) {
+        if (lane < d - j * 64) {
             bad |= (uint32_t)col[j] >= a.cols;
-            atomicAdd(&my[col_group(col[j], ng)], 1);
+            where[j] += my[col_group(col[j], ng)];
+            st[where[j]] = col[j];
         }
     }
     report_bad(a, bad);
+    int pay[R];
+    load_payloads<R>(a, src0, d, lane, pay);
     __builtin_amdgcn_wave_barrier();
-    const int c = my[lane];                              // lane g holds the size of group g
-    if (counts) counts[(int64_t)lr * kMaxGroups + lane] = c;
-    int inc = c;
+    if (a.idx_out) {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int t = __shfl_up(inc, off);
-        if (lane >= off) inc += t;
+        for (int j = 0; j < R; j++)
+            if (lane < d - j * 64) (a.idx_out + dst0 + j * 64)[lane] = st[j * 64 + lane];
     }
     __builtin_amdgcn_wave_barrier();
-    my[lane] = inc - c;                                  // where group g starts; moves on as it fills
+#pragma unroll
+    for (int j = 0; j < R; j++)
+        if (lane < d - j * 64) st[where[j]] = pay[j];
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int j = 0; j < R; j++) {
-        if (j * 64 >= d) break;                          // uniform
-        const bool valid = j * 64 + lane < d;
-        const int g = col_group(col[j], ng);
-        const unsigned long long peers = wave_match(g, bits, valid);
-        const int rank = lanes_below(peers, lane);
-        const int pos = my[g] + rank;
-        __builtin_amdgcn_wave_barrier();
-        if (valid) {
-            st[pos] = make_int2(col[j], pay[j]);
-            if (rank == 0) my[g] = pos + __popcll(peers);    // one lane per group present
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        const int e = j * 64 + lane;
-        if (e < d) {
-            const int2 v = st[e];
-            if (a.idx_out) a.idx_out[dst0 + e] = v.x;
-            a.pay_out[dst0 + e] = v.y;
-        }
-    }
+    for (int j = 0; j < R; j++)
+        if (lane < d - j * 64) (a.pay_out + dst0 + j * 64)[lane] = st[j * 64 + lane];
 }
 
 // Longer rows ("wide") in chunks of kWideChunk non-zeros, a workgroup per chunk, so that a row of
-// 200,000 is 49 workgroups and not a chain of 200 rounds in one: count the chunk's groups, place.  chunk_row[c] = the long row of chunk c, first_chunk[i] = the
+// 200,000 is 49 workgroups and not a chain of 200 rounds in one.  A row of one chunk is placed at once; of the
+// others the chunks' groups are counted first.  chunk_row[c] = the long row of chunk c, first_chunk[i] = the
 // first chunk of long row i.
 struct WideArgs {
     const int *chunk_row, *first_chunk;
@@ -887,21 +929,22 @@ struct WideArgs {
     int *chunk_count;                         // [chunks][64]: non-zeros of each group
 };
 struct WideChunk {
-    int64_t src;
+    int src, row;                             // in the caller's arrays; where the row starts in the sorted ones
     int n, ng;
+    bool whole;                               // the row has no other chunk
 };
 __device__ __forceinline__ WideChunk wide_chunk(const CopyArgs &a, const WideArgs &wa, int c)
 {
-    const int i = wa.chunk_row[c];
+    const int i = __builtin_amdgcn_readfirstlane(wa.chunk_row[c]);
     const int64_t r = wa.first_long + i;
-    const int d = a.sr.s_indptr[r + 1] - a.sr.s_indptr[r], off = (c - wa.first_chunk[i]) * kWideChunk;
-    return {(int64_t)a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r] + off, min(kWideChunk, d - off),
-            row_groups(d, wa.forced_groups)};
+    const int from = __builtin_amdgcn_readfirstlane(a.sr.s_indptr[r]);
+    const int d = __builtin_amdgcn_readfirstlane(a.sr.s_indptr[r + 1]) - from, off = (c - wa.first_chunk[i]) * kWideChunk;
+    return {__builtin_amdgcn_readfirstlane(a.sr.indptr[a.sr.perm ? a.sr.perm[r] : r]) + off, from, min(kWideChunk, d - off),
+            row_groups(d, wa.forced_groups), d <= kWideChunk};
 }
 
-__device__ __forceinline__ void wide_count(const CopyArgs &a, const WideArgs &wa, int *cnt, int c)
+__device__ __forceinline__ void wide_count(const CopyArgs &a, const WideChunk &ch, int *cnt, int *__restrict__ count)
 {
-    const WideChunk ch = wide_chunk(a, wa, c);
     if ((int)threadIdx.x < kMaxGroups) cnt[threadIdx.x] = 0;
     __syncthreads();
     int col[kWideChunk / kThreads];
@@ -920,7 +963,82 @@ __device__ __forceinline__ void wide_count(const CopyArgs &a, const WideArgs &wa
     }
     report_bad(a, bad);
     __syncthreads();
-    if ((int)threadIdx.x < kMaxGroups) wa.chunk_count[(int64_t)c * kMaxGroups + threadIdx.x] = cnt[threadIdx.x];
+    if ((int)threadIdx.x < kMaxGroups) count[threadIdx.x] = cnt[threadIdx.x];
+}
+
+// A chunk's non-zeros to their places, by W wavefronts.  kWhole: the chunk is the row, whose groups are counted here
+// (count); else sum says how many non-zeros of each group the row has and how many the chunks before this one, to be added
+// up over the wavefronts.
+template <int W> struct ChunkLds {
+    int buf[kWideChunk];
+    int at[W][kMaxGroups], off[kMaxGroups];
+};
+template <int W, bool kWhole>
+__device__ __forceinline__ void place_chunk(const CopyArgs &a, ChunkLds<W> &l, const WideChunk &ch, int *__restrict__ count,
+                                            int (*sum)[W][kMaxGroups])
+{
+    constexpr int R = kWideChunk / (W * 64);             // rounds of a wavefront at most: each takes as many
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int share = (ch.n + W * 64 - 1) / (W * 64) * 64, first = w * share, n = min(share, ch.n - first);
+    l.at[w][lane] = 0;
+    __builtin_amdgcn_wave_barrier();
+    int col[R], where[R];
+    load_columns<R>(a, ch.src, ch.n, first + lane, col);
+    rank_in_groups<R>(col, n, ch.ng, l.at[w], where);
+    __syncthreads();
+    if (w == 0) {
+        int v[W], total = 0;
+#pragma unroll
+        for (int q = 0; q < W; q++) { v[q] = l.at[q][lane]; total += v[q]; }
+        int run = wave_exclusive_sum(total);             // where the chunk's group `lane` starts in LDS
+        if constexpr (kWhole) {
+            count[lane] = total;
+        } else {
+            int all = 0, before = 0;
+#pragma unroll
+            for (int q = 0; q < W; q++) {
+                all += sum[0][q][lane];
+                before += sum[1][q][lane];
+            }
+            l.off[lane] = (int)ch.row + wave_exclusive_sum(all) + before - run;
+        }
+#pragma unroll
+        for (int q = 0; q < W; q++) { l.at[q][lane] = run; run += v[q]; }
+    }
+    __syncthreads();
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        if (lane < n - j * 64) {
+            bad |= (uint32_t)col[j] >= a.cols;
+            where[j] += l.at[w][col_group(col[j], ch.ng)];
+            l.buf[where[j]] = col[j];
+        }
+    }
+    if (kWhole) report_bad(a, bad);                      // (else reported by wide_count)
+    int pay[R];
+    load_payloads<R>(a, ch.src, ch.n, first + lane, pay);
+    __syncthreads();
+    int to[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const int e = j * W * 64 + (int)threadIdx.x;
+        if (e < ch.n) {
+            const int c = l.buf[e];
+            to[j] = (kWhole ? (int)ch.row : l.off[col_group(c, ch.ng)]) + e;
+            if (a.idx_out) a.idx_out[to[j]] = c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; j++)
+        if (lane < n - j * 64) l.buf[where[j]] = pay[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const int e = j * W * 64 + (int)threadIdx.x;
+        if (e < ch.n) a.pay_out[to[j]] = l.buf[e];
+    }
 }
 
 // The units of whole rows, for which everything is known when the rows are placed.
@@ -954,7 +1072,7 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
         PermuteLds permute;
         GroupLds<kMidRounds> mid;
         GroupLds<kSmallRounds> small;
-        int cnt[kMaxGroups];
+        ChunkLds<kWaves4> chunk;
     };
     __shared__ __attribute__((aligned(16))) char raw[sizeof(Lds)];
     Lds &l = *reinterpret_cast<Lds *>(raw);
@@ -968,16 +1086,22 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
         return;
     }
     b -= u.groups;
-    if (b < cp.n_chunks) { wide_count(a, wa, l.cnt, b); return; }
+    if (b < cp.n_chunks) {
+        const WideChunk ch = wide_chunk(a, wa, b);
+        int *const count = wa.chunk_count + (int64_t)b * kMaxGroups;
+        if (ch.whole) place_chunk<kWaves4, true>(a, l.chunk, ch, count, nullptr);
+        else wide_count(a, ch, l.chunk.off, count);
+        return;
+    }
     b -= cp.n_chunks;
     if (b < cp.mid_groups) {                  // a wavefront without a row leaves; no barriers inside
-        const int i = b * kWaves4 + (threadIdx.x >> 6);
+        const int i = b * kWaves4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if (i < cp.n_mid) group_row<kMidRounds>(a, l.mid, cp.first_mid + i, cp.n_small + i, wa.forced_groups, cp.counts);
         return;
     }
     b -= cp.mid_groups;
     if (b < cp.small_groups) {
-        const int i = b * kWaves4 + (threadIdx.x >> 6);
+        const int i = b * kWaves4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if (i < cp.n_small) group_row<kSmallRounds>(a, l.small, cp.first_small + i, i, wa.forced_groups, cp.counts);
         return;
     }
@@ -987,100 +1111,30 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
 // Counts the split rows for the plan and, in the workgroups behind, places the chunks of wide rows, one each (both
 // come behind the counts of the chunks and nothing else: as launches of their own, with another that added up the
 // chunks' counts, they took 12 us more on 2.45 M non-zeros).
-constexpr int kPlaceThreads = 1024;
-__global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, WideArgs wa, int split_groups, SplitArgs split)
+template <int kPlaceThreads>
+__global__ __launch_bounds__(kPlaceThreads) void wide_place_kernel(CopyArgs a, WideArgs wa, int first, SplitArgs split)
 {
     constexpr int kWaves = kPlaceThreads / 64;
-    constexpr int R = kWideChunk / kPlaceThreads;        // rounds of a wavefront, which takes a sixteenth of the chunk
-    __shared__ int2 buf[kWideChunk];
-    __shared__ int at[kWaves][kMaxGroups], off[kMaxGroups], sum[2][kWaves][kMaxGroups];
-    if ((int)blockIdx.x < split_groups) {
-        count_split_rows<kPlaceThreads>(split, (int)blockIdx.x, split_groups, reinterpret_cast<int (*)[kXcds]>(&sum[0][0][0]));
+    __shared__ ChunkLds<kWaves> l;
+    __shared__ int sum[2][kWaves][kMaxGroups];
+    if ((int)blockIdx.x < split.n_groups) {
+        count_split_rows<kPlaceThreads>(split, (int)blockIdx.x, reinterpret_cast<int (*)[kXcds]>(&sum[0][0][0]));
         return;
     }
-    const int chunk = (int)blockIdx.x - split_groups;
+    const int chunk = first + (int)blockIdx.x - split.n_groups;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const WideChunk ch = wide_chunk(a, wa, chunk);
-    const int bits = 31 - __clz(ch.ng);
-    at[w][lane] = 0;
-    __builtin_amdgcn_wave_barrier();
     // the row's non-zeros of each group, and those of the chunks before this one
-    {
-        const int i = wa.chunk_row[chunk], c0 = wa.first_chunk[i], c1 = wa.first_chunk[i + 1];
-        int all = 0, before = 0;
+    const int i = wa.chunk_row[chunk], c0 = wa.first_chunk[i], c1 = wa.first_chunk[i + 1];
+    int all = 0, before = 0;
 #pragma unroll 4
-        for (int c = c0 + w; c < c1; c += kWaves) {
-            const int v = wa.chunk_count[(int64_t)c * kMaxGroups + lane];
-            all += v;
-            before += c < chunk ? v : 0;
-        }
-        sum[0][w][lane] = all;
-        sum[1][w][lane] = before;
+    for (int c = c0 + w; c < c1; c += kWaves) {
+        const int v = wa.chunk_count[(int64_t)c * kMaxGroups + lane];
+        all += v;
+        before += c < chunk ? v : 0;
     }
-    int col[R], pay[R];
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        const int e = (w * R + j) * 64 + lane;
-        col[j] = pay[j] = 0;
-        if (e < ch.n) {
-            col[j] = a.idx[ch.src + e];
-            pay[j] = payload(a, ch.src + e);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < R; j++)
-        if ((w * R + j) * 64 + lane < ch.n) atomicAdd(&at[w][col_group(col[j], ch.ng)], 1);
-    __syncthreads();
-    if (w == 0) {
-        int v[kWaves], total = 0;
-#pragma unroll
-        for (int q = 0; q < kWaves; q++) { v[q] = at[q][lane]; total += v[q]; }
-        int inc = total;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(inc, o);
-            if (lane >= o) inc += t;
-        }
-        int run = inc - total;                           // where the chunk's group `lane` starts in LDS
-        int all = 0, before = 0;
-#pragma unroll
-        for (int q = 0; q < kWaves; q++) {
-            all += sum[0][q][lane];
-            before += sum[1][q][lane];
-        }
-        int upto = all;                                  // the row's non-zeros of the groups up to this one
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(upto, o);
-            if (lane >= o) upto += t;
-        }
-        off[lane] = a.sr.s_indptr[wa.first_long + wa.chunk_row[chunk]] + upto - all + before - run;
-#pragma unroll
-        for (int q = 0; q < kWaves; q++) { at[q][lane] = run; run += v[q]; }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-        if ((w * R + j) * 64 >= ch.n) break;             // uniform
-        const bool valid = (w * R + j) * 64 + lane < ch.n;
-        const int g = col_group(col[j], ch.ng);
-        const unsigned long long peers = wave_match(g, bits, valid);
-        const int rank = lanes_below(peers, lane);
-        const int pos = at[w][g] + rank;
-        __builtin_amdgcn_wave_barrier();
-        if (valid) {
-            buf[pos] = make_int2(col[j], pay[j]);
-            if (rank == 0) at[w][g] = pos + __popcll(peers);
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < ch.n; e += kPlaceThreads) {
-        const int2 v = buf[e];
-        const int64_t to = (int64_t)off[col_group(v.x, ch.ng)] + e;
-        if (a.idx_out) a.idx_out[to] = v.x;
-        a.pay_out[to] = v.y;
-    }
+    sum[0][w][lane] = all;
+    sum[1][w][lane] = before;
+    place_chunk<kWaves, false>(a, l, wide_chunk(a, wa, chunk), nullptr, sum);
 }
 
 // Columns of a matrix whose arrays are used in place (sorted, no split row).
@@ -1587,7 +1641,7 @@ static int choose_plan_split(int64_t nnz, bool team) { return team || nnz < kSma
 
 // Launches that fill the sorted copy (see CopyArgs).  Needs perm (or none), s_indptr, the bins' runs,
 // n_split_rows and, for wide rows, the chunk tables, as the preprocessing leaves them on the handle.  The units of
-// whole rows are listed (u.groups > 0) and the split rows counted for the plan (split.n_split > 0) on the way.
+// whole rows are listed (u.groups > 0) and the split rows counted for the plan (split.n_groups > 0) on the way.
 static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, int64_t nnz_short, const UnitsArgs &u,
                          SplitArgs split, hipStream_t s)
 {
@@ -1612,11 +1666,10 @@ static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, i
     split.n_wide = n_wide;
     split.first_chunk = wa.first_chunk ? wa.first_chunk + wa.n_narrow : nullptr;
     split.chunk_count = wa.chunk_count;
-    // (each workgroup of split rows ends on eight atomics to the same eight words)
-    constexpr unsigned kSplitGroups = 1024;
-    const unsigned split_groups = std::min((unsigned)((split.n_split + kPlaceThreads / 64 - 1) / (kPlaceThreads / 64)), kSplitGroups);
-    if (cp.n_chunks + split_groups > 0)
-        wide_place_kernel<<<dim3((unsigned)cp.n_chunks + split_groups), dim3(kPlaceThreads), 0, s>>>(a, wa, (int)split_groups, split);
+    const int lone = (int)h->n_lone_chunks, placed = cp.n_chunks - lone, threads = place_threads(placed);
+    if (placed + split.n_groups > 0)
+        (threads == 256 ? wide_place_kernel<256> : wide_place_kernel<1024>)<<<
+            dim3((unsigned)(placed + split.n_groups)), dim3((unsigned)threads), 0, s>>>(a, wa, lone, split);
     ACCEL_HIP(hipGetLastError());
     return ACCEL_OK;
 }
@@ -1735,7 +1788,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     h->n_blocks = h->n_long_blocks = h->n_long_rows = h->n_zero_rows = 0;
     h->max_degree = 0;
     h->n_units = h->n_long_units = 0;
-    h->n_split_rows = h->n_big_rows = h->n_wide_rows = h->n_chunks = 0;
+    h->n_split_rows = h->n_big_rows = h->n_wide_rows = h->n_chunks = h->n_lone_chunks = 0;
     h->plan_team = h->plan_team_option == 2 || (h->plan_team_option == 0 && choose_plan_team(rows, nnz));
     h->plan_unit = h->plan_unit_option > 0 ? h->plan_unit_option : choose_plan_unit(nnz, h->plan_team);
     h->plan_split = h->plan_split_option > 0 ? h->plan_split_option : choose_plan_split(nnz, h->plan_team);
@@ -1780,6 +1833,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     h->n_long_blocks = st[kStatLongBlocks];
     h->n_wide_rows = st[kStatWideRows];
     h->n_chunks = st[kStatWideChunks];
+    h->n_lone_chunks = st[kStatLoneChunks];
     h->n_big_rows = alt ? st[kStatBigAlt] : st[kStatBig];
     h->n_split_rows = h->n_long_rows;
     for (int d = h->plan_split + 1; d <= kDegBound; d++) h->n_split_rows += mail->hist[d];
@@ -1880,7 +1934,7 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     // ---- sorted CSR; every column is looked at once on the way -------------------------
     DevBuf slot;
     SplitArgs split;
-    if ((rc = prepare_split_rows(&tmp, h, ua.sr, rule, pu, zeroed, mail, &slot, &split))) return rc;
+    if ((rc = prepare_split_rows(&tmp, h, ua.sr, rule, pu, mail, &slot, &split))) return rc;
     split.gcount = gcount;
     if (own_copy) {
         const CopyArgs ca{sorted_rows(h), h->idx, h->val, (uint32_t)h->cols, s_idx, reinterpret_cast<int32_t *>(s_val), 0,

@@ -1,0 +1,46 @@
+"""The sorted copy at the sizes where its kernels change: rows of one chunk, placed by four wavefronts that share their rounds
+evenly, next to rows of several; more than 1,024 chunks, placed by smaller workgroups; tiles of whole rows that hold one
+degree, a few, or very many.  Whole numbers, compared exactly with the oracle; products within its tolerance."""
+import numpy as np
+import pytest
+
+from oracle import spmm_oracle as so
+from test_gpu_preprocess import check_plan, check_preprocess
+from test_gpu_preprocess_shapes import graph
+
+pytestmark = pytest.mark.gpu
+
+
+def check(gpu, deg, cols, groups=0, **options):
+    g = graph(gpu, deg, cols)
+    op = check_preprocess(gpu, g, plan_team=1, plan_groups=groups, **options)
+    check_plan(op, g.n_cols)
+    X = np.random.default_rng(2).uniform(-1, 1, (g.n_cols, 4)).astype(np.float32)
+    assert so.check(op.matmul(X), g.indptr, g.indices, g.values, X) <= so.TOL
+    v = np.random.default_rng(3).uniform(-1, 1, g.nnz).astype(np.float32)
+    op.update_values(v)                                  # the same kernels, with positions instead of values
+    assert so.check(op.matmul(X), g.indptr, g.indices, v, X) <= so.TOL
+    op.close()
+
+
+@pytest.mark.parametrize("groups", [0, 8, 16, 32, 64])
+def test_rows_of_one_chunk(gpu, groups):
+    edges = [64 * k + e for k in (16, 17, 20, 32, 48, 63, 64) for e in (-1, 0, 1)]
+    small = [193, 255, 256, 257, 383, 384, 385, 640, 641, 1023, 1024, 0, 1, 5]
+    check(gpu, np.random.default_rng(5).permutation(edges + small), 50_021, groups, plan_unit=384)
+
+
+def test_many_chunks(gpu):
+    rng = np.random.default_rng(6)
+    check(gpu, rng.permutation(np.concatenate([4097 + 4 * rng.integers(0, 1200, 520), rng.integers(1, 1500, 300)])), 60_013,
+          plan_unit=384)
+
+
+@pytest.mark.parametrize("kind", ["ones", "one run", "two runs", "every degree", "few", "empty rows"])
+@pytest.mark.parametrize("rows", [1, 300, 2047, 2049, 5000])
+def test_tiles_of_whole_rows(gpu, kind, rows):
+    rng = np.random.default_rng(rows)
+    deg = {"ones": np.ones(rows, int), "one run": np.full(rows, 13), "two runs": np.where(np.arange(rows) % 2, 1, 191),
+           "every degree": np.arange(rows) % 193, "few": rng.integers(1, 4, rows), "empty rows": rng.integers(0, 2, rows) * 7}[kind]
+    deg[rng.integers(0, rows)] = 9                       # (at least one row that makes the order another)
+    check(gpu, deg, 10_007, plan_unit=192)
