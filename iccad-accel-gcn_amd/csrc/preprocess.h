@@ -148,17 +148,40 @@ struct DevBuf {  // device memory that is given back on scope exit unless it is 
 
 inline unsigned grid_for(int64_t n) { return (unsigned)((n + kThreads - 1) / kThreads); }
 
+// Scans over a wavefront with all lanes active, by moves between the lanes' registers: through ds_bpermute (__shfl) each
+// of the six steps waits for the LDS, 0.4 us a scan on an idle chip, and the fourteen sums at the end of degree_kernel
+// took 2.7 of its 8 us on 60 k non-zeros.  Lanes that a step has nothing for keep 0 (rows of 16 lanes first).
+template <int kCtrl, int kRows> __device__ __forceinline__ int lanes_moved(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
+}
+template <class F> __device__ __forceinline__ int wave_scan(int v, F f)
+{
+    v = f(v, lanes_moved<0x111, 0xf>(v));                // from 1, 2, 4, 8 lanes below, within rows
+    v = f(v, lanes_moved<0x112, 0xf>(v));
+    v = f(v, lanes_moved<0x114, 0xf>(v));
+    v = f(v, lanes_moved<0x118, 0xf>(v));
+    v = f(v, lanes_moved<0x142, 0xa>(v));                // the last lane of rows 0 and 2 to rows 1 and 3
+    return f(v, lanes_moved<0x143, 0xc>(v));             // lane 31 to rows 2 and 3
+}
+__device__ __forceinline__ int wave_inclusive_sum(int v)
+{
+    return wave_scan(v, [](int a, int b) { return a + b; });
+}
+__device__ __forceinline__ int wave_exclusive_sum(int v) { return wave_inclusive_sum(v) - v; }
+__device__ __forceinline__ int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_inclusive_sum(v), 63); }
+// (of values that are not negative)
+__device__ __forceinline__ int wave_max(int v)
+{
+    return __builtin_amdgcn_readlane(wave_scan(v, [](int a, int b) { return a > b ? a : b; }), 63);
+}
+
 // Exclusive scan of one value per thread over a workgroup of T threads; `lds` holds T / 64 ints.
 template <int T>
 __device__ __forceinline__ int block_exclusive_sum(int v, int *lds, int &total)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int inc = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int t = __shfl_up(inc, off);
-        if (lane >= off) inc += t;
-    }
+    const int inc = wave_inclusive_sum(v);
     if (lane == 63) lds[w] = inc;
     __syncthreads();
     int prefix = 0, tot = 0;
@@ -173,48 +196,19 @@ __device__ __forceinline__ int block_exclusive_sum(int v, int *lds, int &total)
     return prefix + inc - v;
 }
 
-__device__ __forceinline__ int wave_exclusive_sum(int v)
-{
-    const int lane = threadIdx.x & 63;
-    int inc = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int t = __shfl_up(inc, off);
-        if (lane >= off) inc += t;
-    }
-    return inc - v;
-}
-
-__device__ __forceinline__ int wave_sum(int v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
-// Lanes of this wavefront that are `valid` and hold the same value in the low `bits` bits of v.
-__device__ __forceinline__ unsigned long long wave_match(int v, int bits, bool valid)
-{
-    unsigned long long peers = __ballot(valid);
-    for (int b = 0; b < bits; b++) {
-        const bool bit = (v >> b) & 1;
-        const unsigned long long bal = __ballot(bit);
-        peers &= bit ? bal : ~bal;
-    }
-    return peers;
-}
-// The same of a column group of ng (8 to 64): four instructions a bit (seven by the loop above).
-__device__ __forceinline__ unsigned long long match_group(int g, int ng, bool valid)
+// Lanes of this wavefront that are `valid` and hold the same value in the low kBits bits of v: four instructions a bit.
+template <int kBits>
+__device__ __forceinline__ unsigned long long wave_match(int v, bool valid)
 {
     const unsigned long long all = __ballot(valid);
     uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
-    auto bit = [&](int b) {
-        const int m = (g << (31 - b)) >> 31;
-        const unsigned long long bal = __ballot(m != 0);
-        lo &= ~((uint32_t)bal ^ (uint32_t)m);
-        hi &= ~((uint32_t)(bal >> 32) ^ (uint32_t)m);
-    };
-    bit(0); bit(1); bit(2); bit(3); bit(4); bit(5);
+#pragma unroll
+    for (int b = 0; b < kBits; b++) {
+        const int bit = (v << (31 - b)) >> 31;
+        const unsigned long long bal = __ballot(bit != 0);
+        lo &= ~((uint32_t)bal ^ (uint32_t)bit);
+        hi &= ~((uint32_t)(bal >> 32) ^ (uint32_t)bit);
+    }
     return (unsigned long long)hi << 32 | lo;
 }
 __device__ __forceinline__ int lanes_below(unsigned long long m, int lane)
@@ -444,12 +438,7 @@ __device__ __forceinline__ void list_units(const SortedRows &sr, const UnitRule 
             const int nz = d * n;
             const int cost = n > 0 ? unit_cost(nz, n, rule.cost_shift) : 0;
             const unsigned long long heads = __ballot(n > 0), heavies = __ballot(n > 0 && nz > rule.light_nz);
-            int inc = cost;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int t = __shfl_up(inc, off);
-                if (lane >= off) inc += t;
-            }
+            const int inc = wave_inclusive_sum(cost);
             if (n > 0) {
                 int w, rpb;
                 slice_rule(d, w, rpb);
@@ -462,7 +451,7 @@ __device__ __forceinline__ void list_units(const SortedRows &sr, const UnitRule 
             const unsigned long long eights = __ballot(is8);
             if (is8) pu.rank8[p - first_split] = rows8 + lanes_below(eights, lane);
             n_units += __popcll(heads);
-            cost0 += __shfl(inc, 63);
+            cost0 += __builtin_amdgcn_readlane(inc, 63);
             heavy0 += __popcll(heavies);
             rows8 += __popcll(eights);
         }

@@ -123,11 +123,7 @@ __global__ __launch_bounds__(kThreads) void degree_kernel(DegreeArgs a, int *__r
     static_assert(kWideRow < 2 * kXcds * kGroupMinPiece, "rows of 16 and more groups are wide ones");
 #pragma unroll
     for (int k = 0; k < kStatCount; k++) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const int t = __shfl_xor(st[k], off);
-            st[k] = k <= kStatMaxDegree ? max(st[k], t) : st[k] + t;
-        }
+        st[k] = k <= kStatMaxDegree ? wave_max(st[k]) : wave_sum(st[k]);
         if (lane == 0) part[w][k] = st[k];
     }
     __syncthreads();
@@ -156,6 +152,7 @@ __global__ __launch_bounds__(kThreads) void bin_scan_kernel(int *__restrict__ bi
         const int k = threadIdx.x & 15;
         int v = 0;
         if (k < kStatCount)
+#pragma unroll 8                                         // (not unrolled: 17 us for 958 workgroups' statistics, 6 so)
             for (int g = threadIdx.x >> 4; g < n_groups; g += kThreads / 16) {
                 const int t = stats[g * 16 + k];
                 v = k <= kStatMaxDegree ? max(v, t) : v + t;
@@ -283,22 +280,32 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 
     // sorted row pointers and block4 entries of the rows of up to 384 non-zeros, by sorted row
     const int n_binned = run_row[kLongBin];
-    for (int64_t p0 = me - lane; p0 < n_binned; p0 += all) {
-        const int64_t p = p0 + lane;
-        if (p >= n_binned) break;
-        int lo = 0, hi = kLongBin - 1;                    // the last bin that starts at or before p
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (run_row[mid] <= p) lo = mid; else hi = mid - 1;
-        }
-        const int d = lo, i = (int)p - run_row[d], loc = run_nz[d] + i * d;
-        a.s_indptr[p] = loc;
-        if (d > 0) {
-            int wn, rpb;
-            slice_rule(d, wn, rpb);
-            if (i % rpb == 0)
-                a.block4[run_blk[d] + i / rpb] =
-                    make_int4(d, (int)p, loc, (wn << 16) + min(rpb, run_row[d + 1] - run_row[d] - i));
+    // (rows of a thread searched for together, in steps that are selections: one at a time with branches, 3.6 us here)
+    constexpr int kAtOnce = 4;
+    for (int64_t p0 = me; p0 < n_binned; p0 += kAtOnce * all) {
+        int bin[kAtOnce];
+#pragma unroll
+        for (int k = 0; k < kAtOnce; k++) bin[k] = 0;
+#pragma unroll
+        for (int step = 256; step > 0; step >>= 1)            // the last bin that starts at or before the row
+#pragma unroll
+            for (int k = 0; k < kAtOnce; k++) {
+                const bool on = run_row[min(bin[k] + step, kLongBin)] <= p0 + k * all;
+                bin[k] += (on & (bin[k] + step < kLongBin)) ? step : 0;
+            }
+#pragma unroll
+        for (int k = 0; k < kAtOnce; k++) {
+            const int64_t p = p0 + k * all;
+            if (p >= n_binned) break;
+            const int d = bin[k], i = (int)p - run_row[d], loc = run_nz[d] + i * d;
+            a.s_indptr[p] = loc;
+            if (d > 0) {
+                int wn, rpb;
+                slice_rule(d, wn, rpb);
+                if (i % rpb == 0)
+                    a.block4[run_blk[d] + i / rpb] =
+                        make_int4(d, (int)p, loc, (wn << 16) + min(rpb, run_row[d + 1] - run_row[d] - i));
+            }
         }
     }
     if (me == 0) a.s_indptr[a.rows] = a.indptr[a.rows];
@@ -321,7 +328,7 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
             const bool ok = r < r_end;
             const int d = d4[j];
             const int bin = min(d, kLongBin);
-            const unsigned long long peers = wave_match(bin, 9, ok);
+            const unsigned long long peers = wave_match<9>(bin, ok);
             const int rank = lanes_below(peers, lane);
             const int p = next[w][bin] + rank;
             __builtin_amdgcn_wave_barrier();
@@ -763,7 +770,7 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, i
 #pragma unroll
             for (int k = 0; k < kRows; k++) {
                 const bool on = l.run_row[min(bin[k] + step, kBins)] <= row0 + j0 + k * kThreads;
-                bin[k] += on & (bin[k] + step <= d_last) ? step : 0;
+                bin[k] += (on & (bin[k] + step <= d_last)) ? step : 0;
             }
 #pragma unroll
         for (int k = 0; k < kRows; k++) src[k] = a.sr.indptr[src[k]];
@@ -792,7 +799,7 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, i
 #pragma unroll
             for (int q = 0; q < kPermuteNz; q++) {
                 const bool on = l.row_end[min(src[q] + step, n_here) - 1] <= position(q);
-                src[q] += on & (src[q] + step <= n_here) ? step : 0;
+                src[q] += (on & (src[q] + step <= n_here)) ? step : 0;
             }
     }
 #pragma unroll
@@ -850,6 +857,8 @@ __device__ __forceinline__ void load_payloads(const CopyArgs &a, int src, int n,
 }
 // The place of this lane's non-zero among those of its group that the wavefront has met, R rounds in a row.
 // cnt (64 ints of this wavefront, cleared): the sizes of the groups on return.
+constexpr int kGroupBits = 6;
+static_assert(kMaxGroups == 1 << kGroupBits, "a group's number");
 template <int R>
 __device__ __forceinline__ void rank_in_groups(const int (&col)[R], int n, int ng, int *cnt, int (&where)[R])
 {
@@ -859,7 +868,7 @@ __device__ __forceinline__ void rank_in_groups(const int (&col)[R], int n, int n
         if (j * 64 >= n) break;                          // uniform
         const bool valid = lane < n - j * 64;
         const int g = col_group(col[j], ng);
-        const unsigned long long peers = match_group(g, ng, valid);
+        const unsigned long long peers = wave_match<kGroupBits>(g, valid);
         const int rank = lanes_below(peers, lane);
         where[j] = cnt[g] + rank;
         __builtin_amdgcn_wave_barrier();
