@@ -370,61 +370,12 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 // ---------------------------------------------------------------------------
 // Rows of more than 384 non-zeros, by (degree, row).  Up to kFewLong of them: each is compared with all
 // (place_long_kernel), and the non-zeros, blocks and chunks of the rows before it are added up on the way, which is all
-// there is to know (ranking, then a scan by one workgroup, took a launch and 10 us more on 2.45 M non-zeros).  More
-// are ranked by comparison up to kRankMax (rank_long_rows_kernel; one workgroup for 800 rows takes 18 us, thirteen 5),
-// or by a stable radix sort, 8 bits a pass; their scans and blocks are launches of their own.
+// there is to know.  More go through a stable radix sort, 8 bits a pass; their scans and blocks are launches of their own.
+// Comparing costs the square: 19 us on 4,850 rows and 25 on 6,400, where comparing for the rank alone, with the launches for
+// the scans and blocks behind it, took 29 and 34 and the gaps between them; on 8,192 it would be 41, as much as the sort's
+// six to nine launches take on 13,000.
 // ---------------------------------------------------------------------------
-constexpr int kFewLong = 2048;
-constexpr int kRankMax = 8192;
-constexpr int kRankRows = 64;                 // rows ranked by sixteen wavefronts, each against a sixteenth
-
-// How many of the n4 * 4 degrees at `tile` (LDS), the first of which is long row `at0`, rank before
-// long row j of degree d.  Equal degrees rank by row, which is the order they are listed in.
-__device__ __forceinline__ int count_before(const int4 *tile, int n4, int at0, int d, int j)
-{
-    int below = 0;
-#pragma unroll 4
-    for (int i = 0; i < n4; i++) {
-        const int4 e = tile[i];
-        const int at = at0 + 4 * i;
-        below += (e.x < d + (at < j)) + (e.y < d + (at + 1 < j)) + (e.z < d + (at + 2 < j)) + (e.w < d + (at + 3 < j));
-    }
-    return below;
-}
-
-// The first kSums workgroups scan one kind each of the counts per share (sums), which has
-// nothing to do with the rest but that both come behind place_rows; the others rank the long rows.
-__global__ __launch_bounds__(1024) void rank_long_rows_kernel(
-    const int *__restrict__ deg, const uint32_t *__restrict__ row, int n, int64_t first_long,
-    int32_t *__restrict__ perm, uint32_t *__restrict__ place, int *__restrict__ sorted_deg, int *__restrict__ sums,
-    int sum_pitch, int n_shares)
-{
-    __shared__ __attribute__((aligned(16))) int tile[4096];
-    __shared__ int part[16][kRankRows];
-    int b = blockIdx.x;
-    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, tile); return; }
-    b -= kSums;
-    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
-    const int d = j < n ? deg[j] : 0;
-    const uint32_t r = j < n ? row[j] : 0;
-    int below = 0;
-    for (int t0 = 0; t0 < n; t0 += 4096) {
-        const int here = min(4096, n - t0), per = (here + 63) / 64;       // vectors of four per wavefront
-        __syncthreads();
-        for (int i = threadIdx.x; i < per * 64; i += 1024) tile[i] = i < here ? deg[t0 + i] : INT_MAX;
-        __syncthreads();
-        below += count_before(reinterpret_cast<const int4 *>(tile) + seg * per, per, t0 + seg * per * 4, d, j);
-    }
-    part[seg][lane] = below;
-    __syncthreads();
-    if (seg == 0 && j < n) {
-        for (int q = 1; q < 16; q++) below += part[q][lane];
-        const int64_t p = first_long + below;
-        if (perm) perm[p] = (int32_t)r;
-        place[r] = (uint32_t)p;
-        sorted_deg[below] = d;
-    }
-}
+constexpr int kFewLong = 8192;
 
 __host__ __device__ inline int blocks_of(int d) { return (d + kDegBound - 1) / kDegBound; }
 __host__ __device__ inline int chunks_of(int d) { return d > kWideRow ? (d + kWideChunk - 1) / kWideChunk : 0; }
@@ -442,45 +393,63 @@ struct LongArgs {
     int *first_chunk, *chunk_row;             // of long row i (null: none is wide)
 };
 
-// Up to kFewLong long rows, completely: places, row pointers, blocks and chunks, 64 rows per workgroup.  The first kSums
-// workgroups scan the counts per share, as in rank_long_rows_kernel.
+// Up to kFewLong long rows, completely: places, row pointers, blocks and chunks.  kRankRows rows per workgroup, few so that
+// even some hundred rows are work for much of the chip, and selections instead of branches (5.5 us on 1,760 rows, where 64
+// rows a workgroup and a branch per row took 17): a lane compares one of them with every 64th of all rows.  The first kSums workgroups scan the counts per share.
+constexpr int kRankRows = 16, kRankTile = 2048;
 __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__restrict__ sums, int sum_pitch, int n_shares)
 {
-    __shared__ __attribute__((aligned(16))) int deg[kFewLong + 64];
-    __shared__ int part[16][4][kRankRows];
-    __shared__ int4 mine[kRankRows];                     // rank, first non-zero, first block, first chunk
+    __shared__ int4 tile[kRankTile];                     // degree, blocks, chunks
+    __shared__ int4 part[16][kRankRows], mine[kRankRows];
+    __shared__ int deg[kRankRows];
     int b = blockIdx.x;
-    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, deg); return; }
+    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, &tile[0].x); return; }
     b -= kSums;
-    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane;
+    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane % kRankRows;
+    const int d = j < a.n ? a.deg[j] : 0;
     const uint32_t r = j < a.n ? a.row[j] : 0;
-    const int per = (a.n + 15) / 16;                     // of a wavefront
-    for (int i = threadIdx.x; i < a.n; i += 1024) deg[i] = a.deg[i];
-    __syncthreads();
-    const int d = j < a.n ? deg[j] : 0;
     int below = 0, nz = 0, blk = 0, chk = 0;
-    const int to = min(a.n, (seg + 1) * per);
-#pragma unroll 4
-    for (int i = seg * per; i < to; i++) {
-        const int e = deg[i];                            // equal degrees rank by row, which is the order they are listed in
-        if (e < d + (i < j)) {
-            below++;
-            nz += e;
-            blk += blocks_of(e);
-            chk += chunks_of(e);
+    for (int t0 = 0; t0 < a.n; t0 += kRankTile) {
+        constexpr int kStep = 1024 / kRankRows, kUnroll = 4;
+        const int here = (min(kRankTile, a.n - t0) + kStep * kUnroll - 1) / (kStep * kUnroll) * (kStep * kUnroll);
+        if (t0 > 0) __syncthreads();
+        for (int i = threadIdx.x; i < here; i += 1024) {
+            const int e = t0 + i < a.n ? a.deg[t0 + i] : INT_MAX;
+            tile[i] = make_int4(e, blocks_of(e), chunks_of(e), 0);
+        }
+        __syncthreads();
+        for (int i0 = 0; i0 < here; i0 += kStep * kUnroll) {
+#pragma unroll
+            for (int k = 0; k < kUnroll; k++) {
+                const int i = i0 + k * kStep + seg * (64 / kRankRows) + lane / kRankRows;
+                const int4 e = tile[i];
+                // (equal degrees rank by row, which is the order they are listed in)
+                const int take = -(int)(e.x < d + (t0 + i < j));
+                below -= take;
+                nz += e.x & take;
+                blk += e.y & take;
+                chk += e.z & take;
+            }
         }
     }
-    part[seg][0][lane] = below;
-    part[seg][1][lane] = nz;
-    part[seg][2][lane] = blk;
-    part[seg][3][lane] = chk;
+#pragma unroll
+    for (int o = kRankRows; o < 64; o *= 2) {
+        below += __shfl_xor(below, o);
+        nz += __shfl_xor(nz, o);
+        blk += __shfl_xor(blk, o);
+        chk += __shfl_xor(chk, o);
+    }
+    if (lane < kRankRows) part[seg][lane] = make_int4(below, nz, blk, chk);
     __syncthreads();
-    if (seg == 0 && j < a.n) {
-        for (int q = 1; q < 16; q++) {
-            below += part[q][0][lane];
-            nz += part[q][1][lane];
-            blk += part[q][2][lane];
-            chk += part[q][3][lane];
+    if (seg == 0 && lane < kRankRows && j < a.n) {
+        below = nz = blk = chk = 0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int4 v = part[q][lane];
+            below += v.x;
+            nz += v.y;
+            blk += v.z;
+            chk += v.w;
         }
         const int64_t p = a.first_long + below;
         if (a.perm) a.perm[p] = (int32_t)r;
@@ -490,17 +459,18 @@ __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__res
             a.first_chunk[below] = chk;
             if (below == a.n - 1) a.first_chunk[a.n] = chk + chunks_of(d);
         }
+        deg[lane] = d;
         mine[lane] = make_int4(below, a.nz0 + nz, a.block0 + blk, chk);
     }
     __syncthreads();
-    for (int i = seg; i < kRankRows && b * kRankRows + i < a.n; i += 16) {
-        const int di = deg[b * kRankRows + i];
-        const int4 m = mine[i];
-        for (int k = lane; k < blocks_of(di); k += 64)
-            a.block4[m.z + k] = make_int4(di, (int)a.first_long + m.x, m.y + k * kDegBound, min(kDegBound, di - k * kDegBound));
-        if (a.first_chunk)
-            for (int k = lane; k < chunks_of(di); k += 64) a.chunk_row[m.w + k] = m.x;
-    }
+    static_assert(kRankRows == 16, "a row per wavefront");
+    if (b * kRankRows + seg >= a.n) return;
+    const int di = deg[seg];
+    const int4 m = mine[seg];
+    for (int k = lane; k < blocks_of(di); k += 64)
+        a.block4[m.z + k] = make_int4(di, (int)a.first_long + m.x, m.y + k * kDegBound, min(kDegBound, di - k * kDegBound));
+    if (a.first_chunk)
+        for (int k = lane; k < chunks_of(di); k += 64) a.chunk_row[m.w + k] = m.x;
 }
 
 constexpr int kItems = 8;
@@ -663,18 +633,12 @@ int place_long_rows(Arena *tmp, const LongArgs &a, int max_degree, const int32_t
                     int *sums, int pitch, int n_shares, hipStream_t s)
 {
     int rc, *sorted_deg, *blocks, *chunks = nullptr;
-    if (a.n <= kFewLong) {
-        const unsigned groups = kSums + (unsigned)((a.n + kRankRows - 1) / kRankRows);
-        place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
-        return ACCEL_OK;
-    }
-    const int ranked = a.n <= kRankMax ? a.n : 0;
+    const bool few = a.n <= kFewLong;
+    const unsigned groups = kSums + (few ? (unsigned)((a.n + kRankRows - 1) / kRankRows) : 0);
+    place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
+    if (few) return ACCEL_OK;
     if ((rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
-    rank_long_rows_kernel<<<dim3(kSums + (unsigned)((ranked + kRankRows - 1) / kRankRows)), dim3(1024), 0, s>>>(
-        a.deg, a.row, ranked, a.first_long, a.perm, a.place, sorted_deg, sums, pitch, n_shares);
-    if (a.n > kRankMax &&
-        (rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s)))
-        return rc;
+    if ((rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s))) return rc;
     if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
     if (a.first_chunk && (rc = tmp->alloc(&chunks, (size_t)a.n))) return rc;
     long_sizes_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(sorted_deg, a.n, blocks, chunks);

@@ -44,3 +44,12 @@ def test_tiles_of_whole_rows(gpu, kind, rows):
            "every degree": np.arange(rows) % 193, "few": rng.integers(1, 4, rows), "empty rows": rng.integers(0, 2, rows) * 7}[kind]
     deg[rng.integers(0, rows)] = 9                       # (at least one row that makes the order another)
     check(gpu, deg, 10_007, plan_unit=192)
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 4096, 4097, 8191, 8192, 8193])
+def test_number_of_long_rows(gpu, n):
+    """Long rows compared with each other, sixteen to a workgroup and against 2,048 at a time, up to 8,192 of them."""
+    rng = np.random.default_rng(n)
+    deg = np.concatenate([385 + rng.integers(0, 3, n), rng.integers(0, 20, 300)])
+    deg[:5] = (1024, 1025, 4097, 9000, 1025)
+    check(gpu, rng.permutation(deg), 30_011, plan_unit=384)
