@@ -273,22 +273,23 @@ struct Shares {
     unsigned groups() const { return (unsigned)(pitch / kWaves4); }
 };
 
-// Exclusive scan of the counts per share, in place, by a workgroup of 1,024 threads; the total goes
+// Exclusive scan of the counts per share, in place, by a workgroup of T threads; the total goes
 // behind the last share.
-__device__ __forceinline__ void scan_shares(int *__restrict__ s, int n, int *lds /* 16 ints */)
+template <int T>
+__device__ __forceinline__ void scan_shares(int *__restrict__ s, int n, int *lds /* T / 64 ints */)
 {
-    static_assert(kMaxShares <= 4 * 1024, "four shares per thread");
-    int v[4], acc = 0;
+    constexpr int kEach = kMaxShares / T;
+    int v[kEach], acc = 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = (int)threadIdx.x * 4 + j;
+    for (int j = 0; j < kEach; j++) {
+        const int i = (int)threadIdx.x * kEach + j;
         v[j] = i < n ? s[i] : 0;
         acc += v[j];
     }
-    int total, run = block_exclusive_sum<1024>(acc, lds, total);
+    int total, run = block_exclusive_sum<T>(acc, lds, total);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = (int)threadIdx.x * 4 + j;
+    for (int j = 0; j < kEach; j++) {
+        const int i = (int)threadIdx.x * kEach + j;
         if (i < n) s[i] = run;
         run += v[j];
     }

@@ -370,10 +370,10 @@ __global__ __launch_bounds__(kThreads) void place_rows_kernel(PlaceArgs a)
 // ---------------------------------------------------------------------------
 // Rows of more than 384 non-zeros, by (degree, row).  Up to kFewLong of them: each is compared with all
 // (place_long_kernel), and the non-zeros, blocks and chunks of the rows before it are added up on the way, which is all
-// there is to know.  More go through a stable radix sort, 8 bits a pass; their scans and blocks are launches of their own.
+// there is to know.  More go through a stable radix sort, 8 bits a pass; their scan and their blocks are launches of their own.
 // Comparing costs the square: 19 us on 4,850 rows and 25 on 6,400, where comparing for the rank alone, with the launches for
-// the scans and blocks behind it, took 29 and 34 and the gaps between them; on 8,192 it would be 41, as much as the sort's
-// six to nine launches take on 13,000.
+// the scans and blocks behind it, took 29 and 34 and the gaps between them; on 8,192 it would be 41, as much as the six
+// launches behind the sort take on 13,000 (39).
 // ---------------------------------------------------------------------------
 constexpr int kFewLong = 8192;
 
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__res
     __shared__ int4 part[16][kRankRows], mine[kRankRows];
     __shared__ int deg[kRankRows];
     int b = blockIdx.x;
-    if (b < kSums) { scan_shares(sums + (int64_t)b * sum_pitch, n_shares, &tile[0].x); return; }
+    if (b < kSums) { scan_shares<1024>(sums + (int64_t)b * sum_pitch, n_shares, &tile[0].x); return; }
     b -= kSums;
     const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6, j = b * kRankRows + lane % kRankRows;
     const int d = j < a.n ? a.deg[j] : 0;
@@ -476,11 +476,20 @@ __global__ __launch_bounds__(1024) void place_long_kernel(LongArgs a, int *__res
 constexpr int kItems = 8;
 constexpr int kTile = kThreads * kItems;      // elements per workgroup in the sort's passes and the scans
 
+// Digits of the tile's keys.  hist: [tile][digit] for kSelfScan tiles and fewer, which the scatter adds up itself, else
+// [digit][tile], scanned by small_scan_kernel.  The workgroups behind the tiles (first pass only) scan one kind each of the
+// counts per share (sums), which has nothing to do with the rest but that both come behind place_rows.
+constexpr int64_t kSelfScan = 64;
 __global__ __launch_bounds__(kThreads) void radix_hist(const uint32_t *__restrict__ keys,
                                                        int64_t n, int shift,
-                                                       int *__restrict__ hist, int64_t tiles)
+                                                       int *__restrict__ hist, int64_t tiles,
+                                                       int *__restrict__ sums, int sum_pitch, int n_shares)
 {
     __shared__ int h[256];
+    if ((int64_t)blockIdx.x >= tiles) {
+        scan_shares<kThreads>(sums + (blockIdx.x - tiles) * sum_pitch, n_shares, h);
+        return;
+    }
     h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kTile;
@@ -490,73 +499,92 @@ __global__ __launch_bounds__(kThreads) void radix_hist(const uint32_t *__restric
         if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1);
     }
     __syncthreads();
-    hist[(int64_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];  // digit-major
+    hist[tiles <= kSelfScan ? (int64_t)blockIdx.x * 256 + threadIdx.x : (int64_t)threadIdx.x * tiles + blockIdx.x] =
+        h[threadIdx.x];
 }
 
+// What the last pass writes instead of keys and their order: the long rows' places and sizes.
+struct LongSorted {
+    const uint32_t *row;                      // of the unsorted long rows (null: not the last pass)
+    int64_t first_long;
+    int32_t *perm;                            // null: in order already
+    uint32_t *place;
+    int *deg, *blocks, *chunks;               // in sorted order; chunks null: no row is wide
+};
+
+// A wavefront takes 512 keys in a row and ranks them without a barrier; then the tile's digits are placed.  With the counts
+// added up here and the last pass writing what two more kernels made of its order, the sort is four launches and not nine:
+// 20 M non-zeros with 13,000 long rows 397 -> 387 us from the graph to its first product, 60 M with 51,000 1028 -> 1011.
+// (A workgroup reads all tiles' counts: 64 KB of them at kSelfScan tiles.)
 __global__ __launch_bounds__(kThreads) void radix_scatter(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out, int64_t n, int shift,
-    const int *__restrict__ hist_scanned, int64_t tiles)
+    const int *__restrict__ hist, int64_t tiles, LongSorted out)
 {
-    __shared__ int running[256];               // next output slot of each digit for this tile
-    __shared__ int wave_cnt[kThreads / 64][256];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    running[threadIdx.x] = hist_scanned[(int64_t)threadIdx.x * tiles + blockIdx.x];
-    const int64_t base = (int64_t)blockIdx.x * kTile;
+    __shared__ int cnt[kWaves4][256], lds[kWaves4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, digit = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * kTile + w * (kTile / kWaves4) + lane;
+    uint32_t key[kItems], val[kItems];
+    int where[kItems];
+#pragma unroll
     for (int j = 0; j < kItems; j++) {
-        const int64_t i = base + j * kThreads + threadIdx.x;
-        const bool valid = i < n;
-        const uint32_t key = valid ? keys_in[i] : 0u;
-        const uint32_t val = valid ? (vals_in ? vals_in[i] : (uint32_t)i) : 0u;
-        const uint32_t dg = (key >> shift) & 255u;
-#pragma unroll
-        for (int q = 0; q < kThreads / 64; q++) wave_cnt[q][threadIdx.x] = 0;
-        __syncthreads();
-        // lanes of this wave that hold the same digit
-        unsigned long long peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const bool bit = (dg >> b) & 1u;
-            const unsigned long long bal = __ballot(bit);
-            peers &= bit ? bal : ~bal;
-        }
-        const int rank = __popcll(peers & ((1ull << lane) - 1ull));
-        if (valid && rank == 0) wave_cnt[w][dg] = __popcll(peers);
-        __syncthreads();
-        if (valid) {
-            int pos = running[dg] + rank;
-            for (int q = 0; q < w; q++) pos += wave_cnt[q][dg];
-            keys_out[pos] = key;
-            vals_out[pos] = val;
-        }
-        __syncthreads();
-        int add = 0;
-#pragma unroll
-        for (int q = 0; q < kThreads / 64; q++) add += wave_cnt[q][threadIdx.x];
-        running[threadIdx.x] += add;
+        const int64_t i = first + j * 64;
+        key[j] = i < n ? keys_in[i] : 0u;
+        val[j] = i < n && vals_in ? vals_in[i] : (uint32_t)i;
     }
-}
-
-
-__global__ __launch_bounds__(kThreads) void apply_long_order_kernel(
-    const uint32_t *__restrict__ order, const uint32_t *__restrict__ sorted_key, const uint32_t *__restrict__ row, int n,
-    int64_t first_long, int32_t *__restrict__ perm, uint32_t *__restrict__ place, int *__restrict__ sorted_deg)
-{
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t r = row[order[i]];
-    if (perm) perm[first_long + i] = (int32_t)r;
-    place[r] = (uint32_t)(first_long + i);
-    sorted_deg[i] = (int)sorted_key[i];
-}
-
-__global__ __launch_bounds__(kThreads) void long_sizes_kernel(const int *__restrict__ sorted_deg, int n,
-                                                              int *__restrict__ blocks, int *__restrict__ chunks)
-{
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    blocks[i] = blocks_of(sorted_deg[i]);
-    if (chunks) chunks[i] = chunks_of(sorted_deg[i]);
+    int at = 0;                                // where this tile's keys of the thread's digit go
+    if (tiles <= kSelfScan) {
+        int all = 0, before = 0;
+#pragma unroll 8
+        for (int t = 0; t < (int)tiles; t++) {
+            const int c = hist[t * 256 + digit];
+            all += c;
+            before += t < (int)blockIdx.x ? c : 0;
+        }
+        int total;
+        at = block_exclusive_sum<kThreads>(all, lds, total) + before;
+    } else {
+        at = hist[(int64_t)digit * tiles + blockIdx.x];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) cnt[w][j * 64 + lane] = 0;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < kItems; j++) {
+        const bool valid = first + j * 64 < n;
+        const int dg = (key[j] >> shift) & 255u;
+        const unsigned long long peers = wave_match<8>(dg, valid);
+        const int rank = lanes_below(peers, lane);
+        where[j] = cnt[w][dg] + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) cnt[w][dg] = where[j] + __popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kWaves4; q++) {
+        const int c = cnt[q][digit];
+        cnt[q][digit] = at;
+        at += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kItems; j++) {
+        if (first + j * 64 >= n) continue;
+        const int pos = where[j] + cnt[w][(key[j] >> shift) & 255u];
+        if (!out.row) {
+            keys_out[pos] = key[j];
+            vals_out[pos] = val[j];
+            continue;
+        }
+        const uint32_t r = out.row[val[j]];
+        const int d = (int)key[j];
+        if (out.perm) out.perm[out.first_long + pos] = (int32_t)r;
+        out.place[r] = (uint32_t)(out.first_long + pos);
+        out.deg[pos] = d;
+        out.blocks[pos] = blocks_of(d);
+        if (out.chunks) out.chunks[pos] = chunks_of(d);
+    }
 }
 
 // Exclusive scan of n ints in place by one workgroup (the radix sort's counts).
@@ -583,9 +611,9 @@ __global__ __launch_bounds__(1024) void small_scan_kernel(int *__restrict__ v, i
     }
 }
 
-// Sorts many long rows (perm, place and the degrees in sorted order).
-int sort_long_rows(Arena *tmp, const int *deg, const uint32_t *row, int n, int max_degree, int64_t first_long,
-                   int32_t *perm, uint32_t *place, int *sorted_deg, hipStream_t s)
+// Sorts many long rows (their places, and degrees, blocks and chunks in sorted order), and scans the counts per share.
+int sort_long_rows(Arena *tmp, const int *deg, int n, int max_degree, const LongSorted &sorted, int *sums, int pitch,
+                   int n_shares, hipStream_t s)
 {
     uint32_t *keys[2], *vals[2];
     int *hist, rc;
@@ -597,15 +625,15 @@ int sort_long_rows(Arena *tmp, const int *deg, const uint32_t *row, int n, int m
     if ((rc = tmp->alloc(&hist, (size_t)(256 * tiles)))) return rc;
     const uint32_t *kin = reinterpret_cast<const uint32_t *>(deg), *vin = nullptr;
     for (int shift = 0, to = 0; shift < 32 && (max_degree >> shift) != 0; shift += 8, to ^= 1) {
-        radix_hist<<<dim3((unsigned)tiles), dim3(kThreads), 0, s>>>(kin, n, shift, hist, tiles);
-        small_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(hist, 256 * tiles);
+        const bool last = shift == 24 || (max_degree >> (shift + 8)) == 0;
+        radix_hist<<<dim3((unsigned)tiles + (shift == 0 ? kSums : 0)), dim3(kThreads), 0, s>>>(kin, n, shift, hist, tiles, sums,
+                                                                                              pitch, n_shares);
+        if (tiles > kSelfScan) small_scan_kernel<<<dim3(1), dim3(1024), 0, s>>>(hist, 256 * tiles);
         radix_scatter<<<dim3((unsigned)tiles), dim3(kThreads), 0, s>>>(kin, vin, keys[to], vals[to], n, shift, hist,
-                                                                     tiles);
+                                                                     tiles, last ? sorted : LongSorted{});
         kin = keys[to];
         vin = vals[to];
     }
-    apply_long_order_kernel<<<dim3(grid_for(n)), dim3(kThreads), 0, s>>>(vin, kin, row, n, first_long, perm, place,
-                                                                        sorted_deg);
     return ACCEL_OK;
 }
 
@@ -633,15 +661,16 @@ int place_long_rows(Arena *tmp, const LongArgs &a, int max_degree, const int32_t
                     int *sums, int pitch, int n_shares, hipStream_t s)
 {
     int rc, *sorted_deg, *blocks, *chunks = nullptr;
-    const bool few = a.n <= kFewLong;
-    const unsigned groups = kSums + (few ? (unsigned)((a.n + kRankRows - 1) / kRankRows) : 0);
-    place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
-    if (few) return ACCEL_OK;
+    if (a.n <= kFewLong) {
+        const unsigned groups = kSums + (unsigned)((a.n + kRankRows - 1) / kRankRows);
+        place_long_kernel<<<dim3(groups), dim3(1024), 0, s>>>(a, sums, pitch, n_shares);
+        return ACCEL_OK;
+    }
     if ((rc = tmp->alloc(&sorted_deg, (size_t)a.n))) return rc;
-    if ((rc = sort_long_rows(tmp, a.deg, a.row, a.n, max_degree, a.first_long, a.perm, a.place, sorted_deg, s))) return rc;
     if ((rc = tmp->alloc(&blocks, (size_t)a.n + 1))) return rc;
     if (a.first_chunk && (rc = tmp->alloc(&chunks, (size_t)a.n))) return rc;
-    long_sizes_kernel<<<dim3(grid_for(a.n)), dim3(kThreads), 0, s>>>(sorted_deg, a.n, blocks, chunks);
+    const LongSorted sorted{a.row, a.first_long, a.perm, a.place, sorted_deg, blocks, chunks};
+    if ((rc = sort_long_rows(tmp, a.deg, a.n, max_degree, sorted, sums, pitch, n_shares, s))) return rc;
     ScanJobs jobs{};
     int n_jobs = 0;
     auto add = [&](const int *in, int *out, int first) {

@@ -53,3 +53,18 @@ def test_number_of_long_rows(gpu, n):
     deg = np.concatenate([385 + rng.integers(0, 3, n), rng.integers(0, 20, 300)])
     deg[:5] = (1024, 1025, 4097, 9000, 1025)
     check(gpu, rng.permutation(deg), 30_011, plan_unit=384)
+
+
+@pytest.mark.parametrize("n", [64 * 2048, 64 * 2048 + 1])
+def test_tiles_of_the_long_rows_sort(gpu, n):
+    """Up to 64 tiles of 2,048 long rows the sort's second kernel adds up the counts of all tiles itself."""
+    rng = np.random.default_rng(n)
+    deg = rng.permutation(np.concatenate([385 + rng.integers(0, 9, n - 2), [1025, 70_000], rng.integers(0, 3, 100)]))
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    op = gpu.AccelSpMM(indptr, np.zeros(indptr[-1], np.int32), np.ones(indptr[-1], np.float32), 4).preprocess()
+    assert op.info.n_long_rows == n
+    order = np.argsort(deg, kind="stable")
+    assert np.array_equal(op.perm(), order)
+    Y = op.matmul(np.ones((4, 4), np.float32))
+    assert np.array_equal(Y, np.repeat(deg[:, None], 4, 1))           # whole numbers below 2^24: exact
+    op.close()
