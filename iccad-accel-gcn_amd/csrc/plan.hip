@@ -198,7 +198,7 @@ __global__ __launch_bounds__(512) void plan_head_kernel(const int *__restrict__ 
     }
 }
 
-// Writes the list.  The first workgroups take split rows, a wavefront each (lane = column group),
+// Writes the list.  The first workgroups take split rows, a lane per column group (see SplitLane),
 // and write their pieces; the others the units of whole rows, one per thread.
 // Inside its queue a unit goes behind the pieces, in the order of the caller's row ids,
 // except that the queue's last kTailLight light units (few non-zeros: short chains of
@@ -223,25 +223,21 @@ struct EmitArgs {
     int4 *work;
 };
 
-__device__ __forceinline__ void emit_pieces(const EmitArgs &a, int lr)
+__device__ __forceinline__ void emit_pieces(const EmitArgs &a, int item)
 {
-    const int lane = threadIdx.x & 63;
+    const SplitLane at = split_lane(a.cl, a.n_split, item);
+    const int lr = at.lr, g = at.group;
     const SplitRow s = split_row(a.s_indptr, a.first_split, a.n_split, lr, a.rank8, a.cl, a.forced);
-    const int c = lane < s.groups ? a.gcount[(int64_t)lr * kMaxGroups + lane] : 0;
+    const int c = at.valid && g < s.groups ? a.gcount[(int64_t)lr * kMaxGroups + g] : 0;
     const int u = (c + a.piece - 1) / a.piece;
-    int c_inc = c, u_inc = u;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int tc = __shfl_up(c_inc, o), tu = __shfl_up(u_inc, o);
-        if (lane >= o) { c_inc += tc; u_inc += tu; }
-    }
+    const int c_inc = row_inclusive_sum(c, at.eight), u_inc = row_inclusive_sum(u, at.eight);
     if (c == 0) return;
     const int row = (int)(a.first_split + lr);
     const int loc = a.s_indptr[row] + c_inc - c, sl = a.slot[lr] + u_inc - u;
-    const int bin0 = a.cl.base[s.cls] + lane * a.cl.rows[s.cls];
-    const int pos0 = a.head->bin_off[plan_bin(s.groups, lane)] + a.bins[bin0 + s.rank] - a.bins[bin0];
+    const int bin0 = a.cl.base[s.cls] + g * a.cl.rows[s.cls];
+    const int pos0 = a.head->bin_off[plan_bin(s.groups, g)] + a.bins[bin0 + s.rank] - a.bins[bin0];
     for (int k = 0, off = 0; off < c; k++, off += a.piece)
-        a.work[plan_index(lane % a.n_queues, pos0 + k, a.n_queues)] =
+        a.work[plan_index(g % a.n_queues, pos0 + k, a.n_queues)] =
             make_int4(kDegBound + 1 + sl + k, row, loc + off, min(a.piece, c - off));
 }
 
@@ -250,8 +246,8 @@ __global__ __launch_bounds__(kThreads) void emit_plan_kernel(EmitArgs a)
     const int per_queue = a.head->per_queue;
     if (per_queue > a.room) return;                    // the host makes room and launches again
     if ((int)blockIdx.x < a.piece_groups) {
-        const int lr = (int)blockIdx.x * kWaves4 + (threadIdx.x >> 6);
-        if (lr < a.n_split) emit_pieces(a, lr);
+        const int item = (int)blockIdx.x * kWaves4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (item < split_items(a.cl, a.n_split)) emit_pieces(a, item);
         return;
     }
     const int tid = ((int)blockIdx.x - a.piece_groups) * kThreads + threadIdx.x;
@@ -313,7 +309,7 @@ int prepare_split_rows(Arena *tmp, const accel_handle *h, const SortedRows &sr, 
     a.piece = std::max(h->plan_unit, h->plan_split);
     a.cost_shift = rule.cost_shift;
     a.n_queues = h->plan_queues;                       // 8 interleaved queues, or 1 (plain order)
-    a.n_groups = split_groups(n_split, place_threads(h->n_chunks - h->n_lone_chunks));
+    a.n_groups = split_groups(split_items(a.cl, n_split), place_threads(h->n_chunks - h->n_lone_chunks));
     // the slots of each split row, and behind them two counters per split row (zero between launches)
     if ((rc = slot->alloc(sizeof(int) * (size_t)(3 * (int64_t)n_split + 1)))) return rc;
     a.row_done = slot->as<int>() + n_split + 1;
@@ -362,7 +358,7 @@ int build_work_list(Arena *tmp, accel_handle *h, const SortedRows &sr, const Uni
             return ACCEL_ERR_ARG;
         }
         if ((rc = dwork.alloc(sizeof(int4) * (size_t)(room * nq)))) return rc;
-        const int piece_groups = (int)grid_for((int64_t)n_split * 64);
+        const int piece_groups = (int)grid_for((int64_t)split_items(cl, n_split) * 64);
         const EmitArgs ea{gcount, sr.s_indptr, first_split, n_split, piece_groups, slot, bins, rank8, cl, forced, piece_nz,
                           units, running, heavy, (int)n_short_units, head, nq, (int)room, dwork.as<int4>()};
         emit_plan_kernel<<<dim3(piece_groups + grid_for(std::max<int64_t>(n_short_units, kThreads))), dim3(kThreads), 0,

@@ -488,7 +488,37 @@ __device__ __forceinline__ SplitRow split_row(const int32_t *__restrict__ s_indp
     return s;
 }
 
-// A wavefront per split row, lane = column group: pieces per group (into `bins`) and per row,
+// Which split row and which of its column groups a lane of wavefront `item` looks at: rows of 8 groups eight to a
+// wavefront, the others (behind them) one.  (Of 82,000 split rows 75,000 have 8 groups; a wavefront each, of which 56 lanes had
+// nothing to do, the counting and the writing of their pieces took 43 and 33 us on 60 M non-zeros; 27 and 20 so.)
+struct SplitLane {
+    int lr, group;
+    bool eight, valid;
+};
+inline __host__ __device__ int split_items(const ClassLayout &cl, int n_split) { return (cl.rows[0] + 7) / 8 + n_split - cl.rows[0]; }
+__device__ __forceinline__ SplitLane split_lane(const ClassLayout &cl, int n_split, int item)
+{
+    const int lane = threadIdx.x & 63, n8 = cl.rows[0], items8 = (n8 + 7) / 8;
+    if (item < items8) {
+        const int lr = item * 8 + lane / 8;
+        return {min(lr, n8 - 1), lane % 8, true, lr < n8};
+    }
+    return {n8 + item - items8, lane, false, true};
+}
+// Sum over the lanes of the row up to this one.
+__device__ __forceinline__ int row_inclusive_sum(int v, bool eight)
+{
+    if (!eight) return wave_inclusive_sum(v);
+    const int at = threadIdx.x & 7;
+    int t = lanes_moved<0x111, 0xf>(v);
+    v += at >= 1 ? t : 0;
+    t = lanes_moved<0x112, 0xf>(v);
+    v += at >= 2 ? t : 0;
+    t = lanes_moved<0x114, 0xf>(v);
+    return v + (at >= 4 ? t : 0);
+}
+
+// A lane per column group of a split row: pieces per group (into `bins`) and per row,
 // and what they cost per queue (column group g belongs to queue g % n_queues).
 struct SplitArgs {
     int *gcount;                              // [split row][64]: non-zeros per group; those of wide rows are added up here
@@ -509,7 +539,7 @@ struct SplitArgs {
 // latter: 2.45 M non-zeros (35 chunks) 10.4 us with 256 threads, 6.8 with 1,024; 30 M (4,200) 62 and 76; 125 M (5,100) 90
 // and 101.  The line lies where the large workgroups stop being on the card all at once, twice over.
 inline int place_threads(int64_t chunks) { return chunks > 1024 ? 256 : 1024; }
-// Workgroups that count n rows: a row per wavefront, a few rows where there are very many.
+// Workgroups that count: an item (see SplitLane) per wavefront, a few items where there are very many.
 constexpr int kSplitGroups = 1024;
 inline int split_groups(int64_t n, int threads) { return (int)std::min<int64_t>((n + threads / 64 - 1) / (threads / 64), kSplitGroups); }
 // (What the rows cost is added up by plan_head_kernel: eight atomics per workgroup, all of them to the same eight words,
@@ -517,26 +547,31 @@ inline int split_groups(int64_t n, int threads) { return (int)std::min<int64_t>(
 template <int T>
 __device__ __forceinline__ void count_split_rows(const SplitArgs &a, int workgroup, int (*part)[kXcds])
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int kWaves = T / 64;
     int cost = 0;
-    for (int lr = workgroup * kWaves + w; lr < a.n_split; lr += a.n_groups * kWaves) {
+    const int n_items = split_items(a.cl, a.n_split);
+    for (int item = workgroup * kWaves + w; item < n_items; item += a.n_groups * kWaves) {
+        const SplitLane at = split_lane(a.cl, a.n_split, item);
+        const int lr = at.lr;
         const SplitRow s = split_row(a.s_indptr, a.first_split, a.n_split, lr, a.rank8, a.cl, a.forced);
         const int wide = lr - (a.n_split - a.n_wide);
+        const bool mine = at.valid && at.group < s.groups;
         int c = 0;
         if (wide >= 0) {
             const int to = a.first_chunk[wide + 1];
 #pragma unroll 4
-            for (int i = a.first_chunk[wide]; i < to; i++) c += a.chunk_count[(int64_t)i * kMaxGroups + lane];
-            a.gcount[(int64_t)lr * kMaxGroups + lane] = c;
-        } else if (lane < s.groups) {
-            c = a.gcount[(int64_t)lr * kMaxGroups + lane];
+            for (int i = a.first_chunk[wide]; i < to; i++) c += a.chunk_count[(int64_t)i * kMaxGroups + at.group];
+            if (mine) a.gcount[(int64_t)lr * kMaxGroups + at.group] = c;
+        } else if (mine) {
+            c = a.gcount[(int64_t)lr * kMaxGroups + at.group];
         }
+        if (!mine) c = 0;
         const int u = (c + a.piece - 1) / a.piece;
-        if (lane < s.groups) a.bins[a.cl.base[s.cls] + lane * a.cl.rows[s.cls] + s.rank] = u;
+        if (mine) a.bins[a.cl.base[s.cls] + at.group * a.cl.rows[s.cls] + s.rank] = u;
         if (c > 0) cost += ((c + 9 * u) >> a.cost_shift) + u;
-        const int total = wave_sum(u);
-        if (lane == 0) {
+        const int total = row_inclusive_sum(u, at.eight);
+        if (at.valid && lane % (at.eight ? 8 : 64) == (at.eight ? 7 : 63)) {
             a.row_units[lr] = total;
             a.row_done[lr] = a.row_done[a.n_split + lr] = 0;
         }
