@@ -20,6 +20,15 @@ constexpr int kWavesPerGroup = 4;                     // wavefronts (work units)
 
 constexpr int kMaxGroups = 64;                        // column groups of the launch plan (8..64)
 
+// The order in which the preprocessing copies tiles of whole rows (see permute_rows in preprocess.hip).
+constexpr int kMaxBands = 256;
+struct TileOrder {
+    int log2_bands = 3;
+    int per_die = 0;                                  // workgroups per die, the most any has
+    // tiles in the bands before (as kernel arguments: a table that a kernel makes costs 3 us more on small matrices)
+    int first[kMaxBands + 1] = {};
+};
+
 // Column group of a non-zero.  Eight consecutive columns share a group so that
 // neighbouring short rows of X (one 128-byte line holds 8 rows at N = 4) stay
 // together.  Group g belongs to die g % 8; with more than 8 groups a die works
@@ -134,6 +143,7 @@ struct accel_handle {
     int64_t n_split_rows = 0;         // rows with more than plan_split non-zeros
     int64_t n_big_rows = 0;           // of those, rows with more than 32 * plan_split
     int64_t nnz_short = 0;            // non-zeros of the rows that are not split
+    accel::TileOrder tiles;           // ... and the order they are copied in
     int64_t n_wide_rows = 0;          // rows with more than 1,024 non-zeros, regrouped in chunks
     int64_t n_chunks = 0;             // ... of 4,096 non-zeros
     int64_t n_lone_chunks = 0;        // of those, the first ones, that are all there is of their row

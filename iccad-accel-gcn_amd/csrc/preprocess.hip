@@ -710,93 +710,111 @@ __device__ __forceinline__ void report_bad(const CopyArgs &a, bool bad)
     if (a.mail && __ballot(bad) && (threadIdx.x & 63) == 0) a.mail->bad_index = 1;
 }
 
-// Rows that stay whole (up to 384 non-zeros): a workgroup copies kPermuteTile consecutive non-zeros
-// of the sorted matrix.  Which rows those are is a closed form of the position (runs of equal
-// degree); their source offsets are put in LDS, and where the tile lies inside one run, as nearly
-// all do on a large matrix, each thread finds the row of its non-zeros by a multiplication, elsewhere by
-// a search without branches.  Bound by reading row segments of some hundred bytes at arbitrary addresses (about twice
-// their bytes in 128-byte lines; 64 M non-zeros: 290 us) on a large matrix, by the chain of a tile on a small one: all of
-// a thread's searches and row pointers are under way together (one after the other this kernel took 13.1 us instead of
-// 8.4 on 60 k non-zeros, 22.3 instead of 17.3 on 2.45 M).
+// Rows that stay whole (up to 384 non-zeros): a workgroup copies a tile, up to kPermuteTile consecutive non-zeros of one
+// run of equal degree in the sorted matrix, so that the row of a non-zero is a multiplication away; the rows'
+// source offsets are put in LDS.  Bound by the lines that row segments of some hundred bytes at arbitrary addresses touch,
+// twice their bytes and, for the offsets, a line per row: unless rows that are neighbours in the caller's
+// matrix, which share those lines, are copied by the same die at about the same time.  So tiles go by bands of the caller's
+// rows.  A run's rows are in the caller's order: tile i of its n tiles comes from about the i-th n-th of the matrix, and
+// belongs to about band i B / n of B (shifted by less than a tile, each run differently, so that runs of one tile do not all
+// end in the last band).  A die takes an eighth of the bands, one after the other, all runs' tiles of a band together.
+// In sorted order, several runs to a tile, found by search: 16 M non-zeros 361 MB read in 80.5 us, so 183 MB in 71 (whole
+// launch); 125 M 1.79 GB and 457 us, 1.28 GB and 430; 2.45 M 17.5 and 14.6 us, 60 k 8.8 and 6.0.  Tiles of 1,024
+// and of 4,096: 77 and 79 us on the 16 M, 469 and 436 on the 125 M.
 constexpr int kPermuteNz = 8;                        // non-zeros per thread
 constexpr int kPermuteTile = kThreads * kPermuteNz;  // non-zeros per workgroup
-struct PermuteLds {
-    int run_row[kBins + 1], run_nz[kBins];
-    int row_end[kPermuteTile + 1];                   // first non-zero of the row behind, per row of the tile
-    int shift[kPermuteTile + 1];                     // source position minus sorted position, per row
-};
-__device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, int tile, int n_take)
+__host__ __device__ inline int tiles_of_run(int nz) { return nz / kPermuteTile + (nz % kPermuteTile > 0); }
+
+// Tiles of the run of degree d, n in all, that the bands before `band` hold.
+__host__ __device__ inline int tiles_before(int band, int n, int d, int log2_bands)
 {
-    const int p0 = tile * kPermuteTile, p1 = min(p0 + kPermuteTile, n_take);
-    // degrees of the rows that hold the tile's first and last non-zero: as many bins (from 1 up) as
-    // start at or before it
-    int d_first = 0, d_last = 0;
-    {
-        constexpr int kLoads = kDegBound / 64;
-        int nz[kLoads];
-#pragma unroll
-        for (int j = 0; j < kLoads; j++) nz[j] = a.sr.run_nz[1 + 64 * j + (threadIdx.x & 63)];
-        for (int i = threadIdx.x; i <= kBins; i += kThreads) l.run_row[i] = a.sr.run_row[i];
-        for (int i = threadIdx.x; i < kBins; i += kThreads) l.run_nz[i] = a.sr.run_nz[i];
-#pragma unroll
-        for (int j = 0; j < kLoads; j++) {
-            d_first += __popcll(__ballot(nz[j] <= p0));
-            d_last += __popcll(__ballot(nz[j] <= p1 - 1));
-        }
+    const int shift = d * 159 & ((1 << log2_bands) - 1);
+    return (band * n + shift) >> log2_bands;                                    // below 2^29
+}
+
+static TileOrder order_tiles(const int *hist, int most)
+{
+    TileOrder t;
+    int64_t all = 0;
+    for (int d = 1; d <= most; d++) all += tiles_of_run(hist[d] * d);
+    while ((2 << t.log2_bands) <= kMaxBands && all >> (t.log2_bands + 1) >= 64) t.log2_bands++;
+    const int bands = 1 << t.log2_bands, per = bands / kXcds;
+    for (int d = 1; d <= most; d++) {
+        const int n = tiles_of_run(hist[d] * d);
+        if (n == 0) continue;
+        for (int b = 1; b <= bands; b++) t.first[b] += tiles_before(b, n, d, t.log2_bands);
     }
-    __syncthreads();
-    const int row0 = l.run_row[d_first] + (p0 - l.run_nz[d_first]) / d_first;
-    const int row1 = l.run_row[d_last] + (p1 - 1 - l.run_nz[d_last]) / d_last;
-    const int n_here = row1 - row0 + 1;              // at most kPermuteTile: every row holds a non-zero of the tile
-    const bool one_run = d_first == d_last;
+    for (int x = 0; x < kXcds; x++) t.per_die = std::max(t.per_die, t.first[(x + 1) * per] - t.first[x * per]);
+    return t;
+}
+
+struct PermuteLds {
+    int shift[kPermuteTile + 1];                     // source position minus sorted position, per row of the tile
+};
+// i: the number of the workgroup among those that copy tiles, i % 8 being its die's.
+__device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, const TileOrder &order, int i, int n_take)
+{
+    const int lane = threadIdx.x & 63;
+    const int per = 1 << (order.log2_bands - 3), band0 = i % kXcds * per;
+    const int t = order.first[band0] + i / kXcds;
+    if (t >= order.first[band0 + per]) return;
+    static_assert(kMaxBands / kXcds <= 64, "a lane per band of a die");
+    const int band = band0 + __popcll(__ballot(lane < per && order.first[band0 + min(lane, per - 1)] <= t)) - 1;
+    // which of the band's tiles: six degrees per lane
+    constexpr int kEach = kDegBound / 64;
+    int nz[kEach + 1], from[kEach], count[kEach], mine = 0;
+#pragma unroll
+    for (int k = 0; k <= kEach; k++) nz[k] = min(a.sr.run_nz[1 + lane * kEach + k], n_take);
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        const int n = tiles_of_run(nz[k + 1] - nz[k]);
+        const int degree = 1 + lane * kEach + k;
+        from[k] = tiles_before(band, n, degree, order.log2_bands);
+        count[k] = tiles_before(band + 1, n, degree, order.log2_bands) - from[k];
+        mine += count[k];
+    }
+    int j = t - order.first[band] - wave_exclusive_sum(mine);
+    const int owner = 63 - __clzll((long long)__ballot(j >= 0));        // (behind it the sums are larger)
+    int d = 0, at = 0, end = 0, run0 = 0;
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        if (j >= 0 && j < count[k]) {
+            d = 1 + lane * kEach + k;
+            run0 = nz[k];
+            at = run0 + (from[k] + j) * kPermuteTile;
+            end = nz[k + 1];
+        }
+        j -= count[k];
+    }
+    d = __builtin_amdgcn_readlane(d, owner);
+    run0 = __builtin_amdgcn_readlane(run0, owner);
+    const int p0 = __builtin_amdgcn_readlane(at, owner), n = min(kPermuteTile, __builtin_amdgcn_readlane(end, owner) - p0);
+    const int run_row = a.sr.run_row[d];
+    const int first = (p0 - run0) / d, start0 = run0 + first * d, row0 = run_row + first;
+    const int n_here = (p0 + n - 1 - run0) / d - first + 1;      // at most kPermuteTile: every row holds a non-zero of the tile
     constexpr int kRows = 4;                         // rows of a thread under way at once
-    const int bin_step = one_run ? 0 : 1 << (31 - __clz(d_last - d_first));
     for (int j0 = threadIdx.x; j0 < n_here; j0 += kRows * kThreads) {
-        int bin[kRows], src[kRows];
+        int src[kRows];
 #pragma unroll
         for (int k = 0; k < kRows; k++) {
             const int row = row0 + min(j0 + k * kThreads, n_here - 1);
-            bin[k] = d_first;
             src[k] = a.sr.perm ? a.sr.perm[row] : row;
         }
-        for (int step = bin_step; step > 0; step >>= 1)      // the last bin that starts at or before the row
-#pragma unroll
-            for (int k = 0; k < kRows; k++) {
-                const bool on = l.run_row[min(bin[k] + step, kBins)] <= row0 + j0 + k * kThreads;
-                bin[k] += (on & (bin[k] + step <= d_last)) ? step : 0;
-            }
 #pragma unroll
         for (int k = 0; k < kRows; k++) src[k] = a.sr.indptr[src[k]];
 #pragma unroll
-        for (int k = 0; k < kRows; k++) {
-            const int j = j0 + k * kThreads;
-            if (j >= n_here) continue;
-            const int start = l.run_nz[bin[k]] + (row0 + j - l.run_row[bin[k]]) * bin[k];
-            l.row_end[j] = start + bin[k];
-            l.shift[j] = src[k] - start;
-        }
+        for (int k = 0; k < kRows; k++)
+            if (j0 + k * kThreads < n_here) l.shift[j0 + k * kThreads] = src[k] - (start0 + (j0 + k * kThreads) * d);
     }
     __syncthreads();
-    const int start0 = l.row_end[0] - d_first;       // first non-zero of the tile's first row
-    const float inv = 1.0f / (float)d_first;
+    const float inv = 1.0f / (float)d;
     int src[kPermuteNz], col[kPermuteNz], pay[kPermuteNz];
     bool bad = false;
-    auto position = [&](int q) { return min(p0 + q * kThreads + (int)threadIdx.x, p1 - 1); };
-    if (one_run) {
 #pragma unroll
-        for (int q = 0; q < kPermuteNz; q++) src[q] = (int)(((float)(position(q) - start0) + 0.5f) * inv);    // exact: below 2,432
-    } else {
-#pragma unroll
-        for (int q = 0; q < kPermuteNz; q++) src[q] = 0;
-        for (int step = 1 << (31 - __clz(n_here)); step > 0; step >>= 1)     // rows that end at or before the position
-#pragma unroll
-            for (int q = 0; q < kPermuteNz; q++) {
-                const bool on = l.row_end[min(src[q] + step, n_here) - 1] <= position(q);
-                src[q] += (on & (src[q] + step <= n_here)) ? step : 0;
-            }
+    for (int q = 0; q < kPermuteNz; q++) {
+        const int p = p0 + min(q * kThreads + (int)threadIdx.x, n - 1);
+        src[q] = p + l.shift[(int)(((float)(p - start0) + 0.5f) * inv)];       // exact: p - start0 < 2,432
     }
-#pragma unroll
-    for (int q = 0; q < kPermuteNz; q++) src[q] = position(q) + l.shift[src[q]];
 #pragma unroll
     for (int q = 0; q < kPermuteNz; q++) {
         col[q] = a.idx[src[q]];
@@ -804,11 +822,11 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, i
     }
 #pragma unroll
     for (int q = 0; q < kPermuteNz; q++) {
-        const int p = p0 + q * kThreads + (int)threadIdx.x;
+        const int p = q * kThreads + (int)threadIdx.x;
         bad |= (uint32_t)col[q] >= a.cols;
-        if (p >= p1) continue;
-        if (a.idx_out) a.idx_out[p] = col[q];
-        a.pay_out[p] = pay[q];
+        if (p >= n) continue;
+        if (a.idx_out) a.idx_out[p0 + p] = col[q];
+        a.pay_out[p0 + p] = pay[q];
     }
     report_bad(a, bad);
 }
@@ -1067,7 +1085,7 @@ struct CopyPlan {
     int n_take;                               // non-zeros of whole rows
     int *counts;                              // [split row][64], or null
 };
-__global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArgs wa, CopyPlan cp, UnitsArgs u)
+__global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArgs wa, CopyPlan cp, UnitsArgs u, TileOrder order)
 {
     union Lds {
         UnitsLds units;
@@ -1107,7 +1125,7 @@ __global__ __launch_bounds__(kThreads) void copy_rows_kernel(CopyArgs a, WideArg
         if (i < cp.n_small) group_row<kSmallRounds>(a, l.small, cp.first_small + i, i, wa.forced_groups, cp.counts);
         return;
     }
-    permute_rows(a, l.permute, b - cp.small_groups, cp.n_take);
+    permute_rows(a, l.permute, order, b - cp.small_groups, cp.n_take);
 }
 
 // Counts the split rows for the plan and, in the workgroups behind, places the chunks of wide rows, one each (both
@@ -1662,9 +1680,10 @@ static int copy_nonzeros(Arena *tmp, const accel_handle *h, const CopyArgs &a, i
     cp.first_small = rows - n_split;
     cp.n_take = (int)nnz_short;
     cp.counts = split.gcount;
-    const int64_t groups = (int64_t)u.groups + cp.n_chunks + cp.mid_groups + cp.small_groups +
-                           (nnz_short + kPermuteTile - 1) / kPermuteTile;
-    if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp, u);
+    // the tiles' workgroups start at a multiple of 8, so that the i-th of them is on die i % 8
+    cp.small_groups += -(u.groups + cp.n_chunks + cp.mid_groups + cp.small_groups) & (kXcds - 1);
+    const int64_t groups = (int64_t)u.groups + cp.n_chunks + cp.mid_groups + cp.small_groups + (int64_t)h->tiles.per_die * kXcds;
+    if (groups > 0) copy_rows_kernel<<<dim3((unsigned)groups), dim3(kThreads), 0, s>>>(a, wa, cp, u, h->tiles);
     split.n_wide = n_wide;
     split.first_chunk = wa.first_chunk ? wa.first_chunk + wa.n_narrow : nullptr;
     split.chunk_count = wa.chunk_count;
@@ -1939,11 +1958,12 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
     if ((rc = prepare_split_rows(&tmp, h, ua.sr, rule, pu, mail, &slot, &split))) return rc;
     split.gcount = gcount;
     if (own_copy) {
+        h->tiles = order_tiles(mail->hist, h->plan_split);
         const CopyArgs ca{sorted_rows(h), h->idx, h->val, (uint32_t)h->cols, s_idx, reinterpret_cast<int32_t *>(s_val), 0,
                           mail};
         if ((rc = copy_nonzeros(&tmp, h, ca, whole.nnz, ua, split, s))) return rc;
     } else {
-        copy_rows_kernel<<<dim3((unsigned)ua.groups), dim3(kThreads), 0, s>>>(CopyArgs{}, WideArgs{}, CopyPlan{}, ua);
+        copy_rows_kernel<<<dim3((unsigned)ua.groups), dim3(kThreads), 0, s>>>(CopyArgs{}, WideArgs{}, CopyPlan{}, ua, TileOrder{});
         if (nnz > 0) {
             const unsigned g = (unsigned)std::min<int64_t>((nnz / 4 + kThreads - 1) / kThreads + 1, 16384);
             index_check_kernel<<<dim3(g), dim3(kThreads), 0, s>>>(h->idx, nnz, h->cols, mail);

@@ -68,3 +68,19 @@ def test_tiles_of_the_long_rows_sort(gpu, n):
     Y = op.matmul(np.ones((4, 4), np.float32))
     assert np.array_equal(Y, np.repeat(deg[:, None], 4, 1))           # whole numbers below 2^24: exact
     op.close()
+
+
+@pytest.mark.parametrize("rows, degrees", [(70_000, (3, 30)), (9_000, (1, 193)), (4_000_000, (1, 2)), (300_000, (60, 64))])
+def test_bands_of_tiles(gpu, rows, degrees):
+    """8 to 256 bands of tiles, runs of one tile and of hundreds: every non-zero of the whole rows is copied once."""
+    rng = np.random.default_rng(rows)
+    deg = rng.integers(*degrees, rows)
+    deg[rng.integers(0, rows, 3)] = (5, 9, 11)
+    g = graph(gpu, deg, 20_011, seed=rows)
+    op = gpu.AccelSpMM(g.indptr, g.indices, g.values, g.n_cols).preprocess()
+    order = np.argsort(deg, kind="stable")
+    start = np.concatenate([[0], np.cumsum(deg[order])])
+    source = np.arange(g.nnz) - np.repeat(start[:-1] - g.indptr[order], deg[order])
+    ip, ix, v = op.sorted_csr()
+    assert np.array_equal(ip, start) and np.array_equal(ix, g.indices[source]) and np.array_equal(v, g.values[source])
+    op.close()
