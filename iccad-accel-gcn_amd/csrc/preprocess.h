@@ -15,7 +15,7 @@ constexpr int kWaves4 = kThreads / 64;
 constexpr int kBins = kDegBound + 2;
 constexpr int kLongBin = kDegBound + 1;
 
-// Split rows of more than this many non-zeros are regrouped in pieces of kWideChunk by a
+// Split rows of more than kWideRow non-zeros are regrouped in pieces of kWideChunk by a
 // workgroup per piece, shorter ones by a wavefront each.
 constexpr int kWideRow = 1024;
 constexpr int kWideChunk = 4096;

@@ -18,9 +18,9 @@
 // and its place in the bin: its sorted place, its first non-zero, the block and the unit of the
 // launch plan that it opens.  One pass counts (degree_kernel), one workgroup per bin scans the
 // counts over the shares of rows (bin_scan_kernel), one pass places the rows and writes all of
-// that (place_rows_kernel).  The longer rows, few on most graphs, are ranked by comparison (or
+// that (place_rows_kernel).  The longer rows, few on most graphs, are placed by comparison (or
 // by a radix sort when there are many).
-// Nine launches on a graph of 2.45 M non-zeros (ten more where thousands of rows are longer than 384) and two
+// Nine launches on a graph of 2.45 M non-zeros (five more where more than 8,192 rows are longer than 384) and two
 // synchronisations; a radix sort of all rows with scans for every product took 100 and four.
 #include <chrono>
 #include <climits>
@@ -839,8 +839,8 @@ __device__ __forceinline__ void permute_rows(const CopyArgs &a, PermuteLds &l, c
 // long as enough of them are under way: columns and payload together in LDS (33 KB a workgroup instead of 17) let four
 // workgroups on a compute unit instead of seven, the tiles of whole rows in the same launch among them.  With that, with
 // the ranks kept in registers instead of groups counted by atomics first, and with rows of one chunk placed here
-// (place_chunk), the copying of 125 M non-zeros of a power-law matrix takes 548 us where it took 683, that of 30 M with hub
-// rows 155 where it took 202 (with wide_place_kernel).
+// (place_chunk), the copying of 125 M non-zeros of a power-law matrix took 548 us where it had taken 683, that of 30 M with hub
+// rows 155 where it had taken 202 (with wide_place_kernel; 513 and 142 since whole rows go by bands).
 template <int R> struct GroupLds {
     int buf[kWaves4][R * 64];
     int cnt[kWaves4][kMaxGroups];
@@ -1074,7 +1074,7 @@ struct UnitsLds {
 };
 
 // All of the above in one launch (on a small matrix each would take its few microseconds after the
-// other): workgroups take, in this order, shares of rows whose units are listed, chunks of wide rows to count, split rows
+// other): workgroups take, in this order, shares of rows whose units are listed, chunks of wide rows to place or count, split rows
 // of up to 1,024 and of up to 384 non-zeros (four each), tiles of whole rows.  The units have nothing to do with the rest
 // but that both come behind the placing of the rows; a launch of their own took 8 to 10 us.
 constexpr int kSmallRounds = kDegBound / 64, kMidRounds = kWideRow / 64;
