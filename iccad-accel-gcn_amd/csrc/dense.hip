@@ -113,12 +113,12 @@ __device__ __forceinline__ float w_at(const float *__restrict__ W, int K, int N,
 struct DenseStepAt {
     int64_t row_block;
     int tile, k0;
-    __device__ void advance(int K, int last_tile, int64_t stride)
+    __device__ void advance(int K, int first_tile, int last_tile, int64_t stride)
     {
         k0 += kDenseStep;
         if (k0 >= K) {
             k0 = 0;
-            if (tile == last_tile) { tile = 0; row_block += stride; } else { tile++; }
+            if (tile == last_tile) { tile = first_tile; row_block += stride; } else { tile++; }
         }
     }
 };
@@ -128,7 +128,7 @@ struct DenseArgs {
     float *Z;
     int64_t rows, ldx, ldz, n_row_blocks;
     int K, N, n_col_tiles, n_steps;
-    int apart;                   // the column tiles of a block of rows are workgroups of their own
+    int apart;                   // the column tiles of a block of rows are workgroups of their own (asked for, then decided by dense_launch)
     const u32x4 *image;          // walk_fp16: W taken apart (dense_prepare_kernel), and what is in front of that
     const int *head;
 };
@@ -137,7 +137,9 @@ struct DenseArgs {
 __device__ __forceinline__ DenseStepAt first_step(const DenseArgs &a)
 {
     const int64_t b = blockIdx.x;
-    return a.apart ? DenseStepAt{b % a.n_row_blocks, (int)(b / a.n_row_blocks), 0} : DenseStepAt{b, 0, 0};
+    // the workgroups of a block's tiles are eight apart: on one die, at about the same time
+    const int64_t slot = b / kXcds;
+    return a.apart ? DenseStepAt{slot / a.n_col_tiles * kXcds + b % kXcds, (int)(slot % a.n_col_tiles), 0} : DenseStepAt{b, 0, 0};
 }
 
 // A workgroup's block of W of a step on its way through registers, taken apart, into LDS.
@@ -221,8 +223,8 @@ __device__ __forceinline__ void add_in_fp32(const DenseArgs &a, int64_t row0, in
 // rows, gridDim.x apart, as one sequence of steps: the reads of a block's first steps are
 // issued while the matrix cores work on the last steps of the block before, and that block's
 // rows of Z are stored behind them, so the memory latency is paid once per workgroup, not
-// once per block.  The column tiles of one block of rows (N > 128) follow each other in the
-// same workgroup: the rows of X they share come from L2 for all but the first.
+// once per block.  The column tiles of one block of rows (N > 128) belong to workgroups next to each other on
+// one die, or follow each other in the same one (see dense_launch).
 // Loads are the same in number on every path (clamped, not branched around), which keeps the
 // compiler's waits for them exact.  Starts at `now`, at the start of a tile.
 template <int NT>
@@ -277,13 +279,12 @@ __device__ __forceinline__ void walk_bf16(const DenseArgs &a, char (*w_lds)[kPar
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[t][v] = 0.f;
 
-    // gridDim.x is at most the number of blocks of rows (or of their tiles): every workgroup has work
-    const int64_t stride = a.apart ? a.n_row_blocks : gridDim.x;
-    const int last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
+    const int64_t stride = a.apart ? gridDim.x / a.n_col_tiles : gridDim.x;
+    const int first_tile = a.apart ? now.tile : 0, last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
     DenseStepAt next = now, after;
-    next.advance(a.K, last_tile, stride);
+    next.advance(a.K, first_tile, last_tile, stride);
     after = next;
-    after.advance(a.K, last_tile, stride);
+    after.advance(a.K, first_tile, last_tile, stride);
     v4f x0[4], x1[4];
     WStage<NT> w;
     bf16x8 apart[2][kParts];                   // this step's values of X, taken apart
@@ -396,7 +397,7 @@ __device__ __forceinline__ void walk_bf16(const DenseArgs &a, char (*w_lds)[kPar
         }
         now = next;
         next = after;
-        after.advance(a.K, last_tile, stride);
+        after.advance(a.K, first_tile, last_tile, stride);
         step++;
     };
     while (now.row_block < a.n_row_blocks) {
@@ -410,7 +411,8 @@ template <int NT>
 __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_xw_kernel(DenseArgs a)
 {
     __shared__ __attribute__((aligned(16))) char w_lds[2][kParts * NT * 32 * kWStride];
-    walk_bf16<NT>(a, w_lds, first_step(a));
+    const DenseStepAt at = first_step(a);
+    if (at.row_block < a.n_row_blocks) walk_bf16<NT>(a, w_lds, at);
 }
 
 // ---- two fp16 values per fp32 value -----------------------------------------------------------------------------
@@ -662,12 +664,12 @@ __device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_ld
 #pragma unroll
         for (int t = 0; t < kTiles; t++) high[r][t] = low[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int64_t stride = a.apart ? a.n_row_blocks : gridDim.x;       // (as in the other walk)
-    const int last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
+    const int64_t stride = a.apart ? gridDim.x / a.n_col_tiles : gridDim.x;       // (as in the other walk)
+    const int first_tile = a.apart ? now.tile : 0, last_tile = a.apart ? now.tile : a.n_col_tiles - 1;
     DenseStepAt next = now, after;
-    next.advance(a.K, last_tile, stride);
+    next.advance(a.K, first_tile, last_tile, stride);
     after = next;
-    after.advance(a.K, last_tile, stride);
+    after.advance(a.K, first_tile, last_tile, stride);
     v4f x0[4], x1[4];
     f16x8 apart[2][kParts16];                  // this step's values of X, taken apart
     int scale = 0, scale_next = 0;             // X is multiplied by 2^scale: in this step's tile, in the next step's
@@ -832,7 +834,7 @@ __device__ __forceinline__ DenseStepAt walk_fp16(const DenseArgs &a, char (*w_ld
         scale = scale_next;
         now = next;
         next = after;
-        after.advance(a.K, last_tile, stride);
+        after.advance(a.K, first_tile, last_tile, stride);
         step++;
     };
     // At a barrier: this step's block of W is in place, the other one's readers are done, and what was counted is there.
@@ -864,6 +866,7 @@ __global__ __launch_bounds__(kDenseThreads, 2) void dense_xw_fp16_kernel(DenseAr
     __shared__ __attribute__((aligned(16))) char w_lds[2 * kParts * NT * 32 * kWStride];
     __shared__ int bad, early;
     DenseStepAt at = first_step(a);
+    if (at.row_block >= a.n_row_blocks) return;             // (uniform; of the last eight blocks of rows, with tiles apart)
     if (!a.head[0]) {
         if (threadIdx.x == 0) bad = early = 0;
         at = walk_fp16<NT>(a, reinterpret_cast<char (*)[kParts16 * NT * 32 * 64]>(w_lds), at, &bad, &early);
@@ -995,7 +998,7 @@ __global__ __launch_bounds__(kDenseThreads, NT == 4 ? 2 : 3) void dense_short_ke
 constexpr int kDenseDevices = 64;
 static std::atomic<int> g_resident[kDenseDevices][12];    // [device][kernel]: workgroups the device holds, 0 = not asked yet
 
-static int dense_launch(void (*kernel)(DenseArgs), int which, const DenseArgs &a, hipStream_t s)
+static int dense_launch(void (*kernel)(DenseArgs), int which, DenseArgs a, hipStream_t s)
 {
     int dev = 0;
     ACCEL_HIP(hipGetDevice(&dev));
@@ -1007,8 +1010,20 @@ static int dense_launch(void (*kernel)(DenseArgs), int which, const DenseArgs &a
         resident = (cus > 0 ? cus : 256) * (per_cu > 0 ? per_cu : 1);
         if (dev >= 0 && dev < kDenseDevices) g_resident[dev][which].store(resident, std::memory_order_relaxed);
     }
-    const unsigned grid = a.apart ? (unsigned)(a.n_row_blocks * a.n_col_tiles)
-                                  : (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
+    unsigned grid = (unsigned)(a.n_row_blocks < resident ? a.n_row_blocks : resident);
+    // Column tiles in workgroups of their own: where that is fewer tiles one after the other in a workgroup, and where the blocks
+    // of rows are more than are under way at once: the tiles of a block are worked on together then, by
+    // one die, whose L2 has the rows of X that they share; one after the other they are fetched for each tile.  Rows x K x N, in turn
+    // and so: 200,000 x 602 x 256 287 and 246 us, 100,000 x 250 x 160 75 and 60, 500,000 x 512 x 256 520 and 470, 2.45 M x 512
+    // x 256 2,423 and 2,340, 300,000 x 100 x 515 328 and 263, 30,000 x 100 x 300 31.4 and 27.4.  As many either way, and at
+    // once: 50,000 x 602 x 256 75.0 and 76.0, 60,000 x 40 x 200 23.0 and 23.6.
+    if (a.apart) {
+        const int64_t set = (int64_t)kXcds * a.n_col_tiles;   // workgroups: the tiles of eight blocks of rows, one per die
+        const int64_t sets = (a.n_row_blocks + kXcds - 1) / kXcds, at_once = resident / set;
+        a.apart = at_once > 0 && ((sets + at_once - 1) / at_once < a.n_col_tiles * ((a.n_row_blocks + resident - 1) / resident) ||
+                                  a.n_row_blocks > resident);
+        if (a.apart) grid = (unsigned)(std::min(sets, at_once) * set);
+    }
     kernel<<<grid, kDenseThreads, 0, s>>>(a);
     return ACCEL_OK;
 }
@@ -1050,8 +1065,7 @@ static int dense_product(DenseArgs a, hipStream_t s, bool may_prepare)
     return dense_launch(dense_xw_kernel<NT>, which + 3, a, s);
 }
 
-// Few rows: a workgroup takes one column tile, and a narrower one, as long as there is a compute unit for each (with
-// one tile each, two).  A step takes a microsecond whatever its width.  Rows x K x N, 128 columns and all tiles to a workgroup
+// Few rows: a workgroup takes one column tile, and a narrower one, as long as there is a compute unit for each.  A step takes a microsecond whatever its width.  Rows x K x N, 128 columns and all tiles to a workgroup
 // and so: 2,000 x 250 x 256 31.0 -> 9.4 us, 10,000 x 602 x 128 32.7 -> 21.3, 10,000 x 602 x 256 48.4 -> 29.9, 20,000 x
 // 602 x 256 48.7 -> 39.3.  Beyond the line: 20,000 x 602 x 64 in halves (314 workgroups) 21.4 -> 25.6.
 constexpr int64_t kFewGroups = 256;
@@ -1072,7 +1086,7 @@ int dense_xw_launch(const float *X, const float *W, float *Z, int64_t rows, int 
     auto groups = [&](int of) { return a.n_row_blocks * ((N + of * 32 - 1) / (of * 32)); };
     if (K >= kDenseHalf) {
         while (nt > 1 && groups(nt / 2) <= kFewGroups) nt /= 2;
-        a.apart = groups(nt) > a.n_row_blocks && groups(nt) <= 2 * kFewGroups;
+        a.apart = groups(nt) > a.n_row_blocks;
     }
     a.n_col_tiles = (N + nt * 32 - 1) / (nt * 32);
     const int rc = nt == 1   ? dense_product<1>(a, s, may_prepare)

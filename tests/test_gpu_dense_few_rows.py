@@ -41,3 +41,19 @@ def test_two_parts_with_tiles_apart(gpu, K, rows, N, what):
     assert (np.abs(Z[pick] - want) <= (K + 1) * 2.0 ** -24 * scale).all()
     if what == "ordinary":
         assert so.check_dense(Z[pick], X[pick], W) <= 2 * 2.0 ** -23 + 2.0 ** -24
+
+
+@pytest.mark.parametrize("K,rows,N", [(17, 66_000, 129), (40, 70_001, 200), (64, 70_000, 300), (100, 130_945, 515), (33, 200_000, 257)])
+@pytest.mark.parametrize("what", ["ordinary", "far apart"])
+def test_more_blocks_of_rows_than_are_under_way(gpu, K, rows, N, what):
+    """Workgroups that keep their column tile and go from block to block (512 or 768 of them: more than 65,536 rows)."""
+    rng = np.random.default_rng(K)
+    X = rng.standard_normal((rows, K), dtype=np.float32)
+    if what == "far apart":
+        X *= np.exp2(rng.integers(-50, 50, X.shape)).astype(np.float32)
+    W = rng.standard_normal((K, N)).astype(np.float32)
+    Z = product(gpu, X, W)
+    pick = np.unique(np.concatenate([np.arange(0, rows, 128), np.arange(127, rows, 128), np.arange(rows - 300, rows)]))
+    want = X[pick].astype(np.float64) @ W.astype(np.float64)
+    scale = np.abs(X[pick]).astype(np.float64) @ np.abs(W).astype(np.float64)
+    assert (np.abs(Z[pick] - want) <= (K + 1) * 2.0 ** -24 * scale).all()
