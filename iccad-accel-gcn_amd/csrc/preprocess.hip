@@ -1526,18 +1526,21 @@ static int count_rows(Arena *tmp, const int32_t *indptr, const int32_t *idx, int
 struct RunTotals {
     int64_t blocks = 0, nnz = 0, units = 0;
 };
-static RunTotals run_totals(const int *hist, int most, int unit_nz)
+// (The GPU waits for this: 32-bit divisions, and up to `whole_most` on the way, when that is asked for.)
+static RunTotals run_totals(const int *hist, int most, int unit_nz, int whole_most = 0, RunTotals *whole = nullptr)
 {
     RunTotals t;
     for (int d = 1; d <= most; d++) {
-        if (!hist[d]) continue;
-        int w, rpb;
-        slice_rule(d, w, rpb);
-        const int64_t n = hist[d], full = n / rpb, rest = n % rpb;
-        const int rpu = std::max(1, unit_nz / d);
-        t.blocks += full + (rest > 0);
-        t.nnz += n * d;
-        t.units += full * ((rpb + rpu - 1) / rpu) + (rest + rpu - 1) / rpu;
+        if (hist[d]) {
+            int w, rpb;
+            slice_rule(d, w, rpb);
+            const unsigned n = (unsigned)hist[d], b = (unsigned)rpb, full = n / b, rest = n % b;
+            const unsigned rpu = std::max(1u, (unsigned)unit_nz / (unsigned)d);
+            t.blocks += full + (rest > 0);
+            t.nnz += (int64_t)n * d;
+            t.units += (int64_t)full * ((b + rpu - 1) / rpu) + (rest + rpu - 1) / rpu;
+        }
+        if (d == whole_most) *whole = t;
     }
     return t;
 }
@@ -1865,8 +1868,8 @@ int preprocess_device(accel_handle *h, const SavedOrder *given)
         return ACCEL_ERR_META;
     }
     const int64_t n_split = h->n_split_rows;
-    const RunTotals binned = run_totals(mail->hist, kDegBound, h->plan_unit);
-    const RunTotals whole = run_totals(mail->hist, h->plan_split, h->plan_unit);     // the rows that stay whole
+    RunTotals whole;                                                                 // the rows that stay whole
+    const RunTotals binned = run_totals(mail->hist, kDegBound, h->plan_unit, h->plan_split, &whole);
     const int64_t nb = binned.blocks + h->n_long_blocks;
     if (nb + (int64_t)kMaxGroups * n_split + kXcds * kWavesPerGroup > (int64_t)INT_MAX) {
         set_error("the launch plan would exceed 2^31 work units (%lld block4 entries)", (long long)nb);
